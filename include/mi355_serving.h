@@ -110,6 +110,20 @@ int mi355_hgemm_add(const void* A, const void* B, const void* R, void* C, int M,
                     int64_t ldr, int64_t ldc, int layout, void* stream);
 
 /*
+ * mi355_hgemm / mi355_hgemm_add (R may be NULL) for dtype MI355_DTYPE_FP16 or MI355_DTYPE_BF16, with memory of the caller for
+ * aligned copies of operands the fast paths cannot read: rows that are not 16-byte aligned (a dense matrix whose row
+ * length is not a multiple of 8), or K % 8 != 0 in an operand whose K index is contiguous. mi355_gemm_workspace_bytes says
+ * how many bytes the copies of a call take (0: none are made). With that much `workspace` (16-byte aligned, contents
+ * irrelevant before and after the call) such operands are copied first and the product runs on the fast paths (1999 x
+ * 3001 x 2503 NN: 712 us without, 47 with); with less, or NULL, the call runs without copies, like the entry points above.
+ * Calls that share a workspace must be ordered on one stream. The operators of gemm_unified pass memory of torch's
+ * allocator; the reference's kernels take none of these shapes.
+ */
+size_t mi355_gemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout);
+int mi355_gemm_ws(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                  int64_t ldr, int64_t ldc, int layout, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Fused attention forward, O = softmax(scale * Q K^T + mask) V, online softmax with fp32 statistics.
  *
  * Replaces the device side of `torch::Tensor finefmha_N(Q, K, V, causal, is_decode, decode_length)`

@@ -616,3 +616,41 @@ def test_residual_epilogue_full_size_projection(lib, gpu):
     want = lib.hgemm(a, w, "NT") + res
     lib.hgemm(a, w, "NT", out=res, residual=res)
     assert torch.equal(res, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("M,N,K,off_a,off_b,residual", [
+    (257, 255, 129, 0, 0, False), (1001, 1003, 1005, 0, 0, True), (3, 1016, 4483, 0, 0, False), (16, 513, 2049, 0, 0, False),
+    (64, 1031, 333, 0, 0, True), (300, 9, 73, 0, 0, False), (130, 4099, 65, 0, 0, False), (128, 256, 192, 1, 0, False),
+    (40, 264, 520, 0, 3, True), (7, 100, 66, 5, 7, False), (1, 1, 71, 0, 0, False), (2050, 257, 127, 0, 0, False)])
+def test_operands_with_unaligned_rows_through_aligned_copies(lib, gpu, dtype, layout, M, N, K, off_a, off_b, residual):
+    # dense operands whose rows are not 16-byte aligned, views that start off_a / off_b elements into an allocation, and a
+    # contiguous K that ends inside a 16-byte chunk: mi355_gemm_ws copies them first. The workspace and what surrounds the
+    # operands hold NaNs, C's surroundings come back untouched. Up to 64 rows a K tail makes two roundings more.
+    a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
+    a, b = a.to(dtype), b.to(dtype)
+    raw = lambda t, off: torch.cat((torch.full((off,), float("nan"), dtype=dtype), t.reshape(-1),
+                                    torch.full((9,), float("nan"), dtype=dtype))).to(gpu)
+    ag, bg = raw(a, off_a), raw(b, off_b)
+    pa, pb = ag.data_ptr() + 2 * off_a, bg.data_ptr() + 2 * off_b
+    cdll, lay = lib.load(), lib.LAYOUTS[layout]
+    need = cdll.mi355_gemm_workspace_bytes(pa, pb, M, N, K, a.shape[1], b.shape[1], lay)
+    assert (need > 0) == bool(off_a or off_b or a.shape[1] % 8 or b.shape[1] % 8)
+    ws = torch.full((need + 16,), 0xFF, dtype=torch.uint8, device=gpu)
+    c = torch.full((M + 1, N + 3), 5.0, dtype=dtype, device=gpu)
+    r = (torch.randn(M, N, generator=torch.Generator().manual_seed(7)) * 2).to(dtype)
+    rg = r.to(gpu)
+    st = torch.cuda.current_stream(gpu).cuda_stream
+    rc = cdll.mi355_gemm_ws(pa, pb, rg.data_ptr() if residual else None, c.data_ptr(), M, N, K, a.shape[1], b.shape[1],
+                            N if residual else 0, N + 3, lay, lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16,
+                            ws.data_ptr(), need, st)
+    assert rc == 0
+    torch.cuda.synchronize()
+    ref = so.gemm_ref(a, b, layout)
+    got = c[:M, :N].cpu().float()
+    err = (got - (r.float() if residual else 0.0) - ref).abs()
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10
+    bound = 2e-2 * (K / 1024.0) ** 0.5 + max(1e-2, 3 * eps) * ref.abs() + eps * got.abs()
+    assert bool((err <= bound).all()), float((err - bound).max())
+    assert bool((c[M:] == 5.0).all()) and bool((c[:, N:] == 5.0).all())

@@ -34,7 +34,8 @@ extern "C" {
 
 // R == nullptr: the plain product; otherwise the residual operand of the *_add entry points (checked by the caller)
 static int hgemm_impl(const char* fn, int dtype, const void* A, const void* B, void* C, const void* R, int M, int N, int K, int64_t lda,
-                      int64_t ldb, int64_t ldc, int64_t ldr, int layout, void* stream, int variant = 0) {
+                      int64_t ldb, int64_t ldc, int64_t ldr, int layout, void* stream, int variant = 0, void* workspace = nullptr,
+                      size_t workspace_bytes = 0) {
     if (!A || !B || !C) return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer", fn);
     if (M < 1 || N < 1 || K < 1) return fail(MI355_ERR_BAD_ARGUMENT, "%s: M, N, K must be >= 1 (got %d, %d, %d)", fn, M, N, K);
     if (layout != MI355_GEMM_NN && layout != MI355_GEMM_NT && layout != MI355_GEMM_TN)
@@ -48,7 +49,8 @@ static int hgemm_impl(const char* fn, int dtype, const void* A, const void* B, v
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: leading dimension too small (ldr %lld >= %d required)", fn, (long long)ldr, N);
     if (R != nullptr && R == C && ldr != ldc)
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: R aliases C but ldr (%lld) differs from ldc (%lld)", fn, (long long)ldr, (long long)ldc);
-    hipError_t e = mi355::hgemm_dispatch(A, B, C, R, M, N, K, lda, ldb, ldc, R ? ldr : 0, layout, dtype, variant, static_cast<hipStream_t>(stream));
+    hipError_t e = mi355::hgemm_dispatch(A, B, C, R, M, N, K, lda, ldb, ldc, R ? ldr : 0, layout, dtype, variant, workspace, workspace_bytes,
+                                     static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, fn);
     return 0;
 }
@@ -75,6 +77,19 @@ int mi355_gemm_add_bf16(const void* A, const void* B, const void* R, void* C, in
     return hgemm_impl("mi355_gemm_add_bf16", MI355_DTYPE_BF16, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, stream);
 }
 
+
+size_t mi355_gemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout) {
+    if (!A || !B || M < 1 || N < 1 || K < 1 || layout < MI355_GEMM_NN || layout > MI355_GEMM_TN) return 0;
+    return mi355::hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout);
+}
+
+int mi355_gemm_ws(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldr,
+                  int64_t ldc, int layout, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+    if (dtype != MI355_DTYPE_FP16 && dtype != MI355_DTYPE_BF16) return fail(MI355_ERR_BAD_ARGUMENT, "mi355_gemm_ws: unknown dtype %d", dtype);
+    if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        return fail(MI355_ERR_BAD_ARGUMENT, "mi355_gemm_ws: the workspace must be 16-byte aligned (got %p)", workspace);
+    return hgemm_impl("mi355_gemm_ws", dtype, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, stream, 0, workspace, workspace_bytes);
+}
 
 static int fmha_checked(const char* fn, const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                         int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const mi355::FmhaStrides& sd,

@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
     // is stored at position c ^ 2*(r%4) (keeps the 16 lanes of a transposing read on distinct banks)
     const int b_row = lane >> 3;                                  // + 8*i
     const int b_chunk = (lane & 7) ^ (2 * (b_row & 3));           // (8i + b_row) % 4 == b_row % 4
-    const int n_chunk_max = N / 8 - 1;
+    const int n_chunk_max = (N + 7) / 8 - 1;   // the last chunk may end in the padding of B's rows
     const int b_col = min(n0 / 8 + b_chunk, n_chunk_max) * 8;     // clamp: columns past N are never stored
     const T* b_src = B + (long)(s_begin * 32 + b_row) * ldb + b_col;
     // A slab: 16 rows (m) x 64 bytes; row lane/4, chunk position lane%4, chunk c of row r at c ^ ((r>>1)&3)
@@ -927,6 +927,8 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
 #pragma unroll
         for (int q = 0; q < 4; ++q) red[wave * 1024 + (4 * (lane >> 4) + q) * 64 + 16 * j + (lane & 15)] = acc[j][q];
     __syncthreads();
+    // two columns go out in one 4-byte store where the rows of C (and of the residual) allow it
+    const bool pairs = ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(R)) & 3) == 0 && ((ldc | ldr) & 1) == 0;
     for (int o = tid * 2; o < 1024; o += kSmallMWaves * 128) {  // two neighbouring columns of one row
         float s0 = 0.f, s1 = 0.f;
 #pragma unroll
@@ -936,7 +938,13 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
         }
         const int m = m0 + (o >> 6);
         const int n = n0 + (o & 63);
-        if (m < M && n < N) {
+        if (m < M && n < N && (n + 1 == N || !pairs)) {
+            for (int j = 0; j < 2 && n + j < N; ++j) {
+                T v = (T)(j ? s1 : s0);
+                if (R != nullptr) v = (T)((float)v + (float)R[(long)m * ldr + n + j]);
+                C[(long)m * ldc + n + j] = v;
+            }
+        } else if (m < M && n < N) {
             V2 v;
             v[0] = (T)s0;
             v[1] = (T)s1;
@@ -1502,7 +1510,7 @@ static bool few_rows_prefer_deep_ring(int M, int N, int K, bool nn, bool nt) {
 
 template <typename T, bool A_KC, bool B_KC>
 static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
-                                long ldc, long ldr, int variant, hipStream_t stream) {
+                                long ldc, long ldr, int variant, bool k_zero_padded, hipStream_t stream) {
     // the copies of the fast kernels move 16 bytes into LDS: the operands' rows must be 16-byte aligned. C and the residual
     // may lie anywhere; the kernels that assume whole tiles also assume aligned rows of C (c_aligned).
     const bool ab_aligned = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0) &&
@@ -1523,12 +1531,16 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
         dim3 grid((N + 63) / 64, (M + 63) / 64);
         hgemm_edge_kernel<T, A_KC, B_KC><<<grid, dim3(256), 0, stream>>>(a_tail, b_tail, C, nullptr, M, N, k_tail, lda, ldb, ldc, 0);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        return launch_layout<T, A_KC, B_KC>(A, B, C, C, M, N, k_main, lda, ldb, ldc, ldc, variant, stream);
+        return launch_layout<T, A_KC, B_KC>(A, B, C, C, M, N, k_main, lda, ldb, ldc, ldc, variant, k_zero_padded, stream);
     }
     // the tiled kernels address a tile with 32-bit byte offsets: up to 256 rows of lda (ldb) elements
     // Any N: an operand stored [K,N] is copied in 16-byte chunks of its rows, and the chunk that straddles N ends in the
     // padding a leading dimension of a multiple of 8 leaves (what it holds only reaches columns that are never stored).
-    const bool ragged_ok = ab_aligned && K % 8 == 0 && K >= 8 && lda < (1L << 22) && ldb < (1L << 22);
+    // Any K, if the rows of an operand whose K index is contiguous hold zeros from K up to the next multiple of 8 (the
+    // copies of gemm_pack.hip do, k_zero_padded) or no operand is stored that way: the copies of the other operand take
+    // single rows of K.
+    const bool k_ok = K % 8 == 0 || k_zero_padded || (!A_KC && !B_KC);
+    const bool ragged_ok = ab_aligned && k_ok && lda < (1L << 22) && ldb < (1L << 22);
     const bool small_m = M <= 64 && !(ragged_ok && few_rows_prefer_tiles(M, N, K, A_KC && B_KC));
     // 17 .. 256 rows against a narrow second operand: split-K, where a workspace is to be had
     if (ragged_ok && variant == 0) {
@@ -1559,7 +1571,7 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
         return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
     }
     if constexpr (!B_KC) {   // NN and TN
-        if (aligned && small_m && K % 32 == 0 && K >= 32 && N % 8 == 0 && ldc % 2 == 0)
+        if (ab_aligned && small_m && K % 32 == 0 && K >= 32)
             return launch_smallm_nn<T, A_KC>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
     }
     if constexpr (A_KC && B_KC) {
@@ -1655,7 +1667,7 @@ static hipError_t silu_mul_dispatch_t(const void* A, const void* B, void* C, int
 // MI355_HGEMM_PART: undefined = everything in this translation unit; 0 = the fp16 kernels and the two entry points, 1 =
 // only the bf16 kernels behind the two *_bf16 functions (the build compiles the two parts side by side).
 hipError_t hgemm_dispatch_bf16(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                               long ldc, long ldr, int layout, int variant, hipStream_t stream);
+                               long ldc, long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream);
 hipError_t hgemm_silu_mul_dispatch_bf16(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb,
                                         long ldc, int layout, hipStream_t stream);
 
@@ -1675,30 +1687,51 @@ hipError_t hgemm_silu_mul_dispatch(const void* A, const void* B, void* C, int M,
 
 template <typename T>
 static hipError_t gemm_dispatch_t(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda,
-                                  long ldb, long ldc, long ldr, int layout, int variant, hipStream_t stream) {
+                                  long ldb, long ldc, long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream) {
     const T* a = static_cast<const T*>(A);
     const T* b = static_cast<const T*>(B);
     T* c = static_cast<T*>(C);
     const T* r = static_cast<const T*>(R);
     switch (layout) {
-        case MI355_GEMM_NN: return launch_layout<T, true, false>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, stream);
-        case MI355_GEMM_NT: return launch_layout<T, true, true>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, stream);
-        case MI355_GEMM_TN: return launch_layout<T, false, false>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, stream);
+        case MI355_GEMM_NN: return launch_layout<T, true, false>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
+        case MI355_GEMM_NT: return launch_layout<T, true, true>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
+        case MI355_GEMM_TN: return launch_layout<T, false, false>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
         default: return hipErrorInvalidValue;
     }
 }
 
 #if !defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 1
 hipError_t hgemm_dispatch_bf16(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                               long ldc, long ldr, int layout, int variant, hipStream_t stream) {
-    return gemm_dispatch_t<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
+                               long ldc, long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream) {
+    return gemm_dispatch_t<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
 }
 #endif
 #if !defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 0
+// An operand with unaligned rows is worth an aligned copy from a few K steps on: below that the bounds-checked kernel is
+// done before a second launch would start.
+size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
+    if (K <= 64) return 0;
+    const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
+    return plan.a.pack || plan.b.pack ? plan.bytes() : 0;
+}
+
 hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                          long ldc, long ldr, int layout, int dtype, int variant, hipStream_t stream) {
-    if (dtype == MI355_DTYPE_BF16) return hgemm_dispatch_bf16(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
-    return gemm_dispatch_t<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
+                          long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream) {
+    bool k_zero_padded = false;
+    if (const size_t need = workspace ? hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout) : 0; need > 0 && need <= workspace_bytes) {
+        const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
+        char* a_copy = static_cast<char*>(workspace);
+        char* b_copy = a_copy + plan.b_offset();
+        if (hipError_t e = gemm_pack_launch(plan, A, B, lda, ldb, a_copy, b_copy, stream); e != hipSuccess) return e;
+        if (plan.a.pack) A = a_copy;
+        if (plan.b.pack) B = b_copy;
+        lda = plan.a.ld;
+        ldb = plan.b.ld;
+        k_zero_padded = true;
+    }
+    if (dtype == MI355_DTYPE_BF16) return hgemm_dispatch_bf16(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
+    return gemm_dispatch_t<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
 }
 #endif
 

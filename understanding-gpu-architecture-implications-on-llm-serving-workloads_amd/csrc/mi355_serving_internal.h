@@ -25,9 +25,29 @@ struct DynamicLdsOnce {
 };
 
 // Launches the GEMM kernels; arguments as mi355_hgemm_add after validation (R == nullptr: no residual).
-// `variant` pins a tile shape instead of the choice by shape (0); see mi355_internal_hgemm_variant below.
+// `variant` pins a tile shape instead of the choice by shape (0); see mi355_internal_hgemm_variant below. `workspace`
+// (16-byte aligned device memory, may be null): where aligned copies of operands with unaligned rows may be kept.
 hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                          long ldc, long ldr, int layout, int dtype, int variant, hipStream_t stream);
+                          long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream);
+
+// Aligned copies of GEMM operands (gemm_pack.hip): which operands need one, and the rows and bytes of the copies.
+struct GemmPackPlan {
+    struct Operand {
+        bool pack = false;
+        int cols = 0;       // elements of a stored row
+        long ld = 0;        // row stride of the copy (of the operand itself where none is made)
+        size_t bytes = 0;   // of the copy
+    };
+    Operand a, b;
+    size_t b_offset() const { return (a.bytes + 255) / 256 * 256; }   // where B's copy starts behind A's
+    size_t bytes() const { return b_offset() + b.bytes; }
+};
+GemmPackPlan gemm_pack_plan(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
+hipError_t gemm_pack_launch(const GemmPackPlan& plan, const void* A, const void* B, long lda, long ldb, void* a_copy, void* b_copy,
+                            hipStream_t stream);
+// Bytes of workspace a product can use (0: none, nothing to copy or not worth it).
+size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
 
 // Element strides of the attention operands: tensor[b][h][s][d] lives at b*batch + h*head + s*row + d (d contiguous).
 struct FmhaStrides {

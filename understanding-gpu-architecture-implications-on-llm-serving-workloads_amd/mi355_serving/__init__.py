@@ -17,6 +17,7 @@ ERR_BAD_ARGUMENT, ERR_UNSUPPORTED = 10001, 10002
 
 EXPORTED_SYMBOLS = ("mi355_hgemm", "mi355_fmha_fwd", "mi355_fmha_fwd_strided", "mi355_fmha_fwd_bf16", "mi355_hgemm_silu_mul", "mi355_hgemm_add", "mi355_rmsnorm", "mi355_rope", "mi355_rope_qkv", "mi355_silu_mul",
                     "mi355_gemm_bf16", "mi355_gemm_silu_mul_bf16", "mi355_gemm_add_bf16", "mi355_rmsnorm_bf16", "mi355_rope_bf16", "mi355_rope_qkv_bf16", "mi355_silu_mul_bf16",
+                    "mi355_gemm_workspace_bytes", "mi355_gemm_ws",
                     "mi355_fmha_fwd_workspace_bytes", "mi355_fmha_fwd_ws", "mi355_fmha_fwd_noalloc",
                     "mi355_last_error", "mi355_serving_version")
 # exported for tests and tuning runs, declared in csrc/mi355_serving_internal.h and not in the public header
@@ -75,6 +76,10 @@ def load():
     lib.mi355_last_error.restype = ctypes.c_char_p
     lib.mi355_serving_version.argtypes = []
     lib.mi355_serving_version.restype = i32
+    lib.mi355_gemm_workspace_bytes.argtypes = [vp, vp, i32, i32, i32, i64, i64, i32]
+    lib.mi355_gemm_workspace_bytes.restype = ctypes.c_size_t
+    lib.mi355_gemm_ws.argtypes = [vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i64, i32, i32, vp, ctypes.c_size_t, vp]
+    lib.mi355_gemm_ws.restype = i32
     lib.mi355_fmha_fwd_workspace_bytes.argtypes = [i32] * 6
     lib.mi355_fmha_fwd_workspace_bytes.restype = ctypes.c_size_t
     lib.mi355_fmha_fwd_ws.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, f32, i32, i32, ctypes.POINTER(i64), i32,
@@ -140,19 +145,22 @@ def hgemm(a, b, layout="NN", out=None, residual=None, variant=0):
     stream = torch.cuda.current_stream(a.device).cuda_stream
     # leading dimensions of the contiguous operands (stride(0) of a size-1 dimension is arbitrary in torch)
     lda, ldb = a.shape[1], b.shape[1]
+    dtype = DTYPE_BF16 if a.dtype == torch.bfloat16 else DTYPE_FP16
     if residual is not None:
         if tuple(residual.shape) != (M, N) or residual.dtype != a.dtype or residual.stride(1) != 1:
             raise ValueError("residual must be [%d, %d] %s with a contiguous last dimension" % (M, N, a.dtype))
-        entry = load().mi355_gemm_add_bf16 if a.dtype == torch.bfloat16 else load().mi355_hgemm_add
-        _check(entry(_ptr(a), _ptr(b), _ptr(residual), _ptr(out), M, N, K, lda, ldb, max(residual.stride(0), N),
-                     max(out.stride(0), N), lay, stream))
-        return out
-    if variant:
+    elif variant:
         _check(load().mi355_internal_hgemm_variant(_ptr(a), _ptr(b), _ptr(out), M, N, K, lda, ldb, max(out.stride(0), N), lay,
-                                                   DTYPE_BF16 if a.dtype == torch.bfloat16 else DTYPE_FP16, int(variant), stream))
+                                                   dtype, int(variant), stream))
         return out
-    entry = load().mi355_gemm_bf16 if a.dtype == torch.bfloat16 else load().mi355_hgemm
-    _check(entry(_ptr(a), _ptr(b), _ptr(out), M, N, K, lda, ldb, max(out.stride(0), N), lay, stream))
+    # operands with unaligned rows (or a contiguous K that is not a multiple of 8): room for aligned copies of them
+    need = 0
+    if (lda | ldb) & 7 or (_ptr(a) | _ptr(b)) & 15:
+        need = load().mi355_gemm_workspace_bytes(_ptr(a), _ptr(b), M, N, K, lda, ldb, lay)
+    ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+    _check(load().mi355_gemm_ws(_ptr(a), _ptr(b), _ptr(residual), _ptr(out), M, N, K, lda, ldb,
+                                max(residual.stride(0), N) if residual is not None else 0, max(out.stride(0), N), lay, dtype,
+                                _ptr(ws), need, stream))
     return out
 
 
