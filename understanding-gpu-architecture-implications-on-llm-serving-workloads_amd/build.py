@@ -5,6 +5,7 @@ Produces, inside the three packages:
     mi355_serving/libmi355_serving_timeline.so   profiling twin: the attention kernels also record per-workgroup time stamps
     gemm_unified/_C.so                  torch operators gemm_unified::finegemm_N, linked against the library above
     fmha_unified/_C.so                  torch operators fmha_unified::finefmha_N
+    mi355_serving/_C.so                 the launches of a decoder layer's forward pass (llama_layer.py)
 Each _C.so finds the library through RUNPATH $ORIGIN/../mi355_serving: the packages sit side by side both in the source
 tree and in site-packages.
 
@@ -155,11 +156,12 @@ def build_all(verbose=True):
     build_library(verbose)
     build_operator("gemm_unified", "gemm_ops.cpp", verbose)
     build_operator("fmha_unified", "fmha_ops.cpp", verbose)
+    build_operator("mi355_serving", "layer_ops.cpp", verbose)
 
 
 def is_built():
     return all(os.path.exists(p) for p in (LIB_PATH, os.path.join(HERE, "gemm_unified", "_C.so"),
-                                           os.path.join(HERE, "fmha_unified", "_C.so")))
+                                           os.path.join(HERE, "fmha_unified", "_C.so"), os.path.join(LIB_DIR, "_C.so")))
 
 
 def run_setup(dist_name, op_packages, rel, py_modules=()):
@@ -192,7 +194,7 @@ def run_setup(dist_name, op_packages, rel, py_modules=()):
 
     packages = list(op_packages) + ["mi355_serving"]
     data = {p: ["_C.so"] for p in op_packages}
-    data["mi355_serving"] = [LIB_NAME]
+    data["mi355_serving"] = [LIB_NAME, "_C.so"]
     setup(
         name=dist_name,
         version="2.0.0",
@@ -214,5 +216,6 @@ if __name__ == "__main__":
     elif only == "ops":
         build_operator("gemm_unified", "gemm_ops.cpp")
         build_operator("fmha_unified", "fmha_ops.cpp")
+        build_operator("mi355_serving", "layer_ops.cpp")
     else:
         build_all()

@@ -19,6 +19,7 @@ concatenating q/k/v and interleaving gate/up along the output dimension once at 
 import torch
 
 import mi355_serving as lib
+from mi355_serving import _C
 
 __all__ = ["FineKVCache", "FineLlamaDecoderLayer", "rope_tables"]
 
@@ -94,42 +95,23 @@ class FineLlamaDecoderLayer:
 
     def forward(self, hidden_states, position_ids=None, kv_cache=None, time_attention=False):
         B, S, H = hidden_states.shape
-        D, Hq, Hkv = self.head_dim, self.n_q, self.n_kv
-        x = hidden_states.reshape(B * S, H)
-        past = kv_cache.length if kv_cache is not None else 0
-        if position_ids is None:
-            pos = self.all_positions[past:past + S]   # one [S] table shared by every batch row, no kernel launched
-        else:
-            pos = position_ids.to(torch.int32).contiguous()
-
-        h1 = lib.rmsnorm(x, self.ln1, self.eps)
-        if time_attention:
-            torch.cuda.synchronize()
-            t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            t0.record()
-        qkv = lib.hgemm(h1, self.w_qkv, "NT").view(B, S, Hq + 2 * Hkv, D)
-        q = qkv[:, :, :Hq]
-        if kv_cache is None:
-            lib.rope(qkv[:, :, :Hq + Hkv], self.cos, self.sin, pos)           # q and k heads are adjacent
-            k, v = qkv[:, :, Hq:Hq + Hkv], qkv[:, :, Hq + Hkv:]
-        else:
+        past, kv, first = 0, None, 0
+        if kv_cache is not None:
+            past, kv = kv_cache.length, kv_cache.kv
             if past + S > kv_cache.max_len:
                 raise ValueError("KV cache of %d tokens cannot take %d more after %d" % (kv_cache.max_len, S, past))
-            # one launch: q rotated in place, rotated keys and plain values of the new tokens into the cache
-            lib.rope_qkv(qkv, kv_cache.rows(past, S), self.cos, self.sin, pos, Hq, Hkv)
+        if position_ids is None:
+            pos, first = self.all_positions, past   # a window of one table shared by every batch row, no kernel launched
+            assert past + S <= pos.numel(), "max_positions is %d" % pos.numel()
+        else:
+            pos = position_ids.to(torch.int32).reshape(-1, S).contiguous()   # [1, S] (shared) or [B, S]
+            assert pos.shape[0] in (1, B)
+        out, ms = _C.layer_forward(hidden_states, self.w_qkv, self.w_o, self.w_gu, self.w_d, self.ln1, self.ln2, self.cos, self.sin, pos,
+                                   first, kv, past, self.n_q, self.n_kv, self.eps, self.gu_block, time_attention)
+        if kv_cache is not None:
             kv_cache.length = past + S
-            k, v = kv_cache.k[:, :past + S], kv_cache.v[:, :past + S]
-        attn = torch.empty((B, S, Hq, D), dtype=self.dtype, device=x.device)
-        # [B, S, heads, D] viewed as [B, heads, S, D]: the kernel reads and writes these layouts in place
-        lib.fmha_fwd(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), causal=True, return_lse=False,
-                     out=attn.transpose(1, 2))
-        res = lib.hgemm(attn.view(B * S, Hq * D), self.w_o, "NT", residual=x)   # x + o_proj(attn)
         if time_attention:
-            t1.record()
-            torch.cuda.synchronize()
-            self.attn_ms["decode" if (S == 1 and past > 0) else "prefill"].append(t0.elapsed_time(t1))
-        h2 = lib.rmsnorm(res, self.ln2, self.eps)
-        act = lib.hgemm_silu_mul(h2, self.w_gu, "NT") if self.gu_block else lib.silu_mul(lib.hgemm(h2, self.w_gu, "NT"))
-        return lib.hgemm(act, self.w_d, "NT", out=res, residual=res).view(B, S, H)   # res + down_proj(act), in place
+            self.attn_ms["decode" if (S == 1 and past > 0) else "prefill"].append(ms)
+        return out
 
     __call__ = forward
