@@ -34,11 +34,12 @@ DEVICE_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wno-inline-asm", "-Wno-unused-command-line-argument",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/gemm_pack.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip", "csrc/glue.hip", "csrc/capi.hip"]
+KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/hgemm_dispatch.hip", "csrc/gemm_pack.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip", "csrc/glue.hip", "csrc/capi.hip"]
 # A source listed here is compiled once per entry, each time with that entry's defines, into objects of its own (side by
 # side with the others): the GEMM source holds every tile shape for two element types and three layouts, and one
-# compiler process per element type halves the time the build waits for it.
-SOURCE_PARTS = {"csrc/hgemm.hip": (("fp16", ["-DMI355_HGEMM_PART=0"]), ("bf16", ["-DMI355_HGEMM_PART=1"]))}
+# compiler process each cuts the time the build waits for it to a third of what one per element type takes.
+SOURCE_PARTS = {"csrc/hgemm.hip": [(t + "." + l.lower(), ["-DMI355_HGEMM_T=%s_t" % {"fp16": "half"}.get(t, t), "-DMI355_HGEMM_LAYOUT=MI355_GEMM_" + l])
+                                   for t in ("fp16", "bf16") for l in ("NN", "NT", "TN")]}
 # Per-source additions. The GEMM keeps its MFMA accumulators in ordinary VGPRs: left to itself the compiler moves part of
 # them to AGPRs in the 4-wave kernels and then shuffles them back and forth inside the K loop.
 SOURCE_FLAGS = {"csrc/hgemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
@@ -74,7 +75,7 @@ def _run(cmd, quiet_patterns=("is not a recognized feature for this target",)):
 TIMELINE_LIB_NAME = "libmi355_serving_timeline.so"
 TIMELINE_LIB_PATH = os.path.join(LIB_DIR, TIMELINE_LIB_NAME)
 # Sources that carry per-workgroup time stamps when compiled with -DMI355_TIMELINE (csrc/mi355_timeline.h).
-TIMELINE_SOURCES = ("csrc/hgemm.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip")
+TIMELINE_SOURCES = ("csrc/hgemm.hip", "csrc/hgemm_dispatch.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip")
 # Yardstick kernels that exist in the profiling twin only (a read-only kernel, matrix instructions on registers, matrix and
 # VALU instructions side by side on one SIMD).
 TIMELINE_ONLY_SOURCES = ("csrc/timeline_probes.hip",)

@@ -32,8 +32,6 @@
 //     The MFMA is issued with the B fragment as first operand, i.e. it produces the transposed block, so a
 //     lane ends up with 4 consecutive N of one row of C; the epilogue parks the sub-tile in LDS and stores whole
 //     128-byte lines.
-#include <map>
-#include <mutex>
 #include <type_traits>
 #include <utility>
 #include "mi355_common.h"
@@ -44,7 +42,10 @@ namespace mi355 {
 
 // profiling build: per workgroup of hgemm_main_kernel [wall: entry, loop start, loop end, exit; cycles: loop start, loop
 // end; K tiles; 0]
-MI355_TL(static __device__ unsigned long long hgemm_stamps[timeline::kMaxWorkgroups * timeline::kSlots];)
+MI355_TL(static __device__ unsigned long long hgemm_stamps[timeline::kMaxWorkgroups * timeline::kSlots];
+         static hipError_t read_hgemm_stamps(void* dst, size_t bytes) {   // of this translation unit's kernels
+             return hipMemcpyFromSymbol(dst, HIP_SYMBOL(hgemm_stamps), bytes < sizeof(hgemm_stamps) ? bytes : sizeof(hgemm_stamps));
+         })
 
 // ---------------------------------------------------------------------------------------------------------
 // LDS tile descriptions
@@ -1303,6 +1304,7 @@ static hipError_t launch_main(const T* A, const T* B, T* C, const T* R, int M, i
     const long nblocks = (long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
     int blocks = (int)nblocks;
+    MI355_TL(timeline_hgemm_reader = &read_hgemm_stamps;)
     kern<<<dim3(blocks), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, stream>>>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, nullptr, nullptr, 1);
     return hipGetLastError();
 }
@@ -1316,42 +1318,6 @@ static hipError_t launch_main(const T* A, const T* B, T* C, const T* R, int M, i
 // kernels without split-K instead. The ticket counters, in front of the partial tiles, are zeroed when a buffer is new
 // (a fill kernel on the calling stream) and left at zero by every launch.
 // ---------------------------------------------------------------------------------------------------------
-constexpr size_t kSplitKCounterBytes = 16 * 1024;   // one counter per tile: up to 4096 tiles
-
-static __global__ void hgemm_clear_kernel(unsigned* p, int n) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
-}
-
-static hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, bool* fresh) {
-    struct Buf {
-        void* ptr = nullptr;
-        size_t size = 0;
-    };
-    static std::mutex mu;
-    static std::map<std::pair<int, hipStream_t>, Buf> bufs;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mu);
-    Buf& b = bufs[std::make_pair(dev, stream)];
-    *fresh = false;
-    if (b.size < bytes) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        e = hipStreamIsCapturing(stream, &cap);
-        if (e != hipSuccess) return e;
-        if (cap != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
-        const size_t want = bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes + bytes / 2;
-        void* fresh_buf = nullptr;
-        e = hipMalloc(&fresh_buf, want);
-        if (e != hipSuccess) return e;
-        b.ptr = fresh_buf;   // the previous buffer, if any, stays allocated (see above)
-        b.size = want;
-        *fresh = true;
-    }
-    *out = static_cast<char*>(b.ptr);
-    return hipSuccess;
-}
-
 // Number of ranges K is cut into, or 0 where split-K does not apply: 17 .. 256 rows, K a multiple of 64, few enough
 // 64x64 tiles for at least four ranges at about two workgroups per CU (up to 128 tiles; up to 192 with a long K), at
 // least eight K tiles per range, ranges of equal length. Measured with weights that come from HBM, layout NT (us, without / with split-K): 64 x 4096 x 14336 55 / 32,
@@ -1420,12 +1386,7 @@ static hipError_t launch_split_k(const T* A, const T* B, T* C, const T* R, int M
     if (tiles * sizeof(unsigned) > kSplitKCounterBytes) return hipErrorOutOfMemory;
     const size_t bytes = kSplitKCounterBytes + (size_t)tiles * splits * Cfg::NTHREADS * Cfg::TM * Cfg::TN * 16;
     char* ws = nullptr;
-    bool fresh = false;
-    if (hipError_t e = split_k_workspace(bytes, stream, &ws, &fresh); e != hipSuccess) return e;
-    if (fresh) {
-        hgemm_clear_kernel<<<dim3(4), dim3(256), 0, stream>>>(reinterpret_cast<unsigned*>(ws), (int)(kSplitKCounterBytes / sizeof(unsigned)));
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    }
+    if (hipError_t e = split_k_workspace(bytes, stream, &ws); e != hipSuccess) return e;
     kern<<<dim3((unsigned)tiles, (unsigned)splits), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, stream>>>(
         A, B, C, R, M, N, K, lda, ldb, ldc, ldr, reinterpret_cast<float*>(ws + kSplitKCounterBytes), reinterpret_cast<unsigned*>(ws), splits);
     return hipGetLastError();
@@ -1651,96 +1612,35 @@ static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, in
     return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 1, true>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
 }
 
-template <typename T>
-static hipError_t silu_mul_dispatch_t(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
-                                      int layout, hipStream_t stream) {
-    const T* a = static_cast<const T*>(A);
-    const T* b = static_cast<const T*>(B);
-    T* c = static_cast<T*>(C);
-    switch (layout) {
-        case MI355_GEMM_NN: return launch_silu_mul<T, true, false>(a, b, c, M, N2, K, lda, ldb, ldc, stream);
-        case MI355_GEMM_NT: return launch_silu_mul<T, true, true>(a, b, c, M, N2, K, lda, ldb, ldc, stream);
-        default: return hipErrorNotSupported;
-    }
+// One translation unit per element type and layout (the build compiles the six side by side): MI355_HGEMM_T and
+// MI355_HGEMM_LAYOUT select it; without them everything is instantiated here.
+template <typename T, int LAYOUT>
+hipError_t gemm_layout(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc,
+                       long ldr, int variant, bool k_zero_padded, hipStream_t stream) {
+    return launch_layout<T, LAYOUT != MI355_GEMM_TN, LAYOUT == MI355_GEMM_NT>(
+        static_cast<const T*>(A), static_cast<const T*>(B), static_cast<T*>(C), static_cast<const T*>(R), M, N, K, lda, ldb, ldc, ldr,
+        variant, k_zero_padded, stream);
 }
-
-// MI355_HGEMM_PART: undefined = everything in this translation unit; 0 = the fp16 kernels and the two entry points, 1 =
-// only the bf16 kernels behind the two *_bf16 functions (the build compiles the two parts side by side).
-hipError_t hgemm_dispatch_bf16(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                               long ldc, long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream);
-hipError_t hgemm_silu_mul_dispatch_bf16(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb,
-                                        long ldc, int layout, hipStream_t stream);
-
-#if !defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 1
-hipError_t hgemm_silu_mul_dispatch_bf16(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb,
-                                        long ldc, int layout, hipStream_t stream) {
-    return silu_mul_dispatch_t<bf16_t>(A, B, C, M, N2, K, lda, ldb, ldc, layout, stream);
+template <typename T, int LAYOUT>
+hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
+                                hipStream_t stream) {
+    if constexpr (LAYOUT == MI355_GEMM_TN) return hipErrorNotSupported;
+    else return launch_silu_mul<T, true, LAYOUT == MI355_GEMM_NT>(static_cast<const T*>(A), static_cast<const T*>(B), static_cast<T*>(C),
+                                                                  M, N2, K, lda, ldb, ldc, stream);
 }
-#endif
-#if !defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 0
-hipError_t hgemm_silu_mul_dispatch(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
-                                   int layout, int dtype, hipStream_t stream) {
-    if (dtype == MI355_DTYPE_BF16) return hgemm_silu_mul_dispatch_bf16(A, B, C, M, N2, K, lda, ldb, ldc, layout, stream);
-    return silu_mul_dispatch_t<half_t>(A, B, C, M, N2, K, lda, ldb, ldc, layout, stream);
-}
-#endif
-
-template <typename T>
-static hipError_t gemm_dispatch_t(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda,
-                                  long ldb, long ldc, long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream) {
-    const T* a = static_cast<const T*>(A);
-    const T* b = static_cast<const T*>(B);
-    T* c = static_cast<T*>(C);
-    const T* r = static_cast<const T*>(R);
-    switch (layout) {
-        case MI355_GEMM_NN: return launch_layout<T, true, false>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
-        case MI355_GEMM_NT: return launch_layout<T, true, true>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
-        case MI355_GEMM_TN: return launch_layout<T, false, false>(a, b, c, r, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-#if !defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 1
-hipError_t hgemm_dispatch_bf16(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                               long ldc, long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream) {
-    return gemm_dispatch_t<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
-}
-#endif
-#if !defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 0
-// An operand with unaligned rows is worth an aligned copy from a few K steps on: below that the bounds-checked kernel is
-// done before a second launch would start.
-size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
-    if (K <= 64) return 0;
-    const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
-    return plan.a.pack || plan.b.pack ? plan.bytes() : 0;
-}
-
-hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
-                          long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream) {
-    bool k_zero_padded = false;
-    if (const size_t need = workspace ? hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout) : 0; need > 0 && need <= workspace_bytes) {
-        const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
-        char* a_copy = static_cast<char*>(workspace);
-        char* b_copy = a_copy + plan.b_offset();
-        if (hipError_t e = gemm_pack_launch(plan, A, B, lda, ldb, a_copy, b_copy, stream); e != hipSuccess) return e;
-        if (plan.a.pack) A = a_copy;
-        if (plan.b.pack) B = b_copy;
-        lda = plan.a.ld;
-        ldb = plan.b.ld;
-        k_zero_padded = true;
-    }
-    if (dtype == MI355_DTYPE_BF16) return hgemm_dispatch_bf16(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
-    return gemm_dispatch_t<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
-}
+#define MI355_HGEMM_INSTANTIATE(T, LAYOUT)                                                                                     \
+    template hipError_t gemm_layout<T, LAYOUT>(const void*, const void*, void*, const void*, int, int, int, long, long, long,  \
+                                               long, int, bool, hipStream_t);                                                  \
+    template hipError_t gemm_silu_mul_layout<T, LAYOUT>(const void*, const void*, void*, int, int, int, long, long, long, hipStream_t);
+#ifdef MI355_HGEMM_T
+MI355_HGEMM_INSTANTIATE(MI355_HGEMM_T, MI355_HGEMM_LAYOUT)
+#else
+MI355_HGEMM_INSTANTIATE(half_t, MI355_GEMM_NN)
+MI355_HGEMM_INSTANTIATE(half_t, MI355_GEMM_NT)
+MI355_HGEMM_INSTANTIATE(half_t, MI355_GEMM_TN)
+MI355_HGEMM_INSTANTIATE(bf16_t, MI355_GEMM_NN)
+MI355_HGEMM_INSTANTIATE(bf16_t, MI355_GEMM_NT)
+MI355_HGEMM_INSTANTIATE(bf16_t, MI355_GEMM_TN)
 #endif
 
 }  // namespace mi355
-
-#if defined(MI355_TIMELINE) && (!defined(MI355_HGEMM_PART) || MI355_HGEMM_PART == 0)
-// profiling build: copies the records of the last tiled fp16 GEMM launch (kMaxWorkgroups x kSlots 64-bit values) to the host
-extern "C" int mi355_timeline_read_hgemm(void* dst, size_t bytes) {
-    const size_t all = sizeof(unsigned long long) * mi355::timeline::kMaxWorkgroups * mi355::timeline::kSlots;
-    return (int)hipMemcpyFromSymbol(dst, HIP_SYMBOL(mi355::hgemm_stamps), bytes < all ? bytes : all);
-}
-#endif

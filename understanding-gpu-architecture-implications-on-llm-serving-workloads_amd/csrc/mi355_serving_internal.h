@@ -31,6 +31,23 @@ hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, 
                           long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
                           hipStream_t stream);
 
+// The kernels of one element type and layout (hgemm.hip, one translation unit each). k_zero_padded: rows whose K index is
+// contiguous hold zeros from K up to the next multiple of 8.
+template <typename T, int LAYOUT>
+hipError_t gemm_layout(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc,
+                       long ldr, int variant, bool k_zero_padded, hipStream_t stream);
+template <typename T, int LAYOUT>
+hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
+                                hipStream_t stream);
+
+// Workspace of the split-K path: ticket counters (one per tile, at zero between launches), then `bytes` minus those for
+// partial tiles. hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: none to be had.
+constexpr size_t kSplitKCounterBytes = 16 * 1024;   // up to 4096 tiles
+hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out);
+#ifdef MI355_TIMELINE
+extern hipError_t (*timeline_hgemm_reader)(void*, size_t);   // of the translation unit whose tiled kernel was launched last
+#endif
+
 // Aligned copies of GEMM operands (gemm_pack.hip): which operands need one, and the rows and bytes of the copies.
 struct GemmPackPlan {
     struct Operand {
