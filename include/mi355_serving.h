@@ -18,10 +18,10 @@
  *     was captured on (or use mi355_fmha_fwd_ws with memory of your own). Only the calling stream's capture state is
  *     visible to the library: a first (or growing) call made while ANOTHER stream captures in global capture mode is a
  *     hipMalloc inside that capture and invalidates it, so make such calls before any capture starts.
- *     The GEMM entry points keep a second buffer of the same kind per (device, stream) for the partial tiles of their
- *     split-K path (17 .. 1024 rows against a second operand of up to 8192 columns, K a multiple of 128; >= 8 MiB, up to
- *     72 MiB); a GEMM call that cannot get it (its stream is being captured and has none yet, or hipMalloc fails) does not fail: it
- *     runs the kernels without split-K, so a captured call is faster when the step ran once on that stream before.
+ *     The GEMM entry points keep a second buffer of the same kind per (device, stream) for the partial tiles of products
+ *     that are cut into ranges of K because their tiles do not fill the machine (>= 8 MiB, up to 96 MiB); a GEMM call
+ *     that cannot get it (its stream is being captured and has none yet, or hipMalloc fails) does not fail: it
+ *     runs the kernels without ranges of K, so a captured call is faster when the step ran once on that stream before.
  *     The attention entry points other than mi355_fmha_fwd_ws (which takes the caller's) and mi355_fmha_fwd_noalloc
  *     (which walks all keys in one kernel) keep a third buffer of that kind
  *     for a chunk of queries against a long cache (at most 128 work items of 128 or 256 queries, kv_valid_len >= 2048: the keys
@@ -73,7 +73,7 @@ extern "C" {
  *                                  gemm_15_amd.cpp:291-313)
  * lda/ldb/ldc are in elements and refer to the stored matrices (e.g. lda >= M for layout TN).
  * Any M, N, K >= 1 is accepted. The fast paths need A and B 16-byte aligned with lda and ldb multiples of 8, and
- * K % 8 == 0 (K % 64 != 0 with M <= 64 and no residual: one more launch for the last K % 64 columns); M and N are free
+ * K % 8 == 0 unless no operand's K index is contiguous (layout TN; other operands: mi355_gemm_ws); M and N are free
  * (ragged tile edges are handled inside the kernels; an operand whose M or N index is contiguous is read in 16-byte
  * chunks, up to 7 elements into the padding that its leading dimension, a multiple of 8, leaves behind M or N). C (and
  * a residual) may have any row stride and alignment (global memory takes 16-byte accesses at any element; only the
@@ -102,8 +102,7 @@ int mi355_hgemm_silu_mul(const void* A, const void* B, void* C, int M, int N, in
  * projections of a decoder layer whose result is added to the residual stream (`hidden_states = residual + hidden_states`
  * after o_proj and after down_proj, benchmarks/flashattn-cuda/modeling_llama.py:776,781; an elementwise kernel of its own
  * in the reference). The product is rounded to fp16 first and the sum once more, so the result equals that of the two
- * separate operations bit for bit (one exception: with K % 64 != 0 and M <= 64, mi355_hgemm forms its product in two
- * passes and this entry point in one, so the two may differ in the last bit of the product). R may be C (in place; then ldr must equal ldc), otherwise R and C must not overlap;
+ * separate operations bit for bit. R may be C (in place; then ldr must equal ldc), otherwise R and C must not overlap;
  * ldr >= N. Layouts, shapes and fast-path conditions as mi355_hgemm (R and ldr aligned like C and ldc).
  */
 int mi355_hgemm_add(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb,

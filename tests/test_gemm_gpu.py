@@ -654,3 +654,51 @@ def test_operands_with_unaligned_rows_through_aligned_copies(lib, gpu, dtype, la
     bound = 2e-2 * (K / 1024.0) ** 0.5 + max(1e-2, 3 * eps) * ref.abs() + eps * got.abs()
     assert bool((err <= bound).all()), float((err - bound).max())
     assert bool((c[M:] == 5.0).all()) and bool((c[:, N:] == 5.0).all())
+
+
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("M,N,K,splits,own_merge", [(150, 200, 1000, 3, False), (150, 203, 1000, 3, True), (257, 64, 712, 5, False),
+                                                    (33, 391, 136, 2, True), (70, 72, 2112, 16, False), (1, 8, 192, 3, True)])
+def test_ranges_of_k_of_any_length_on_every_tile_shape(lib, gpu, layout, shape, M, N, K, splits, own_merge):
+    # ranges that are no equal shares of K, the last one with a K tail; merged by the last workgroup of a tile or by a kernel of
+    # their own: the same bits on every launch, since the ranges are added in their order either way
+    if shape == 7 and layout == "TN":
+        pytest.skip("32-row tiles exist for layouts with a K-contiguous A")
+    a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
+    pad = lambda t: torch.cat((t, torch.full((t.shape[0], -t.shape[1] % 8), float("nan"), dtype=t.dtype)), 1).to(gpu)
+    ag, bg = pad(a), pad(b)
+    c = torch.full((M + 1, N + 5), 4.0, dtype=torch.float16, device=gpu)
+    st = torch.cuda.current_stream(gpu).cuda_stream
+    got = []
+    for _ in range(3):
+        c[:M, :N] = 0
+        assert lib.load().mi355_internal_hgemm_variant(ag.data_ptr(), bg.data_ptr(), c.data_ptr(), M, N, K, ag.shape[1], bg.shape[1], N + 5,
+                                                       lib.LAYOUTS[layout], 0, shape + 16 * splits + 4096 * own_merge, st) == 0
+        torch.cuda.synchronize()
+        got.append(c[:M, :N].cpu())
+    ok, stt = so.gemm_tolerance_ok(got[0], so.gemm_ref(a, b, layout), K)
+    assert ok, stt
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("M,N,K", [(1, 24, 8), (16, 77, 40), (3, 130, 72), (17, 513, 1000), (64, 40, 4136), (8, 16, 248)])
+def test_k_tails_and_odd_widths_on_the_small_m_kernels(lib, gpu, dtype, layout, M, N, K):
+    # the last K % 32 (layout NT: 64) columns are taken by the last wave with zeros behind K; what lies in the rows' padding are NaNs
+    a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
+    a, b = a.to(dtype), b.to(dtype)
+    pad = lambda t: torch.cat((t, torch.full((t.shape[0], -t.shape[1] % 8), float("nan"), dtype=t.dtype)), 1).to(gpu)
+    ag, bg = pad(a), pad(b)
+    c = torch.full((M + 1, N + 5), 4.0, dtype=dtype, device=gpu)
+    st = torch.cuda.current_stream(gpu).cuda_stream
+    assert lib.load().mi355_internal_hgemm_variant(ag.data_ptr(), bg.data_ptr(), c.data_ptr(), M, N, K, ag.shape[1], bg.shape[1], N + 5, lib.LAYOUTS[layout],
+                                                   lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, 8, st) == 0
+    torch.cuda.synchronize()
+    ref = so.gemm_ref(a, b, layout)
+    err = (c[:M, :N].cpu().float() - ref).abs()
+    bound = 2e-2 * (K / 1024.0) ** 0.5 + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10) * ref.abs()
+    assert bool((err <= bound).all()), float((err - bound).max())
+    assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())

@@ -132,7 +132,7 @@ static int fmha_checked(const char* fn, const void* Q, const void* K, const void
 }
 
 static int hgemm_silu_mul_impl(const char* fn, int dtype, const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-                         int layout, void* stream) {
+                         int layout, void* stream, int variant = 0) {
     if (!A || !B || !C) return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer", fn);
     if (M < 1 || N < 1 || K < 1) return fail(MI355_ERR_BAD_ARGUMENT, "%s: M, N, K must be >= 1", fn);
     if (layout != MI355_GEMM_NN && layout != MI355_GEMM_NT)
@@ -141,7 +141,7 @@ static int hgemm_silu_mul_impl(const char* fn, int dtype, const void* A, const v
     if (lda < K || ldb < b_min || ldc < N)
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: leading dimension too small", fn);
     if (N > 0x3fffffff) return fail(MI355_ERR_BAD_ARGUMENT, "%s: N too large", fn);
-    hipError_t e = mi355::hgemm_silu_mul_dispatch(A, B, C, M, 2 * N, K, lda, ldb, ldc, layout, dtype, static_cast<hipStream_t>(stream));
+    hipError_t e = mi355::hgemm_silu_mul_dispatch(A, B, C, M, 2 * N, K, lda, ldb, ldc, layout, dtype, variant, static_cast<hipStream_t>(stream));
     if (e == hipErrorNotSupported)
         return fail(MI355_ERR_UNSUPPORTED,
                     "%s: needs M <= 16 with layout NT, or M > 64 (or M > 16 with enough columns to fill the machine), N a multiple of 32, K a multiple of 64 and 16-byte aligned operands; "
@@ -153,6 +153,11 @@ static int hgemm_silu_mul_impl(const char* fn, int dtype, const void* A, const v
 int mi355_hgemm_silu_mul(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                          int layout, void* stream) {
     return hgemm_silu_mul_impl("mi355_hgemm_silu_mul", MI355_DTYPE_FP16, A, B, C, M, N, K, lda, ldb, ldc, layout, stream);
+}
+
+int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                                          int64_t ldc, int layout, int dtype, int variant, void* stream) {
+    return hgemm_silu_mul_impl("mi355_internal_hgemm_silu_mul_variant", dtype, A, B, C, M, N, K, lda, ldb, ldc, layout, stream, variant);
 }
 
 int mi355_gemm_silu_mul_bf16(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,

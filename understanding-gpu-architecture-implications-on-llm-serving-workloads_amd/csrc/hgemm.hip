@@ -32,6 +32,7 @@
 //     The MFMA is issued with the B fragment as first operand, i.e. it produces the transposed block, so a
 //     lane ends up with 4 consecutive N of one row of C; the epilogue parks the sub-tile in LDS and stores whole
 //     128-byte lines.
+#include <cmath>
 #include <type_traits>
 #include <utility>
 #include "mi355_common.h"
@@ -355,9 +356,11 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     tile_of_block(blockIdx.x, (M + Cfg::BM - 1) / Cfg::BM, (N + Cfg::BN - 1) / Cfg::BN, tile_m, tile_n);
     const long m0 = (long)tile_m * Cfg::BM;
     const long n0 = (long)tile_n * Cfg::BN;
-    if constexpr (SPLIT_K) {   // this workgroup's range of K
-        K /= splits;
-        const long k0 = (long)blockIdx.y * K;
+    if constexpr (SPLIT_K) {   // this workgroup's range of K: whole K tiles, the last range ends with K
+        const int all = (K + BK - 1) / BK;
+        const int t0 = (int)((long)blockIdx.y * all / splits), t1 = (int)((long)(blockIdx.y + 1) * all / splits);
+        const long k0 = (long)t0 * BK;
+        K = min(K, t1 * BK) - (int)k0;
         A += A_KC ? k0 : k0 * lda;
         B += B_KC ? k0 : k0 * ldb;
     }
@@ -686,19 +689,30 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     wait_vmcnt<0>();  // the last tiles' copies (on the empty buffer) have written their zeros
     __syncthreads();  // every wave has finished reading the operand stages
     if constexpr (SPLIT_K) {
-        // partial tile (block, range): element q of lane t's accumulator block b at float (b * 4 + q) * NTHREADS + t, so
-        // that every store and load instruction of a wave covers 256 contiguous bytes
-        const long tile_floats = (long)Cfg::NTHREADS * TM * TN * 4;
-        float* tile_part = part + (long)blockIdx.x * splits * tile_floats;
-        float* mine = tile_part + (long)blockIdx.y * tile_floats + tid;
-        // (device-scope atomic stores, i.e. `global_store_dword .. sc1`, written as such so that the compiler places the
+        if (counters == nullptr) {   // the partial tiles are merged by a kernel of their own: [range][padded M][padded N]
+            const long np = (long)((N + BN - 1) / BN) * BN, mp = (long)((M + BM - 1) / BM) * BM;
+            float* dst = part + ((long)blockIdx.y * mp + m0 + wm * TM * 16 + (lane & 15)) * np + n0 + wn * TN * 16 + 4 * (lane >> 4);
+#pragma unroll
+            for (int b = 0; b < TM * TN; ++b) *(float4v*)(dst + (long)(b / TN) * 16 * np + (b % TN) * 16) = acc[b / TN][b % TN];
+            return;
+        }
+        // partial tile (tile, range): pair p (two floats) of lane t's accumulator block b at pair (b * 2 + p) * NTHREADS + t,
+        // so that every store and load instruction of a wave covers 512 contiguous bytes
+        constexpr int NB = TM * TN;
+        constexpr long kTilePairs = (long)Cfg::NTHREADS * NB * 2;
+        uint64_t* const tile_part = reinterpret_cast<uint64_t*>(part) + (long)blockIdx.x * splits * kTilePairs + tid;
+        uint64_t* const mine = tile_part + (long)blockIdx.y * kTilePairs;
+        // (device-scope atomic stores, i.e. `global_store_dwordx2 .. sc1`, written as such so that the compiler places the
         // wait states between the last matrix instructions and the first memory instruction that reads their result: a
         // wave that arrives last at the barrier above is only a few cycles behind its last MFMA)
 #pragma unroll
-        for (int b = 0; b < TM * TN; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                __hip_atomic_store(mine + (long)(b * 4 + q) * Cfg::NTHREADS, acc[b / TN][b % TN][q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int p = 0; p < 2; ++p) {
+                const float4v v = acc[b / TN][b % TN];
+                const uint64_t w = (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2 * p]) | (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2 * p + 1]) << 32;
+                __hip_atomic_store(mine + (long)(b * 2 + p) * Cfg::NTHREADS, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's part has reached memory before the ticket is drawn
         __syncthreads();
         MI355_LDS unsigned* ticket_sh = (MI355_LDS unsigned*)smem;
@@ -707,26 +721,38 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
         const unsigned ticket = *ticket_sh;
         __syncthreads();   // the epilogue below reuses that LDS
         if (ticket != (unsigned)(splits - 1)) return;
-        // the last one: every other workgroup of this tile drew its ticket after its part had reached memory. The parts
-        // are read with device-coherent loads (sc1), 16 in flight per lane, and added in the order of the ranges.
+        // The last one: every other workgroup of this tile drew its ticket after its part had reached memory. The parts
+        // are read with device-coherent loads and added in the order of the ranges, this workgroup's own part too (it is
+        // what the registers hold, but a fixed place for it would cost more registers than the load costs time). A batch
+        // of loads is a round trip to memory of ~1 us whatever its size, so a batch is as large as the registers allow:
+        // 64 registers of a lane, all blocks of one to four ranges.
+        constexpr int kChunk = NB < 16 ? NB : 16, kBatch = 16 / kChunk < 4 ? 16 / kChunk : 4;
+        static_assert(NB % kChunk == 0, "whole chunks of blocks");
 #pragma unroll
-        for (int b = 0; b < TM * TN; ++b) {
-            float4v sum = float4v{0.f, 0.f, 0.f, 0.f};
-            for (int r0 = 0; r0 < splits; r0 += 4) {
-                float4v v[4];
+        for (int b0 = 0; b0 < NB; b0 += kChunk) {
+            float4v sum[kChunk];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const float* pa = tile_part + (long)min(r0 + u, splits - 1) * tile_floats + (long)(b * 4) * Cfg::NTHREADS + tid;
+            for (int b = 0; b < kChunk; ++b) sum[b] = float4v{0.f, 0.f, 0.f, 0.f};
+            for (int r0 = 0; r0 < splits; r0 += kBatch) {
+                uint64_t v[kBatch][kChunk][2];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        asm volatile("global_load_dword %0, %1, off sc1" : "=v"(v[u][q]) : "v"(pa + (long)q * Cfg::NTHREADS) : "memory");
+                for (int u = 0; u < kBatch; ++u) {
+                    const uint64_t* pa = tile_part + (long)min(r0 + u, splits - 1) * kTilePairs + (long)b0 * 2 * Cfg::NTHREADS;
+#pragma unroll
+                    for (int b = 0; b < kChunk * 2; ++b)
+                        v[u][b / 2][b % 2] = __hip_atomic_load(pa + (long)b * Cfg::NTHREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) :: "memory");
+                __builtin_amdgcn_sched_barrier(0);   // all loads of the batch are issued before the first is waited for
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (r0 + u < splits) sum += v[u];
+                for (int u = 0; u < kBatch; ++u)
+                    if (r0 + u < splits)
+#pragma unroll
+                        for (int b = 0; b < kChunk; ++b)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) sum[b][q] += __builtin_bit_cast(float, (uint32_t)(v[u][b][q / 2] >> (32 * (q & 1))));
             }
-            acc[b / TN][b % TN] = sum;
+#pragma unroll
+            for (int b = 0; b < kChunk; ++b) acc[(b0 + b) / TN][(b0 + b) % TN] = sum[b];
         }
         if (tid == 0) __hip_atomic_store(&counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -740,6 +766,55 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
             rec[0] = tl_w[0]; rec[1] = tl_w[1]; rec[2] = tl_w[2]; rec[3] = tl_w[3];
             rec[4] = tl_c[0]; rec[5] = tl_c[1]; rec[6] = (unsigned long long)ktiles; rec[7] = 0;
         })
+}
+
+// Merges the partial tiles of a split-K launch without counters: C = sum over the ranges, in their order (+ R after the
+// rounding, as in the epilogue). A thread takes 8 columns of a row. Bandwidth-bound: every partial tile is read once, mostly
+// from the memory-side cache, by all CUs, where the last workgroup of a tile would read its tile's parts alone.
+template <typename T>
+static __global__ __launch_bounds__(256) void hgemm_merge_kernel(const float* __restrict__ part, T* C, const T* R, int M, int N, long mp, long np,
+                                                          long ldc, long ldr, int splits) {
+    using V8 = typename Elem<T>::v8;
+    const int chunks = (int)(np / 8);
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    const long row = i / chunks;
+    const int col = (int)(i - row * chunks) * 8;
+    if (row >= M || col >= N) return;
+    const float* p = part + row * np + col;
+    float4v lo = *(const float4v*)p, hi = *(const float4v*)(p + 4);
+    int r = 1;
+    for (; r + 2 < splits; r += 3) {   // three ranges in flight
+        float4v a[3], b[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            a[u] = *(const float4v*)(p + (r + u) * mp * np);
+            b[u] = *(const float4v*)(p + (r + u) * mp * np + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u) { lo += a[u]; hi += b[u]; }
+    }
+    for (; r < splits; ++r) {
+        lo += *(const float4v*)(p + r * mp * np);
+        hi += *(const float4v*)(p + r * mp * np + 4);
+    }
+    V8 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[j] = (T)lo[j]; v[4 + j] = (T)hi[j]; }
+    T* c = C + row * ldc + col;
+    const T* res = R + row * ldr + col;
+    if (col + 8 <= N) {
+        if (R != nullptr) {
+            V8 x;
+            __builtin_memcpy(&x, res, 16);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (T)((float)v[j] + (float)x[j]);
+        }
+        __builtin_memcpy(c, &v, 16);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (col + j < N) c[j] = R != nullptr ? (T)((float)v[j] + (float)res[j]) : v[j];
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -885,6 +960,17 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
     float4v acc[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = float4v{0.f, 0.f, 0.f, 0.f};
+    auto k_step = [&](MI355_LDS const char* st) {
+        V8 af;
+        if constexpr (A_KC) af = Elem<T>::frag(lds_read_b128(st + a_off));
+        else af = Elem<T>::frag(concat(lds_read_tr16_b64(st + a_off), lds_read_tr16_b64(st + a_off + 256)));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            half4 lo = lds_read_tr16_b64(st + b_off[j]);
+            half4 hi = lds_read_tr16_b64(st + b_off[j] + 4 * 128);
+            acc[j] = Elem<T>::mfma16(af, Elem<T>::frag(concat(lo, hi)), acc[j]);
+        }
+    };
 
     // ---- pipeline ---------------------------------------------------------------------------------------------
     int issued = s_begin;
@@ -904,19 +990,20 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
         } else {
             wait_vmcnt<0>();
         }
-        MI355_LDS char* st = wbase + slot * kSmallMStageBytes;
+        k_step(wbase + slot * kSmallMStageBytes);
         slot = (slot + 1 == kSmallMStages) ? 0 : slot + 1;
-        V8 af;
-        if constexpr (A_KC) af = Elem<T>::frag(lds_read_b128(st + a_off));
-        else af = Elem<T>::frag(concat(lds_read_tr16_b64(st + a_off), lds_read_tr16_b64(st + a_off + 256)));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            half4 lo = lds_read_tr16_b64(st + b_off[j]);
-            half4 hi = lds_read_tr16_b64(st + b_off[j] + 4 * 128);
-            acc[j] = Elem<T>::mfma16(af, Elem<T>::frag(concat(lo, hi)), acc[j]);
-        }
         // the reads of this slot must be complete before a later copy refills it
         wait_lgkmcnt<0>();
+    }
+    if (const int k0 = ksteps * 32; k0 < K && wave == kSmallMWaves - 1) {
+        // the last K % 32 rows of B (columns of A), by the last wave, whose copies have all landed: zeros behind K
+        const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *(MI355_LDS half8*)(wbase + i * 1024 + lane * 16) = k0 + 8 * i + b_row < K ? *(const half8*)(b_src + (long)(8 * i) * ldb) : zero;
+        *(MI355_LDS half8*)(wbase + 4096 + lane * 16) = k0 + (A_KC ? 8 * a_chunk : at_k) < K ? *(const half8*)a_src : zero;
+        wait_lgkmcnt<0>();
+        k_step(wbase);
     }
 
     // ---- reduce the 8 partial tiles through LDS ---------------------------------------------------------------
@@ -1047,6 +1134,14 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
     for (int sub = 0; sub < 2; ++sub) f_off[sub] = f_row * 128 + (((4 * sub + (lane >> 4)) ^ (f_row & 7)) << 4);
 
     float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
+    auto k_step = [&](MI355_LDS const char* st) {
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+            V8 bf = Elem<T>::frag(lds_read_b128(st + f_off[sub]));
+            V8 af = Elem<T>::frag(lds_read_b128(st + 2048 + f_off[sub]));
+            acc = Elem<T>::mfma16(af, bf, acc);
+        }
+    };
 
     int issued = s_begin;
 #pragma unroll
@@ -1065,15 +1160,21 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
         } else {
             wait_vmcnt<0>();
         }
-        MI355_LDS char* st = wbase + slot * kSmallMNtStageBytes;
+        k_step(wbase + slot * kSmallMNtStageBytes);
         slot = (slot + 1 == kSmallMNtStages) ? 0 : slot + 1;
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-            V8 bf = Elem<T>::frag(lds_read_b128(st + f_off[sub]));
-            V8 af = Elem<T>::frag(lds_read_b128(st + 2048 + f_off[sub]));
-            acc = Elem<T>::mfma16(af, bf, acc);
-        }
         wait_lgkmcnt<0>();  // the reads of this slot are complete before a later copy refills it
+    }
+    if (const int k0 = ksteps * 64; k0 < K && wave == kSmallMNtWaves - 1) {
+        // the last K % 64 columns, by the last wave, whose copies have all landed: zeros behind K (K is a multiple of 8, or
+        // the rows hold zeros up to the next one)
+        const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+        const bool in = k0 + 8 * c_chunk < K;
+        *(MI355_LDS half8*)(wbase + lane * 16) = in ? *(const half8*)b_src0 : zero;
+        *(MI355_LDS half8*)(wbase + 1024 + lane * 16) = in ? *(const half8*)b_src1 : zero;
+        *(MI355_LDS half8*)(wbase + 2048 + lane * 16) = in ? *(const half8*)a_src0 : zero;
+        if constexpr (!HALF_A) *(MI355_LDS half8*)(wbase + 3072 + lane * 16) = in ? *(const half8*)a_src1 : zero;
+        wait_lgkmcnt<0>();
+        k_step(wbase);
     }
 
     // acc[q] is D[m = 4*(lane/16) + q][n = lane%16]; reduce the 8 partial tiles through LDS
@@ -1309,164 +1410,202 @@ static hipError_t launch_main(const T* A, const T* B, T* C, const T* R, int M, i
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------------------------------------
-// Split-K on 64x64 tiles (and, further down, on 128x128 tiles), for 17 .. 256 rows against a second operand that is too narrow to give every CU a tile: the
-// ranges of K of a tile run on different workgroups (see SPLIT_K of hgemm_main_kernel) and meet in a workspace of the
-// library's own: one buffer per (device, stream), allocated at first use and replaced by a larger one when a call needs
-// more; a buffer that has been handed to a kernel is never freed (a HIP graph captured earlier may hold its address).
-// Nothing can be allocated while the stream is capturing: such a call (no buffer yet, or too small a one) takes the
-// kernels without split-K instead. The ticket counters, in front of the partial tiles, are zeroed when a buffer is new
-// (a fill kernel on the calling stream) and left at zero by every launch.
-// ---------------------------------------------------------------------------------------------------------
-// Number of ranges K is cut into, or 0 where split-K does not apply: 17 .. 256 rows, K a multiple of 64, few enough
-// 64x64 tiles for at least four ranges at about two workgroups per CU (up to 128 tiles; up to 192 with a long K), at
-// least eight K tiles per range, ranges of equal length. Measured with weights that come from HBM, layout NT (us, without / with split-K): 64 x 4096 x 14336 55 / 32,
-// 17 x 4096 x 14336 35 / 29, 128 x 4096 x 14336 54 / 44, 64 x 4096 x 4096 17.4 / 15.7, 96 x 4096 x 4096 17.3 / 15.5,
-// 48 x 6144 x 4096 16.6 / 17.4; two ranges only lose (96 x 6144 x 4096 20 / 24, 192 x 4096 x 4096 21 / 25), and so do up to
-// 32 rows with a short K, where the small-M kernels are at their best (32 x 4096 x 4096 11 / 15). 129 .. 192 tiles get
-// four ranges where K is long (192 x 4096 x 14336 70 / 58, NN 81 / 59; with K = 4096 22 against 21 without; 256 tiles:
-// 69 / 73).
-static int split_k_ranges(int M, int N, int K) {
-    if (M < 17 || M > 256 || K % 64 != 0) return 0;
-    if (M <= 32 && K < 8192) return 0;
-    const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
-    if (tiles > 192 || (tiles > 128 && K < 8192)) return 0;
-    const int ktiles = K / 64;
-    int s = tiles > 128 ? 4 : (int)(512 / tiles);
-    if (s > 16) s = 16;
-    while (s >= 4 && (ktiles % s != 0 || ktiles / s < 8)) --s;
-    return s >= 4 ? s : 0;
-}
-
-// The same on 128x128 tiles (64 KiB of partial tile per workgroup), for 193 .. 1024 rows against a long K (the down
-// projection): at most 128 tiles, two to four ranges so that about every CU has a workgroup (640 x 3072 x 12288 NT:
-// 96 / 76). Measured, weights from HBM
-// (us, best tile shape without / with split-K): NT 256 x 4096 x 14336 70 / 54, 384 rows 99 / 83, 512 rows 100 / 86,
-// 320 x 2048 x 16384 68 / 47; NN 256 x 4096 x 8192 47 / 38, 384 rows 61 / 54, 512 x 4096 x 14336 108 / 85. Layout NT with
-// K = 8192 loses to its 128x64 tiles (384 x 4096 x 8192: 49 / 52), so it needs a longer K; 640 rows (160 tiles) and every
-// product with K = 4096 lose 10-60 %.
-static int split_k_ranges_128(int M, int N, int K, bool nt) {
-    if (M < 193 || M > 1024 || K < (nt ? 12288 : 8192) || K % 64 != 0) return 0;
-    const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-    const int ktiles = K / 64;
-    if (tiles > 128) {
-        // 129 .. 255 tiles leave CUs idle for a whole walk over K. With s ranges the walk takes rounds(s) / s of that time,
-        // rounds(s) = ceil(tiles * s / 256), plus about 0.05 s of it for the partial tiles (measured, us without / with: NT
-        // 896 x 3072 x 12288, 168 tiles, three ranges 124 / 102; 768 x 4096 x 14336, 192 tiles, four ranges 136 / 130;
-        // 768 x 3072 x 12288, 144 tiles, three ranges 123 / 98; 640 x 4096 x 12288, 160 tiles, three ranges 124 / 102;
-        // eight ranges lose: 896 x 4096 x 14336 138 / 176, 513 rows 102 / 117): the best s up to four, if it saves 4 %; a
-        // saving below 10 % only with a last row of tiles that is at least three quarters full (700 x 4096 x 12288, 192
-        // tiles with 60 rows in the last six of every column: 102 / 107)
-        if (tiles >= 256 || K < 12288) return 0;
-        int best = 0;
-        double best_cost = 0.96;
-        for (int s = 2; s <= 4; ++s) {
-            if (ktiles % s != 0 || ktiles / s < 16) continue;
-            const double cost = (double)((tiles * s + 255) / 256) / s + 0.05 * s;
-            if (cost < best_cost) { best_cost = cost; best = s; }
-        }
-        if (best_cost > 0.9 && M % 128 != 0 && M % 128 < 96) return 0;
-        return best;
-    }
-    int s = (int)(256 / tiles);
-    if (s > 4) s = 4;
-    while (s >= 2 && (ktiles % s != 0 || ktiles / s < 8)) --s;
-    return s >= 2 ? s : 0;
-}
-
-// hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: no workspace to be had, the caller takes another kernel
-template <typename T, bool A_KC, bool B_KC, int BT = 64, int STAGES = 4, int PER_CU = 2>
+// hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: no workspace to be had, the caller takes another kernel.
+// own_merge: the partial tiles are merged by hgemm_merge_kernel instead of the last workgroup of each tile.
+template <typename T, bool A_KC, bool B_KC, int BM, int BN, int WM, int WN, int STAGES = 0, int PER_CU = 1>
 static hipError_t launch_split_k(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb, long ldc,
-                                 long ldr, int splits, hipStream_t stream) {
-    using Cfg = MainCfg<A_KC, B_KC, BT, BT, 2, 2, STAGES>;
-    auto kern = hgemm_main_kernel<T, A_KC, B_KC, BT, BT, 2, 2, 0, true, STAGES, PER_CU, true>;
+                                 long ldr, int splits, bool own_merge, hipStream_t stream) {
+    using Cfg = MainCfg<A_KC, B_KC, BM, BN, WM, WN, STAGES>;
+    auto kern = hgemm_main_kernel<T, A_KC, B_KC, BM, BN, WM, WN, 0, true, STAGES, PER_CU, true>;
     static DynamicLdsOnce lds_once;
     if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES); e != hipSuccess) return e;
-    const long tiles = (long)((M + BT - 1) / BT) * ((N + BT - 1) / BT);
-    if (tiles * sizeof(unsigned) > kSplitKCounterBytes) return hipErrorOutOfMemory;
-    const size_t bytes = kSplitKCounterBytes + (size_t)tiles * splits * Cfg::NTHREADS * Cfg::TM * Cfg::TN * 16;
+    const long tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+    if (!own_merge && tiles * sizeof(unsigned) > kSplitKCounterBytes) return hipErrorOutOfMemory;
+    const size_t bytes = kSplitKCounterBytes + (size_t)tiles * splits * BM * BN * 4;
     char* ws = nullptr;
     if (hipError_t e = split_k_workspace(bytes, stream, &ws); e != hipSuccess) return e;
+    float* part = reinterpret_cast<float*>(ws + kSplitKCounterBytes);
+    MI355_TL(timeline_hgemm_reader = &read_hgemm_stamps;)
     kern<<<dim3((unsigned)tiles, (unsigned)splits), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, stream>>>(
-        A, B, C, R, M, N, K, lda, ldb, ldc, ldr, reinterpret_cast<float*>(ws + kSplitKCounterBytes), reinterpret_cast<unsigned*>(ws), splits);
+        A, B, C, R, M, N, K, lda, ldb, ldc, ldr, part, own_merge ? nullptr : reinterpret_cast<unsigned*>(ws), splits);
+    if (own_merge) {
+        const long mp = tiles_m * BM, np = tiles_n * BN, threads = (long)M * (np / 8);
+        hgemm_merge_kernel<T><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream>>>(part, C, R, M, N, mp, np, ldc, ldr, splits);
+    }
     return hipGetLastError();
 }
 
-// 17..64 rows: the small-M kernels stream B once per 16 rows (the L2 catches part of the repeats), the 128x128 tiles
-// stream it once but run K / 64 dependent tile steps of ~0.4 us on at most one workgroup per 128 columns. Cost models
-// from measurements of both at Llama projection shapes; true = the tiles are expected to be faster.
-static double small_m_us(int M, int N, int K, bool nn) {
-    return (double)((M + 15) / 16) * (double)N * (double)K * 2.0 / 6.5e6 + (nn ? 2.3 : 4.0);
+enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile128x256, kTile256x128, kTile32x64, kSmallM, kDeepRing };
+struct KernelChoice {
+    int shape = kTile128x128;
+    int splits = 1;           // ranges of K
+    bool own_merge = false;   // their partial tiles are merged by a kernel of its own
+};
+// see mi355_internal_hgemm_variant
+static KernelChoice pinned_kernel(int variant) {
+    KernelChoice k;
+    k.shape = variant & 15;
+    k.splits = (variant >> 4) & 0xff;
+    if (k.splits < 1) k.splits = 1;
+    k.own_merge = (variant >> 12) != 0;
+    return k;
 }
-static double few_row_tiles_us(int M, int N, int K, bool nt) {
-    long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-    double step_us = 0.42;
-    if (nt && tiles < 192) {   // layout NT runs 128x64 tiles then
-        tiles = (long)((M + 127) / 128) * ((N + 63) / 64);
-        step_us = 0.34;
+// The kernel that is expected to finish a product first, by a model of the time of each. The constants (microseconds) were
+// fitted to ~32 000 timings of pinned kernels over 600 products (1 .. 8192 rows, 256 .. 16384 columns, K 256 .. 14336, all
+// layouts, ragged and round sizes); over those the choice takes 2.2 % longer than the best kernel on average.
+//   * A tiled kernel runs in rounds of one workgroup per CU (two for the small tiles) of `K tiles * step + fixed`. The step
+//     is set by the CU's intake of 64 bytes per cycle as much as by the matrix instructions (see the tile shapes' rings at
+//     MainCfg), and by half again (small tiles) or a fifth (256x256) where the second operand is too large to stay in the
+//     memory-side cache between calls.
+//   * Ranges of K fill the machine where the tiles of a product do not. Merged by the last workgroup of a tile: a round
+//     trip through memory, and one more of 64 KiB per range and 128x128 tile. Merged by a kernel of their own: its launch,
+//     and the partial tiles once through memory: the better one for large tiles and more than a few ranges (512 x 4096 x
+//     14336 NT, 256x128 tiles in four ranges: 72.0 us against 68.7; 128 x 4096 x 14336, 128x128 in eight: 37.7 / 34.7).
+//   * Nothing is faster than its bytes take, ~5.6 TB/s behind ~3 us.
+// Against the thresholds this replaced (us, before / after): 288 x 776 x 12160 NN 46 / 30, 42 x 520 x 4336 NN 23 / 9, 212 x
+// 9012 x 12208 TN 126 / 78, 131 x 7808 x 13952 NT 89 / 68, 8 x 640 x 13440 TN 22 / 11, 500 x 4096 x 14336 NT 84 / 69.
+struct ShapeCost {
+    int shape, bm, bn, per_cu;
+    float step, step_full, fixed;   // K tile alone on its CU, with `per_cu` workgroups there; outside the K loop
+    float uncached;                 // factor on the steps for a large second operand
+};
+// gate_up: among the shapes whose waves hold 64 columns, the gate and the up of the same outputs.
+static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles_ok, bool split_ok, bool gate_up) {
+    static const ShapeCost shapes[] = {
+        {kTile256x256, 256, 256, 1, 1.30f, 1.30f, 7.1f, 1.19f}, {kTile128x256, 128, 256, 1, .667f, .667f, 5.2f, 1.31f},
+        {kTile256x128, 256, 128, 1, .617f, .617f, 5.7f, 1.31f}, {kTile128x128, 128, 128, 1, .417f, .417f, 3.9f, 1.33f},
+        {kTileHalf, 64, 128, 1, .274f, .274f, 3.5f, 1.43f},     {kTile64x64, 64, 64, 2, .177f, .382f, 2.9f, 1.53f},
+        {kTile32x64, 32, 64, 2, .146f, .270f, 2.9f, 1.65f},     {kDeepRing, 64, 64, 1, .151f, .151f, 3.5f, 1.53f}};
+    static const int ranges[] = {2, 3, 4, 5, 6, 8, 10, 12, 16};
+    const bool nt = a_kc && b_kc;
+    const float layout = nt ? .914f : a_kc ? 1.f : 1.043f;
+    const float b_bytes = 2.f * (float)N * (float)K, bytes = b_bytes + 2.f * (float)M * ((float)K + (float)N);
+    const float floor_us = bytes / 5.6e6f + 3.1f;
+    const int ktiles = (K + 63) / 64;
+    KernelChoice best;
+    best.shape = 0;
+    float best_us = 1e30f;
+    const auto consider = [&](float us, int shape, int splits, bool own_merge) {
+        if (us >= best_us) return;
+        best_us = us;
+        best.shape = shape;
+        best.splits = splits;
+        best.own_merge = own_merge;
+    };
+    if (M <= 64 && !gate_up) {   // the small-M kernels: workgroups of 16 rows and 64 (layout NT: 16) columns, the whole of K
+        const int row_blocks = (M + 15) / 16;
+        const long wgs = (long)row_blocks * ((N + (nt ? 15 : 63)) / (nt ? 16 : 64));
+        const float k = (float)K / 64.f * (b_bytes > 20e6f ? 2.2f : 1.f);
+        if (nt) consider(fmaxf(3.8f + k * .019f * fmaxf(1.f, wgs * .004f), b_bytes * (1.f + (row_blocks - 1) * .55f) / 5.5e6f + 2.f), kSmallM, 1, false);
+        else consider(fmaxf(3.3f + k * .095f * fmaxf(1.f, wgs * .003f), b_bytes * (1.f + (row_blocks - 1) * .79f) / 6.3e6f + 3.4f), kSmallM, 1, false);
     }
-    return (double)(K / 64) * step_us * (double)((tiles + 255) / 256);
-}
-static bool few_rows_prefer_tiles(int M, int N, int K, bool nt) {
-    if (M <= 16) return false;
-    return few_row_tiles_us(M, N, K, nt) < small_m_us(M, N, K, false) - 4.0;
-}
-// Which tile shape is expected to finish a product of more than 64 rows first (1 = 256x256, 2 = 128x128, 3 = 64x128 or
-// 128x64, 4 = 64x64 two to a CU, 5 = 128x256, 6 = 256x128, 7 = 32x64). A CU takes in 64 bytes per cycle from the memory system, so
-// the time of a K tile is set by the tile's bytes as much as by its matrix instructions (the operands of a 128x128 tile
-// need the same 512 cycles to arrive that its matrix instructions take): measured cycles per K tile of 64 of one
-// workgroup alone on its CU are 2470 (256x256; matrix pipes 2048), 1340 (128x256 and 256x128 on a ring of three stages;
-// pipes 1024), 770 (128x128; pipes 512), 576 (half tile) and 384 (64x64). A workgroup spends another 5000-12000 cycles
-// outside its K loop (first tiles in flight, epilogue). The workgroups run in rounds of one per CU (two for the 64x64
-// tiles); the last round may be a partial one. The model reproduces the measured times of 1024^3 .. 8192^3,
-// 2048 x 4096 x 4096 and 1536 x 1536 x 8192 within ~10 %. The 128x128 figure used below is 840, that of the 128x256
-// tiles 1400: on N(0,1) operands, under the board's power limit, the larger tiles do better against the smaller ones
-// than on zeros (3072 x 3072 x 4096: 75 us against 87 where zeros give 70 against 71). The 128x256 tiles are for the
-// products that fill the chip once with them, where 256x256 tiles leave CUs idle and 128x128 tiles need two rounds
-// (2048 x 4096 x 4096: 59 us against 66 on 128x128 tiles and 89 on 256x256; 2048 x 4096 x 14336: 186 against 216); of
-// the two orientations the one with fewer rounds, 256x128 if they tie (768 x 28672 x 4096: 163 us against 168,
-// 1536 x 4096 x 14336: 157 against 161, 768 x 6144 x 4096: 40.7 against 42.1; 2048 x 4096 x 4096 the same either way).
-// The 32x64 tiles (ring of 8 stages of 12 KiB, 335 cycles per K tile) are for 65 .. 128 rows against a narrow second
-// operand (generation steps of that many sequences through the O and down projections), where 64x64 tiles are only
-// half as many as CUs: 128 x 4096 x 14336 NT 41 -> 33 us, 128 x 4096 x 4096 13.2 -> 11.2, 96 x 4096 x 14336 40 -> 32
-// (with 256 rows, or 6144 columns, they would need two rounds and lose: 63 us against 45, 20 against 14).
-static int cheapest_tile_shape(int M, int N, int K, bool a_k_contiguous, bool nt) {
-    struct Cand { int shape, bm, bn, per_cu; double step, fixed; };
-    static const Cand cands[] = {{1, 256, 256, 1, 2470., 12000.}, {2, 128, 128, 1, 840., 7000.}, {3, 64, 128, 1, 576., 6000.},
-                                 {4, 64, 64, 2, 384., 5000.}, {5, 128, 256, 1, 1400., 9000.}, {6, 256, 128, 1, 1400., 9000.},
-                                 {7, 32, 64, 1, 335., 5000.}};
-    const double ktiles = (double)((K + 63) / 64);
-    int best = 2;
-    double best_t = 0.;
-    for (const Cand& c : cands) {
-        if (c.shape == 7 && !a_k_contiguous) continue;   // 32-row tiles exist for a K-contiguous A only
-        const int bm = (c.shape == 3 && nt) ? c.bn : c.bm, bn = (c.shape == 3 && nt) ? c.bm : c.bn;   // layout NT: 128x64
+    if (!tiles_ok) return best;   // (shape 0: none of these kernels)
+    for (const ShapeCost& c : shapes) {
+        if ((c.shape == kTile32x64 && !a_kc) || (c.shape == kDeepRing && M > 64)) continue;
+        if (gate_up && (c.shape == kTile32x64 || c.shape == kTileHalf)) continue;
+        if (c.bm > 64 && c.bm >= 2 * M) continue;   // more than half of every tile would be padding
+        const bool half_nt = c.shape == kTileHalf && nt;   // 128x64 for layout NT
+        const int bm = half_nt ? c.bn : c.bm, bn = half_nt ? c.bm : c.bn;
         const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        const long cap = 256L * c.per_cu, full = tiles / cap, rem = tiles % cap;
-        double t = (double)full * (c.per_cu * ktiles * c.step + c.fixed);
-        if (rem) t += (double)((rem + 255) / 256) * ktiles * c.step + c.fixed;
-        if (c.shape == 6) t -= 1.;   // a tie between the two orientations
-        if (best_t == 0. || t < best_t) { best_t = t; best = c.shape; }
+        const float factor = layout * (b_bytes > 20e6f ? c.uncached : 1.f);
+        const auto loop_us = [&](int splits, int per_cu) {
+            const float kt = (float)((ktiles + splits - 1) / splits), one = kt * c.step * factor + c.fixed;
+            const long wgs = tiles * splits;
+            if (per_cu == 1) return (float)((wgs + 255) / 256) * one;
+            const float two = kt * c.step_full * factor + c.fixed;
+            const long rem = wgs % 512;
+            return (float)(wgs / 512) * two + (rem > 256 ? two : rem > 0 ? one : 0.f);
+        };
+        // (unsplit, the 32x64 tiles run on a ring of eight stages, one workgroup to a CU)
+        consider(fmaxf(loop_us(1, c.shape == kTile32x64 ? 1 : c.per_cu), floor_us), c.shape, 1, false);
+        if (!split_ok || c.shape == kDeepRing || tiles > 400) continue;
+        for (const int s : ranges) {
+            if (tiles * s > 1200 || ktiles < 2 * s) break;
+            const float us = fmaxf(loop_us(s, c.per_cu), floor_us), tile_kib = (float)(bm * bn) / 256.f;
+            const float part_mb = (float)(tiles * s) * tile_kib / 1024.f;
+            if (part_mb > 64.f) break;
+            consider(us + 1.67f + s * tile_kib * (1.207f / 64.f) + part_mb * .2f, c.shape, s, false);
+            consider(us + 3.07f + part_mb * .36f, c.shape, s, true);
+        }
     }
     return best;
 }
+// The same, remembered for the last few products of the calling thread: going through the candidates takes the host ~0.5 us,
+// a tenth of what the smallest products take altogether.
+static KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles_ok, bool split_ok, bool gate_up = false) {
+    struct Entry {
+        int M = 0, N = 0, K = 0, flags = 0;
+        KernelChoice choice;
+    };
+    static thread_local Entry seen[64];
+    const int flags = a_kc | b_kc << 1 | tiles_ok << 2 | split_ok << 3 | gate_up << 4;
+    const uint32_t hash = ((uint32_t)M * 0x9e3779b1u) ^ ((uint32_t)N * 0x85ebca6bu) ^ ((uint32_t)K * 0xc2b2ae35u) ^ (uint32_t)flags * 0x27d4eb2fu;
+    Entry& e = seen[hash >> 26];
+    if (e.M != M || e.N != N || e.K != K || e.flags != flags) {
+        e.choice = cheapest_kernel(M, N, K, a_kc, b_kc, tiles_ok, split_ok, gate_up);
+        e.M = M; e.N = N; e.K = K; e.flags = flags;
+    }
+    return e.choice;
+}
 
-// Up to 64 rows on 64x64 tiles with an 8-deep ring: the second operand is streamed once whatever M is, by N / 64
-// workgroups that each sustain ~38 GB/s until HBM saturates (~6.3 TB/s); layout NN pays ~10 % for its 128-byte row
-// segments. True when that is expected to beat both alternatives above (measured at Llama projection shapes:
-// 16 x 14336 x 4096 NT 19 us against 22, 64 rows NN 22 against 31, 64 x 4096 x 4096 NT 15 against 17; but
-// 16 x 4096 x 14336 NT 41 against 19 on the split-K small-M kernel, and 16 x 14336 x 4096 NN 21 against 20).
-// Layout NT with up to 16 rows always takes the split-K small-M kernel: with weights that are in no cache (a different
-// weight matrix on every launch, as in a decoder stack) it is the faster one at every Llama projection shape
-// (8 x 28672 x 4096: 39 us against 46, 8 x 14336 x 4096: 23 against 26, 16 x 14336 x 4096: 24.6 against 25.8).
-static bool few_rows_prefer_deep_ring(int M, int N, int K, bool nn, bool nt) {
-    if (nt && M <= 16) return false;
-    const double bytes = (double)N * (double)K * 2.0;
-    const double rate = fmin(6.3e6, (double)((N + 63) / 64) * 38e3);   // bytes per microsecond
-    const double deep_us = (bytes / rate + 1.0) * (nn ? 1.1 : 1.0);
-    double other_us = small_m_us(M, N, K, nn);
-    if (M > 16) other_us = fmin(other_us, few_row_tiles_us(M, N, K, nt) + 4.0);
-    return deep_us < other_us;
+// hipErrorNotSupported: no such kernel for this layout
+template <typename T, bool A_KC, bool B_KC>
+static hipError_t run_kernel(const KernelChoice& k, const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
+                             long ldc, long ldr, bool c_aligned, hipStream_t stream) {
+#define MI355_ARGS A, B, C, R, M, N, K, lda, ldb, ldc, ldr
+    if (k.splits > 1) {
+        switch (k.shape) {
+            case kTile128x128: return launch_split_k<T, A_KC, B_KC, 128, 128, 2, 2>(MI355_ARGS, k.splits, k.own_merge, stream);
+            case kTileHalf:
+                if constexpr (A_KC && B_KC) return launch_split_k<T, A_KC, B_KC, 128, 64, 2, 2>(MI355_ARGS, k.splits, k.own_merge, stream);
+                else return launch_split_k<T, A_KC, B_KC, 64, 128, 1, 4>(MI355_ARGS, k.splits, k.own_merge, stream);
+            case kTile64x64: return launch_split_k<T, A_KC, B_KC, 64, 64, 2, 2, 4, 2>(MI355_ARGS, k.splits, k.own_merge, stream);
+            case kTile128x256: return launch_split_k<T, A_KC, B_KC, 128, 256, 2, 4>(MI355_ARGS, k.splits, k.own_merge, stream);
+            case kTile256x128: return launch_split_k<T, A_KC, B_KC, 256, 128, 4, 2>(MI355_ARGS, k.splits, k.own_merge, stream);
+            case kTile256x256: return launch_split_k<T, A_KC, B_KC, 256, 256, 2, 4>(MI355_ARGS, k.splits, k.own_merge, stream);
+            case kTile32x64:
+                if constexpr (A_KC) return launch_split_k<T, A_KC, B_KC, 32, 64, 2, 2, 4, 2>(MI355_ARGS, k.splits, k.own_merge, stream);
+                else return hipErrorNotSupported;
+            default: return hipErrorNotSupported;
+        }
+    }
+    const auto whole = [&](int bm, int bn) { return c_aligned && M % bm == 0 && N % bn == 0; };
+    switch (k.shape) {
+        case kTile256x256:
+            if (whole(256, 256)) return launch_main<T, A_KC, B_KC, 256, 256, 2, 4>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 0, true>(MI355_ARGS, stream);
+        case kTile128x128:
+            if (whole(128, 128)) return launch_main<T, A_KC, B_KC, 128, 128, 2, 2>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 0, true>(MI355_ARGS, stream);
+        case kTileHalf:
+            if constexpr (A_KC && B_KC) {
+                if (whole(128, 64)) return launch_main<T, A_KC, B_KC, 128, 64, 2, 2>(MI355_ARGS, stream);
+                return launch_main<T, A_KC, B_KC, 128, 64, 2, 2, 0, true>(MI355_ARGS, stream);
+            } else {
+                if (whole(64, 128)) return launch_main<T, A_KC, B_KC, 64, 128, 1, 4>(MI355_ARGS, stream);
+                return launch_main<T, A_KC, B_KC, 64, 128, 1, 4, 0, true>(MI355_ARGS, stream);
+            }
+        case kTile64x64:
+            if (whole(64, 64)) return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, false, 4, 2>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, true, 4, 2>(MI355_ARGS, stream);
+        case kTile128x256:
+            if (whole(128, 256)) return launch_main<T, A_KC, B_KC, 128, 256, 2, 4>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 128, 256, 2, 4, 0, true>(MI355_ARGS, stream);
+        case kTile256x128:
+            if (whole(256, 128)) return launch_main<T, A_KC, B_KC, 256, 128, 4, 2>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 256, 128, 4, 2, 0, true>(MI355_ARGS, stream);
+        case kTile32x64:
+            if constexpr (A_KC) return launch_main<T, A_KC, B_KC, 32, 64, 2, 2, 0, true, 8>(MI355_ARGS, stream);
+            else return hipErrorNotSupported;
+        case kDeepRing:
+            return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, true>(MI355_ARGS, stream);
+        case kSmallM:
+            if constexpr (!B_KC) return launch_smallm_nn<T, A_KC>(MI355_ARGS, stream);
+            else if constexpr (A_KC) return launch_smallm_nt<T>(MI355_ARGS, stream);
+            else return hipErrorNotSupported;
+        default: return hipErrorNotSupported;
+    }
+#undef MI355_ARGS
 }
 
 template <typename T, bool A_KC, bool B_KC>
@@ -1478,105 +1617,25 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
                             (lda % 8 == 0) && (ldb % 8 == 0);
     const bool c_aligned = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && (ldc % 8 == 0) &&
                            (reinterpret_cast<uintptr_t>(R) % 16 == 0) && (ldr % 8 == 0);
-    const bool aligned = ab_aligned && c_aligned;
-    // K that is not a multiple of the tiles' depth (the reference's own tiled kernels take K % 16 == 0,
-    // kernels/gemm/pkg/gemm_unified/csrc/auto/gemm_7.cu:115-135): the tiled kernels take any multiple of 8, their
-    // prologue handles the K % 64 columns at the end. Up to 64 rows are better served by the small-M kernels, which
-    // need whole k-steps: there the last K % 64 columns go through the bounds-checked kernel first, into C, and the
-    // product over the first K - K % 64 is added to it as a residual (two roundings more than a single pass; 16 x 4096 x
-    // 4104 NT: 10 us, against 16 on tiles). A call that brings a residual of its own takes the tiles.
-    if (aligned && R == nullptr && M <= 64 && K > 64 && K % 64 != 0 && variant == 0) {
-        const int k_tail = K % 64, k_main = K - k_tail;
-        const T* a_tail = A_KC ? A + k_main : A + (long)k_main * lda;
-        const T* b_tail = B_KC ? B + k_main : B + (long)k_main * ldb;
-        dim3 grid((N + 63) / 64, (M + 63) / 64);
-        hgemm_edge_kernel<T, A_KC, B_KC><<<grid, dim3(256), 0, stream>>>(a_tail, b_tail, C, nullptr, M, N, k_tail, lda, ldb, ldc, 0);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        return launch_layout<T, A_KC, B_KC>(A, B, C, C, M, N, k_main, lda, ldb, ldc, ldc, variant, k_zero_padded, stream);
-    }
-    // the tiled kernels address a tile with 32-bit byte offsets: up to 256 rows of lda (ldb) elements
-    // Any N: an operand stored [K,N] is copied in 16-byte chunks of its rows, and the chunk that straddles N ends in the
-    // padding a leading dimension of a multiple of 8 leaves (what it holds only reaches columns that are never stored).
     // Any K, if the rows of an operand whose K index is contiguous hold zeros from K up to the next multiple of 8 (the
     // copies of gemm_pack.hip do, k_zero_padded) or no operand is stored that way: the copies of the other operand take
-    // single rows of K.
+    // single rows of K. Any N: an operand stored [K,N] is copied in 16-byte chunks of its rows, and the chunk that straddles
+    // N ends in the padding a leading dimension of a multiple of 8 leaves (what it holds only reaches columns that are
+    // never stored).
     const bool k_ok = K % 8 == 0 || k_zero_padded || (!A_KC && !B_KC);
-    const bool ragged_ok = ab_aligned && k_ok && lda < (1L << 22) && ldb < (1L << 22);
-    const bool small_m = M <= 64 && !(ragged_ok && few_rows_prefer_tiles(M, N, K, A_KC && B_KC));
-    // 17 .. 256 rows against a narrow second operand: split-K, where a workspace is to be had
-    if (ragged_ok && variant == 0) {
-        if (const int splits = split_k_ranges(M, N, K); splits > 0) {
-            const hipError_t e = launch_split_k<T, A_KC, B_KC>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, splits, stream);
-            if (e != hipErrorStreamCaptureUnsupported && e != hipErrorOutOfMemory) return e;
+    if (ab_aligned && k_ok) {
+        // the tiled kernels address a tile with 32-bit byte offsets: up to 256 rows of lda (ldb) elements
+        const bool tiles_ok = lda < (1L << 22) && ldb < (1L << 22);
+        KernelChoice pick = variant > 0 && (A_KC || (variant & 15) != kTile32x64) && (tiles_ok || (variant & 15) == kSmallM) ? pinned_kernel(variant) : choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, true);
+        for (;;) {
+            const hipError_t e = run_kernel<T, A_KC, B_KC>(pick, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, c_aligned, stream);
+            // no workspace to be had (the stream is being captured and has none yet): the best kernel without split-K
+            if (pick.splits <= 1 || variant > 0 || (e != hipErrorStreamCaptureUnsupported && e != hipErrorOutOfMemory)) {
+                if (e != hipErrorNotSupported) return e;
+                break;
+            }
             (void)hipGetLastError();
-        } else if (const int splits128 = split_k_ranges_128(M, N, K, A_KC && B_KC); splits128 > 0) {
-            const hipError_t e = launch_split_k<T, A_KC, B_KC, 128, 0, 1>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, splits128, stream);
-            if (e != hipErrorStreamCaptureUnsupported && e != hipErrorOutOfMemory) return e;
-            (void)hipGetLastError();
-        }
-    }
-    // 33 .. 64 rows against a second operand of up to 8192 columns (generation steps of that many sequences through the
-    // QKV, O and down projections): 32x64 tiles, two rows of up to 128 workgroups. The 64x64 tiles below put half as many
-    // workgroups on the stream of the second operand, the small-M kernels stream it once per 16 rows; with weights that
-    // come from HBM (us, 64x64 tiles with the 8-deep ring / 32x64 tiles): NT 64 x 4096 x 14336 71 / 55, 48 x 4096 x 4096
-    // 19.9 / 15.8, 40 x 6144 x 4096 19.8 / 15.6; NN 64 x 4096 x 14336 84 / 69, 33 x 4096 x 4096 23.5 / 19.5. Up to 32 rows
-    // are one row of such tiles, and the small-M kernels stay ahead (NT 32 x 4096 x 14336 37 / 56).
-    if constexpr (A_KC) {
-        if (ragged_ok && variant == 0 && M > 32 && M <= 64 && (N + 63) / 64 <= 128)
-            return launch_main<T, A_KC, B_KC, 32, 64, 2, 2, 0, true, 8>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-    }
-    // Up to 64 rows (generation-step projections): 64x64 tiles with an 8-deep ring stream the second operand once, on
-    // N / 64 workgroups with ~50 KiB each in flight, where the split-K small-M kernels below stream it once per 16 rows.
-    if (ragged_ok && M <= 64 && variant == 0 && few_rows_prefer_deep_ring(M, N, K, A_KC && !B_KC, A_KC && B_KC)) {
-        if (M == 64 && N % 64 == 0 && c_aligned) return launch_main<T, A_KC, B_KC, 64, 64, 2, 2>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-        return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-    }
-    if constexpr (!B_KC) {   // NN and TN
-        if (ab_aligned && small_m && K % 32 == 0 && K >= 32)
-            return launch_smallm_nn<T, A_KC>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-    }
-    if constexpr (A_KC && B_KC) {
-        // (this kernel stores element by element: C and the residual may lie anywhere)
-        if (ab_aligned && small_m && K % 64 == 0 && K >= 64) return launch_smallm_nt<T>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-    }
-    // Tiled kernels: M and N need not be multiples of the tile, nor of 8. Shapes: 1 = 256x256 (8 waves, ring of 2),
-    // 2 = 128x128 (4 waves, ring of 3), 3 = half of that (64x128, for layout NT 128x64, which keeps the 128-byte rows of
-    // both K-contiguous operands; ring of 5), 4 = 64x64 with a ring of 4 (64 KiB: two workgroups fit on a CU), 5 = 128x256
-    // and 6 = 256x128 (8 waves of 64x64, ring of 3), 7 = 32x64 (4 waves of 16x32, ring of 8; layouts with a K-contiguous
-    // A). More than 64 rows: the shape with the least
-    // estimated time. Up to 64 rows (products that few_rows_prefer_tiles sends here): 64x64 tiles, two to a CU, for layout
-    // NT (17 .. 64 x 28672 x 4096 with weights from HBM: 45 - 52 us against 53 - 57 on 128x64 tiles and 51 on 128x128),
-    // 128x128 otherwise (layout NN: 42 - 47 us against 52 - 64).
-    if (ragged_ok) {
-        int shape = variant >= 1 && variant <= (A_KC ? 7 : 6) ? variant : M <= 64 ? ((A_KC && B_KC) ? 4 : 2) : cheapest_tile_shape(M, N, K, A_KC, A_KC && B_KC);
-        const auto whole = [&](int bm, int bn) { return c_aligned && M % bm == 0 && N % bn == 0; };
-        switch (shape) {
-            case 1:
-                if (whole(256, 256)) return launch_main<T, A_KC, B_KC, 256, 256, 2, 4>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-            case 3:
-                if constexpr (A_KC && B_KC) {
-                    if (whole(128, 64)) return launch_main<T, A_KC, B_KC, 128, 64, 2, 2>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                    return launch_main<T, A_KC, B_KC, 128, 64, 2, 2, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                } else {
-                    if (whole(64, 128)) return launch_main<T, A_KC, B_KC, 64, 128, 1, 4>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                    return launch_main<T, A_KC, B_KC, 64, 128, 1, 4, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                }
-            case 5:
-                if (whole(128, 256)) return launch_main<T, A_KC, B_KC, 128, 256, 2, 4>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                return launch_main<T, A_KC, B_KC, 128, 256, 2, 4, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-            case 6:
-                if (whole(256, 128)) return launch_main<T, A_KC, B_KC, 256, 128, 4, 2>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                return launch_main<T, A_KC, B_KC, 256, 128, 4, 2, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-            case 7:
-                if constexpr (A_KC) return launch_main<T, A_KC, B_KC, 32, 64, 2, 2, 0, true, 8>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                [[fallthrough]];
-            case 4:
-                if (whole(64, 64)) return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, false, 4, 2>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                return launch_main<T, A_KC, B_KC, 64, 64, 2, 2, 0, true, 4, 2>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-            default:
-                if (whole(128, 128)) return launch_main<T, A_KC, B_KC, 128, 128, 2, 2>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
-                return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 0, true>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, stream);
+            pick = choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, false);
         }
     }
     dim3 grid((N + 63) / 64, (M + 63) / 64);
@@ -1589,27 +1648,30 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
 // caller runs the product and mi355_silu_mul separately.
 template <typename T, bool A_KC, bool B_KC>
 static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, int K, long lda, long ldb,
-                                  long ldc, hipStream_t stream) {
+                                  long ldc, int variant, hipStream_t stream) {
     const bool aligned = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0) &&
                          (reinterpret_cast<uintptr_t>(C) % 16 == 0) && (lda % 8 == 0) && (ldb % 8 == 0) && (ldc % 8 == 0);
     // N = columns of op(B); gate/up pairs are 64 columns wide. Few rows are better served by the small-M product.
     if (!aligned || K % 64 != 0 || K < 64 || N % 64 != 0 || lda >= (1L << 22) || ldb >= (1L << 22)) return hipErrorNotSupported;
     if constexpr (A_KC && B_KC) {   // generation step: the split-K small-M kernel with the same epilogue
-        if (M <= 16) return launch_smallm_nt_gate_up<T>(A, B, C, M, N, K, lda, ldb, ldc, stream);
+        if (M <= 16 && (variant == 0 || variant == kSmallM)) return launch_smallm_nt_gate_up<T>(A, B, C, M, N, K, lda, ldb, ldc, stream);
     }
-    // up to 64 rows (generation steps of a few dozen sequences): 64x64 tiles with an 8-deep ring as for the plain product,
-    // four waves side by side along M so that every wave holds the gate and the up columns of its rows
-    if (M <= 64 && !few_rows_prefer_tiles(M, N, K, false))
-        return launch_main<T, A_KC, B_KC, 64, 64, 4, 1, 1, true>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
-    const bool fits128 = M % 128 == 0 && N % 128 == 0;
-    const bool fits256 = M % 256 == 0 && N % 256 == 0;
-    const long t256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-    if (t256 >= 192) {
-        if (fits256) return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 1>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
-        return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 1, true>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
+    // More rows: the tile shape by the same model as the plain product's. On 64x64 tiles four waves lie side by side along M,
+    // so that every wave holds the gate and the up columns of its rows.
+#define MI355_ARGS A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0
+    switch (variant > 0 ? variant : choose_kernel(M, N, K, A_KC, B_KC, true, false, true).shape) {
+        case kTile256x256:
+            if (M % 256 == 0 && N % 256 == 0) return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 1>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 1, true>(MI355_ARGS, stream);
+        case kTile128x256: return launch_main<T, A_KC, B_KC, 128, 256, 2, 4, 1, true>(MI355_ARGS, stream);
+        case kTile256x128: return launch_main<T, A_KC, B_KC, 256, 128, 4, 2, 1, true>(MI355_ARGS, stream);
+        case kTile64x64: return launch_main<T, A_KC, B_KC, 64, 64, 4, 1, 1, true, 4, 2>(MI355_ARGS, stream);
+        case kDeepRing: return launch_main<T, A_KC, B_KC, 64, 64, 4, 1, 1, true>(MI355_ARGS, stream);
+        default:
+            if (M % 128 == 0 && N % 128 == 0) return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 1>(MI355_ARGS, stream);
+            return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 1, true>(MI355_ARGS, stream);
     }
-    if (fits128) return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 1>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
-    return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 1, true>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
+#undef MI355_ARGS
 }
 
 // One translation unit per element type and layout (the build compiles the six side by side): MI355_HGEMM_T and
@@ -1623,15 +1685,15 @@ hipError_t gemm_layout(const void* A, const void* B, void* C, const void* R, int
 }
 template <typename T, int LAYOUT>
 hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
-                                hipStream_t stream) {
+                                int variant, hipStream_t stream) {
     if constexpr (LAYOUT == MI355_GEMM_TN) return hipErrorNotSupported;
     else return launch_silu_mul<T, true, LAYOUT == MI355_GEMM_NT>(static_cast<const T*>(A), static_cast<const T*>(B), static_cast<T*>(C),
-                                                                  M, N2, K, lda, ldb, ldc, stream);
+                                                                  M, N2, K, lda, ldb, ldc, variant, stream);
 }
 #define MI355_HGEMM_INSTANTIATE(T, LAYOUT)                                                                                     \
     template hipError_t gemm_layout<T, LAYOUT>(const void*, const void*, void*, const void*, int, int, int, long, long, long,  \
                                                long, int, bool, hipStream_t);                                                  \
-    template hipError_t gemm_silu_mul_layout<T, LAYOUT>(const void*, const void*, void*, int, int, int, long, long, long, hipStream_t);
+    template hipError_t gemm_silu_mul_layout<T, LAYOUT>(const void*, const void*, void*, int, int, int, long, long, long, int, hipStream_t);
 #ifdef MI355_HGEMM_T
 MI355_HGEMM_INSTANTIATE(MI355_HGEMM_T, MI355_HGEMM_LAYOUT)
 #else

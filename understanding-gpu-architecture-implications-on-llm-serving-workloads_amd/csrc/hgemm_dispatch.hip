@@ -91,12 +91,12 @@ hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, 
 }
 
 hipError_t hgemm_silu_mul_dispatch(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
-                                   int layout, int dtype, hipStream_t stream) {
+                                   int layout, int dtype, int variant, hipStream_t stream) {
     const bool bf16 = dtype == MI355_DTYPE_BF16, nn = layout == MI355_GEMM_NN;
     if (!nn && layout != MI355_GEMM_NT) return hipErrorNotSupported;
     const auto entry = bf16 ? (nn ? &gemm_silu_mul_layout<bf16_t, MI355_GEMM_NN> : &gemm_silu_mul_layout<bf16_t, MI355_GEMM_NT>)
                             : (nn ? &gemm_silu_mul_layout<half_t, MI355_GEMM_NN> : &gemm_silu_mul_layout<half_t, MI355_GEMM_NT>);
-    return entry(A, B, C, M, N2, K, lda, ldb, ldc, stream);
+    return entry(A, B, C, M, N2, K, lda, ldb, ldc, variant, stream);
 }
 
 #ifdef MI355_TIMELINE

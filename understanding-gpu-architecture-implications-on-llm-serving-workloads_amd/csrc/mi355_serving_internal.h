@@ -38,7 +38,7 @@ hipError_t gemm_layout(const void* A, const void* B, void* C, const void* R, int
                        long ldr, int variant, bool k_zero_padded, hipStream_t stream);
 template <typename T, int LAYOUT>
 hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
-                                hipStream_t stream);
+                                int variant, hipStream_t stream);
 
 // Workspace of the split-K path: ticket counters (one per tile, at zero between launches), then `bytes` minus those for
 // partial tiles. hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: none to be had.
@@ -76,7 +76,7 @@ struct FmhaStrides {
 
 // The product fused with silu(gate) * up (see hgemm_main_kernel's EPI); hipErrorNotSupported for shapes without it.
 hipError_t hgemm_silu_mul_dispatch(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
-                                   int layout, int dtype, hipStream_t stream);
+                                   int layout, int dtype, int variant, hipStream_t stream);
 
 // Where the split-KV and key-range attention paths keep their partial results.
 struct FmhaWorkspace {
@@ -123,13 +123,16 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 // Test and tuning hooks: exported from the shared library but not part of its public header. They take the kernel
 // variant as an argument (no process-wide state): variants that do not fit the shape fall back to the choice by shape.
 //   gemm: 0 = by shape; 1 = 256x256 tiles, 2 = 128x128, 3 = 64x128 (layout NT: 128x64), 4 = 64x64 with a ring of four
-//         stages, 5 = 128x256, 6 = 256x128, 7 = 32x64 (layouts NN and NT): the tiled kernel of that shape for any product the tiled kernels take (M and N need not be multiples
-//         of the tile); products of up to 64 rows that the small-M kernels take stay on those
+//         stages, 5 = 128x256, 6 = 256x128, 7 = 32x64 (layouts NN and NT), 8 = the small-M kernels (up to 64 rows), 9 = 64x64 with
+//         a ring of eight; shapes 1 .. 7 take s ranges of K with variant + 16 s, merged by a kernel of their own (instead of
+//         the last workgroup of a tile) with variant + 16 s + 4096. The gate/up product: 1, 2, 4, 5, 6, 8, 9
 //   fmha: 0 = by shape, 1 = 128-query workgroups, 2 = 256-query workgroups (1 and 2 also keep generation-step shapes off
 //         the split-KV path), 3 = keys cut into ranges and merged (an error where the choice by shape would not do that)
 extern "C" {
 int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int layout, int dtype, int variant, void* stream);
+int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                                          int64_t ldc, int layout, int dtype, int variant, void* stream);
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                     int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides,
                                     int dtype, int variant, void* stream);
