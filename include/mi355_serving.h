@@ -8,7 +8,7 @@
  * Conventions
  *   - every pointer is a DEVICE pointer owned by the caller; none is retained. The only memory the library ever
  *     allocates are three kinds of workspace. One holds the partial results of the split-KV attention path (taken when
- *     Hq/Hkv * Sq <= 32 and kv_valid_len >= 512, i.e. generation steps): one buffer per (device, stream), obtained
+ *     Hq/Hkv * Sq <= 32 and kv_valid_len >= 512, i.e. generation steps over long caches): one buffer per (device, stream), obtained
  *     with hipMalloc at first use (>= 4 MiB; when a later call needs more, a larger buffer is allocated and the old
  *     one is kept, because a HIP graph captured earlier may still hold its address; nothing is freed before the
  *     process ends, and every stream that ever made such a call keeps its buffer), so steady-state calls allocate

@@ -683,3 +683,23 @@ def test_torch_operator_bfloat16_and_mixed_dtype_rejection(gpu):
     assert out.dtype == torch.bfloat16 and (out.float().cpu() - o_ref).abs().max() <= 1.6e-2
     with pytest.raises(RuntimeError, match="dtype"):
         fmha_unified.ops.fine_fmha(q.to(gpu), k.half().to(gpu), v.to(gpu), True, False, 5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal,kvv", [
+    (1, 8, 2, 1, 1, False, None), (2, 8, 8, 1, 31, False, 30), (3, 32, 8, 1, 300, False, None),      # one key range
+    (1, 4, 1, 8, 511, True, None), (2, 4, 1, 5, 3, True, None),       # several query rows; queries that see no key
+    (40, 16, 8, 1, 77, False, 76), (17, 32, 16, 1, 1024, False, None), (260, 2, 1, 2, 40, True, 39),   # more workgroups than CUs: two waves each
+    (1, 8, 2, 1, 512, False, None), (1, 8, 2, 1, 575, False, 570), (2, 4, 2, 1, 1025, False, None)])    # ranges of two tiles
+def test_generation_step_over_short_caches(lib, gpu, dtype, B, Hq, Hkv, Sq, Sk, causal, kvv):
+    q, k, v = (bf16_inputs if dtype == torch.bfloat16 else so.fmha_inputs)(B, Hq, Hkv, Sq, Sk, seed=B + Sk)
+    kvv = Sk if kvv is None else kvv
+    o_ref, lse_ref = so.attention_ref(q, k, v, causal=causal, kv_valid_len=kvv)
+    k, v = k.clone(), v.clone()
+    k[:, :, kvv:] = float("nan")
+    v[:, :, kvv:] = float("nan")
+    o, lse = lib.fmha_fwd(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal, kv_valid_len=kvv)
+    torch.cuda.synchronize()
+    assert float((o.cpu().float() - o_ref).abs().max()) <= (1.6e-2 if dtype == torch.bfloat16 else 2e-3)
+    seen = torch.isfinite(lse_ref)
+    assert torch.equal(torch.isfinite(lse.cpu()), seen) and float((lse.cpu() - lse_ref)[seen].abs().max()) <= 1e-3

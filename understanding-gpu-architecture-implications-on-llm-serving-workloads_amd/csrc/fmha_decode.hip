@@ -1,4 +1,4 @@
-// Decode-shaped attention forward for gfx950 (MI355X): few query rows per kv head, long key sequence.
+// Decode-shaped attention forward for gfx950 (MI355X): few query rows per kv head, any number of keys.
 //
 // The reference runs its generation step (`is_decode`, one query row padded to 64 by ops.py:19-25) through the
 // prefill kernel, one workgroup per (batch, q head) walking all keys (semi/fmha_2_amd.cpp:341-356); that leaves
@@ -67,7 +67,7 @@ __device__ __forceinline__ float other_half(float x) {
 }  // namespace dec
 
 // Workgroup wg = (b * Hkv + hkv) * splits + s covers key tiles [s * tiles_per_split, (s + 1) * tiles_per_split).
-// WAVES waves with NSTAGE pipeline stages of 16 KiB each. <4, 2> (one wave per SIMD, one tile in flight behind the one
+// WAVES waves with NSTAGE pipeline stages of 16 KiB each (two waves: a single key range only). <4, 2> (one wave per SIMD, one tile in flight behind the one
 // being consumed, 128 KiB of LDS) measured better than <3, 3> for short and for long key ranges alike.
 template <typename T, int WAVES, int NSTAGE>
 __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
@@ -482,7 +482,7 @@ __global__ void fmha_decode_clear_kernel(unsigned* counters, int n) {
 
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
     const int group = Hq / Hkv;
-    return (long)group * Sq <= 32 && kv_valid_len >= 512 && Sk >= kv_valid_len && B >= 1;
+    return (long)group * Sq <= 32 && Sk >= kv_valid_len && B >= 1;
 }
 
 namespace dec {
@@ -501,12 +501,29 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     const int ncols = (Hq / Hkv) * Sq;
     const int tiles = (kv_valid + TK - 1) / TK;
     const long pairs = (long)B * Hkv;
-    // about one workgroup per CU; a key range is at least 8 tiles (two per wave)
-    long splits = (256 + pairs / 2) / pairs;
-    splits = (splits < 1 || pairs > kMaxSplitPairs) ? 1 : splits;
-    const long max_splits = (tiles + 7) / 8;
-    if (splits > max_splits) splits = max_splits;
-    if (splits > kMaxSplits) splits = kMaxSplits;
+    // The number of key ranges that is expected to be done first. A workgroup (one to a CU) takes ~3 us and, per tile, what it
+    // gets of the memory's rate: 0.32 us while up to 64 of them run, 0.38 with 128, 0.69 with all 256 (measured over
+    // 8192 keys); more ranges than one also take the merge. Below 512 keys one workgroup walks
+    // them all: no workspace is needed, and the merge would take as long as the walk. us, with as many ranges as make about 256
+    // workgroups of at least eight tiles / by this model: 8 pairs over 1000 keys 9.3 / 8.4, 52 pairs over 9777 keys (five
+    // ranges would be 260 workgroups: a second round for four of them) 66.8 / 50.4, 160 pairs over 4500 keys 80.5 / 65.0.
+    long splits = 1;
+    if (pairs <= kMaxSplitPairs && kv_valid >= 512) {
+        float best_us = 1e30f;
+        const long most = (tiles + 1) / 2 < kMaxSplits ? (tiles + 1) / 2 : kMaxSplits;   // at least two tiles to a range
+        for (long s = 1; s <= most && pairs * s <= 512; ++s) {
+            const float range_tiles = (float)(((tiles + s - 1) / s + 3) / 4 * 4);   // the four waves walk equal pieces
+            const long full = pairs * s / 256, rest = pairs * s % 256;
+            const auto round_us = [&](long wgs) {
+                return 3.f + range_tiles * (wgs <= 64 ? .32f : wgs <= 128 ? .32f + .001f * (float)(wgs - 64) : .38f + .00242f * (float)(wgs - 128));
+            };
+            const float us = (float)full * round_us(256) + (rest > 0 ? round_us(rest) : 0.f) + (s > 1 ? 2.5f + .04f * (float)s + (s > 24 ? .03f * (float)(s - 24) : 0.f) : 0.f);
+            if (us < best_us) {
+                best_us = us;
+                splits = s;
+            }
+        }
+    }
     DecodePlan p;
     p.tiles_per_split = (int)((tiles + splits - 1) / splits);
     p.splits = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
@@ -601,7 +618,7 @@ static hipError_t launch_decode(const T* Q, const T* K, const T* V, T* O, float*
                                 int tiles_per_split, long workgroups, const FmhaStrides& sd, hipStream_t stream) {
     constexpr int LDS = WAVES * NSTAGE * dec::STAGE_BYTES;
     static_assert(LDS >= WAVES * (32 * dec::D + 64) * 4 + 64, "the combine step reuses the pipeline memory");
-    static_assert(LDS >= (3 * dec::kMaxSplits * 32 + 32 + 64) * 4, "so does the merge of the key ranges");
+    static_assert(WAVES < 4 || LDS >= (3 * dec::kMaxSplits * 32 + 32 + 64) * 4, "so does the merge of the key ranges");
     auto kern = fmha_decode_kernel<T, WAVES, NSTAGE>;
     static DynamicLdsOnce lds_once;
     if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(kern), LDS); e != hipSuccess) return e;
@@ -650,6 +667,16 @@ hipError_t fmha_decode_dispatch(const T* Q, const T* K, const T* V, T* O, float*
     float* part = reinterpret_cast<float*>(wsp + plan.counter_bytes);
     unsigned* counters = reinterpret_cast<unsigned*>(wsp);
     const float scale_log2 = scale * 1.4426950408889634f;
+    // More workgroups than CUs with up to 1024 keys each: two waves and 64 KiB per workgroup, so that two share a CU and one's
+    // start-up and combine hide under the other's keys (us, four / two waves: 512 workgroups, 128 keys 13.7 / 10.1, 300
+    // keys 20.2 / 17.8, 700 keys 36.7 / 34.2; 1024 workgroups, 128 keys 23.8 / 16.6, 300 keys 35.2 / 31.0; at 1500 keys they
+    // are equal, and 8192 keys lose: 345 / 363). Above 320 keys the last round of 512 workgroups must not be much emptier
+    // than the last one of 256 would be (736 workgroups, 1000 keys: 66.4 / 70.1).
+    const long rest4 = plan.workgroups % 256, rest2 = plan.workgroups % 512;
+    const bool whole_rounds = rest2 == 0 || rest2 >= 384 || (rest4 > 0 && rest4 < 128);
+    if (plan.splits == 1 && plan.workgroups > 256 && (kv_valid <= 320 || (kv_valid <= 1024 && whole_rounds)))
+        return launch_decode<T, 2, 2>(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits,
+                                      plan.tiles_per_split, plan.workgroups, sd, stream);
     return launch_decode<T, 4, 2>(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits,
                                   plan.tiles_per_split, plan.workgroups, sd, stream);
 }
