@@ -702,3 +702,38 @@ def test_k_tails_and_odd_widths_on_the_small_m_kernels(lib, gpu, dtype, layout, 
     bound = 2e-2 * (K / 1024.0) ** 0.5 + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10) * ref.abs()
     assert bool((err <= bound).all()), float((err - bound).max())
     assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())
+
+
+def test_two_threads_on_one_stream_keep_their_partial_results_apart(lib, gpu):
+    # ranges of K merged by a kernel of its own, and attention key ranges: two launches that share the stream's workspace; no launch
+    # of another thread on the same stream may come between them
+    import threading
+
+    stream = torch.cuda.Stream(gpu)
+    work = []
+    for i, (M, N, K, variant) in enumerate([(200, 512, 2048, 2 + 16 * 4 + 4096), (130, 640, 1024, 2 + 16 * 2)]):
+        a, b = operands(M, N, K, "NT", seed=i, b_std=0.05)
+        a, b = a.to(gpu), b.to(gpu)
+        work.append(lambda a=a, b=b, v=variant: lib.hgemm(a, b, "NT", variant=v))
+    for i, Sq in enumerate((64, 100)):
+        q, k, v = (t.to(gpu) for t in so.fmha_inputs(1, 8, 2, Sq, 4096, seed=i))
+        work.append(lambda q=q, k=k, v=v: lib.fmha_fwd(q, k, v, causal=True, return_lse=False))
+
+    def run_one(f, out, n):
+        with torch.cuda.stream(stream):
+            out.extend(f() for _ in range(n))
+
+    torch.cuda.synchronize()
+    want = [[] for _ in work]
+    for f, w in zip(work, want):
+        run_one(f, w, 1)
+    got = [[] for _ in work]
+    threads = [threading.Thread(target=run_one, args=(f, g, 200)) for f, g in zip(work, got)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    stream.synchronize()
+    for w, g in zip(want, got):
+        w = w[0][0] if isinstance(w[0], tuple) else w[0]
+        assert len(g) == 200 and all(torch.equal(w, x[0] if isinstance(x, tuple) else x) for x in g)

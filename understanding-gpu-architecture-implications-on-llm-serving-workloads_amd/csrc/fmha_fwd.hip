@@ -730,18 +730,25 @@ __global__ __launch_bounds__(256) void fmha_merge_segments_kernel(const T* __res
     if (LSE != nullptr && lane == 0) LSE[row] = denom > 0.f ? m + __logf(denom) : -INFINITY;
 }
 
-static hipError_t segment_workspace(size_t bytes, hipStream_t stream, char** out) {
+// `order` comes back holding the lock of that (device, stream), see split_k_workspace.
+static hipError_t segment_workspace(size_t bytes, hipStream_t stream, char** out, std::unique_lock<std::mutex>* order) {
     struct Buf {
         void* ptr = nullptr;
         size_t size = 0;
+        std::mutex order;
     };
     static std::mutex mu;
     static std::map<std::pair<int, hipStream_t>, Buf> bufs;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mu);
-    Buf& b = bufs[std::make_pair(dev, stream)];
+    Buf* entry = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        entry = &bufs[std::make_pair(dev, stream)];
+    }
+    Buf& b = *entry;
+    *order = std::unique_lock<std::mutex>(b.order);
     if (b.size < bytes) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         e = hipStreamIsCapturing(stream, &cap);
@@ -821,8 +828,9 @@ static hipError_t launch_fmha_segmented(const T* Q, const T* K, const T* V, T* O
     const size_t o_bytes = (size_t)segments * rows * fmha::D * sizeof(T);
     const size_t bytes = o_bytes + (size_t)segments * rows * sizeof(float);
     char* ws = caller_ws;   // memory of the caller (large enough: see fmha_fwd_dispatch), or the library's own
+    std::unique_lock<std::mutex> order;   // both launches follow one another on the stream
     if (ws == nullptr)
-        if (hipError_t e = segment_workspace(bytes, stream, &ws); e != hipSuccess) return e;
+        if (hipError_t e = segment_workspace(bytes, stream, &ws, &order); e != hipSuccess) return e;
     T* o_part = reinterpret_cast<T*>(ws);
     float* lse_part = reinterpret_cast<float*>(ws + o_bytes);
     const int q_tiles = (Sq + 128 * QB - 1) / (128 * QB);

@@ -1423,7 +1423,8 @@ static hipError_t launch_split_k(const T* A, const T* B, T* C, const T* R, int M
     if (!own_merge && tiles * sizeof(unsigned) > kSplitKCounterBytes) return hipErrorOutOfMemory;
     const size_t bytes = kSplitKCounterBytes + (size_t)tiles * splits * BM * BN * 4;
     char* ws = nullptr;
-    if (hipError_t e = split_k_workspace(bytes, stream, &ws); e != hipSuccess) return e;
+    std::unique_lock<std::mutex> order;   // the launches below follow one another on the stream
+    if (hipError_t e = split_k_workspace(bytes, stream, &ws, &order); e != hipSuccess) return e;
     float* part = reinterpret_cast<float*>(ws + kSplitKCounterBytes);
     MI355_TL(timeline_hgemm_reader = &read_hgemm_stamps;)
     kern<<<dim3((unsigned)tiles, (unsigned)splits), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, stream>>>(

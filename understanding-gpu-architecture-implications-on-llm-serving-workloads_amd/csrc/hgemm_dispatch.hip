@@ -17,19 +17,26 @@ static __global__ void hgemm_clear_kernel(unsigned* p, int n) {
 // address). Nothing can be allocated while the stream is capturing: such a call (no buffer yet, or too small a one) fails
 // with hipErrorStreamCaptureUnsupported and its caller takes the kernels without split-K instead. The ticket counters, in
 // front of the partial tiles, are zeroed when a buffer is new (a fill kernel on the calling stream) and left at zero by
-// every launch.
-hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out) {
+// every launch. `order` comes back holding the lock of that (device, stream): the caller keeps it until its launches are
+// issued, so that of two threads with one stream neither's partial tiles are overwritten in front of the other's merge.
+hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, std::unique_lock<std::mutex>* order) {
     struct Buf {
         void* ptr = nullptr;
         size_t size = 0;
+        std::mutex order;
     };
     static std::mutex mu;
     static std::map<std::pair<int, hipStream_t>, Buf> bufs;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mu);
-    Buf& b = bufs[std::make_pair(dev, stream)];
+    Buf* entry = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        entry = &bufs[std::make_pair(dev, stream)];   // entries stay where they are
+    }
+    Buf& b = *entry;
+    *order = std::unique_lock<std::mutex>(b.order);
     if (b.size < bytes) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         e = hipStreamIsCapturing(stream, &cap);

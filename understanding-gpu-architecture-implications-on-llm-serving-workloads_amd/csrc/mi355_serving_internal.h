@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include <cstddef>
+#include <mutex>
 #include "../../include/mi355_serving.h"
 
 namespace mi355 {
@@ -43,7 +44,7 @@ hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, in
 // Workspace of the split-K path: ticket counters (one per tile, at zero between launches), then `bytes` minus those for
 // partial tiles. hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: none to be had.
 constexpr size_t kSplitKCounterBytes = 16 * 1024;   // up to 4096 tiles
-hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out);
+hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, std::unique_lock<std::mutex>* order);
 #ifdef MI355_TIMELINE
 extern hipError_t (*timeline_hgemm_reader)(void*, size_t);   // of the translation unit whose tiled kernel was launched last
 #endif
