@@ -175,3 +175,22 @@ def test_product_code_does_not_touch_the_oracle():
             if f.endswith((".py", ".cpp", ".hip", ".h")):
                 text = open(os.path.join(dirpath, f)).read()
                 assert "serving_oracle" not in text and "oracle/" not in text, os.path.join(dirpath, f)
+
+
+def test_generation_step_partial_results_fit_where_256_workgroups_would(lib):
+    # The number of key ranges is chosen by a model of their time. No call may need more than the 4 MiB static array (what
+    # mi355_fmha_fwd_noalloc has, and the smallest buffer a captured call finds) that would fit it cut into ranges of at least
+    # eight 32-key tiles, one per CU in all; and no call that would then need no memory at all may need some.
+    wsb = lib.load().mi355_fmha_fwd_workspace_bytes
+    limit = 4 << 20
+    for pairs in list(range(1, 40)) + list(range(40, 256, 7)):
+        for cols in (1, 4, 8, 12, 16, 24, 32):
+            for tiles in list(range(16, 64, 5)) + [64, 100, 141, 256, 257, 400, 1000]:
+                even = max(1, min((256 + pairs // 2) // pairs, (tiles + 7) // 8, 256))
+                per = -(-tiles // even)
+                even = -(-tiles // per)
+                need = wsb(pairs, cols, 1, 1, tiles * 32, tiles * 32)
+                if 65536 + pairs * even * cols * 528 <= limit:
+                    assert need <= limit, (pairs, cols, tiles, need)
+                if even == 1:
+                    assert need == 0, (pairs, cols, tiles, need)

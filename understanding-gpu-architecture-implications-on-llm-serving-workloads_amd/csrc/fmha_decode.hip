@@ -19,6 +19,7 @@
 //
 // Mask semantics are those of the prefill kernel (keys >= kv_valid_len masked; causal: key j visible to query i
 // iff j <= i + Sk - Sq).
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -485,9 +486,10 @@ bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid
     return (long)group * Sq <= 32 && Sk >= kv_valid_len && B >= 1;
 }
 
+constexpr size_t kStaticScratchBytes = size_t(4) << 20;   // see `scratch` below
 namespace dec {
 constexpr int kMaxSplits = 256;   // key ranges per (batch, kv head)
-}   // up to this many tiles per wave: <4 waves, 2 stages>
+}
 
 // How a call is cut into workgroups, and what its workspace holds: one counter per (batch, kv head), kCounterStride
 // words apart, then the partial results [workgroup][column][PART_STRIDE].
@@ -511,7 +513,12 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     if (pairs <= kMaxSplitPairs && kv_valid >= 512) {
         float best_us = 1e30f;
         const long most = (tiles + 1) / 2 < kMaxSplits ? (tiles + 1) / 2 : kMaxSplits;   // at least two tiles to a range
+        // More ranges than about one workgroup per CU of at least eight tiles each only where the partial results fit the static
+        // array (and with it the smallest buffer of a stream): such a call needs no more memory than it would with that many.
+        const long even = std::max(1L, std::min({(256 + pairs / 2) / pairs, (long)(tiles + 7) / 8, (long)kMaxSplits}));
+        const long even_tiles = (tiles + even - 1) / even, even_splits = (tiles + even_tiles - 1) / even_tiles;
         for (long s = 1; s <= most && pairs * s <= 512; ++s) {
+            if (s > even_splits && kCounterBytes + (size_t)(pairs * s * ncols) * PART_STRIDE * sizeof(float) > kStaticScratchBytes) break;
             const float range_tiles = (float)(((tiles + s - 1) / s + 3) / 4 * 4);   // the four waves walk equal pieces
             const long full = pairs * s / 256, rest = pairs * s % 256;
             const auto round_us = [&](long wgs) {
@@ -589,7 +596,6 @@ static hipError_t decode_workspace(size_t bytes, hipStream_t stream, char** out,
 // (a kernel that is aborted, overlapping calls) leaves a counter that is not zero. From then on no workgroup of that
 // (batch, kv head) draws the last ticket, O and LSE of its rows are not written and no error is reported, until the
 // process ends; mi355_fmha_fwd_ws (counters zeroed on every call) is the entry point that does not depend on history.
-constexpr size_t kStaticScratchBytes = size_t(4) << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 size_t fmha_decode_static_scratch_bytes() { return kStaticScratchBytes; }
