@@ -89,8 +89,8 @@ int mi355_hgemm(const void* A, const void* B, void* C, int M, int N, int K, int6
  * applied to the accumulators before the single rounding to fp16. Replaces `self.act_fn(self.gate_proj(x)) * self.up_proj(x)`
  * (benchmarks/flashattn-cuda/modeling_llama.py:227): two GEMMs, a SiLU kernel and a multiply kernel in the reference.
  * Layouts NN and NT; N a multiple of 32, K a multiple of 64, 16-byte aligned operands and leading dimensions. Every such
- * shape is one launch: up to 16 rows in layout NT on the split-K small-M kernel, up to 64 rows otherwise on 64x64 tiles
- * with a deep ring (both stream the weight once), more rows on the 128x128 / 256x256 tiles, all with the same epilogue.
+ * shape is one launch: up to 16 rows in layout NT on the split-K small-M kernel, otherwise on the tile shape that a cost model
+ * expects to be fastest, all with the same epilogue.
  * Other shapes (K or N off those multiples, unaligned operands, layout TN) return MI355_ERR_UNSUPPORTED and nothing is
  * launched: run mi355_hgemm on the same operands followed by mi355_silu_mul with interleave = 32.
  */
