@@ -227,6 +227,30 @@ def test_decoder_layer_prefill(lib, gpu, B, S, H, n_q, n_kv, F):
     assert ok, st
 
 
+@pytest.mark.parametrize("B,S,F", [(2, 37, 1024), (3, 1, 1000)])      # an MLP width of 1000 has no gate/up epilogue
+@pytest.mark.parametrize("cached", [False, True])
+def test_decoder_layer_positions_of_each_row_and_strided_hidden_states(lib, gpu, B, S, F, cached):
+    from llama_layer import FineKVCache, FineLlamaDecoderLayer
+    H, n_q, n_kv = 512, 4, 2
+    w = layer_weights(H, n_q, n_kv, F, seed=40)
+    layer = FineLlamaDecoderLayer({k: v.to(gpu) for k, v in w.items()}, n_q, n_kv, max_positions=256)
+    x = so.randn_fp16((B, S, H), 3)
+    xg = torch.cat((x, x), 2).to(gpu)[:, :, H:]      # rows 2 H apart
+    b = torch.arange(B)[:, None]
+    rows = torch.arange(S)[None] * (1 + b) + 50 * b   # other distances too: attention does not see a common offset
+    for pos in (rows, rows[1], rows[1:2]):           # one row of positions per sequence; one for all of them
+        cache = FineKVCache(B, S + 3, n_kv, device=gpu) if cached else None
+        out = layer(xg, pos.to(gpu), kv_cache=cache)
+        ref, k_ref, _ = so.llama_decoder_layer_ref(x, w, pos.reshape(-1, S).expand(B, S), n_q, n_kv)
+        ok, st = layer_close(out, ref)
+        assert ok, (tuple(pos.shape), st)
+        if cached:
+            assert (cache.k[:, :S].transpose(1, 2).float().cpu() - k_ref).abs().max() <= 2e-2
+    for bad in (rows[:, :, None].expand(B, S, 2), rows.repeat(2, 1)):
+        with pytest.raises((AssertionError, RuntimeError)):
+            layer(xg, bad.to(gpu))
+
+
 def test_decoder_layer_generation_steps_with_cache(lib, gpu):
     from llama_layer import FineKVCache, FineLlamaDecoderLayer
     B, S0, H, n_q, n_kv, F, steps = 2, 600, 512, 8, 2, 1024, 3
