@@ -194,3 +194,28 @@ def test_generation_step_partial_results_fit_where_256_workgroups_would(lib):
                     assert need <= limit, (pairs, cols, tiles, need)
                 if even == 1:
                     assert need == 0, (pairs, cols, tiles, need)
+
+
+def decode_plan(lib, B, Hq, Hkv, Sq, kv):
+    splits, waves = ctypes.c_int(), ctypes.c_int()
+    assert lib.load().mi355_internal_fmha_decode_plan(B, Hq, Hkv, Sq, kv, ctypes.byref(splits), ctypes.byref(waves)) == 0
+    return splits.value, waves.value
+
+
+def even_cut(pairs, tiles):
+    """Ranges of the even cut: about 256 workgroups of at least eight 32-key tiles."""
+    even = max(1, min((256 + pairs // 2) // pairs, (tiles + 7) // 8, 256))
+    return -(-tiles // -(-tiles // even))
+
+
+def test_generation_step_has_no_fewer_key_ranges_and_waves_than_its_precision_needs(lib):
+    # A wave rounds its probabilities against the maximum of its first tile; with fewer ranges or waves than the even cut on
+    # four waves the pieces get longer and the error of O against float64 grows by up to 5 %.
+    for pairs in list(range(1, 40)) + list(range(40, 256, 7)) + [300, 512, 1024]:
+        for cols in (1, 4, 8, 32):
+            for kv in (1, 32, 64, 65, 128, 300, 511, 512, 513, 700, 1000, 2208, 2336, 4500, 8191, 8192, 16384, 32768):
+                splits, waves = decode_plan(lib, pairs, cols, 1, 1, kv)
+                tiles = (kv + 31) // 32
+                assert splits >= (even_cut(pairs, tiles) if kv >= 512 and pairs < 256 else 1), (pairs, cols, kv, splits)
+                assert waves == 4 or (splits == 1 and kv <= 64), (pairs, cols, kv, waves)
+    assert decode_plan(lib, 1, 32, 8, 1, 8191) == (32, 4)      # one sequence, 8 kv heads: the even cut itself

@@ -226,6 +226,13 @@ int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V,
                         strides ? strides_from(strides) : contiguous_strides(Hq, Hkv, Sq, Sk, D), dtype, stream, variant);
 }
 
+int mi355_internal_fmha_decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves) {
+    if (B < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv != 0 || Sq < 1 || kv_valid_len < 1 || !splits || !waves)
+        return fail(MI355_ERR_BAD_ARGUMENT, "mi355_internal_fmha_decode_plan: bad argument");
+    mi355::fmha_decode_plan_of(B, Hq, Hkv, Sq, kv_valid_len, splits, waves);
+    return 0;
+}
+
 int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int layout, int dtype, int variant, void* stream) {
     return hgemm_impl("mi355_internal_hgemm_variant", dtype, A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, layout, stream, variant);

@@ -495,36 +495,52 @@ constexpr int kMaxSplits = 256;   // key ranges per (batch, kv head)
 // words apart, then the partial results [workgroup][column][PART_STRIDE].
 struct DecodePlan {
     int splits, tiles_per_split;
+    int waves;                     // of a workgroup
     long workgroups;
     size_t counter_bytes, bytes;   // bytes == 0: a single key range per (batch, kv head), no workspace
 };
+// The most key ranges the model may choose: at least two tiles each, at most 512 workgroups, the partial results within the
+// static array.
+static long finer_splits(long pairs, int tiles, int ncols) {
+    using namespace dec;
+    const long fit = (long)((kStaticScratchBytes - kCounterBytes) / (PART_STRIDE * sizeof(float))) / (pairs * ncols);
+    return std::min({(long)(tiles + 1) / 2, (long)kMaxSplits, 512 / pairs, fit});
+}
+
 static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     using namespace dec;
     const int ncols = (Hq / Hkv) * Sq;
     const int tiles = (kv_valid + TK - 1) / TK;
     const long pairs = (long)B * Hkv;
-    // The number of key ranges that is expected to be done first. A workgroup (one to a CU) takes ~3 us and, per tile, what it
-    // gets of the memory's rate: 0.32 us while up to 64 of them run, 0.38 with 128, 0.69 with all 256 (measured over
-    // 8192 keys); more ranges than one also take the merge. Below 512 keys one workgroup walks
-    // them all: no workspace is needed, and the merge would take as long as the walk. us, with as many ranges as make about 256
-    // workgroups of at least eight tiles / by this model: 8 pairs over 1000 keys 9.3 / 8.4, 52 pairs over 9777 keys (five
-    // ranges would be 260 workgroups: a second round for four of them) 66.8 / 50.4, 160 pairs over 4500 keys 80.5 / 65.0.
+    // The number of key ranges. At least about one workgroup per CU of at least eight tiles each, and more of them where that
+    // is expected to be done first; never fewer, although fewer would often be faster where that many workgroups start a second
+    // round for a few of them. A wave rounds its probabilities against the maximum of its first tile: the largest ones,
+    // which carry most of the error, are exact there, and a longer piece more often holds larger ones behind that tile
+    // (relative error of O against float64 with a half or a third of the ranges: 1.01 .. 1.05 times as large; with two to
+    // four times as many 0.91 .. 1.00). The model: a workgroup (one to a CU) takes ~3 us and, per tile, what it gets of the
+    // memory's rate: 0.32 us while up to 64 of them run, 0.38 with 128, 0.69 with all 256 (measured over 8192 keys); then
+    // the merge. Below 512 keys one workgroup walks them all: no workspace is needed, and the merge would take as long as
+    // the walk. us, with the even cut / by this rule: 8 pairs over 1000 keys 9.1 / 8.0, 52 pairs over 8191 keys (five ranges are
+    // 260 workgroups) 56.8 / 45.9, 160 pairs over 4500 keys 82.8 / 70.0.
     long splits = 1;
     if (pairs <= kMaxSplitPairs && kv_valid >= 512) {
-        float best_us = 1e30f;
-        const long most = (tiles + 1) / 2 < kMaxSplits ? (tiles + 1) / 2 : kMaxSplits;   // at least two tiles to a range
-        // More ranges than about one workgroup per CU of at least eight tiles each only where the partial results fit the static
-        // array (and with it the smallest buffer of a stream): such a call needs no more memory than it would with that many.
         const long even = std::max(1L, std::min({(256 + pairs / 2) / pairs, (long)(tiles + 7) / 8, (long)kMaxSplits}));
-        const long even_tiles = (tiles + even - 1) / even, even_splits = (tiles + even_tiles - 1) / even_tiles;
-        for (long s = 1; s <= most && pairs * s <= 512; ++s) {
-            if (s > even_splits && kCounterBytes + (size_t)(pairs * s * ncols) * PART_STRIDE * sizeof(float) > kStaticScratchBytes) break;
+        const long even_tiles = (tiles + even - 1) / even;
+        splits = (tiles + even_tiles - 1) / even_tiles;
+        const auto split_us = [&](long s) {
             const float range_tiles = (float)(((tiles + s - 1) / s + 3) / 4 * 4);   // the four waves walk equal pieces
             const long full = pairs * s / 256, rest = pairs * s % 256;
             const auto round_us = [&](long wgs) {
                 return 3.f + range_tiles * (wgs <= 64 ? .32f : wgs <= 128 ? .32f + .001f * (float)(wgs - 64) : .38f + .00242f * (float)(wgs - 128));
             };
-            const float us = (float)full * round_us(256) + (rest > 0 ? round_us(rest) : 0.f) + (s > 1 ? 2.5f + .04f * (float)s + (s > 24 ? .03f * (float)(s - 24) : 0.f) : 0.f);
+            return (float)full * round_us(256) + (rest > 0 ? round_us(rest) : 0.f) + 2.5f + .04f * (float)s + (s > 24 ? .03f * (float)(s - 24) : 0.f);
+        };
+        // More only where the partial results fit the static array (and with it the smallest buffer of a stream): such a call
+        // needs no more memory than it would with the even cut.
+        const long most = splits > 1 ? finer_splits(pairs, tiles, ncols) : 1;
+        float best_us = most > splits ? .97f * split_us(splits) : 0.f;   // (a predicted gain of less than 3 % is none)
+        for (long s = splits + 1; s <= most; ++s) {
+            const float us = split_us(s);
             if (us < best_us) {
                 best_us = us;
                 splits = s;
@@ -535,9 +551,19 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     p.tiles_per_split = (int)((tiles + splits - 1) / splits);
     p.splits = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
     p.workgroups = pairs * p.splits;
+    // Two tiles or fewer and more workgroups than CUs: two waves and 64 KiB per workgroup, so that two share a CU and one's
+    // start-up and combine hide under the other's keys (us, four / two waves, 64 keys: 512 workgroups of 4 columns 10.4 / 7.5, 1024
+    // workgroups 20.3 / 14.3). Each wave has one tile either way; beyond that, longer pieces would round coarser (see above).
+    p.waves = kv_valid <= 2 * TK && p.workgroups > 256 ? 2 : 4;
     p.counter_bytes = p.splits > 1 ? kCounterBytes : 0;
     p.bytes = p.splits > 1 ? p.counter_bytes + (size_t)p.workgroups * ncols * PART_STRIDE * sizeof(float) : 0;
     return p;
+}
+
+void fmha_decode_plan_of(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves) {
+    const DecodePlan plan = decode_plan(B, Hq, Hkv, Sq, kv_valid_len);
+    *splits = plan.splits;
+    *waves = plan.waves;
 }
 
 size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
@@ -673,14 +699,7 @@ hipError_t fmha_decode_dispatch(const T* Q, const T* K, const T* V, T* O, float*
     float* part = reinterpret_cast<float*>(wsp + plan.counter_bytes);
     unsigned* counters = reinterpret_cast<unsigned*>(wsp);
     const float scale_log2 = scale * 1.4426950408889634f;
-    // More workgroups than CUs with up to 1024 keys each: two waves and 64 KiB per workgroup, so that two share a CU and one's
-    // start-up and combine hide under the other's keys (us, four / two waves: 512 workgroups, 128 keys 13.7 / 10.1, 300
-    // keys 20.2 / 17.8, 700 keys 36.7 / 34.2; 1024 workgroups, 128 keys 23.8 / 16.6, 300 keys 35.2 / 31.0; at 1500 keys they
-    // are equal, and 8192 keys lose: 345 / 363). Above 320 keys the last round of 512 workgroups must not be much emptier
-    // than the last one of 256 would be (736 workgroups, 1000 keys: 66.4 / 70.1).
-    const long rest4 = plan.workgroups % 256, rest2 = plan.workgroups % 512;
-    const bool whole_rounds = rest2 == 0 || rest2 >= 384 || (rest4 > 0 && rest4 < 128);
-    if (plan.splits == 1 && plan.workgroups > 256 && (kv_valid <= 320 || (kv_valid <= 1024 && whole_rounds)))
+    if (plan.waves == 2)
         return launch_decode<T, 2, 2>(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits,
                                       plan.tiles_per_split, plan.workgroups, sd, stream);
     return launch_decode<T, 4, 2>(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits,

@@ -95,6 +95,8 @@ hipError_t fmha_fwd_dispatch(const void* Q, const void* K, const void* V, void* 
 
 // Split-KV path for few query rows per kv head (generation step); see fmha_decode.hip.
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len);
+// Key ranges per (batch, kv head) and waves per workgroup of that path.
+void fmha_decode_plan_of(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves);
 // Bytes of workspace a call with these sizes uses (0 when it does not take the split-KV path).
 size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len);
 // Bytes of workspace the key-range path of fmha_fwd.hip uses for a call with these sizes (0 when it does not take it), and
@@ -137,4 +139,6 @@ int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C,
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                     int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides,
                                     int dtype, int variant, void* stream);
+// how a generation step over `kv_valid_len` keys is cut: key ranges per (batch, kv head), waves per workgroup
+int mi355_internal_fmha_decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves);
 }
