@@ -251,7 +251,9 @@ int mi355_silu_mul_bf16(const void* gate_up, void* out, int64_t rows, int inter,
  * The attention forward with a workspace owned by the caller, for callers that manage all device memory themselves
  * (HIP graph capture, arena allocators). mi355_fmha_fwd_workspace_bytes returns how many bytes a call with these sizes
  * needs: on the split-KV path 64 KiB of ticket counters plus the size of its partial results (at most ~9 MiB; 0 when
- * B * Hkv is large enough for one key range per (batch, kv head)); for a chunk of queries against a long cache (see the
+ * B * Hkv is large enough for one key range per (batch, kv head), or kv_valid_len < 512), asked for so that the bytes of the
+ * longest cache of a generation loop serve its shorter ones (the exception: more than 4 MiB, of which a shorter cache may need
+ * up to a tenth more); for a chunk of queries against a long cache (see the
  * conventions above) ranges * B * Hq * Sq * 260 bytes, which the call uses if `workspace_bytes` covers them and otherwise
  * does without (it then walks all keys in one kernel; a split-KV call with too small a workspace fails); 0 for every
  * other shape (then `workspace` may be NULL). mi355_fmha_fwd_ws is mi355_fmha_fwd_strided (strides == NULL:

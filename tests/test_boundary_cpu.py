@@ -219,3 +219,21 @@ def test_generation_step_has_no_fewer_key_ranges_and_waves_than_its_precision_ne
                 assert splits >= (even_cut(pairs, tiles) if kv >= 512 and pairs < 256 else 1), (pairs, cols, kv, splits)
                 assert waves == 4 or (splits == 1 and kv <= 64), (pairs, cols, kv, waves)
     assert decode_plan(lib, 1, 32, 8, 1, 8191) == (32, 4)      # one sequence, 8 kv heads: the even cut itself
+
+
+@pytest.mark.parametrize("B,Hq,Hkv", [(1, 8, 2), (1, 32, 8), (3, 32, 8), (16, 32, 8), (20, 32, 8), (13, 16, 4), (1, 64, 8), (2, 32, 1)])
+def test_workspace_asked_for_at_the_longest_cache_serves_the_shorter_ones(lib, B, Hq, Hkv):
+    # a generation loop asks once for mi355_fmha_fwd_ws. Where the even cut of the shorter cache has no more ranges than that
+    # of the longer one, the shorter one must not need more (the even cut alone may: 32 ranges of 8 tiles, 29 of 9).
+    wsb = lib.load().mi355_fmha_fwd_workspace_bytes
+    lengths = list(range(512, 12000, 32)) + [16384, 16416, 32768]
+    need = [wsb(B, Hq, Hkv, 1, 32768, kv) for kv in lengths]
+    cuts = [even_cut(B * Hkv, (kv + 31) // 32) for kv in lengths]
+    most_need = most_cut = 0
+    for kv, n, c in zip(lengths, need, cuts):
+        assert (n > 0) == (c > 1), (kv, n, c)      # memory is asked for exactly where the even cut takes some
+        if c >= most_cut:
+            assert n >= most_need, (kv, n, most_need)
+        splits, _ = decode_plan(lib, B, Hq, Hkv, 1, kv)
+        assert n >= (65536 + B * Hkv * splits * (Hq // Hkv) * 528 if splits > 1 else 0), (kv, n, splits)
+        most_need, most_cut = max(most_need, n), max(most_cut, c)

@@ -498,6 +498,7 @@ struct DecodePlan {
     int waves;                     // of a workgroup
     long workgroups;
     size_t counter_bytes, bytes;   // bytes == 0: a single key range per (batch, kv head), no workspace
+    size_t ask_bytes;              // what a caller is asked for: as much as any cut the model may choose would take
 };
 // The most key ranges the model may choose: at least two tiles each, at most 512 workgroups, the partial results within the
 // static array.
@@ -522,7 +523,7 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     // the merge. Below 512 keys one workgroup walks them all: no workspace is needed, and the merge would take as long as
     // the walk. us, with the even cut / by this rule: 8 pairs over 1000 keys 9.1 / 8.0, 52 pairs over 8191 keys (five ranges are
     // 260 workgroups) 56.8 / 45.9, 160 pairs over 4500 keys 82.8 / 70.0.
-    long splits = 1;
+    long splits = 1, most = 1;
     if (pairs <= kMaxSplitPairs && kv_valid >= 512) {
         const long even = std::max(1L, std::min({(256 + pairs / 2) / pairs, (long)(tiles + 7) / 8, (long)kMaxSplits}));
         const long even_tiles = (tiles + even - 1) / even;
@@ -537,7 +538,7 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
         };
         // More only where the partial results fit the static array (and with it the smallest buffer of a stream): such a call
         // needs no more memory than it would with the even cut.
-        const long most = splits > 1 ? finer_splits(pairs, tiles, ncols) : 1;
+        most = splits > 1 ? std::max(splits, finer_splits(pairs, tiles, ncols)) : 1;
         float best_us = most > splits ? .97f * split_us(splits) : 0.f;   // (a predicted gain of less than 3 % is none)
         for (long s = splits + 1; s <= most; ++s) {
             const float us = split_us(s);
@@ -555,8 +556,13 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     // start-up and combine hide under the other's keys (us, four / two waves, 64 keys: 512 workgroups of 4 columns 10.4 / 7.5, 1024
     // workgroups 20.3 / 14.3). Each wave has one tile either way; beyond that, longer pieces would round coarser (see above).
     p.waves = kv_valid <= 2 * TK && p.workgroups > 256 ? 2 : 4;
+    const auto bytes_of = [&](long s) { return s > 1 ? kCounterBytes + (size_t)(pairs * s) * ncols * PART_STRIDE * sizeof(float) : 0; };
     p.counter_bytes = p.splits > 1 ? kCounterBytes : 0;
-    p.bytes = p.splits > 1 ? p.counter_bytes + (size_t)p.workgroups * ncols * PART_STRIDE * sizeof(float) : 0;
+    p.bytes = bytes_of(p.splits);
+    // The number the model chooses goes up and down as the cache grows; the most it may choose only goes up (and the even cut
+    // by less than a tenth down, where its last range is a short one). A caller who asks once, for the longest cache, has
+    // enough for the shorter ones.
+    p.ask_bytes = bytes_of(most);
     return p;
 }
 
@@ -568,7 +574,7 @@ void fmha_decode_plan_of(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* 
 
 size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
     if (!fmha_decode_applicable(B, Hq, Hkv, Sq, Sk, kv_valid_len)) return 0;
-    return decode_plan(B, Hq, Hkv, Sq, kv_valid_len).bytes;
+    return decode_plan(B, Hq, Hkv, Sq, kv_valid_len).ask_bytes;
 }
 
 // The library's own workspace: one buffer per (device, stream), allocated on first use and replaced by a larger one when

@@ -97,7 +97,7 @@ hipError_t fmha_fwd_dispatch(const void* Q, const void* K, const void* V, void* 
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len);
 // Key ranges per (batch, kv head) and waves per workgroup of that path.
 void fmha_decode_plan_of(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves);
-// Bytes of workspace a call with these sizes uses (0 when it does not take the split-KV path).
+// Bytes of workspace a caller is asked for (0 when a call with these sizes does not take the split-KV path, or has one range).
 size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len);
 // Bytes of workspace the key-range path of fmha_fwd.hip uses for a call with these sizes (0 when it does not take it), and
 // the bytes a call uses on whichever of the two paths it takes.
