@@ -703,3 +703,29 @@ def test_generation_step_over_short_caches(lib, gpu, dtype, B, Hq, Hkv, Sq, Sk, 
     assert float((o.cpu().float() - o_ref).abs().max()) <= (1.6e-2 if dtype == torch.bfloat16 else 2e-3)
     seen = torch.isfinite(lse_ref)
     assert torch.equal(torch.isfinite(lse.cpu()), seen) and float((lse.cpu() - lse_ref)[seen].abs().max()) <= 1e-3
+
+
+def test_two_threads_whose_first_generation_step_is_on_one_stream(lib, gpu):
+    # the stream has no workspace yet: whichever thread allocates it, the ticket counters are cleared in front of the first kernel
+    # that draws tickets from them, and a larger buffer that another thread asks for meanwhile has its own cleared as well
+    import threading
+    shapes = [(1, 32, 8, 2048), (8, 32, 1, 16384), (3, 16, 4, 3000)]       # 4 MiB, more than 4 MiB, 4 MiB
+    data = [[t.to(gpu) for t in so.fmha_inputs(B, Hq, Hkv, 1, Sk, seed=i)] for i, (B, Hq, Hkv, Sk) in enumerate(shapes)]
+    want = [lib.fmha_fwd(*d)[0].clone() for d in data]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        stream = torch.cuda.Stream(gpu)       # (of torch's pool: the first of these uses of a pooled stream are its first at all)
+        outs = [torch.full_like(d[0], float("nan")) for d in data]
+        gate = threading.Barrier(len(data))
+
+        def step(i):
+            with torch.cuda.stream(stream):
+                gate.wait()
+                lib.fmha_fwd(*data[i], return_lse=False, out=outs[i])
+        threads = [threading.Thread(target=step, args=(i,)) for i in range(len(data))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        stream.synchronize()
+        assert all(torch.equal(o, w) for o, w in zip(outs, want))

@@ -481,6 +481,11 @@ __global__ void fmha_decode_clear_kernel(unsigned* counters, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) counters[i] = 0u;
 }
 
+static hipError_t clear_counters(void* counters, long n, hipStream_t stream) {
+    fmha_decode_clear_kernel<<<dim3(4), dim3(256), 0, stream>>>(static_cast<unsigned*>(counters), (int)n);
+    return hipGetLastError();
+}
+
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
     const int group = Hq / Hkv;
     return (long)group * Sq <= 32 && Sk >= kv_valid_len && B >= 1;
@@ -587,22 +592,29 @@ size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int k
 // hipErrorStreamCaptureUnsupported unless an earlier call on the same stream already made the buffer large enough (run
 // the step once before capturing it, or hand in a workspace of your own). Only the calling stream's capture state can be
 // seen from here: while ANOTHER stream of the process captures in global capture mode, a first or growing call (a
-// hipMalloc) would invalidate that capture, so make those calls before any capture starts. `fresh_counters` tells the
-// caller that the buffer is new and its ticket counters still have to be set to zero (on the calling stream, in front of
-// the kernel: no synchronous fill of the whole buffer on the null stream).
-static hipError_t decode_workspace(size_t bytes, hipStream_t stream, char** out, bool* fresh_counters) {
+// hipMalloc) would invalidate that capture, so make those calls before any capture starts. The ticket
+// counters of a new buffer are set to zero here, on the calling stream, in front of whatever uses it (no synchronous fill of the
+// whole buffer on the null stream). `order` comes back holding the lock of that (device, stream): the caller keeps it until
+// its kernel is issued, so that no call of another thread on the same stream, with a buffer that has grown meanwhile or not
+// been cleared yet, comes between.
+static hipError_t decode_workspace(size_t bytes, hipStream_t stream, char** out, std::unique_lock<std::mutex>* order) {
     struct Buf {
         void* ptr = nullptr;
         size_t size = 0;
+        std::mutex order;
     };
     static std::mutex mu;
     static std::map<std::pair<int, hipStream_t>, Buf> bufs;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mu);
-    Buf& b = bufs[std::make_pair(dev, stream)];
-    *fresh_counters = false;
+    Buf* entry = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        entry = &bufs[std::make_pair(dev, stream)];   // entries stay where they are
+    }
+    Buf& b = *entry;
+    *order = std::unique_lock<std::mutex>(b.order);
     if (b.size < bytes) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         e = hipStreamIsCapturing(stream, &cap);
@@ -614,7 +626,10 @@ static hipError_t decode_workspace(size_t bytes, hipStream_t stream, char** out,
         if (e != hipSuccess) return e;
         b.ptr = fresh;   // the previous buffer, if any, stays allocated (see above)
         b.size = want;
-        *fresh_counters = true;
+        if (e = clear_counters(b.ptr, (long)(dec::kCounterBytes / sizeof(unsigned)), stream); e != hipSuccess) {
+            b.size = 0;   // counters not cleared: the next call starts over
+            return e;
+        }
     }
     *out = static_cast<char*>(b.ptr);
     return hipSuccess;
@@ -674,31 +689,24 @@ hipError_t fmha_decode_dispatch(const T* Q, const T* K, const T* V, T* O, float*
     const DecodePlan plan = decode_plan(B, Hq, Hkv, Sq, kv_valid);
     char* wsp = nullptr;
     hipError_t e = hipSuccess;
+    std::unique_lock<std::mutex> order;   // of the library's buffer, until the kernel below is issued
     if (plan.bytes > 0) {
         // Ticket counters must be zero when the kernel starts. The library's buffers and the static array are zeroed once
-        // (a fresh buffer by the fill kernel below, the static array by the loader) and every call leaves its counters at
-        // zero; a caller's memory holds anything, so its counters are zeroed on every call.
-        bool clear_counters = false;
-        long n_counters = (long)B * Hkv * kCounterStride;   // this call's counters
+        // (a fresh buffer by decode_workspace, the static array by the loader) and every call leaves its counters at
+        // zero; a caller's memory holds anything, so this call's counters are zeroed on every call.
         switch (ws.kind) {
             case FmhaWorkspace::kCaller:
                 if (ws.ptr == nullptr || ws.bytes < plan.bytes || reinterpret_cast<uintptr_t>(ws.ptr) % 16 != 0) return hipErrorInvalidValue;
                 wsp = static_cast<char*>(ws.ptr);
-                clear_counters = true;
+                e = clear_counters(wsp, (long)B * Hkv * kCounterStride, stream);
                 break;
             case FmhaWorkspace::kStatic:
                 if (plan.bytes > kStaticScratchBytes) return hipErrorOutOfMemory;   // the entry point checks first and says why
                 e = static_scratch_ptr(&wsp);
                 break;
             default:
-                e = decode_workspace(plan.bytes, stream, &wsp, &clear_counters);
-                n_counters = kCounterBytes / (long)sizeof(unsigned);   // a fresh buffer: the whole counter region, once
+                e = decode_workspace(plan.bytes, stream, &wsp, &order);
                 break;
-        }
-        if (e != hipSuccess) return e;
-        if (clear_counters) {
-            fmha_decode_clear_kernel<<<dim3(4), dim3(256), 0, stream>>>(reinterpret_cast<unsigned*>(wsp), (int)n_counters);
-            e = hipGetLastError();
         }
         if (e != hipSuccess) return e;
     }
