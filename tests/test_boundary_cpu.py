@@ -216,6 +216,9 @@ def test_generation_step_has_no_fewer_key_ranges_and_waves_than_its_precision_ne
             for kv in (1, 32, 64, 65, 128, 300, 511, 512, 513, 700, 1000, 2208, 2336, 4500, 8191, 8192, 16384, 32768):
                 splits, waves = decode_plan(lib, pairs, cols, 1, 1, kv)
                 tiles = (kv + 31) // 32
+                if splits == 0:      # the prefill kernel's
+                    assert kv < 512, (pairs, cols, kv)
+                    continue
                 assert splits >= (even_cut(pairs, tiles) if kv >= 512 and pairs < 256 else 1), (pairs, cols, kv, splits)
                 assert waves == 4 or (splits == 1 and kv <= 64), (pairs, cols, kv, waves)
     assert decode_plan(lib, 1, 32, 8, 1, 8191) == (32, 4)      # one sequence, 8 kv heads: the even cut itself
@@ -237,3 +240,13 @@ def test_workspace_asked_for_at_the_longest_cache_serves_the_shorter_ones(lib, B
         splits, _ = decode_plan(lib, B, Hq, Hkv, 1, kv)
         assert n >= (65536 + B * Hkv * splits * (Hq // Hkv) * 528 if splits > 1 else 0), (kv, n, splits)
         most_need, most_cut = max(most_need, n), max(most_cut, c)
+
+
+def test_short_caches_take_the_kernel_that_is_done_first(lib):
+    # several queries over a short cache: the prefill kernel, until its query heads need several rounds of workgroups
+    for B, Hq, Hkv, Sq, kv in ((1, 32, 8, 8, 32), (1, 32, 8, 8, 64), (8, 32, 8, 8, 511), (4, 32, 32, 32, 128), (4, 32, 32, 20, 300), (1, 64, 8, 2, 64),
+                               (32, 32, 32, 32, 511), (1, 8, 2, 5, 128)):
+        assert decode_plan(lib, B, Hq, Hkv, Sq, kv)[0] == 0, (B, Hq, Hkv, Sq, kv)
+    for B, Hq, Hkv, Sq, kv in ((1, 32, 8, 1, 300), (1, 8, 2, 1, 301), (1, 32, 32, 1, 128), (16, 32, 8, 2, 300), (64, 32, 8, 5, 64), (128, 32, 8, 8, 300),
+                               (32, 32, 32, 1, 64), (1, 32, 8, 8, 512), (4, 32, 32, 32, 700)):
+        assert decode_plan(lib, B, Hq, Hkv, Sq, kv)[0] > 0, (B, Hq, Hkv, Sq, kv)

@@ -21,6 +21,7 @@
 // iff j <= i + Sk - Sq).
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -486,9 +487,24 @@ static hipError_t clear_counters(void* counters, long n, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Few query rows per kv head: this kernel, except over a short cache where the prefill kernel is expected to be done first. It
+// walks up to 32 columns of queries side by side and combines its waves column by column, which with many columns takes
+// longer than a short walk over the keys; the prefill kernel pads every head's queries to 128 rows, but has a workgroup per
+// query head, and pays only from 256 of those on. us, prefill kernel / this one: 1 x 32/8 heads, 8 queries over 64 keys 5.6 / 11.6,
+// over 300 9.2 / 13.8; 4 x 32/32, 20 queries over 128 keys 7.1 / 10.0; 1 x 32/8, one query over 300 keys 9.1 / 7.9; 64 x 32/8,
+// one query over 300 keys 65 / 17, 5 queries 65 / 23. The model is within 4 % of the faster one on average over 24 head
+// configurations, 1 .. 32 queries and 32 .. 511 keys (0.66 of the prefill kernel's time, nowhere more than 1.09).
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
-    const int group = Hq / Hkv;
-    return (long)group * Sq <= 32 && Sk >= kv_valid_len && B >= 1;
+    const long cols = (long)(Hq / Hkv) * Sq;
+    if (cols > 32 || Sk < kv_valid_len || B < 1) return false;
+    if (kv_valid_len >= 512) return true;
+    const float tiles64 = (float)((kv_valid_len + 63) / 64), tiles32 = (float)((kv_valid_len + 31) / 32);
+    const long items = (long)B * Hq, wgs = (long)B * Hkv;
+    const float prefill_us = 4.9f + .78f * tiles64 + (float)((items + 255) / 256 - 1) * (2.4f + 1.09f * tiles64);
+    const float step_us = kv_valid_len <= 64 && wgs > 256   // two waves, two workgroups to a CU
+                              ? (float)((wgs + 511) / 512) * (2.8f + .34f * (float)cols + .0403f * (float)kv_valid_len)
+                              : (float)((wgs + 255) / 256) * (3.5f + .225f * (float)cols + 1.1f * ceilf(tiles32 / 4.f));
+    return step_us <= 1.03f * prefill_us;
 }
 
 constexpr size_t kStaticScratchBytes = size_t(4) << 20;   // see `scratch` below
@@ -573,7 +589,7 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
 
 void fmha_decode_plan_of(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves) {
     const DecodePlan plan = decode_plan(B, Hq, Hkv, Sq, kv_valid_len);
-    *splits = plan.splits;
+    *splits = fmha_decode_applicable(B, Hq, Hkv, Sq, kv_valid_len, kv_valid_len) ? plan.splits : 0;
     *waves = plan.waves;
 }
 

@@ -95,7 +95,7 @@ hipError_t fmha_fwd_dispatch(const void* Q, const void* K, const void* V, void* 
 
 // Split-KV path for few query rows per kv head (generation step); see fmha_decode.hip.
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len);
-// Key ranges per (batch, kv head) and waves per workgroup of that path.
+// Key ranges per (batch, kv head), 0 where a call does not take that path, and waves per workgroup.
 void fmha_decode_plan_of(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves);
 // Bytes of workspace a caller is asked for (0 when a call with these sizes does not take the split-KV path, or has one range).
 size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len);
@@ -139,6 +139,6 @@ int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C,
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                     int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides,
                                     int dtype, int variant, void* stream);
-// how a generation step over `kv_valid_len` keys is cut: key ranges per (batch, kv head), waves per workgroup
+// how few queries over `kv_valid_len` keys are cut: key ranges per (batch, kv head), 0 = by the prefill kernel; waves per workgroup
 int mi355_internal_fmha_decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves);
 }
