@@ -250,3 +250,23 @@ def test_short_caches_take_the_kernel_that_is_done_first(lib):
     for B, Hq, Hkv, Sq, kv in ((1, 32, 8, 1, 300), (1, 8, 2, 1, 301), (1, 32, 32, 1, 128), (16, 32, 8, 2, 300), (64, 32, 8, 5, 64), (128, 32, 8, 8, 300),
                                (32, 32, 32, 1, 64), (1, 32, 8, 8, 512), (4, 32, 32, 32, 700)):
         assert decode_plan(lib, B, Hq, Hkv, Sq, kv)[0] > 0, (B, Hq, Hkv, Sq, kv)
+
+
+@pytest.mark.parametrize("layout,few_rows,shapes", [
+    # up to 16 rows against an nn.Linear weight: the small-M kernels, which stream it fastest, also beyond a layer's widths
+    ("NT", (1, 4, 8), [(50304, 4096), (50257, 4096), (128256, 2048), (28672, 8192), (14336, 14336), (14336, 4096), (4096, 14336), (4096, 4096)]),
+    ("NT", (16,), [(50304, 4096), (32000, 4096), (28672, 4096), (28672, 8192), (14336, 4096), (4096, 14336), (8192, 8192), (4096, 4096)]),
+    # a short K, where a kernel that starts fast is done first
+    ("NT", (1, 4, 11), [(3520, 448), (4096, 384), (576, 320), (1024, 192)]), ("NN", (1, 8), [(1088, 448), (320, 384)]),
+    ("NN", (1, 16), [(14336, 4096)])])
+def test_products_of_few_rows_that_the_small_m_kernels_finish_first(lib, layout, few_rows, shapes):
+    for M in few_rows:
+        for N, K in shapes:
+            choice = lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout])
+            assert choice == 8, (M, N, K, layout, choice)
+
+
+@pytest.mark.parametrize("M,N,K,layout", [(20, 220928, 128, "NT"), (45, 258816, 128, "TN"), (64, 10240, 8192, "NN"), (12, 13494, 12872, "NT"),
+                                          (16, 50264, 4096, "NN"), (16, 28672, 4096, "NN"), (64, 14336, 4096, "NT")])
+def test_products_of_few_rows_that_the_tiles_finish_first(lib, M, N, K, layout):
+    assert lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout]) != 8

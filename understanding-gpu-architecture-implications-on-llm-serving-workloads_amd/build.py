@@ -34,7 +34,7 @@ DEVICE_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wno-inline-asm", "-Wno-unused-command-line-argument",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/hgemm_dispatch.hip", "csrc/gemm_pack.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip", "csrc/glue.hip", "csrc/capi.hip"]
+KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/hgemm_dispatch.hip", "csrc/hgemm_choice.hip", "csrc/gemm_pack.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip", "csrc/glue.hip", "csrc/capi.hip"]
 # A source listed here is compiled once per entry, each time with that entry's defines, into objects of its own (side by
 # side with the others): the GEMM source holds every tile shape for two element types and three layouts, and one
 # compiler process each cuts the time the build waits for it to a third of what one per element type takes.

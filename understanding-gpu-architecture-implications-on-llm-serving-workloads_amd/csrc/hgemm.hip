@@ -1320,20 +1320,6 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_rega_kern
     }
 }
 
-// Tiles per workgroup for the kernel above, or 0 when it does not apply: K = 4096, at most 16 rows, whole tiles, and at
-// least 192 workgroups left to keep the memory system busy. Measured on weights that come from HBM (a different weight
-// matrix on every launch), against one tile per workgroup: 16 x 14336 x 4096 24.5 -> 21.7 us with four tiles (22.1 with
-// two), 16 x 6144 x 4096 13.1 -> 11.4 (two), 16 x 28672 x 4096 43.2 -> 40.5 (four; 42.2 with two). Up to 8 rows, where
-// the activation slab is half as large to begin with: 8 x 14336 x 4096 22.3 -> 20.5 us with two tiles (21.2 with four),
-// 8 x 28672 x 4096 39.1 -> 39.4-39.9 either way, so the widest products keep one tile per workgroup there.
-static int smallm_nt_rega_tpw(int M, int n_tiles, int K, long lda, long ldb) {
-    if (M > 16 || K != 4096 || lda >= (1L << 22) || ldb >= (1L << 22)) return 0;   // lane offsets of up to 40 rows in 32 bits
-    if (M <= 8) return n_tiles % 2 == 0 && n_tiles / 2 >= 192 && n_tiles / 2 <= 512 ? 2 : 0;
-    for (int tpw : {4, 2})
-        if (n_tiles % tpw == 0 && n_tiles / tpw >= 192) return tpw;
-    return 0;
-}
-
 template <typename T, bool HALF_A, bool GATE_UP>
 static hipError_t launch_smallm_nt_rega(const T* A, const T* B, T* C, const T* R, int M, int N, long lda, long ldb, long ldc,
                                         long ldr, int n_tiles, int tpw, hipStream_t stream) {
@@ -1436,12 +1422,6 @@ static hipError_t launch_split_k(const T* A, const T* B, T* C, const T* R, int M
     return hipGetLastError();
 }
 
-enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile128x256, kTile256x128, kTile32x64, kSmallM, kDeepRing };
-struct KernelChoice {
-    int shape = kTile128x128;
-    int splits = 1;           // ranges of K
-    bool own_merge = false;   // their partial tiles are merged by a kernel of its own
-};
 // see mi355_internal_hgemm_variant
 static KernelChoice pinned_kernel(int variant) {
     KernelChoice k;
@@ -1451,104 +1431,6 @@ static KernelChoice pinned_kernel(int variant) {
     k.own_merge = (variant >> 12) != 0;
     return k;
 }
-// The kernel that is expected to finish a product first, by a model of the time of each. The constants (microseconds) were
-// fitted to ~32 000 timings of pinned kernels over 600 products (1 .. 8192 rows, 256 .. 16384 columns, K 256 .. 14336, all
-// layouts, ragged and round sizes); over those the choice takes 2.2 % longer than the best kernel on average.
-//   * A tiled kernel runs in rounds of one workgroup per CU (two for the small tiles) of `K tiles * step + fixed`. The step
-//     is set by the CU's intake of 64 bytes per cycle as much as by the matrix instructions (see the tile shapes' rings at
-//     MainCfg), and by half again (small tiles) or a fifth (256x256) where the second operand is too large to stay in the
-//     memory-side cache between calls.
-//   * Ranges of K fill the machine where the tiles of a product do not. Merged by the last workgroup of a tile: a round
-//     trip through memory, and one more of 64 KiB per range and 128x128 tile. Merged by a kernel of their own: its launch,
-//     and the partial tiles once through memory: the better one for large tiles and more than a few ranges (512 x 4096 x
-//     14336 NT, 256x128 tiles in four ranges: 72.0 us against 68.7; 128 x 4096 x 14336, 128x128 in eight: 37.7 / 34.7).
-//   * Nothing is faster than its bytes take, ~5.6 TB/s behind ~3 us.
-// Against the thresholds this replaced (us, before / after): 288 x 776 x 12160 NN 46 / 30, 42 x 520 x 4336 NN 23 / 9, 212 x
-// 9012 x 12208 TN 126 / 78, 131 x 7808 x 13952 NT 89 / 68, 8 x 640 x 13440 TN 22 / 11, 500 x 4096 x 14336 NT 84 / 69.
-struct ShapeCost {
-    int shape, bm, bn, per_cu;
-    float step, step_full, fixed;   // K tile alone on its CU, with `per_cu` workgroups there; outside the K loop
-    float uncached;                 // factor on the steps for a large second operand
-};
-// gate_up: among the shapes whose waves hold 64 columns, the gate and the up of the same outputs.
-static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles_ok, bool split_ok, bool gate_up) {
-    static const ShapeCost shapes[] = {
-        {kTile256x256, 256, 256, 1, 1.30f, 1.30f, 7.1f, 1.19f}, {kTile128x256, 128, 256, 1, .667f, .667f, 5.2f, 1.31f},
-        {kTile256x128, 256, 128, 1, .617f, .617f, 5.7f, 1.31f}, {kTile128x128, 128, 128, 1, .417f, .417f, 3.9f, 1.33f},
-        {kTileHalf, 64, 128, 1, .274f, .274f, 3.5f, 1.43f},     {kTile64x64, 64, 64, 2, .177f, .382f, 2.9f, 1.53f},
-        {kTile32x64, 32, 64, 2, .146f, .270f, 2.9f, 1.65f},     {kDeepRing, 64, 64, 1, .151f, .151f, 3.5f, 1.53f}};
-    static const int ranges[] = {2, 3, 4, 5, 6, 8, 10, 12, 16};
-    const bool nt = a_kc && b_kc;
-    const float layout = nt ? .914f : a_kc ? 1.f : 1.043f;
-    const float b_bytes = 2.f * (float)N * (float)K, bytes = b_bytes + 2.f * (float)M * ((float)K + (float)N);
-    const float floor_us = bytes / 5.6e6f + 3.1f;
-    const int ktiles = (K + 63) / 64;
-    KernelChoice best;
-    best.shape = 0;
-    float best_us = 1e30f;
-    const auto consider = [&](float us, int shape, int splits, bool own_merge) {
-        if (us >= best_us) return;
-        best_us = us;
-        best.shape = shape;
-        best.splits = splits;
-        best.own_merge = own_merge;
-    };
-    if (M <= 64 && !gate_up) {   // the small-M kernels: workgroups of 16 rows and 64 (layout NT: 16) columns, the whole of K
-        const int row_blocks = (M + 15) / 16;
-        const long wgs = (long)row_blocks * ((N + (nt ? 15 : 63)) / (nt ? 16 : 64));
-        const float k = (float)K / 64.f * (b_bytes > 20e6f ? 2.2f : 1.f);
-        if (nt) consider(fmaxf(3.8f + k * .019f * fmaxf(1.f, wgs * .004f), b_bytes * (1.f + (row_blocks - 1) * .55f) / 5.5e6f + 2.f), kSmallM, 1, false);
-        else consider(fmaxf(3.3f + k * .095f * fmaxf(1.f, wgs * .003f), b_bytes * (1.f + (row_blocks - 1) * .79f) / 6.3e6f + 3.4f), kSmallM, 1, false);
-    }
-    if (!tiles_ok) return best;   // (shape 0: none of these kernels)
-    for (const ShapeCost& c : shapes) {
-        if ((c.shape == kTile32x64 && !a_kc) || (c.shape == kDeepRing && M > 64)) continue;
-        if (gate_up && (c.shape == kTile32x64 || c.shape == kTileHalf)) continue;
-        if (c.bm > 64 && c.bm >= 2 * M) continue;   // more than half of every tile would be padding
-        const bool half_nt = c.shape == kTileHalf && nt;   // 128x64 for layout NT
-        const int bm = half_nt ? c.bn : c.bm, bn = half_nt ? c.bm : c.bn;
-        const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        const float factor = layout * (b_bytes > 20e6f ? c.uncached : 1.f);
-        const auto loop_us = [&](int splits, int per_cu) {
-            const float kt = (float)((ktiles + splits - 1) / splits), one = kt * c.step * factor + c.fixed;
-            const long wgs = tiles * splits;
-            if (per_cu == 1) return (float)((wgs + 255) / 256) * one;
-            const float two = kt * c.step_full * factor + c.fixed;
-            const long rem = wgs % 512;
-            return (float)(wgs / 512) * two + (rem > 256 ? two : rem > 0 ? one : 0.f);
-        };
-        // (unsplit, the 32x64 tiles run on a ring of eight stages, one workgroup to a CU)
-        consider(fmaxf(loop_us(1, c.shape == kTile32x64 ? 1 : c.per_cu), floor_us), c.shape, 1, false);
-        if (!split_ok || c.shape == kDeepRing || tiles > 400) continue;
-        for (const int s : ranges) {
-            if (tiles * s > 1200 || ktiles < 2 * s) break;
-            const float us = fmaxf(loop_us(s, c.per_cu), floor_us), tile_kib = (float)(bm * bn) / 256.f;
-            const float part_mb = (float)(tiles * s) * tile_kib / 1024.f;
-            if (part_mb > 64.f) break;
-            consider(us + 1.67f + s * tile_kib * (1.207f / 64.f) + part_mb * .2f, c.shape, s, false);
-            consider(us + 3.07f + part_mb * .36f, c.shape, s, true);
-        }
-    }
-    return best;
-}
-// The same, remembered for the last few products of the calling thread: going through the candidates takes the host ~0.5 us,
-// a tenth of what the smallest products take altogether.
-static KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles_ok, bool split_ok, bool gate_up = false) {
-    struct Entry {
-        int M = 0, N = 0, K = 0, flags = 0;
-        KernelChoice choice;
-    };
-    static thread_local Entry seen[64];
-    const int flags = a_kc | b_kc << 1 | tiles_ok << 2 | split_ok << 3 | gate_up << 4;
-    const uint32_t hash = ((uint32_t)M * 0x9e3779b1u) ^ ((uint32_t)N * 0x85ebca6bu) ^ ((uint32_t)K * 0xc2b2ae35u) ^ (uint32_t)flags * 0x27d4eb2fu;
-    Entry& e = seen[hash >> 26];
-    if (e.M != M || e.N != N || e.K != K || e.flags != flags) {
-        e.choice = cheapest_kernel(M, N, K, a_kc, b_kc, tiles_ok, split_ok, gate_up);
-        e.M = M; e.N = N; e.K = K; e.flags = flags;
-    }
-    return e.choice;
-}
-
 // hipErrorNotSupported: no such kernel for this layout
 template <typename T, bool A_KC, bool B_KC>
 static hipError_t run_kernel(const KernelChoice& k, const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
@@ -1627,7 +1509,8 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
     if (ab_aligned && k_ok) {
         // the tiled kernels address a tile with 32-bit byte offsets: up to 256 rows of lda (ldb) elements
         const bool tiles_ok = lda < (1L << 22) && ldb < (1L << 22);
-        KernelChoice pick = variant > 0 && (A_KC || (variant & 15) != kTile32x64) && (tiles_ok || (variant & 15) == kSmallM) ? pinned_kernel(variant) : choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, true);
+        const bool whole_lines = ldb % 64 == 0;
+        KernelChoice pick = variant > 0 && (A_KC || (variant & 15) != kTile32x64) && (tiles_ok || (variant & 15) == kSmallM) ? pinned_kernel(variant) : choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, true, whole_lines);
         for (;;) {
             const hipError_t e = run_kernel<T, A_KC, B_KC>(pick, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, c_aligned, stream);
             // no workspace to be had (the stream is being captured and has none yet): the best kernel without split-K
@@ -1636,7 +1519,7 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
                 break;
             }
             (void)hipGetLastError();
-            pick = choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, false);
+            pick = choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, false, whole_lines);
         }
     }
     dim3 grid((N + 63) / 64, (M + 63) / 64);
@@ -1660,7 +1543,7 @@ static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, in
     // More rows: the tile shape by the same model as the plain product's. On 64x64 tiles four waves lie side by side along M,
     // so that every wave holds the gate and the up columns of its rows.
 #define MI355_ARGS A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0
-    switch (variant > 0 ? variant : choose_kernel(M, N, K, A_KC, B_KC, true, false, true).shape) {
+    switch (variant > 0 ? variant : choose_kernel(M, N, K, A_KC, B_KC, true, false, ldb % 64 == 0, true).shape) {
         case kTile256x256:
             if (M % 256 == 0 && N % 256 == 0) return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 1>(MI355_ARGS, stream);
             return launch_main<T, A_KC, B_KC, 256, 256, 2, 4, 1, true>(MI355_ARGS, stream);

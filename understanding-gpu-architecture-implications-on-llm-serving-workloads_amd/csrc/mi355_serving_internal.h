@@ -41,6 +41,33 @@ template <typename T, int LAYOUT>
 hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
                                 int variant, hipStream_t stream);
 
+// The kernel of a product (hgemm_choice.hip); the shapes' numbers are those of mi355_internal_hgemm_variant below.
+enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile128x256, kTile256x128, kTile32x64, kSmallM, kDeepRing };
+struct KernelChoice {
+    int shape = kTile128x128;
+    int splits = 1;           // ranges of K
+    bool own_merge = false;   // their partial tiles are merged by a kernel of their own
+};
+// a_kc, b_kc: the operand's K index is contiguous. tiles_ok, split_ok: the tiled kernels, ranges of K may be chosen. whole_lines: the
+// second operand's rows are multiples of 128 bytes. gate_up: among the shapes whose waves hold 64 columns, the gate and the up
+// of the same outputs. shape 0: none of these kernels.
+KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles_ok, bool split_ok, bool whole_lines, bool gate_up = false);
+
+// Row tiles per workgroup of the small-M kernel that keeps the activation rows in registers (hgemm_smallm_nt_rega_kernel), or 0 when
+// it does not apply: K = 4096, at most 16 rows, whole tiles, and at
+// least 192 workgroups left to keep the memory system busy. Measured on weights that come from HBM (a different weight
+// matrix on every launch), against one tile per workgroup: 16 x 14336 x 4096 24.5 -> 21.7 us with four tiles (22.1 with
+// two), 16 x 6144 x 4096 13.1 -> 11.4 (two), 16 x 28672 x 4096 43.2 -> 40.5 (four; 42.2 with two). Up to 8 rows, where
+// the activation slab is half as large to begin with: 8 x 14336 x 4096 22.3 -> 20.5 us with two tiles (21.2 with four),
+// 8 x 28672 x 4096 39.1 -> 39.4-39.9 either way, so the widest products keep one tile per workgroup there.
+inline int smallm_nt_rega_tpw(int M, int n_tiles, int K, long lda, long ldb) {
+    if (M > 16 || K != 4096 || lda >= (1L << 22) || ldb >= (1L << 22)) return 0;   // lane offsets of up to 40 rows in 32 bits
+    if (M <= 8) return n_tiles % 2 == 0 && n_tiles / 2 >= 192 && n_tiles / 2 <= 512 ? 2 : 0;
+    for (int tpw : {4, 2})
+        if (n_tiles % tpw == 0 && n_tiles / tpw >= 192) return tpw;
+    return 0;
+}
+
 // Workspace of the split-K path: ticket counters (one per tile, at zero between launches), then `bytes` minus those for
 // partial tiles. hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: none to be had.
 constexpr size_t kSplitKCounterBytes = 16 * 1024;   // up to 4096 tiles
@@ -134,6 +161,8 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 extern "C" {
 int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int layout, int dtype, int variant, void* stream);
+// the variant that the choice by shape takes for a product of 16-byte aligned operands (ldb: row stride of the second one)
+int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout);
 int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                           int64_t ldc, int layout, int dtype, int variant, void* stream);
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
