@@ -72,10 +72,10 @@ extern "C" {
  *   layout NT  <- finegemm_13..15 (manual/gemm_13_amd.cpp:248-270, gemm_14_amd.cpp:268-290,
  *                                  gemm_15_amd.cpp:291-313)
  * lda/ldb/ldc are in elements and refer to the stored matrices (e.g. lda >= M for layout TN).
- * Any M, N, K >= 1 is accepted. The fast paths need A and B 16-byte aligned with lda and ldb multiples of 8, and
- * K % 8 == 0 unless no operand's K index is contiguous (layout TN; other operands: mi355_gemm_ws); M and N are free
- * (ragged tile edges are handled inside the kernels; an operand whose M or N index is contiguous is read in 16-byte
- * chunks, up to 7 elements into the padding that its leading dimension, a multiple of 8, leaves behind M or N). C (and
+ * Any M, N, K >= 1 is accepted. The fast paths need A and B 16-byte aligned with lda and ldb multiples of 8
+ * (other operands: mi355_gemm_ws); M, N and K are free (ragged tile edges and the end of K are handled inside the
+ * kernels; an operand is read in aligned 16-byte chunks of its rows, up to 7 elements into the padding that its leading
+ * dimension, a multiple of 8, leaves behind M, N or K; what is read there does not reach C). C (and
  * a residual) may have any row stride and alignment (global memory takes 16-byte accesses at any element; only the
  * last N % 8 columns of a row are stored element by element).
  */
@@ -111,9 +111,9 @@ int mi355_hgemm_add(const void* A, const void* B, const void* R, void* C, int M,
 /*
  * mi355_hgemm / mi355_hgemm_add (R may be NULL) for dtype MI355_DTYPE_FP16 or MI355_DTYPE_BF16, with memory of the caller for
  * aligned copies of operands the fast paths cannot read: rows that are not 16-byte aligned (a dense matrix whose row
- * length is not a multiple of 8), or K % 8 != 0 in an operand whose K index is contiguous. mi355_gemm_workspace_bytes says
- * how many bytes the copies of a call take (0: none are made). With that much `workspace` (16-byte aligned, contents
- * irrelevant before and after the call) such operands are copied first and the product runs on the fast paths (1999 x
+ * length is not a multiple of 8, a view that starts at an odd element). mi355_gemm_workspace_bytes says how many bytes the
+ * copies of a call take (0: none are made). With that much `workspace` (16-byte aligned, contents irrelevant before and
+ * after the call) such operands are copied first and the product runs on the fast paths (1999 x
  * 3001 x 2503 NN: 712 us without, 47 with); with less, or NULL, the call runs without copies, like the entry points above.
  * Calls that share a workspace must be ordered on one stream. The operators of gemm_unified pass memory of torch's
  * allocator; the reference's kernels take none of these shapes.

@@ -737,3 +737,32 @@ def test_two_threads_on_one_stream_keep_their_partial_results_apart(lib, gpu):
     for w, g in zip(want, got):
         w = w[0][0] if isinstance(w[0], tuple) else w[0]
         assert len(g) == 200 and all(torch.equal(w, x[0] if isinstance(x, tuple) else x) for x in g)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 2 + 16 * 3, 4 + 16 * 2 + 4096])
+@pytest.mark.parametrize("M,N,K", [(1, 24, 9), (16, 77, 41), (33, 200, 1003), (64, 40, 4135), (300, 264, 261), (130, 65, 318)])
+def test_k_that_ends_inside_a_chunk_of_padded_rows(lib, gpu, dtype, layout, variant, M, N, K):
+    # rows padded to multiples of 8, K no multiple of 8: no copies are asked for, the last chunk of a row whose K index is
+    # contiguous holds NaNs behind K, which the kernels replace by zeros; one rounding of the product
+    shape, splits = variant & 15, max(1, variant >> 4 & 0xff)
+    if (shape == 7 and layout == "TN") or (shape in (8, 9) and M > 64) or (K + 63) // 64 < 2 * splits and splits > 1:
+        pytest.skip("no such kernel for this product")
+    a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
+    a, b = a.to(dtype), b.to(dtype)
+    pad = lambda t: torch.cat((t, torch.full((t.shape[0], -t.shape[1] % 8), float("nan"), dtype=t.dtype)), 1).to(gpu)
+    ag, bg = pad(a), pad(b)
+    lda, ldb, lay = ag.shape[1], bg.shape[1], lib.LAYOUTS[layout]
+    assert lib.load().mi355_gemm_workspace_bytes(ag.data_ptr(), bg.data_ptr(), M, N, K, lda, ldb, lay) == 0
+    c = torch.full((M + 1, N + 5), 4.0, dtype=dtype, device=gpu)
+    assert lib.load().mi355_internal_hgemm_variant(ag.data_ptr(), bg.data_ptr(), c.data_ptr(), M, N, K, lda, ldb, N + 5, lay,
+                                                   lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, variant,
+                                                   torch.cuda.current_stream(gpu).cuda_stream) == 0
+    torch.cuda.synchronize()
+    ref = so.gemm_ref(a, b, layout)
+    # fp32 sums: the order of K additions, at most K 2^-24 of the sum of magnitudes (far below); then one rounding
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    mags = so.gemm_ref(a.abs(), b.abs(), layout)
+    assert bool(((c[:M, :N].cpu().float() - ref).abs() <= eps * ref.abs() + K * 2.0 ** -23 * mags + 2.0 ** -24).all())
+    assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())

@@ -1,5 +1,5 @@
 // Aligned copies of GEMM operands whose rows are not 16-byte aligned (a dense matrix whose row length is not a multiple of
-// 8, a view that starts at an odd element), or whose contiguous K index ends inside a 16-byte chunk. The GEMM's
+// 8, a view that starts at an odd element). The GEMM's
 // global -> LDS copies move 16 aligned bytes; without this pass such products run the bounds-checked kernel, which gathers
 // its operands element by element, one memory round trip (~600 ns) per 16 columns of K. Measured without / with the copies:
 // 1999 x 3001 x 2503 NN 712 / 47 us, 3789 x 8336 x 5632 TN 2555 / 309, 998 x 12720 x 6719 NN 4231 / 163, 2 x 13248 x 5824 TN
@@ -71,16 +71,16 @@ PackJob job_of(const void* src, void* dst, long ld, const GemmPackPlan::Operand&
 GemmPackPlan gemm_pack_plan(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
     GemmPackPlan p;
     const bool a_kc = layout != MI355_GEMM_TN, b_kc = layout == MI355_GEMM_NT;
-    const auto operand = [](const void* ptr, long ld, int rows, int cols, bool k_contiguous) {
+    const auto operand = [](const void* ptr, long ld, int rows, int cols) {
         GemmPackPlan::Operand op;
         op.cols = cols;
-        op.pack = reinterpret_cast<uintptr_t>(ptr) % 16 != 0 || ld % 8 != 0 || (k_contiguous && cols % 8 != 0);
+        op.pack = reinterpret_cast<uintptr_t>(ptr) % 16 != 0 || ld % 8 != 0;
         op.ld = op.pack ? ((long)cols + 7) / 8 * 8 : ld;
         op.bytes = op.pack ? (size_t)op.ld * rows * 2 : 0;
         return op;
     };
-    p.a = operand(A, lda, a_kc ? M : K, a_kc ? K : M, a_kc);
-    p.b = operand(B, ldb, b_kc ? N : K, b_kc ? K : N, b_kc);
+    p.a = operand(A, lda, a_kc ? M : K, a_kc ? K : M);
+    p.b = operand(B, ldb, b_kc ? N : K, b_kc ? K : N);
     // the kernels that read the copies address rows of up to 2^22 elements; chunks are counted in 32 bits
     if (p.a.ld >= (1L << 22) || p.b.ld >= (1L << 22) || p.a.bytes / 16 >= (size_t(1) << 31) || p.b.bytes / 16 >= (size_t(1) << 31))
         p.a.pack = p.b.pack = false;

@@ -21,9 +21,9 @@
 //     inside their buffer resources; every tile issues the same instructions (the copies of the last tiles run on a
 //     resource whose size is set to zero: out of range, nothing is fetched), so the waits never change and the loop has
 //     one body per stage. Per K tile and wave of the 256x256 kernel: 64 MFMAs and ~58 other instructions.
-//   * K is any multiple of 8: the tile that holds the last K % 64 columns is taken first, by the prologue, whose copies
-//     point the lanes at k >= K out of the resource's range (such a copy writes zeros to LDS); the loop is the same code
-//     for every K.
+//   * K is free: the tile that holds the last K % 64 columns is taken first, by the prologue, whose copies point the lanes at
+//     k >= K out of the resource's range (such a copy writes zeros to LDS; where K ends inside a 16-byte chunk, the prologue
+//     puts zeros behind it in LDS itself); the loop is the same code for every K.
 //   * an operand whose K index is contiguous in memory is read from LDS with ds_read_b128; an operand whose
 //     M/N index is contiguous (B in the NN case) is read with the transposing ds_read_b64_tr_b16, so no
 //     transpose pass over B is ever made.
@@ -172,6 +172,19 @@ __device__ __forceinline__ int sign_mask_scalar(int x) {
     return r;
 }
 
+// the first `left` of the 8 elements of a 16-byte chunk, zeros behind them (nothing is read where left <= 0)
+template <typename T>
+__device__ __forceinline__ half8 first_of_chunk(const T* p, int left) {
+    int4v v = {0, 0, 0, 0};
+    if (left > 0) v = *(const int4v*)p;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        if (2 * w >= left) v[w] = 0;
+        else if (2 * w + 1 == left) v[w] &= 0xffff;
+    }
+    return __builtin_bit_cast(half8, v);
+}
+
 // f(std::integral_constant<int, I>) for I = BEGIN .. END-1, unrolled at compile time
 template <int BEGIN, int END, class F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -312,7 +325,7 @@ __device__ __forceinline__ void store_wave_tile(const float4v (&acc)[TM][TN], MI
 // column blocks, at the same accumulator positions, and C has N / 2 columns.
 // R (may be null, may be C itself): a residual of C's shape added to the rounded product, `residual + proj(x)` of
 // modeling_llama.py:776,781 with the rounding of the unfused sequence (product to T, then the sum to T).
-// RAGGED: M and N need not be multiples of the tile, nor of 8. Copies of rows past the end are redirected to the last row
+// RAGGED: M and N need not be multiples of the tile, nor of 8, nor K of 8. Copies of rows past the end are redirected to the last row
 // (or, for an operand whose M/N index is contiguous, to the last 8 columns of its extent rounded up to a multiple of 8: the
 // columns between the extent and that multiple lie in the padding of the operand's rows, because its leading dimension is
 // a multiple of 8, and what they hold only reaches rows / columns of the product that are never stored), so every load
@@ -433,7 +446,7 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // K need not be a multiple of the tile depth: the last K tile, which then holds K % 64 columns (rows) of the
     // operands, is taken FIRST, by the prologue, with copies of its own (below); the loop never sees it.
     const int ktiles = (K + BK - 1) / BK;
-    const int k_first = K - (ktiles - 1) * BK;   // depth of that tile: 8 .. 64
+    const int k_first = K - (ktiles - 1) * BK;   // depth of that tile: 1 .. 64
     const long first_tile = k_first < BK ? ktiles - 1 : 0;   // position along K, in tiles, of the tile taken first
     int4v a_res = make_buffer_resource(a_base + first_tile * a_k_step);
     int4v b_res = make_buffer_resource(b_base + first_tile * b_k_step);
@@ -654,6 +667,21 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     });
     wait_vmcnt<NCOPY * (NSTAGE - 1)>();
     __syncthreads();
+    if constexpr (RAGGED && (A_KC || B_KC)) {
+        if ((k_first & 7) != 0) {   // K ends inside a 16-byte chunk of the rows: zeros for what its copy brought from behind K
+            const int chunk = k_first >> 3;
+            auto clear = [&](auto tk, MI355_LDS char* stage, int rows) {
+                using TK = decltype(tk);
+                for (int row = tid; row < rows; row += Cfg::NTHREADS) {
+                    MI355_LDS uint16_t* c = (MI355_LDS uint16_t*)(stage + row * TK::kRowBytes + ((chunk ^ TK::swz(row)) << 4));
+                    for (int e = k_first & 7; e < 8; ++e) c[e] = 0;
+                }
+            };
+            if constexpr (A_KC) clear(ATK{}, smem, BM);
+            if constexpr (B_KC) clear(BTK{}, smem + kBRegion, BN);
+            __syncthreads();
+        }
+    }
     load_frags(Sub0{}, Sub0{}, af[0], bf[0]);
 
     // One K tile in stage sc (a compile-time constant: the loop below is unrolled over the ring). Every tile issues the
@@ -997,11 +1025,12 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
     }
     if (const int k0 = ksteps * 32; k0 < K && wave == kSmallMWaves - 1) {
         // the last K % 32 rows of B (columns of A), by the last wave, whose copies have all landed: zeros behind K
+        const int a_left = K - k0 - (A_KC ? 8 * a_chunk : at_k);
         const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             *(MI355_LDS half8*)(wbase + i * 1024 + lane * 16) = k0 + 8 * i + b_row < K ? *(const half8*)(b_src + (long)(8 * i) * ldb) : zero;
-        *(MI355_LDS half8*)(wbase + 4096 + lane * 16) = k0 + (A_KC ? 8 * a_chunk : at_k) < K ? *(const half8*)a_src : zero;
+        *(MI355_LDS half8*)(wbase + 4096 + lane * 16) = A_KC ? first_of_chunk(a_src, a_left) : a_left > 0 ? *(const half8*)a_src : zero;
         wait_lgkmcnt<0>();
         k_step(wbase);
     }
@@ -1165,14 +1194,12 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
         wait_lgkmcnt<0>();  // the reads of this slot are complete before a later copy refills it
     }
     if (const int k0 = ksteps * 64; k0 < K && wave == kSmallMNtWaves - 1) {
-        // the last K % 64 columns, by the last wave, whose copies have all landed: zeros behind K (K is a multiple of 8, or
-        // the rows hold zeros up to the next one)
-        const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-        const bool in = k0 + 8 * c_chunk < K;
-        *(MI355_LDS half8*)(wbase + lane * 16) = in ? *(const half8*)b_src0 : zero;
-        *(MI355_LDS half8*)(wbase + 1024 + lane * 16) = in ? *(const half8*)b_src1 : zero;
-        *(MI355_LDS half8*)(wbase + 2048 + lane * 16) = in ? *(const half8*)a_src0 : zero;
-        if constexpr (!HALF_A) *(MI355_LDS half8*)(wbase + 3072 + lane * 16) = in ? *(const half8*)a_src1 : zero;
+        // the last K % 64 columns, by the last wave, whose copies have all landed: zeros behind K
+        const int left = K - k0 - 8 * c_chunk;
+        *(MI355_LDS half8*)(wbase + lane * 16) = first_of_chunk(b_src0, left);
+        *(MI355_LDS half8*)(wbase + 1024 + lane * 16) = first_of_chunk(b_src1, left);
+        *(MI355_LDS half8*)(wbase + 2048 + lane * 16) = first_of_chunk(a_src0, left);
+        if constexpr (!HALF_A) *(MI355_LDS half8*)(wbase + 3072 + lane * 16) = first_of_chunk(a_src1, left);
         wait_lgkmcnt<0>();
         k_step(wbase);
     }
@@ -1452,7 +1479,7 @@ static hipError_t run_kernel(const KernelChoice& k, const T* A, const T* B, T* C
             default: return hipErrorNotSupported;
         }
     }
-    const auto whole = [&](int bm, int bn) { return c_aligned && M % bm == 0 && N % bn == 0; };
+    const auto whole = [&](int bm, int bn) { return c_aligned && M % bm == 0 && N % bn == 0 && K % 8 == 0; };
     switch (k.shape) {
         case kTile256x256:
             if (whole(256, 256)) return launch_main<T, A_KC, B_KC, 256, 256, 2, 4>(MI355_ARGS, stream);
@@ -1493,20 +1520,17 @@ static hipError_t run_kernel(const KernelChoice& k, const T* A, const T* B, T* C
 
 template <typename T, bool A_KC, bool B_KC>
 static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
-                                long ldc, long ldr, int variant, bool k_zero_padded, hipStream_t stream) {
+                                long ldc, long ldr, int variant, hipStream_t stream) {
     // the copies of the fast kernels move 16 bytes into LDS: the operands' rows must be 16-byte aligned. C and the residual
     // may lie anywhere; the kernels that assume whole tiles also assume aligned rows of C (c_aligned).
     const bool ab_aligned = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0) &&
                             (lda % 8 == 0) && (ldb % 8 == 0);
     const bool c_aligned = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && (ldc % 8 == 0) &&
                            (reinterpret_cast<uintptr_t>(R) % 16 == 0) && (ldr % 8 == 0);
-    // Any K, if the rows of an operand whose K index is contiguous hold zeros from K up to the next multiple of 8 (the
-    // copies of gemm_pack.hip do, k_zero_padded) or no operand is stored that way: the copies of the other operand take
-    // single rows of K. Any N: an operand stored [K,N] is copied in 16-byte chunks of its rows, and the chunk that straddles
-    // N ends in the padding a leading dimension of a multiple of 8 leaves (what it holds only reaches columns that are
-    // never stored).
-    const bool k_ok = K % 8 == 0 || k_zero_padded || (!A_KC && !B_KC);
-    if (ab_aligned && k_ok) {
+    // Any K: where it ends inside a 16-byte chunk of a row, the kernels put zeros in the place of what follows in that chunk.
+    // Any N: an operand stored [K,N] is copied in 16-byte chunks of its rows, and the chunk that straddles N ends in the padding
+    // a leading dimension of a multiple of 8 leaves (what it holds only reaches columns that are never stored).
+    if (ab_aligned) {
         // the tiled kernels address a tile with 32-bit byte offsets: up to 256 rows of lda (ldb) elements
         const bool tiles_ok = lda < (1L << 22) && ldb < (1L << 22);
         const bool whole_lines = ldb % 64 == 0;
@@ -1562,10 +1586,10 @@ static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, in
 // MI355_HGEMM_LAYOUT select it; without them everything is instantiated here.
 template <typename T, int LAYOUT>
 hipError_t gemm_layout(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc,
-                       long ldr, int variant, bool k_zero_padded, hipStream_t stream) {
+                       long ldr, int variant, hipStream_t stream) {
     return launch_layout<T, LAYOUT != MI355_GEMM_TN, LAYOUT == MI355_GEMM_NT>(
         static_cast<const T*>(A), static_cast<const T*>(B), static_cast<T*>(C), static_cast<const T*>(R), M, N, K, lda, ldb, ldc, ldr,
-        variant, k_zero_padded, stream);
+        variant, stream);
 }
 template <typename T, int LAYOUT>
 hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
@@ -1576,7 +1600,7 @@ hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, in
 }
 #define MI355_HGEMM_INSTANTIATE(T, LAYOUT)                                                                                     \
     template hipError_t gemm_layout<T, LAYOUT>(const void*, const void*, void*, const void*, int, int, int, long, long, long,  \
-                                               long, int, bool, hipStream_t);                                                  \
+                                               long, int, hipStream_t);                                                        \
     template hipError_t gemm_silu_mul_layout<T, LAYOUT>(const void*, const void*, void*, int, int, int, long, long, long, int, hipStream_t);
 #ifdef MI355_HGEMM_T
 MI355_HGEMM_INSTANTIATE(MI355_HGEMM_T, MI355_HGEMM_LAYOUT)

@@ -69,11 +69,11 @@ size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, 
 
 template <typename T>
 static hipError_t gemm_of_type(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc,
-                               long ldr, int layout, int variant, bool k_zero_padded, hipStream_t stream) {
+                               long ldr, int layout, int variant, hipStream_t stream) {
     switch (layout) {
-        case MI355_GEMM_NN: return gemm_layout<T, MI355_GEMM_NN>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
-        case MI355_GEMM_NT: return gemm_layout<T, MI355_GEMM_NT>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
-        case MI355_GEMM_TN: return gemm_layout<T, MI355_GEMM_TN>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, variant, k_zero_padded, stream);
+        case MI355_GEMM_NN: return gemm_layout<T, MI355_GEMM_NN>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, variant, stream);
+        case MI355_GEMM_NT: return gemm_layout<T, MI355_GEMM_NT>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, variant, stream);
+        case MI355_GEMM_TN: return gemm_layout<T, MI355_GEMM_TN>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, variant, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -81,7 +81,6 @@ static hipError_t gemm_of_type(const void* A, const void* B, void* C, const void
 hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
                           long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
                           hipStream_t stream) {
-    bool k_zero_padded = false;
     if (const size_t need = workspace ? hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout) : 0; need > 0 && need <= workspace_bytes) {
         const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
         char* a_copy = static_cast<char*>(workspace);
@@ -91,10 +90,9 @@ hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, 
         if (plan.b.pack) B = b_copy;
         lda = plan.a.ld;
         ldb = plan.b.ld;
-        k_zero_padded = true;
     }
-    if (dtype == MI355_DTYPE_BF16) return gemm_of_type<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
-    return gemm_of_type<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, k_zero_padded, stream);
+    if (dtype == MI355_DTYPE_BF16) return gemm_of_type<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
+    return gemm_of_type<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
 }
 
 hipError_t hgemm_silu_mul_dispatch(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,

@@ -32,11 +32,10 @@ hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, 
                           long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
                           hipStream_t stream);
 
-// The kernels of one element type and layout (hgemm.hip, one translation unit each). k_zero_padded: rows whose K index is
-// contiguous hold zeros from K up to the next multiple of 8.
+// The kernels of one element type and layout (hgemm.hip, one translation unit each).
 template <typename T, int LAYOUT>
 hipError_t gemm_layout(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc,
-                       long ldr, int variant, bool k_zero_padded, hipStream_t stream);
+                       long ldr, int variant, hipStream_t stream);
 template <typename T, int LAYOUT>
 hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
                                 int variant, hipStream_t stream);
