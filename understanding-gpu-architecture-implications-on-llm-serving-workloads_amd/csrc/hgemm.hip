@@ -172,16 +172,11 @@ __device__ __forceinline__ int sign_mask_scalar(int x) {
     return r;
 }
 
-// the first `left` of the 8 elements of a 16-byte chunk, zeros behind them (nothing is read where left <= 0)
-template <typename T>
-__device__ __forceinline__ half8 first_of_chunk(const T* p, int left) {
-    int4v v = {0, 0, 0, 0};
-    if (left > 0) v = *(const int4v*)p;
+// the first `left` of the 8 elements of a 16-byte chunk, zeros behind them
+__device__ __forceinline__ half8 first_of_chunk(half8 chunk, int left) {
+    int4v v = __builtin_bit_cast(int4v, chunk);
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        if (2 * w >= left) v[w] = 0;
-        else if (2 * w + 1 == left) v[w] &= 0xffff;
-    }
+    for (int w = 0; w < 4; ++w) v[w] = 2 * w >= left ? 0 : 2 * w + 1 == left ? v[w] & 0xffff : v[w];
     return __builtin_bit_cast(half8, v);
 }
 
@@ -1030,7 +1025,9 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             *(MI355_LDS half8*)(wbase + i * 1024 + lane * 16) = k0 + 8 * i + b_row < K ? *(const half8*)(b_src + (long)(8 * i) * ldb) : zero;
-        *(MI355_LDS half8*)(wbase + 4096 + lane * 16) = A_KC ? first_of_chunk(a_src, a_left) : a_left > 0 ? *(const half8*)a_src : zero;
+        half8 a_chunk8 = a_left > 0 ? *(const half8*)a_src : zero;
+        if (A_KC && (K & 7) != 0) a_chunk8 = first_of_chunk(a_chunk8, a_left);
+        *(MI355_LDS half8*)(wbase + 4096 + lane * 16) = a_chunk8;
         wait_lgkmcnt<0>();
         k_step(wbase);
     }
@@ -1196,10 +1193,17 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
     if (const int k0 = ksteps * 64; k0 < K && wave == kSmallMNtWaves - 1) {
         // the last K % 64 columns, by the last wave, whose copies have all landed: zeros behind K
         const int left = K - k0 - 8 * c_chunk;
-        *(MI355_LDS half8*)(wbase + lane * 16) = first_of_chunk(b_src0, left);
-        *(MI355_LDS half8*)(wbase + 1024 + lane * 16) = first_of_chunk(b_src1, left);
-        *(MI355_LDS half8*)(wbase + 2048 + lane * 16) = first_of_chunk(a_src0, left);
-        if constexpr (!HALF_A) *(MI355_LDS half8*)(wbase + 3072 + lane * 16) = first_of_chunk(a_src1, left);
+        const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+        half8 v[HALF_A ? 3 : 4];   // (all of them in flight before the first is looked at)
+        v[0] = left > 0 ? *(const half8*)b_src0 : zero;
+        v[1] = left > 0 ? *(const half8*)b_src1 : zero;
+        v[2] = left > 0 ? *(const half8*)a_src0 : zero;
+        if constexpr (!HALF_A) v[3] = left > 0 ? *(const half8*)a_src1 : zero;
+#pragma unroll
+        for (int i = 0; i < (HALF_A ? 3 : 4); ++i) {
+            if ((K & 7) != 0) v[i] = first_of_chunk(v[i], left);
+            *(MI355_LDS half8*)(wbase + i * 1024 + lane * 16) = v[i];
+        }
         wait_lgkmcnt<0>();
         k_step(wbase);
     }
