@@ -262,11 +262,21 @@ def test_short_caches_take_the_kernel_that_is_done_first(lib):
 def test_products_of_few_rows_that_the_small_m_kernels_finish_first(lib, layout, few_rows, shapes):
     for M in few_rows:
         for N, K in shapes:
-            choice = lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout])
+            choice = lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout], None)
             assert choice == 8, (M, N, K, layout, choice)
 
 
 @pytest.mark.parametrize("M,N,K,layout", [(20, 220928, 128, "NT"), (45, 258816, 128, "TN"), (64, 10240, 8192, "NN"), (12, 13494, 12872, "NT"),
                                           (16, 50264, 4096, "NN"), (16, 28672, 4096, "NN"), (64, 14336, 4096, "NT")])
 def test_products_of_few_rows_that_the_tiles_finish_first(lib, M, N, K, layout):
-    assert lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout]) != 8
+    assert lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout], None) != 8
+
+
+def test_aligned_copies_of_large_operands_are_asked_for_only_where_they_are_repaid(lib):
+    # unaligned dense operands, bytes of the copies asked for: nothing where reading and writing a large operand takes longer than
+    # the bounds-checked kernel takes for the product
+    ask = lambda M, N, K, lay: lib.load().mi355_gemm_workspace_bytes(4096, 1 << 40, M, N, K, M if lay == "TN" else K, K if lay == "NT" else N, lib.LAYOUTS[lay])
+    for M, N, K, lay in ((1, 128257, 512, "NN"), (1, 256001, 1024, "TN"), (4, 128257, 512, "NN"), (2, 53001, 102, "NN")):
+        assert ask(M, N, K, lay) == 0, (M, N, K, lay)
+    for M, N, K, lay in ((64, 50257, 4096, "NN"), (16, 14337, 4096, "NN"), (16, 128256, 4099, "NT"), (1999, 3001, 2503, "NN"), (256, 4097, 4096, "TN")):
+        assert ask(M, N, K, lay) >= N * K * 2 * (lay != "TN" or N % 8 != 0), (M, N, K, lay)

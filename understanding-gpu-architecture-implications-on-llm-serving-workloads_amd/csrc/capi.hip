@@ -226,8 +226,9 @@ int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V,
                         strides ? strides_from(strides) : contiguous_strides(Hq, Hkv, Sq, Sk, D), dtype, stream, variant);
 }
 
-int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout) {
+int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout, float* us) {
     const mi355::KernelChoice k = mi355::choose_kernel(M, N, K, layout != MI355_GEMM_TN, layout == MI355_GEMM_NT, true, true, ldb % 64 == 0);
+    if (us != nullptr) *us = k.us;
     return k.shape + (k.splits > 1 ? 16 * k.splits : 0) + (k.own_merge ? 4096 : 0);
 }
 

@@ -60,6 +60,7 @@ static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, b
         best.shape = shape;
         best.splits = splits;
         best.own_merge = own_merge;
+        best.us = us;
     };
     if (M <= 64 && !gate_up) {   // the small-M kernels: workgroups of 16 rows and 64 (layout NT: 16) columns, the whole of K
         const int row_blocks = (M + 15) / 16;

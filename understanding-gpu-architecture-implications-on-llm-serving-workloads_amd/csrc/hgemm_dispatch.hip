@@ -1,5 +1,6 @@
 // Host side of the GEMM entry points: aligned copies of operands, the choice of the translation unit that holds the kernels
 // of an element type and layout (hgemm.hip), and the workspace of the split-K path.
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -59,12 +60,27 @@ hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, std::
     return hipSuccess;
 }
 
-// An operand with unaligned rows is worth an aligned copy from a few K steps on: below that the bounds-checked kernel is
-// done before a second launch would start.
+// Whether the copies of a plan are repaid: a launch, each copied operand read and written once, and the product on the fast
+// kernels, against the bounds-checked kernel, whose workgroups of 64 x 64 take 16 columns of K per memory round trip (0.85 us)
+// until more of them than fit wait for each other, longer with more rows and by layout. Constants fitted to 379 products with and
+// without copies (1 .. 512 rows, 64 .. 262144 columns, K 66 .. 8192): over those the rule is 0.4 % off the faster one on average,
+// copying always 7 %. us, without / with copies: 1 x 128257 x 512 NN 49 / 83, 1 x 256001 x 1024 212 / 309, 16 x 128256 x 131 19 / 26,
+// 2 x 300 x 77 4.7 / 7.9; 64 x 50257 x 4096 1071 / 236, 16 x 14337 x 4096 220 / 69, 1 x 1001 x 513 24 / 9.
+static bool copies_pay(const GemmPackPlan& plan, int M, int N, int K, int layout) {
+    const float wgs = (float)((M + 63) / 64) * (float)((N + 63) / 64), rows = (float)(M < 64 ? M : 64);
+    const float per_wg = layout == MI355_GEMM_NT ? 1.94e-4f * (1.f + .0144f * rows) : 4.04e-5f * (1.f + (layout == MI355_GEMM_TN ? .0103f : .0559f) * rows);
+    const float without_us = 2.32f + (float)K * fmaxf(.0533f, per_wg * wgs);
+    const KernelChoice fast = choose_kernel(M, N, K, layout != MI355_GEMM_TN, layout == MI355_GEMM_NT, true, true, plan.b.ld % 64 == 0);
+    return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < without_us;
+}
+
+// Below a few K steps the bounds-checked kernel is done before a second launch would start. Where the copies are not repaid the
+// product runs without them whatever memory there is; large ones are not asked for either.
 size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
     if (K <= 64) return 0;
     const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
-    return plan.a.pack || plan.b.pack ? plan.bytes() : 0;
+    if (!plan.a.pack && !plan.b.pack) return 0;
+    return plan.bytes() <= (size_t(1) << 20) || copies_pay(plan, M, N, K, layout) ? plan.bytes() : 0;
 }
 
 template <typename T>
@@ -83,13 +99,15 @@ hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, 
                           hipStream_t stream) {
     if (const size_t need = workspace ? hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout) : 0; need > 0 && need <= workspace_bytes) {
         const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
-        char* a_copy = static_cast<char*>(workspace);
-        char* b_copy = a_copy + plan.b_offset();
-        if (hipError_t e = gemm_pack_launch(plan, A, B, lda, ldb, a_copy, b_copy, stream); e != hipSuccess) return e;
-        if (plan.a.pack) A = a_copy;
-        if (plan.b.pack) B = b_copy;
-        lda = plan.a.ld;
-        ldb = plan.b.ld;
+        if (copies_pay(plan, M, N, K, layout)) {
+            char* a_copy = static_cast<char*>(workspace);
+            char* b_copy = a_copy + plan.b_offset();
+            if (hipError_t e = gemm_pack_launch(plan, A, B, lda, ldb, a_copy, b_copy, stream); e != hipSuccess) return e;
+            if (plan.a.pack) A = a_copy;
+            if (plan.b.pack) B = b_copy;
+            lda = plan.a.ld;
+            ldb = plan.b.ld;
+        }
     }
     if (dtype == MI355_DTYPE_BF16) return gemm_of_type<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
     return gemm_of_type<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);

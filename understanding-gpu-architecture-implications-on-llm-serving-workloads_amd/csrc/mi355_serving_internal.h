@@ -46,6 +46,7 @@ struct KernelChoice {
     int shape = kTile128x128;
     int splits = 1;           // ranges of K
     bool own_merge = false;   // their partial tiles are merged by a kernel of their own
+    float us = 0.f;           // expected time
 };
 // a_kc, b_kc: the operand's K index is contiguous. tiles_ok, split_ok: the tiled kernels, ranges of K may be chosen. whole_lines: the
 // second operand's rows are multiples of 128 bytes. gate_up: among the shapes whose waves hold 64 columns, the gate and the up
@@ -160,8 +161,9 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 extern "C" {
 int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int layout, int dtype, int variant, void* stream);
-// the variant that the choice by shape takes for a product of 16-byte aligned operands (ldb: row stride of the second one)
-int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout);
+// the variant that the choice by shape takes for a product of 16-byte aligned operands (ldb: row stride of the second one), and the
+// time it expects (us may be null)
+int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout, float* us);
 int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                           int64_t ldc, int layout, int dtype, int variant, void* stream);
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,

@@ -90,7 +90,7 @@ def load():
     lib.mi355_fmha_fwd_noalloc.restype = i32
     lib.mi355_internal_hgemm_variant.argtypes = [vp, vp, vp, i32, i32, i32, i64, i64, i64, i32, i32, i32, vp]
     lib.mi355_internal_hgemm_variant.restype = i32
-    lib.mi355_internal_hgemm_choice.argtypes = [i32, i32, i32, i64, i32]
+    lib.mi355_internal_hgemm_choice.argtypes = [i32, i32, i32, i64, i32, ctypes.POINTER(f32)]
     lib.mi355_internal_hgemm_choice.restype = i32
     lib.mi355_internal_hgemm_silu_mul_variant.argtypes = lib.mi355_internal_hgemm_variant.argtypes
     lib.mi355_internal_hgemm_silu_mul_variant.restype = i32

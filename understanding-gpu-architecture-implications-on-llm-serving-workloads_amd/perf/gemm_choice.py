@@ -76,7 +76,7 @@ def main():
     rows = []
     for i in range(args.products):
         M, N, K, layout = draw(rng, args.rows)
-        chosen = cdll.mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout])
+        chosen = cdll.mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout], None)
         todo = sorted(set(variants(M, N, K, layout)) | {chosen})
         best = {v: time_us(M, N, K, layout, v, 4) for v in todo}
         for _ in range(3):
