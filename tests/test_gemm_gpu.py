@@ -766,3 +766,42 @@ def test_k_that_ends_inside_a_chunk_of_padded_rows(lib, gpu, dtype, layout, vari
     mags = so.gemm_ref(a.abs(), b.abs(), layout)
     assert bool(((c[:M, :N].cpu().float() - ref).abs() <= eps * ref.abs() + K * 2.0 ** -23 * mags + 2.0 ** -24).all())
     assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())
+
+
+def test_products_of_unaligned_operands_run_when_no_memory_for_copies_is_left(lib, gpu):
+    # torch's allocator is limited to a little more than it holds: the output fits, aligned copies of the second operand
+    # (117 MB) do not. The operator, the ctypes wrapper and the decoder layer run the product without copies.
+    import gemm_unified
+    from llama_layer import FineLlamaDecoderLayer
+    M, N, K = 64, 14337, 4096
+    a, b = operands(M, N, K, "NN", seed=1, b_std=0.05)
+    ag, bg = a.to(gpu), b.to(gpu)
+    assert lib.load().mi355_gemm_workspace_bytes(ag.data_ptr(), bg.data_ptr(), M, N, K, K, N, 0) > 100 << 20
+    H, F = 2048, 16384
+    g = torch.Generator().manual_seed(2)
+    w = {n: (torch.randn(s, generator=g) * 0.02).half().to(gpu) for n, s in
+         dict(q=(2048, H), k=(512, H), v=(512, H), o=(H, 2048), gate=(F, H), up=(F, H), down=(H, F)).items()}
+    w.update(ln1=torch.ones(H, dtype=torch.float16, device=gpu), ln2=torch.ones(H, dtype=torch.float16, device=gpu))
+    layer = FineLlamaDecoderLayer(w, 16, 4, max_positions=64)
+    x = (torch.randn(1, 3, H, generator=g)).half().to(gpu)
+    want = layer(x).float()
+    odd = torch.empty(H * F + 1, dtype=torch.float16, device=gpu)      # the same weight, one element off alignment
+    odd[1:] = layer.w_d.reshape(-1)
+    layer.w_d = odd[1:].view(H, F)
+    ref = so.gemm_ref(a, b, "NN")
+    del w
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (40 << 20)) / torch.cuda.get_device_properties(gpu).total_memory)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(60 << 20, dtype=torch.uint8, device=gpu)
+        outs = [gemm_unified.ops.fine_gemm(ag, bg, 0), lib.hgemm(ag, bg, "NN")]
+        got = layer(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    torch.cuda.synchronize()
+    for c in outs:
+        ok, st = so.gemm_tolerance_ok(c.cpu(), ref, K)
+        assert ok, st
+    assert float((got.float() - want).norm() / want.norm()) < 2.0 ** -10      # one more rounding of the last product

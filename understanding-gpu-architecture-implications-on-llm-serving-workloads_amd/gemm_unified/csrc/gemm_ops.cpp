@@ -56,10 +56,17 @@ at::Tensor run_gemm(const at::Tensor& a, const at::Tensor& b, int layout, const 
     // Leading dimensions are the logical row lengths of the contiguous operands, not stride(0): torch ignores the stride of
     // a size-1 dimension when it decides contiguity, so a [1, K] operand may carry any stride(0).
     const int64_t lda = ac.size(1), ldb = bc.size(1);
-    // operands with unaligned rows: room for aligned copies, from torch's allocator (reused in the stream's order)
-    const size_t need = mi355_gemm_workspace_bytes(ac.data_ptr(), bc.data_ptr(), (int)M, (int)N, (int)K, lda, ldb, layout);
+    // operands with unaligned rows: room for aligned copies, from torch's allocator (reused in the stream's order); where there is
+    // none left the product runs without copies
+    size_t need = mi355_gemm_workspace_bytes(ac.data_ptr(), bc.data_ptr(), (int)M, (int)N, (int)K, lda, ldb, layout);
     at::Tensor ws;
-    if (need > 0) ws = at::empty({static_cast<int64_t>(need)}, a.options().dtype(at::kByte));
+    if (need > 0) {
+        try {
+            ws = at::empty({static_cast<int64_t>(need)}, a.options().dtype(at::kByte));
+        } catch (const c10::OutOfMemoryError&) {
+            need = 0;
+        }
+    }
     int rc = mi355_gemm_ws(ac.data_ptr(), bc.data_ptr(), nullptr, c.data_ptr(), (int)M, (int)N, (int)K, lda, ldb, 0, N, layout,
                            bf16 ? MI355_DTYPE_BF16 : MI355_DTYPE_FP16, need > 0 ? ws.data_ptr() : nullptr, need, stream);
     TORCH_CHECK(rc == 0, name, ": ", mi355_last_error(), " (code ", rc, ")");

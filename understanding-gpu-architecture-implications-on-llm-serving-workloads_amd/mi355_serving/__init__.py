@@ -160,11 +160,16 @@ def hgemm(a, b, layout="NN", out=None, residual=None, variant=0):
         _check(load().mi355_internal_hgemm_variant(_ptr(a), _ptr(b), _ptr(out), M, N, K, lda, ldb, max(out.stride(0), N), lay,
                                                    dtype, int(variant), stream))
         return out
-    # operands with unaligned rows (or a contiguous K that is not a multiple of 8): room for aligned copies of them
+    # operands with unaligned rows: room for aligned copies of them, if there is any
     need = 0
     if (lda | ldb) & 7 or (_ptr(a) | _ptr(b)) & 15:
         need = load().mi355_gemm_workspace_bytes(_ptr(a), _ptr(b), M, N, K, lda, ldb, lay)
-    ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+    ws = None
+    if need:
+        try:
+            ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+        except torch.OutOfMemoryError:
+            need = 0
     _check(load().mi355_gemm_ws(_ptr(a), _ptr(b), _ptr(residual), _ptr(out), M, N, K, lda, ldb,
                                 max(residual.stride(0), N) if residual is not None else 0, max(out.stride(0), N), lay, dtype,
                                 _ptr(ws), need, stream))

@@ -38,9 +38,15 @@ struct Events {   // the pair of events around the attention block when it is ti
 // C = A W^T (+ R) for activations [M, K] and an nn.Linear weight [N, K], both with rows side by side
 void linear(const void* a, const at::Tensor& w, const void* r, void* c, int64_t M, int dtype, hipStream_t stream) {
     const int64_t N = w.size(0), K = w.size(1);
-    const size_t need = mi355_gemm_workspace_bytes(a, w.data_ptr(), (int)M, (int)N, (int)K, K, K, MI355_GEMM_NT);
+    size_t need = mi355_gemm_workspace_bytes(a, w.data_ptr(), (int)M, (int)N, (int)K, K, K, MI355_GEMM_NT);
     at::Tensor ws;
-    if (need > 0) ws = at::empty({static_cast<int64_t>(need)}, w.options().dtype(at::kByte));
+    if (need > 0) {
+        try {
+            ws = at::empty({static_cast<int64_t>(need)}, w.options().dtype(at::kByte));
+        } catch (const c10::OutOfMemoryError&) {
+            need = 0;   // the product runs without aligned copies
+        }
+    }
     check(mi355_gemm_ws(a, w.data_ptr(), r, c, (int)M, (int)N, (int)K, K, K, N, N, MI355_GEMM_NT, dtype,
                         need > 0 ? ws.data_ptr() : nullptr, need, stream), "mi355_gemm_ws");
 }
