@@ -805,3 +805,22 @@ def test_products_of_unaligned_operands_run_when_no_memory_for_copies_is_left(li
         ok, st = so.gemm_tolerance_ok(c.cpu(), ref, K)
         assert ok, st
     assert float((got.float() - want).norm() / want.norm()) < 2.0 ** -10      # one more rounding of the last product
+
+
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("K,splits", [(40, 3), (64, 2), (130, 16), (200, 255)])
+@pytest.mark.parametrize("shape,own_merge", [(2, False), (4, True), (1, False)])
+def test_more_ranges_pinned_than_k_has_tiles(lib, gpu, layout, K, splits, shape, own_merge):
+    # as many ranges as there are K tiles, and none that starts behind K
+    M, N = 70, 136
+    a, b = operands(M, N, K, layout, seed=K, b_std=0.05)
+    c = torch.full((M, N), 4.0, dtype=torch.float16, device=gpu)
+    ag = torch.full((a.shape[0], (a.shape[1] + 7) // 8 * 8), float("nan"), dtype=torch.float16, device=gpu)
+    ag[:, :a.shape[1]] = a.to(gpu)
+    bg = torch.full((b.shape[0], (b.shape[1] + 7) // 8 * 8), float("nan"), dtype=torch.float16, device=gpu)
+    bg[:, :b.shape[1]] = b.to(gpu)
+    assert lib.load().mi355_internal_hgemm_variant(ag.data_ptr(), bg.data_ptr(), c.data_ptr(), M, N, K, ag.shape[1], bg.shape[1], N, lib.LAYOUTS[layout],
+                                                   0, shape + 16 * splits + 4096 * own_merge, torch.cuda.current_stream(gpu).cuda_stream) == 0
+    torch.cuda.synchronize()
+    ok, st = so.gemm_tolerance_ok(c.cpu(), so.gemm_ref(a, b, layout), K)
+    assert ok, st

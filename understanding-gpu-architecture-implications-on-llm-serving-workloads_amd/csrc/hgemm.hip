@@ -32,7 +32,7 @@
 //     The MFMA is issued with the B fragment as first operand, i.e. it produces the transposed block, so a
 //     lane ends up with 4 consecutive N of one row of C; the epilogue parks the sub-tile in LDS and stores whole
 //     128-byte lines.
-#include <cmath>
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 #include "mi355_common.h"
@@ -1454,10 +1454,10 @@ static hipError_t launch_split_k(const T* A, const T* B, T* C, const T* R, int M
 }
 
 // see mi355_internal_hgemm_variant
-static KernelChoice pinned_kernel(int variant) {
+static KernelChoice pinned_kernel(int variant, int K) {
     KernelChoice k;
     k.shape = variant & 15;
-    k.splits = (variant >> 4) & 0xff;
+    k.splits = std::min((variant >> 4) & 0xff, (K + 63) / 64);   // a range is at least one K tile: an empty one would copy a whole tile from behind K
     if (k.splits < 1) k.splits = 1;
     k.own_merge = (variant >> 12) != 0;
     return k;
@@ -1538,7 +1538,7 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
         // the tiled kernels address a tile with 32-bit byte offsets: up to 256 rows of lda (ldb) elements
         const bool tiles_ok = lda < (1L << 22) && ldb < (1L << 22);
         const bool whole_lines = ldb % 64 == 0;
-        KernelChoice pick = variant > 0 && (A_KC || (variant & 15) != kTile32x64) && (tiles_ok || (variant & 15) == kSmallM) ? pinned_kernel(variant) : choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, true, whole_lines);
+        KernelChoice pick = variant > 0 && (A_KC || (variant & 15) != kTile32x64) && (tiles_ok || (variant & 15) == kSmallM) ? pinned_kernel(variant, K) : choose_kernel(M, N, K, A_KC, B_KC, tiles_ok, true, whole_lines);
         for (;;) {
             const hipError_t e = run_kernel<T, A_KC, B_KC>(pick, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, c_aligned, stream);
             // no workspace to be had (the stream is being captured and has none yet): the best kernel without split-K

@@ -151,7 +151,8 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 }  // namespace mi355
 
 // Test and tuning hooks: exported from the shared library but not part of its public header. They take the kernel
-// variant as an argument (no process-wide state): variants that do not fit the shape fall back to the choice by shape.
+// variant as an argument (no process-wide state). Where a layout lacks a pinned kernel the choice by shape or the bounds-checked
+// kernel takes its place; of more ranges than K has tiles as many are taken as it has.
 //   gemm: 0 = by shape; 1 = 256x256 tiles, 2 = 128x128, 3 = 64x128 (layout NT: 128x64), 4 = 64x64 with a ring of four
 //         stages, 5 = 128x256, 6 = 256x128, 7 = 32x64 (layouts NN and NT), 8 = the small-M kernels (up to 64 rows), 9 = 64x64 with
 //         a ring of eight; shapes 1 .. 7 take s ranges of K with variant + 16 s, merged by a kernel of their own (instead of
