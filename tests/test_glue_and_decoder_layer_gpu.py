@@ -391,3 +391,29 @@ def test_bfloat16_decoder_layer_prefill_and_step(lib, gpu):
                                            round_stages=False)
     rel = float((out.float().cpu() - ref).norm() / ref.norm())
     assert rel <= 1.5e-2, rel
+
+
+def test_decoder_layer_with_a_cache_of_the_callers_own(lib, gpu):
+    # anything with `length`, `max_len`, `k`, `v` and `rows`: here keys and values token-major side by side, in a wider tensor
+    from llama_layer import FineKVCache, FineLlamaDecoderLayer
+    B, S0, H, n_q, n_kv, F = 2, 70, 512, 8, 2, 1024
+
+    class TokenMajorCache:
+        def __init__(self, max_len):
+            self.all = torch.zeros((B, max_len, 2 * n_kv + 1, 128), dtype=torch.float16, device=gpu)
+            self.k, self.v = self.all[:, :, :n_kv], self.all[:, :, n_kv:2 * n_kv]
+            self.max_len, self.length = max_len, 0
+
+        def rows(self, past, S):
+            return self.all[:, past:past + S, :2 * n_kv]
+
+    w = layer_weights(H, n_q, n_kv, F, seed=50)
+    layer = FineLlamaDecoderLayer({k: v.to(gpu) for k, v in w.items()}, n_q, n_kv, max_positions=256)
+    mine, fine = TokenMajorCache(S0 + 2), FineKVCache(B, S0 + 2, n_kv, device=gpu)
+    for t, S in enumerate((S0, 1, 1)):
+        x = so.randn_fp16((B, S, H), 60 + t).to(gpu)
+        assert torch.equal(layer(x, kv_cache=mine), layer(x, kv_cache=fine))      # the same kernels on the same values
+    assert mine.length == fine.length == S0 + 2
+    assert torch.equal(mine.k, fine.k) and torch.equal(mine.v, fine.v) and bool((mine.all[:, :, 2 * n_kv] == 0).all())
+    with pytest.raises(ValueError):
+        layer(x, kv_cache=mine)

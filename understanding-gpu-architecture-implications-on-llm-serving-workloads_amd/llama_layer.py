@@ -95,11 +95,13 @@ class FineLlamaDecoderLayer:
 
     def forward(self, hidden_states, position_ids=None, kv_cache=None, time_attention=False):
         B, S, H = hidden_states.shape
-        past, kv, first = 0, None, 0
+        past, kv, first = 0, (), 0
         if kv_cache is not None:
-            past, kv = kv_cache.length, kv_cache.kv
+            past = kv_cache.length
             if past + S > kv_cache.max_len:
                 raise ValueError("KV cache of %d tokens cannot take %d more after %d" % (kv_cache.max_len, S, past))
+            # one tensor in the layout above, or any cache with `rows`, `k` and `v` as there
+            kv = (kv_cache.kv,) if type(kv_cache) is FineKVCache else (kv_cache.rows(past, S), kv_cache.k, kv_cache.v)
         if position_ids is None:
             pos, first = self.all_positions, past   # a window of one table shared by every batch row, no kernel launched
             assert past + S <= pos.numel(), "max_positions is %d" % pos.numel()

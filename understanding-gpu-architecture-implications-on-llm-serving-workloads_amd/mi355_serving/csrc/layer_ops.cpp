@@ -12,6 +12,7 @@
 
 #include <cmath>
 #include <tuple>
+#include <vector>
 
 #include "mi355_serving.h"
 
@@ -52,13 +53,14 @@ void linear(const void* a, const at::Tensor& w, const void* r, void* c, int64_t 
 }
 
 // hidden_states [B, S, H] -> (layer output [B, S, H], milliseconds of the attention block if `timed`, else 0). `positions`:
-// int32, [S] for all batch rows or [B, S]. `kv` (or None): the cache tensor [B, 2 n_kv, max_len, 128], whose rows
-// past .. past + S - 1 are written. `gate_up_block`: 32 when w_gu alternates 32 gate rows with their 32 up rows, 0 when all
+// int32, [S] for all batch rows or [B, S]. `kv`: empty without a cache; {cache} for a tensor [B, 2 n_kv, max_len, 128], whose rows
+// past .. past + S - 1 are written; or {rows, k, v} for a cache of any layout: the [B, S, 2 n_kv, 128] view of the new tokens,
+// which are written, and the [B, past + S or more, n_kv, 128] views of all keys and values. `gate_up_block`: 32 when w_gu alternates 32 gate rows with their 32 up rows, 0 when all
 // gate rows precede all up rows.
 std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, const at::Tensor& w_qkv, const at::Tensor& w_o,
                                              const at::Tensor& w_gu, const at::Tensor& w_d, const at::Tensor& ln1, const at::Tensor& ln2,
                                              const at::Tensor& cos, const at::Tensor& sin, const at::Tensor& positions, int64_t first_position,
-                                             const c10::optional<at::Tensor>& kv, int64_t past, int64_t n_q, int64_t n_kv, double eps,
+                                             const std::vector<at::Tensor>& kv, int64_t past, int64_t n_q, int64_t n_kv, double eps,
                                              int64_t gate_up_block, bool timed) {
     constexpr int64_t D = 128;
     TORCH_CHECK(hidden_states.dim() == 3 && hidden_states.is_cuda(), "hidden_states must be a [B, S, H] GPU tensor");
@@ -123,31 +125,47 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
     linear(h, w_qkv, nullptr, qkv, rows, dtype, stream);
     // attention operands read where they lie: q in the fused projection, k and v there or in the cache (batch, head, row strides)
     const int64_t row = heads * D;
-    int64_t kv_batch = S * row, kv_head = D, kv_row = row, keys = S;
-    char *k = qkv + 2 * n_q * D, *v = k + 2 * n_kv * D;
-    if (!kv.has_value()) {
+    struct Rows {   // where a [B, tokens, heads, 128] operand lies: bytes are 2 per element
+        char* ptr;
+        int64_t batch, row, head;
+    };
+    int64_t keys = S;
+    Rows k = {qkv + 2 * n_q * D, S * row, row, D}, v = {k.ptr + 2 * n_kv * D, S * row, row, D};
+    if (kv.empty()) {
         const auto entry = bf16 ? &mi355_rope_bf16 : &mi355_rope;
         check(entry(qkv, qkv, (int)B, (int)S, (int)(n_q + n_kv), 0, (int)D, S * row, row, S * row, row, cos_p, sin_p, pos, pos_batch, n_pos, stream),
               "mi355_rope");
     } else {
-        const at::Tensor& t = *kv;
-        TORCH_CHECK(t.is_cuda() && t.device() == x.device() && t.scalar_type() == type && t.dim() == 4 && t.size(0) == B && t.size(1) == 2 * n_kv &&
-                    t.size(3) == D && t.stride(3) == 1 && past >= 0 && past + S <= t.size(2),
-                    "the KV cache must be a [B, 2 * n_kv, max_len, 128] tensor of the hidden states' type and device with room for the new tokens");
-        kv_batch = t.stride(0);
-        kv_head = t.stride(1);
-        kv_row = t.stride(2);
+        Rows fresh;   // of the new tokens, keys in front of values
         keys = past + S;
-        k = static_cast<char*>(t.data_ptr());
-        v = k + 2 * n_kv * kv_head;
+        if (kv.size() == 1) {
+            const at::Tensor& t = kv[0];
+            TORCH_CHECK(t.is_cuda() && t.device() == x.device() && t.scalar_type() == type && t.dim() == 4 && t.size(0) == B && t.size(1) == 2 * n_kv &&
+                        t.size(3) == D && t.stride(3) == 1 && past >= 0 && past + S <= t.size(2),
+                        "the KV cache must be a [B, 2 * n_kv, max_len, 128] tensor of the hidden states' type and device with room for the new tokens");
+            k = {static_cast<char*>(t.data_ptr()), t.stride(0), t.stride(2), t.stride(1)};
+            v = {k.ptr + 2 * n_kv * k.head, k.batch, k.row, k.head};
+            fresh = {k.ptr + 2 * past * k.row, k.batch, k.row, k.head};
+        } else {
+            TORCH_CHECK(kv.size() == 3 && past >= 0, "kv: nothing, the cache tensor, or (rows, k, v)");
+            const auto view = [&](const at::Tensor& t, int64_t tokens, int64_t n, const char* name) {
+                TORCH_CHECK(t.is_cuda() && t.device() == x.device() && t.scalar_type() == type && t.dim() == 4 && t.size(0) == B && t.size(1) >= tokens &&
+                            t.size(2) == n && t.size(3) == D && t.stride(3) == 1, "the KV cache's ", name, " must be a [", B, ", ", tokens, ", ", n,
+                            ", 128] view of the hidden states' type and device");
+                return Rows{static_cast<char*>(t.data_ptr()), t.stride(0), t.stride(1), t.stride(2)};
+            };
+            fresh = view(kv[0], S, 2 * n_kv, "new rows");
+            k = view(kv[1], keys, n_kv, "keys");
+            v = view(kv[2], keys, n_kv, "values");
+        }
         const auto entry = bf16 ? &mi355_rope_qkv_bf16 : &mi355_rope_qkv;
-        check(entry(qkv, k + 2 * past * kv_row, (int)B, (int)S, (int)n_q, (int)n_kv, (int)D, S * row, row, kv_batch, kv_row, kv_head, cos_p, sin_p, pos,
+        check(entry(qkv, fresh.ptr, (int)B, (int)S, (int)n_q, (int)n_kv, (int)D, S * row, row, fresh.batch, fresh.row, fresh.head, cos_p, sin_p, pos,
                     pos_batch, n_pos, stream), "mi355_rope_qkv");
     }
     {
-        const int64_t strides[12] = {S * row, D, row, kv_batch, kv_head, kv_row, kv_batch, kv_head, kv_row, S * n_q * D, D, n_q * D};
+        const int64_t strides[12] = {S * row, D, row, k.batch, k.head, k.row, v.batch, v.head, v.row, S * n_q * D, D, n_q * D};
         const auto entry = bf16 ? &mi355_fmha_fwd_bf16 : &mi355_fmha_fwd_strided;
-        check(entry(qkv, k, v, attn, nullptr, (int)B, (int)n_q, (int)n_kv, (int)S, (int)keys, (int)D, 1.0f / std::sqrt((float)D), 1, (int)keys,
+        check(entry(qkv, k.ptr, v.ptr, attn, nullptr, (int)B, (int)n_q, (int)n_kv, (int)S, (int)keys, (int)D, 1.0f / std::sqrt((float)D), 1, (int)keys,
                     strides, stream), "mi355_fmha_fwd");
     }
     linear(attn, w_o, x.data_ptr(), out.data_ptr(), rows, dtype, stream);   // x + o_proj(attn)
