@@ -139,9 +139,8 @@ def test_silu_mul(lib, gpu, rows, inter):
                                           (16, 512, 256, "NN"), (17, 1024, 512, "NT"), (48, 7168, 256, "NT"),
                                           (33, 512, 1024, "NN"), (64, 2048, 128, "NN"), (40, 96, 64, "NT"), (5, 256, 192, "NN")])
 def test_gemm_with_gate_up_epilogue(lib, gpu, M, F, K, layout):
-    # silu(x Wg^T) * (x Wu^T) from one launch on the interleaved weight (tiled shapes; up to 16 rows in layout NT on the
-    # split-K kernel, with and without the second half of the A slab; up to 64 rows otherwise on the 64x64 deep-ring tiles)
-    # or, where K is off the tiles' multiple, from the two-step fallback;
+    # silu(x Wg^T) * (x Wu^T) from one launch on the interleaved weight (up to 16 rows in layout NT on the small-M kernel, with
+    # and without the second half of the A slab, otherwise on the tile shape of the choice by shape) or, where K is off the tiles' multiple, from the two-step fallback;
     # compared with the fp32 oracle. One rounding of an fp32 value: |err| <= 2^-10 |ref| + the GEMM's accumulation slack.
     x = so.randn_fp16((M, K), 1)
     wg, wu = so.randn_fp16((F, K), 2, 0.05), so.randn_fp16((F, K), 3, 0.05)
@@ -175,6 +174,31 @@ def test_gate_up_epilogue_is_one_launch_for_every_row_count(lib, gpu):
         ref = so.silu_mul_ref(torch.cat((so.gemm_ref(x, wg, "NT"), so.gemm_ref(x, wu, "NT")), 1))
         err = (out.float().cpu() - ref).abs()
         assert bool((err <= 2.0 ** -10 * ref.abs() + 1e-3).all()), (M, float(err.max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT"])
+@pytest.mark.parametrize("variant", [1, 2, 4, 5, 6, 8, 9])      # 256x256, 128x128, 64x64, 128x256, 256x128, small-M, 64x64 with a deep ring
+@pytest.mark.parametrize("M,F,K", [(256, 256, 128), (13, 96, 192), (300, 160, 128), (130, 288, 64), (512, 128, 320)])
+def test_gate_up_epilogue_on_every_kernel_that_has_it(lib, gpu, dtype, layout, variant, M, F, K):
+    # whole and ragged tiles; the columns and rows around the output stay as they are
+    if variant == 8 and (layout == "NN" or M > 16):
+        pytest.skip("the small-M kernel has it for up to 16 rows in layout NT")
+    x, wg, wu = so.randn_fp16((M, K), 1).to(dtype), so.randn_fp16((F, K), 2, 0.05).to(dtype), so.randn_fp16((F, K), 3, 0.05).to(dtype)
+    gate, up = so.gemm_ref(x, wg, "NT"), so.gemm_ref(x, wu, "NT")
+    ref = gate / (1 + torch.exp(-gate)) * up
+    nt = layout == "NT"
+    w = lib.interleave_gate_up((wg if nt else wg.t().contiguous()).to(gpu), (wu if nt else wu.t().contiguous()).to(gpu), dim=0 if nt else 1)
+    out = torch.full((M + 1, F + 8), 3.0, dtype=dtype, device=gpu)
+    xg = x.to(gpu)
+    assert lib.load().mi355_internal_hgemm_silu_mul_variant(xg.data_ptr(), w.data_ptr(), out.data_ptr(), M, F, K, K, K if nt else 2 * F, F + 8,
+                                                            lib.LAYOUTS[layout], lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, variant, 0) == 0
+    torch.cuda.synchronize()
+    # one rounding of an fp32 value, and the sums' error carried through silu (slope below 1.1) and the product
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10
+    err = (out[:M, :F].float().cpu() - ref).abs()
+    assert bool((err <= eps * ref.abs() + 1e-3).all()), float(err.max())
+    assert bool((out[M:] == 3.0).all()) and bool((out[:, F:] == 3.0).all())
 
 
 def test_gate_up_single_row_activation_with_arbitrary_row_stride(lib, gpu):

@@ -244,6 +244,12 @@ int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, i
     return hgemm_impl("mi355_internal_hgemm_variant", dtype, A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, layout, stream, variant);
 }
 
+int mi355_internal_hgemm_add_variant(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                                     int64_t ldr, int64_t ldc, int layout, int dtype, int variant, void* stream) {
+    if (!R) return fail(MI355_ERR_BAD_ARGUMENT, "mi355_internal_hgemm_add_variant: null pointer");
+    return hgemm_impl("mi355_internal_hgemm_add_variant", dtype, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, stream, variant);
+}
+
 static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 static int rmsnorm_impl(const char* fn, int dtype, const void* x, const void* residual, void* residual_out, const void* weight, void* out, int64_t rows,

@@ -162,6 +162,9 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 extern "C" {
 int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int layout, int dtype, int variant, void* stream);
+// with a residual R (arguments as mi355_hgemm_add)
+int mi355_internal_hgemm_add_variant(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                                     int64_t ldr, int64_t ldc, int layout, int dtype, int variant, void* stream);
 // the variant that the choice by shape takes for a product of 16-byte aligned operands (ldb: row stride of the second one), and the
 // time it expects (us may be null)
 int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout, float* us);

@@ -21,7 +21,8 @@ EXPORTED_SYMBOLS = ("mi355_hgemm", "mi355_fmha_fwd", "mi355_fmha_fwd_strided", "
                     "mi355_fmha_fwd_workspace_bytes", "mi355_fmha_fwd_ws", "mi355_fmha_fwd_noalloc",
                     "mi355_last_error", "mi355_serving_version")
 # exported for tests and tuning runs, declared in csrc/mi355_serving_internal.h and not in the public header
-INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_choice", "mi355_internal_hgemm_silu_mul_variant", "mi355_internal_fmha_fwd_variant",
+INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_add_variant", "mi355_internal_hgemm_choice",
+                    "mi355_internal_hgemm_silu_mul_variant", "mi355_internal_fmha_fwd_variant",
                     "mi355_internal_fmha_decode_plan")
 
 _lib = None
@@ -90,6 +91,8 @@ def load():
     lib.mi355_fmha_fwd_noalloc.restype = i32
     lib.mi355_internal_hgemm_variant.argtypes = [vp, vp, vp, i32, i32, i32, i64, i64, i64, i32, i32, i32, vp]
     lib.mi355_internal_hgemm_variant.restype = i32
+    lib.mi355_internal_hgemm_add_variant.argtypes = [vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i64, i32, i32, i32, vp]
+    lib.mi355_internal_hgemm_add_variant.restype = i32
     lib.mi355_internal_hgemm_choice.argtypes = [i32, i32, i32, i64, i32, ctypes.POINTER(f32)]
     lib.mi355_internal_hgemm_choice.restype = i32
     lib.mi355_internal_hgemm_silu_mul_variant.argtypes = lib.mi355_internal_hgemm_variant.argtypes
