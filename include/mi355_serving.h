@@ -274,8 +274,8 @@ int mi355_fmha_fwd_ws(const void* Q, const void* K, const void* V, void* O, floa
  * counterpart in the reference. It calls no hipMalloc / hipFree or any other allocating routine: the partial results of
  * the split-KV path live in a fixed 4 MiB array in device memory that is part of the library's code object (one copy
  * per GPU the library runs on, held until the process ends; its first 64 KiB hold the ticket counters). A call whose partial results do not fit (more than about
- * 7800 = (4 MiB - 64 KiB) / 528 B (workgroup, query column) pairs; a call runs about 256 workgroups, so this means more than ~30 query
- * rows per kv head at small batch; a Llama generation step has 4) returns MI355_ERR_UNSUPPORTED and launches nothing. Every call on a GPU shares that GPU's array: calls through this entry point
+ * 7800 = (4 MiB - 64 KiB) / 528 B (workgroup, query column) pairs; a call is cut into about 256 workgroups, into up to 512 only where
+ * their results still fit, so this means more than ~30 query rows per kv head at small batch; a Llama generation step has 4) returns MI355_ERR_UNSUPPORTED and launches nothing. Every call on a GPU shares that GPU's array: calls through this entry point
  * that overlap on one GPU (different streams, or threads) race; order them on one stream. The array's ticket counters are
  * zero when the library is loaded and every completed call leaves them at zero; a call that does not complete (an aborted
  * kernel, overlapping calls) can leave one that is not, and later calls for that (batch, kv head) then write no output

@@ -1,6 +1,6 @@
 // C ABI of libmi355_serving.so (see include/mi355_serving.h): argument validation and error reporting around
-// the kernel dispatchers. Nothing here allocates device memory or synchronises (the one allocation the library ever
-// makes, the split-KV workspace of mi355_fmha_fwd*, lives in fmha_decode.hip).
+// the kernel dispatchers. Nothing here allocates device memory or synchronises (the library's workspaces, one per device and
+// stream each, are those of fmha_decode.hip, fmha_fwd.hip and hgemm_dispatch.hip).
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>

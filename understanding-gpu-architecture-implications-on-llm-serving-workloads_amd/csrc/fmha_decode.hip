@@ -5,7 +5,8 @@
 // almost the whole GPU idle and is bound by one workgroup's memory rate. Here the step is a split-KV
 // ("flash-decoding") pass in ONE launch, HBM-bound by the single read of K and V:
 //
-//   * a workgroup = (batch, kv head, key range); about one workgroup per CU. The query rows of all q heads that share
+//   * a workgroup = (batch, kv head, key range); about one workgroup per CU or, where that is expected to be done sooner, up to
+//     two rounds of them (decode_plan). The query rows of all q heads that share
 //     the kv head are packed side by side as the (up to 32) columns of the S^T = K Q^T product, so K and V are read once
 //     per kv head, not once per q head.
 //   * the waves of a workgroup cut its key range into contiguous pieces; each wave streams its piece in tiles of 32 keys

@@ -326,9 +326,10 @@ __device__ __forceinline__ void store_wave_tile(const float4v (&acc)[TM][TN], MI
 // a multiple of 8, and what they hold only reaches rows / columns of the product that are never stored), so every load
 // stays inside the matrices' rows; the epilogue stores only what exists: whole 16-byte pieces wherever a row of C starts
 // (global memory takes such an access at any element), the last N % 8 columns of a row element by element.
-// SPLIT_K: the grid's y index selects one of `splits` equal ranges of K (K a multiple of 64 * splits). A workgroup
-// stores its partial tile (fp32, each lane its own accumulators) to `part`, draws a ticket from the tile's counter, and
-// the workgroup that draws the last one adds the partial tiles of all ranges, in the order of the ranges (so the sum does
+// SPLIT_K: the grid's y index selects one of `splits` ranges of K, whole K tiles each, as equal as that allows, the last one ending
+// with K. Without counters a workgroup stores its partial tile as rows of a padded matrix per range and hgemm_merge_kernel adds them.
+// With counters it stores its partial tile (fp32, each lane its own accumulators) to `part`, draws a ticket from the tile's counter,
+// and the workgroup that draws the last one adds the partial tiles of all ranges, in the order of the ranges (so the sum does
 // not depend on which workgroup arrives last), and runs the epilogue. Ordering without a fence, as in the split-KV
 // attention kernel: the partial tiles are stored device-coherently (`sc1`), every lane waits for its stores to be
 // acknowledged (`s_waitcnt vmcnt(0)`), a workgroup barrier, then one thread draws the ticket with a relaxed device-scope
