@@ -858,3 +858,11 @@ def test_residual_behind_the_merge_of_ranges_of_k(lib, gpu, dtype, layout, shape
         torch.cuda.synchronize()
         assert torch.equal(dst[:M, :N], want)
         assert bool((dst[M:] == 4.0).all()) and bool((dst[:, N:] == 4.0).all())
+
+
+def test_a_pinned_kernel_keeps_its_residual_in_the_ctypes_wrapper(lib, gpu):
+    a, b = operands(70, 136, 200, "NT", seed=3, b_std=0.05)
+    ag, bg = a.to(gpu), b.to(gpu)
+    r = (torch.randn(70, 136, generator=torch.Generator().manual_seed(4)) * 2).half().to(gpu)
+    for variant in (2, 4 + 16 * 2 + 4096):
+        assert torch.equal(lib.hgemm(ag, bg, "NT", residual=r, variant=variant), lib.hgemm(ag, bg, "NT", variant=variant) + r)

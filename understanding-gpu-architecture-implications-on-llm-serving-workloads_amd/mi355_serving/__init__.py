@@ -159,9 +159,13 @@ def hgemm(a, b, layout="NN", out=None, residual=None, variant=0):
     if residual is not None:
         if tuple(residual.shape) != (M, N) or residual.dtype != a.dtype or residual.stride(1) != 1:
             raise ValueError("residual must be [%d, %d] %s with a contiguous last dimension" % (M, N, a.dtype))
-    elif variant:
-        _check(load().mi355_internal_hgemm_variant(_ptr(a), _ptr(b), _ptr(out), M, N, K, lda, ldb, max(out.stride(0), N), lay,
-                                                   dtype, int(variant), stream))
+    if variant:
+        tail = (lay, dtype, int(variant), stream)
+        if residual is None:
+            _check(load().mi355_internal_hgemm_variant(_ptr(a), _ptr(b), _ptr(out), M, N, K, lda, ldb, max(out.stride(0), N), *tail))
+        else:
+            _check(load().mi355_internal_hgemm_add_variant(_ptr(a), _ptr(b), _ptr(residual), _ptr(out), M, N, K, lda, ldb,
+                                                           max(residual.stride(0), N), max(out.stride(0), N), *tail))
         return out
     # operands with unaligned rows: room for aligned copies of them, if there is any
     need = 0
