@@ -866,3 +866,13 @@ def test_a_pinned_kernel_keeps_its_residual_in_the_ctypes_wrapper(lib, gpu):
     r = (torch.randn(70, 136, generator=torch.Generator().manual_seed(4)) * 2).half().to(gpu)
     for variant in (2, 4 + 16 * 2 + 4096):
         assert torch.equal(lib.hgemm(ag, bg, "NT", residual=r, variant=variant), lib.hgemm(ag, bg, "NT", variant=variant) + r)
+
+
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 192, 248, 256, 320, 384, 448, 832])
+def test_256x256_tiles_with_few_k_tiles(lib, gpu, layout, K):
+    """The 256x256 tiles' rings hold two K tiles of A and three of B: K tiles up to and beyond both, round and with a tail, whole
+    and ragged in M and N; NaN behind the operands' rows would show a tile that is read before it has landed."""
+    for M, N in ((256, 512), (300, 520)):
+        a, b = operands(M, N, K, layout, seed=M + K)
+        check(lib, gpu, a, b, layout, K, variant=1)

@@ -7,8 +7,8 @@
 // [N,K]) for 13..15.
 //
 // Main kernel: one workgroup of 8 waves computes a 256x256 tile of C, K is walked in steps of 64.
-//   * global -> LDS staging uses 16-byte direct-to-LDS copies (no VGPR bounce) into a ring of stages (two 64 KiB
-//     stages for the 256x256 tile, three for 128x128, five for 64x128 / 128x64, eight - or four, with two workgroups
+//   * global -> LDS staging uses 16-byte direct-to-LDS copies (no VGPR bounce) into a ring of stages (two of A
+//     and three of B, 32 KiB each, for the 256x256 tile, three for 128x128, five for 64x128 / 128x64, eight - or four, with two workgroups
 //     on a CU - for 64x64); every wave-instruction writes 1 KiB of contiguous LDS, the XOR swizzle is applied on the
 //     global-address side.
 //     The copies are buffer loads (scalar tile base + one 32-bit lane offset): a global load with 64-bit lane
@@ -152,13 +152,21 @@ struct MainCfg {
     static constexpr int A_BYTES = BM * BK * 2;
     static constexpr int B_BYTES = BN * BK * 2;
     static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-    // 64 KiB stages: two of them fit; the 48 KiB stages of the 128x256 tiles and the 32 KiB stages of the 128x128 tile
+    // 64 KiB stages: two of them fit, and a third one of B (below); the 48 KiB stages of the 128x256 tiles and the 32 KiB stages of the 128x128 tile
     // get a third, which gives every copy one more K tile of time to land (small problems run few tiles per workgroup and are bound by that latency). The narrow tiles
     // serve products with few rows, which are bound by the stream of the weight matrix from HBM: their ring is as deep
     // as 128 KiB of LDS allow (5 stages of 24 KiB, 8 of 16 KiB), so that a CU keeps ~50 KiB of that stream in flight.
     // STAGES > 0 sets the depth (the 64x64 tiles of small products run with four stages, two workgroups to a CU).
     static constexpr int NSTAGE = STAGES > 0 ? STAGES : STAGE_BYTES > 48 * 1024 ? 2 : STAGE_BYTES > 24 * 1024 ? 3 : STAGE_BYTES > 16 * 1024 ? 5 : 8;
-    static constexpr int LDS_BYTES = STAGE_BYTES * NSTAGE;
+    // The 256x256 tiles fill the 160 KiB: 2 x 32 KiB of A, 3 x 32 KiB of B. A copy of B then has two K tiles to land instead of
+    // one, and A's, which most workgroups find in L2, wait behind less. Where B (a weight) comes from HBM a K tile takes ~1.1 us to
+    // arrive, longer than its matrix instructions (us, 2 stages of both / 3 of B; operands from HBM): 500 x 28672 x 4096 NT
+    // gate/up 109 / 100, 500 x 6144 x 4096 92 / 77, 8192 x 4096 x 14336 717 / 666, 8192 x 28672 x 4096 gate/up 1405 / 1335, 8192^3 NN
+    // 774 / 757, NT 787 / 751, TN 772 / 772. The third stage to A instead: 104, 88, 653, 1335, 754, 749, 769. (A deeper ring does
+    // nothing for the smaller tiles, which already have two or more K tiles in flight: 128x128 tiles with four or five stages, 64x128
+    // with six, and 128x256 and 256x128 tiles with a fourth stage of either operand are within 1 % of what they are.)
+    static constexpr int NSTAGE_A = NSTAGE, NSTAGE_B = NSTAGE + (STAGE_BYTES > 48 * 1024 ? 1 : 0);
+    static constexpr int LDS_BYTES = A_BYTES * NSTAGE_A + B_BYTES * NSTAGE_B;
     static constexpr int A_INSTS = A_BYTES / (NWAVES * 1024);  // 16-byte copies per lane per K tile
     static constexpr int B_INSTS = B_BYTES / (NWAVES * 1024);
     static constexpr int FRAG_SLOTS = TM > TN ? TM : TN;
@@ -451,7 +459,7 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // A fragments: TM blocks of 16 rows; B fragments: TN blocks of 16 columns; a K tile is two 32-deep substeps.
     constexpr int NSUB = BK / 32;
     static_assert(NSUB == 2, "the pipeline below is written for two substeps per K tile");
-    // LDS layout: the NSTAGE stages of A one behind the other, then those of B. A stage index is a compile-time constant
+    // LDS layout: the stages of A one behind the other, then those of B. A stage index is a compile-time constant
     // wherever fragments are read (the K loop is unrolled over the ring), so a fragment address is a loop-invariant
     // register plus an immediate offset and the loop holds no address arithmetic. The immediate field of an LDS read
     // reaches 64 KiB: where an operand's ring is longer than that (less the largest offset inside a stage), its stages
@@ -459,8 +467,9 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     constexpr int kAImm = A_KC ? (TM - 1) * 16 * ATK::kRowBytes : 36 * ATM::kRowBytes;   // largest offset inside a stage
     constexpr int kBImm = B_KC ? (TN - 1) * 16 * BTK::kRowBytes : 36 * BTN::kRowBytes;
     constexpr int kAPerSet = (65535 - kAImm) / Cfg::A_BYTES + 1, kBPerSet = (65535 - kBImm) / Cfg::B_BYTES + 1;
-    constexpr int kASets = (Cfg::NSTAGE + kAPerSet - 1) / kAPerSet, kBSets = (Cfg::NSTAGE + kBPerSet - 1) / kBPerSet;
-    constexpr int kBRegion = Cfg::NSTAGE * Cfg::A_BYTES;
+    constexpr int NSA = Cfg::NSTAGE_A, NSB = Cfg::NSTAGE_B;
+    constexpr int kASets = (NSA + kAPerSet - 1) / kAPerSet, kBSets = (NSB + kBPerSet - 1) / kBPerSet;
+    constexpr int kBRegion = NSA * Cfg::A_BYTES;
     MI355_LDS char* a_ptr[kASets][Cfg::FRAG_SLOTS];  // K-contiguous operand: one per k-substep; M/N-contiguous: one per 16-wide block
     MI355_LDS char* b_ptr[kBSets][Cfg::FRAG_SLOTS];
 #pragma unroll
@@ -508,9 +517,9 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // fragment f of substep kk, f in the order of first use: A0, B0 .. B(TN-1), A1 .. A(TM-1)
     auto load_frag = [&](auto sc, auto kc, auto fc, V8(&afn)[TM], V8(&bfn)[TN]) {
         constexpr int f = decltype(fc)::value, kk = decltype(kc)::value;
-        constexpr int st = decltype(sc)::value;
-        constexpr int aset = st / kAPerSet, ao = (st % kAPerSet) * Cfg::A_BYTES;   // set, and stage offset inside it
-        constexpr int bset = st / kBPerSet, bo = (st % kBPerSet) * Cfg::B_BYTES;
+        constexpr int sa = decltype(sc)::value % NSA, sb = decltype(sc)::value % NSB;   // stages of that tile
+        constexpr int aset = sa / kAPerSet, ao = (sa % kAPerSet) * Cfg::A_BYTES;   // set, and stage offset inside it
+        constexpr int bset = sb / kBPerSet, bo = (sb % kBPerSet) * Cfg::B_BYTES;
         if constexpr (f == 0 || f > TN) {
             constexpr int i = f == 0 ? 0 : f - TN;
             if constexpr (A_KC) {
@@ -540,8 +549,8 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // 2 = only the load (M0 was set a slot earlier, the matrix instruction in between is the wait state M0 needs)
     auto issue_copy = [&](auto sc, auto dc, auto part) {
         constexpr int d = decltype(dc)::value, pt = decltype(part)::value;
-        constexpr int st = decltype(sc)::value;
         constexpr bool is_a = d < Cfg::A_INSTS;
+        constexpr int st = decltype(sc)::value % (is_a ? NSA : NSB);
         constexpr int e = is_a ? d : d - Cfg::A_INSTS;
         constexpr int dst = is_a ? st * Cfg::A_BYTES + e * Cfg::NWAVES * 1024 : kBRegion + st * Cfg::B_BYTES + e * Cfg::NWAVES * 1024;
         if constexpr (pt == 1) {
@@ -562,14 +571,6 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
         const uint64_t b = (((uint64_t)(uint32_t)res[1] << 32) | (uint32_t)res[0]) + (uint64_t)step;
         res[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
         res[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-    };
-    auto advance_copies = [&]() {
-        advance_base(a_res, a_k_step);
-        advance_base(b_res, b_k_step);
-    };
-    auto issue_copies = [&](auto sc) {
-        static_for<0, NCOPY>([&](auto dc) { issue_copy(sc, dc, std::integral_constant<int, 0>{}); });
-        advance_copies();
     };
     // The MFMA is issued with the B fragment as first operand, i.e. it produces the transposed block: lane l ends up
     // with C[m = l % 16][n = 4 (l / 16) .. +3] of the block, 4 consecutive columns of one row.
@@ -616,10 +617,12 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
                 if constexpr (decltype(dc)::value * kCopySpacingNum / kCopySpacingDen == g) issue_copy(sc, dc, std::integral_constant<int, 1>{});
             });
     };
-    // Ring of NSTAGE stages, tile t in stage t % NSTAGE. The prologue fills every stage; in tile kt, behind the barrier,
-    // the copies of tile kt + NSTAGE go into the stage tile kt has just left. At that barrier tile kt+1 must have
-    // landed: all but the copies of the NSTAGE-2 tiles issued after it.
-    constexpr int NSTAGE = Cfg::NSTAGE;
+    // Rings of NSA stages of A and NSB of B (NSA, or one more), tile t in stages t % NSA and t % NSB. The prologue fills every stage;
+    // in tile kt, behind the barrier, the copies of A's tile kt + NSA, then those of B's tile kt + NSB go into the stages tile kt has
+    // just left. At that barrier tile kt+1 must have landed: all but the copies issued behind A's of that tile, those of NSA - 2
+    // tiles of A and NSB - 2 of B.
+    static_assert(NSB == NSA || NSB == NSA + 1, "the order of the copies, and the wait that counts them");
+    constexpr int kUnroll = NSA == NSB ? NSA : NSA * NSB;   // tiles after which both rings are where they were
     V8 af[2][TM], bf[2][TN];
     using Sub0 = std::integral_constant<int, 0>;
     using Sub1 = std::integral_constant<int, 1>;
@@ -655,13 +658,18 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
         advance_base(a_res, k_first < BK ? -first_tile * a_k_step : a_k_step);
         advance_base(b_res, k_first < BK ? -first_tile * b_k_step : b_k_step);
     }
-    static_for<1, NSTAGE>([&](auto sc) {
-        const int records = sign_mask_scalar(decltype(sc)::value - ktiles);
+    static_for<1, NSB>([&](auto sc) {
+        constexpr int t = decltype(sc)::value;
+        const int records = sign_mask_scalar(t - ktiles);
         a_res[2] = records;
         b_res[2] = records;
-        issue_copies(sc);
+        static_for<0, NCOPY>([&](auto dc) {
+            if constexpr (t < NSA || decltype(dc)::value >= Cfg::A_INSTS) issue_copy(sc, dc, std::integral_constant<int, 0>{});
+        });
+        if constexpr (t < NSA) advance_base(a_res, a_k_step);
+        advance_base(b_res, b_k_step);
     });
-    wait_vmcnt<NCOPY * (NSTAGE - 1)>();
+    wait_vmcnt<Cfg::A_INSTS * (NSA - 1) + Cfg::B_INSTS * (NSB - 1)>();
     __syncthreads();
     if constexpr (RAGGED && (A_KC || B_KC)) {
         if ((k_first & 7) != 0) {   // K ends inside a 16-byte chunk of the rows: zeros for what its copy brought from behind K
@@ -684,25 +692,25 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // same instructions, so the count the waits rely on never changes: once no tile is left to fetch, the copies run on
     // an empty buffer (num_records = 0: out of range, nothing is fetched).
     auto tile = [&](auto sc, int kt) {
-        using Next = std::integral_constant<int, (decltype(sc)::value + 1) % NSTAGE>;
+        using Next = std::integral_constant<int, (decltype(sc)::value + 1) % kUnroll>;
         substep(af[0], bf[0], [&](auto mc) { frags_of_slot(sc, Sub1{}, mc, af[1], bf[1]); });
         // my copies of the next tile have landed and my reads of this stage are complete; after the barrier that holds
         // for every wave, so this stage may be refilled and the next one may be read
-        wait_vmcnt<NCOPY * (NSTAGE - 2)>();
+        wait_vmcnt<Cfg::A_INSTS * (NSA - 2) + Cfg::B_INSTS * (NSB - 2)>();
         __syncthreads();
-        const int records = sign_mask_scalar(kt + NSTAGE - ktiles);   // -1 while a tile is left to fetch, else 0
-        a_res[2] = records;
-        b_res[2] = records;
+        a_res[2] = sign_mask_scalar(kt + NSA - ktiles);   // -1 while a tile is left to fetch, else 0
+        b_res[2] = NSA == NSB ? a_res[2] : sign_mask_scalar(kt + NSB - ktiles);
         substep(af[1], bf[1], [&](auto mc) {
             frags_of_slot(Next{}, Sub0{}, mc, af[0], bf[0]);
-            copies_of_slot(sc, mc);   // tile kt + NSTAGE
+            copies_of_slot(sc, mc);   // tiles kt + NSA of A, kt + NSB of B
         });
-        advance_copies();
+        advance_base(a_res, a_k_step);
+        advance_base(b_res, b_k_step);
     };
     int kt = 0;
     MI355_TL(tl_w[1] = timeline::wall_clock(); tl_c[0] = timeline::shader_cycles();)
-    for (; kt < ktiles; kt += NSTAGE)
-        static_for<0, NSTAGE>([&](auto sc) {
+    for (; kt < ktiles; kt += kUnroll)
+        static_for<0, kUnroll>([&](auto sc) {
             if (kt + decltype(sc)::value < ktiles) tile(sc, kt + decltype(sc)::value);
         });
     MI355_TL(tl_w[2] = timeline::wall_clock(); tl_c[1] = timeline::shader_cycles();)
