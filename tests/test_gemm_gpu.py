@@ -876,3 +876,42 @@ def test_256x256_tiles_with_few_k_tiles(lib, gpu, layout, K):
     for M, N in ((256, 512), (300, 520)):
         a, b = operands(M, N, K, layout, seed=M + K)
         check(lib, gpu, a, b, layout, K, variant=1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("M,N,K,residual", [(4352, 4096, 64, True), (4200, 4104, 200, True), (4200, 4104, 72, False), (8448, 4352, 128, False)])
+def test_256x256_tiles_over_several_rounds(lib, gpu, dtype, layout, M, N, K, residual):
+    """More 256x256 tiles than CUs, so that a workgroup takes two or three of them: 272, 289 and 561 tiles, whole and ragged, K of
+    one to four tiles. Expected: the same kernel on row blocks of the product that are one round each, bit for bit."""
+    a, b = operands(M, N, K, layout, seed=M + K)
+    ag, bg = a.to(gpu, dtype), b.to(gpu, dtype)
+    r = torch.randn(M, N, generator=torch.Generator().manual_seed(9)).to(gpu, dtype) if residual else None
+    c = lib.hgemm(ag, bg, layout, residual=r, variant=1)
+    for i in range(0, M, 3584):
+        rows = slice(i, min(i + 3584, M))
+        part = ag[:, rows].contiguous() if layout == "TN" else ag[rows]
+        assert torch.equal(c[rows], lib.hgemm(part, bg, layout, residual=r[rows] if residual else None, variant=1))
+    ok, st = so.gemm_tolerance_ok(c[:64].cpu() if not residual else (c[:64].float() - r[:64].float()).cpu(),
+                                  so.gemm_ref(a[:, :64].contiguous() if layout == "TN" else a[:64], b, layout), K)
+    assert dtype != torch.float16 or ok, st
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT"])
+@pytest.mark.parametrize("M,F", [(4352, 2048), (4300, 2080)])
+def test_gate_up_256x256_tiles_over_several_rounds(lib, gpu, dtype, layout, M, F):
+    K, cdll, st = 192, lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).to(gpu, dtype), (torch.randn(2 * F, K, generator=g) * 0.05).to(gpu, dtype)
+    w = w if layout == "NT" else w.t().contiguous()
+    out = torch.full((2, M, F), float("nan"), device=gpu, dtype=dtype)
+    code = lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16
+    for o, step in ((out[0], M), (out[1], 3584)):
+        for i in range(0, M, step):
+            rows = x[i:i + step]
+            assert cdll.mi355_internal_hgemm_silu_mul_variant(rows.data_ptr(), w.data_ptr(), o[i:].data_ptr(), rows.shape[0], F, K, K, w.shape[1], F,
+                                                              lib.LAYOUTS[layout], code, 1, st) == 0
+    assert torch.equal(out[0], out[1]) and not out.isnan().any()
+    ref = so.silu_mul_ref(x[:64].cpu().float() @ (w if layout == "NT" else w.t()).reshape(-1, 2, 32, K).transpose(0, 1).reshape(2 * F, K).cpu().float().t())
+    assert (out[0][:64].cpu().float() - ref.float()).norm() <= (2e-3 if dtype == torch.float16 else 1.6e-2) * ref.float().norm()
