@@ -915,3 +915,16 @@ def test_gate_up_256x256_tiles_over_several_rounds(lib, gpu, dtype, layout, M, F
     assert torch.equal(out[0], out[1]) and not out.isnan().any()
     ref = so.silu_mul_ref(x[:64].cpu().float() @ (w if layout == "NT" else w.t()).reshape(-1, 2, 32, K).transpose(0, 1).reshape(2 * F, K).cpu().float().t())
     assert (out[0][:64].cpu().float() - ref.float()).norm() <= (2e-3 if dtype == torch.float16 else 1.6e-2) * ref.float().norm()
+
+
+@pytest.mark.parametrize("variant", [2, 3, 4, 7, 9])
+@pytest.mark.parametrize("M", [33, 128])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 17])
+def test_k_walked_from_different_places_on_each_xcd(lib, gpu, variant, M, tiles):
+    """nn.Linear weights under one or two rows of tiles: XCD x starts x eighths of K in, rounded to whole turns of the ring, and wraps.
+    Every number of K tiles around one and two turns of each ring (3, 4, 5 and 8 stages), round and with a tail (which starts at its end)."""
+    if variant == 9 and M > 64:
+        return
+    for K in (64 * tiles, 64 * tiles - 8):
+        a, b = operands(M, 1096, K, "NT", seed=tiles + M)
+        check(lib, gpu, a, b, "NT", K, variant=variant)

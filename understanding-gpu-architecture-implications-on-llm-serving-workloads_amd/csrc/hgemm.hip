@@ -21,6 +21,7 @@
 //     inside their buffer resources; every tile issues the same instructions (the copies of the last tiles run on a
 //     resource whose size is set to zero: out of range, nothing is fetched), so the waits never change and the loop has
 //     one body per stage. Per K tile and wave of the 256x256 kernel: 64 MFMAs and ~58 other instructions.
+//   * where workgroups share nothing but the rows of A, those of different XCDs walk K from different places (kStagger).
 //   * K is free: the tile that holds the last K % 64 columns is taken first, by the prologue, whose copies point the lanes at
 //     k >= K out of the resource's range (such a copy writes zeros to LDS; where K ends inside a 16-byte chunk, the prologue
 //     puts zeros behind it in LDS itself); the loop is the same code for every K.
@@ -464,7 +465,20 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // operands, is taken FIRST, by the prologue, with copies of its own (below); the loop never sees it.
     const int ktiles = (K + BK - 1) / BK;
     const int k_first = K - (ktiles - 1) * BK;   // depth of that tile: 1 .. 64
-    const long first_tile = k_first < BK ? ktiles - 1 : 0;   // position along K, in tiles, of the tile taken first
+    // A weight stored [N,K] under one or two rows of tiles: every workgroup streams 128-byte pieces of its own rows, a row apart,
+    // and all of them the same columns at the same time, which keeps part of the memory channels busy and the others waiting.
+    // The XCDs therefore start an eighth of K apart from each other and go on at k = 0 behind the last tile. us, in step /
+    // this: 128 x 28672 x 4096 NT 54.3 / 47.7, 64 rows 52.0 / 47.9, 32 rows 49.5 / 43.5, 33 x 50257 85.7 / 82.0, 256 rows 84.6 / 81.8,
+    // 128 x 6144 and 64 x 4096 x 14336 the same; more rows of tiles, and weights stored [K,N], whose rows lie side by side,
+    // gain nothing or lose 1-4 %.
+    constexpr bool kStagger = A_KC && B_KC && !SPLIT_K && !PERSIST && BM <= 128 && BN <= 128;
+    int before_wrap = ktiles;   // K tiles in front of the one at k = 0 that follows the last
+    if (kStagger && tiles_m <= 2 && k_first == BK) {
+        static_assert(!kStagger || Cfg::NSTAGE_A == Cfg::NSTAGE_B, "whole turns of both rings in front of the wrap");
+        const int whole = (ktiles - ktiles * (int)(blockIdx.x & 7) / 8) / Cfg::NSTAGE_A * Cfg::NSTAGE_A;
+        if (whole > 0) before_wrap = whole;
+    }
+    const long first_tile = k_first < BK ? ktiles - 1 : ktiles - before_wrap;   // position along K, in tiles, of the tile taken first
     int4v a_res, b_res;
 
     // ---- LDS fragment read offsets (bytes inside one stage) -------------------------------------------
@@ -751,10 +765,16 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
         };
         int kt = 0;
         MI355_TL(tl_w[1] = timeline::wall_clock(); tl_c[0] = timeline::shader_cycles();)
-        for (; kt < ktiles; kt += kUnroll)
-            static_for<0, kUnroll>([&](auto sc) {
-                if (kt + decltype(sc)::value < ktiles) tile(sc, kt + decltype(sc)::value);
-            });
+        // (the copies run NSA tiles ahead: they go back to k = 0 when the tile NSA in front of the wrap is next)
+        for (int stop = before_wrap < ktiles ? before_wrap - NSA : ktiles;; stop = ktiles) {
+            for (; kt < stop; kt += kUnroll)
+                static_for<0, kUnroll>([&](auto sc) {
+                    if (kt + decltype(sc)::value < ktiles) tile(sc, kt + decltype(sc)::value);
+                });
+            if (!kStagger || stop == ktiles) break;
+            advance_base(a_res, -ktiles * a_k_step);
+            advance_base(b_res, -ktiles * b_k_step);
+        }
         MI355_TL(tl_w[2] = timeline::wall_clock(); tl_c[1] = timeline::shader_cycles();)
 
         // ---- epilogue ------------------------------------------------------------------------------------------------
