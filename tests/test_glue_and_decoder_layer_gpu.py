@@ -218,6 +218,55 @@ def test_gate_up_single_row_activation_with_arbitrary_row_stride(lib, gpu):
         assert bool((err <= 2.0 ** -10 * ref.abs() + 1e-3).all()), (stride0, float(err.max()))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cached", [True, False])
+@pytest.mark.parametrize("B,S,n_q,n_kv,hidden,normed", [
+    (1, 1, 8, 2, 1024, True), (4, 1, 4, 1, 1536, True), (1, 3, 5, 1, 2048, True), (2, 1, 32, 8, 4096, True),    # norm in front
+    (7, 1, 8, 2, 1024, True), (8, 1, 4, 2, 2048, True), (1, 6, 8, 2, 1024, True),
+    (2, 8, 16, 4, 2048, False), (3, 3, 8, 2, 1000, False), (8, 1, 32, 8, 4096, False), (16, 1, 32, 8, 4096, False),
+    (7, 5, 8, 2, 1024, False)])
+def test_step_qkv_equals_the_launches_it_replaces(lib, gpu, dtype, cached, B, S, n_q, n_kv, hidden, normed):
+    # RMSNorm of a few rows, their QKV projection on the small-M kernel and the rotation into a head-major cache (or in place): the
+    # same values in the same order of summation, rounded in the same places
+    rows, heads, past, max_len = B * S, n_q + 2 * n_kv, 5, 5 + S + 2
+    cos, sin = (t.to(gpu) for t in so.rope_tables(64, 128, 10000.0))
+    pos = ((torch.arange(rows, dtype=torch.int32) * 7) % 70).reshape(B, S).to(gpu)      # some beyond the table: clamped
+    x = (3 * so.randn_fp16((rows, hidden), 1)).to(dtype).to(gpu)
+    if rows > 1:
+        x[1] = 0
+    ln, w = (1 + so.randn_fp16((hidden,), 2, 0.1)).to(dtype).to(gpu), so.randn_fp16((heads * 128, hidden), 3, 0.05).to(dtype).to(gpu)
+    ref = lib.hgemm(lib.rmsnorm(x, ln, 1e-5) if normed else x, w, "NT", variant=8).view(B, S, heads, 128)
+    cache = [torch.full((B, 2 * n_kv, max_len, 128), 3.0, dtype=dtype, device=gpu) for _ in range(2)]
+    ref_rows = cache[0][:, :, past:past + S].transpose(1, 2) if cached else ref[:, :, n_q:]
+    lib.rope_qkv(ref, ref_rows, cos, sin, pos, n_q, n_kv)
+    qkv = torch.full((rows + 1, heads * 128), 3.0, dtype=dtype, device=gpu)
+    out = cache[1][:, :, past:past + S].transpose(1, 2) if cached else qkv[:rows].view(B, S, heads, 128)[:, :, n_q:]
+    rc = lib.load().mi355_internal_step_qkv(x.data_ptr(), ln.data_ptr() if normed else None, 1e-5, w.data_ptr(), qkv.data_ptr(), out.data_ptr(), B, S,
+                                            n_q, n_kv, hidden, out.stride(0), out.stride(1), out.stride(2), cos.data_ptr(), sin.data_ptr(),
+                                            pos.data_ptr(), S, 64, lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, 0)
+    assert rc in (0, lib.ERR_UNSUPPORTED)
+    if rc:
+        assert not normed       # a size for which the choice by shape has another kernel
+        pytest.skip("not the small-M kernel")
+    torch.cuda.synchronize()
+    n = n_q if cached else heads
+    assert torch.equal(qkv[:rows].view(B, S, heads, 128)[:, :, :n], ref[:, :, :n]) and torch.equal(cache[1], cache[0])
+    assert bool((qkv[rows:] == 3.0).all()) and (not cached or bool((qkv[:rows, n_q * 128:] == 3.0).all()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,F,hidden", [(1, 2816, 1024), (4, 96, 4096), (3, 160, 1536), (2, 288, 2048), (5, 2816, 1024), (8, 96, 2048)])
+def test_step_gate_up_equals_the_launches_it_replaces(lib, gpu, dtype, rows, F, hidden):
+    x = (3 * so.randn_fp16((rows, hidden), 1)).to(dtype).to(gpu)
+    ln, w = (1 + so.randn_fp16((hidden,), 2, 0.1)).to(dtype).to(gpu), so.randn_fp16((2 * F, hidden), 3, 0.05).to(dtype).to(gpu)
+    ref = lib.hgemm_silu_mul(lib.rmsnorm(x, ln, 1e-5), w, "NT")
+    out = torch.full((rows + 1, F), 3.0, dtype=dtype, device=gpu)
+    assert lib.load().mi355_internal_step_gate_up(x.data_ptr(), ln.data_ptr(), 1e-5, w.data_ptr(), out.data_ptr(), rows, F, hidden,
+                                                  lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, 0) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out[:rows], ref) and bool((out[rows:] == 3.0).all())
+
+
 def layer_weights(H, n_q, n_kv, F, seed=0):
     D = 128
     g = lambda shape, s, std: so.randn_fp16(shape, seed + s, std)

@@ -38,7 +38,8 @@ KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/hgemm_dispatch.hip", "csrc/hgemm_choic
 # A source listed here is compiled once per entry, each time with that entry's defines, into objects of its own (side by
 # side with the others): the GEMM source holds every tile shape for two element types and three layouts, and one
 # compiler process each cuts the time the build waits for it to a third of what one per element type takes.
-SOURCE_PARTS = {"csrc/hgemm.hip": [(t + "." + l.lower(), ["-DMI355_HGEMM_T=%s_t" % {"fp16": "half"}.get(t, t), "-DMI355_HGEMM_LAYOUT=MI355_GEMM_" + l])
+SOURCE_PARTS = {"csrc/hgemm.hip": [(t + "." + l.lower(), ["-DMI355_HGEMM_T=%s_t" % {"fp16": "half"}.get(t, t), "-DMI355_HGEMM_LAYOUT=MI355_GEMM_" + l] +
+                                    (["-DMI355_HGEMM_STEP"] if l == "NT" else []))
                                    for t in ("fp16", "bf16") for l in ("NN", "NT", "TN")]}
 # Per-source additions. The GEMM keeps its MFMA accumulators in ordinary VGPRs: left to itself the compiler moves part of
 # them to AGPRs in the 4-wave kernels and then shuffles them back and forth inside the K loop.

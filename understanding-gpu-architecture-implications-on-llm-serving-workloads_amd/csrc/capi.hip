@@ -301,9 +301,9 @@ static int rope_impl(const char* fn, int dtype, const void* x, void* out, int B,
     return 0;
 }
 
-static int rope_qkv_impl(const char* fn, int dtype, void* qkv, void* kv_out, int B, int S, int q_heads, int kv_heads, int D,
-                         int64_t x_batch, int64_t x_row, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
-                         const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions, void* stream) {
+static int rope_qkv_check(const char* fn, const void* qkv, const void* kv_out, int B, int S, int q_heads, int kv_heads, int D,
+                          int64_t x_batch, int64_t x_row, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
+                          const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions) {
     if (!qkv || !kv_out || !cos_table || !sin_table || !positions) return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer", fn);
     if (D != 128) return fail(MI355_ERR_UNSUPPORTED, "%s: head_dim must be 128 (got %d)", fn, D);
     if (B < 1 || S < 1 || q_heads < 1 || kv_heads < 1 || n_positions < 1 || pos_batch < 0)
@@ -319,6 +319,14 @@ static int rope_qkv_impl(const char* fn, int dtype, void* qkv, void* kv_out, int
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: out_row / out_head make the heads of a token overlap those of the next", fn);
     if (!aligned16(qkv) || !aligned16(kv_out) || !aligned16(cos_table) || !aligned16(sin_table))
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: pointers must be 16-byte aligned", fn);
+    return 0;
+}
+
+static int rope_qkv_impl(const char* fn, int dtype, void* qkv, void* kv_out, int B, int S, int q_heads, int kv_heads, int D,
+                         int64_t x_batch, int64_t x_row, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
+                         const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions, void* stream) {
+    if (const int rc = rope_qkv_check(fn, qkv, kv_out, B, S, q_heads, kv_heads, D, x_batch, x_row, out_batch, out_row, out_head, cos_table, sin_table,
+                                      positions, pos_batch, n_positions); rc != 0) return rc;
     hipError_t e = mi355::rope_dispatch(qkv, kv_out, B, S, q_heads, q_heads + kv_heads, kv_heads, x_batch, x_row, out_batch, out_row,
                                         out_head, cos_table, sin_table, positions, pos_batch, n_positions, dtype, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, fn);
@@ -374,6 +382,38 @@ int mi355_silu_mul(const void* gate_up, void* out, int64_t rows, int inter, int 
 int mi355_silu_mul_bf16(const void* gate_up, void* out, int64_t rows, int inter, int interleave, int64_t ld_in, int64_t ld_out,
                    void* stream) {
     return silu_mul_impl("mi355_silu_mul_bf16", MI355_DTYPE_BF16, gate_up, out, rows, inter, interleave, ld_in, ld_out, stream);
+}
+
+
+// Used by the decoder layer only (declared in mi355_serving_internal.h).
+int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, const void* w_qkv, void* qkv, void* kv_out, int B, int S, int q_heads,
+                            int kv_heads, int hidden, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
+                            const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions, int dtype, void* stream) {
+    const char* fn = "mi355_internal_step_qkv";
+    if (!x || !w_qkv || hidden < 1) return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer or no columns", fn);
+    if (B < 1 || S < 1 || (int64_t)B * S > 64) return fail(MI355_ERR_UNSUPPORTED, "%s: at most 64 rows", fn);
+    if (q_heads < 1 || kv_heads < 1 || q_heads > (1 << 20) || kv_heads > (1 << 20))
+        return fail(MI355_ERR_BAD_ARGUMENT, "%s: q_heads and kv_heads must be >= 1", fn);
+    const int64_t width = ((int64_t)q_heads + 2 * (int64_t)kv_heads) * 128;
+    if (const int rc = rope_qkv_check(fn, qkv, kv_out, B, S, q_heads, kv_heads, 128, S * width, width, out_batch, out_row, out_head, cos_table,
+                                      sin_table, positions, pos_batch, n_positions); rc != 0) return rc;
+    const mi355::RopeEpilogue rope = {kv_out, (long)out_batch, (long)out_row, (long)out_head, cos_table, sin_table, positions, (long)pos_batch,
+                                      n_positions, S, q_heads, kv_heads};
+    const hipError_t e = mi355::gemm_step_qkv_dispatch(x, {norm_weight, eps}, w_qkv, qkv, B * S, (int)width, hidden, rope, dtype,
+                                                       static_cast<hipStream_t>(stream));
+    if (e == hipErrorNotSupported) return fail(MI355_ERR_UNSUPPORTED, "%s: no such kernel for these sizes", fn);
+    return e == hipSuccess ? 0 : hip_fail(e, fn);
+}
+
+int mi355_internal_step_gate_up(const void* x, const void* norm_weight, float eps, const void* w_gu, void* out, int rows, int inter, int hidden,
+                                int dtype, void* stream) {
+    const char* fn = "mi355_internal_step_gate_up";
+    if (!x || !norm_weight || !w_gu || !out || rows < 1 || inter < 1 || inter > 0x3fffffff || hidden < 1)
+        return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer or empty operand", fn);
+    const hipError_t e = mi355::gemm_step_gate_up_dispatch(x, {norm_weight, eps}, w_gu, out, rows, 2 * inter, hidden, dtype,
+                                                           static_cast<hipStream_t>(stream));
+    if (e == hipErrorNotSupported) return fail(MI355_ERR_UNSUPPORTED, "%s: no such kernel for these sizes", fn);
+    return e == hipSuccess ? 0 : hip_fail(e, fn);
 }
 
 

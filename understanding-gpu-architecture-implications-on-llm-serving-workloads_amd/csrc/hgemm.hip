@@ -1195,10 +1195,61 @@ static_assert(kSmallMNtLdsBytes >= kSmallMNtWaves * 256 * 4, "the reduction reus
 // GATE_UP: the rows of B come in groups of [32 gate | 32 up] (the operand of the tiled kernels' gate/up epilogue) and C is
 // silu(gate) * up, half as wide. Workgroup t then takes the 8 gate rows 64 (t / 4) + 8 (t % 4) .. +7 and the 8 up rows 32
 // further on, and stores the 8 columns 32 (t / 4) + 8 (t % 4) .. +7 of C.
-template <typename T, bool HALF_A, bool GATE_UP>
+// kEpiRope: the rows of B are the heads of a fused QKV projection, 128 each. Workgroup t takes 8 rows of the lower half of head
+// t / 8 and their partners 64 rows further on, rounds the sums as the plain product stores them, rotates the pairs and writes
+// query heads into C, key and value heads where rope.kv_out says: what rope_kernel (glue.hip) makes of the stored product, bit for
+// bit, without its launch and its round trip through memory.
+enum SmallMEpilogue { kEpiPlain, kEpiGateUp, kEpiRope };
+struct NoEpilogueArgs {};
+template <int EPI>
+using EpilogueArgs = std::conditional_t<EPI == kEpiRope, RopeEpilogue, NoEpilogueArgs>;
+
+// first of the 16 weight rows of tile t, and how far its second 8 rows lie behind its first 8
+template <int EPI>
+__device__ __forceinline__ int smallm_nt_first_row(int t) {
+    return EPI == kEpiGateUp ? 64 * (t >> 2) + 8 * (t & 3) : EPI == kEpiRope ? 128 * (t >> 3) + 8 * (t & 7) : t * 16;
+}
+template <int EPI>
+constexpr int kSmallMNtSecondRows = EPI == kEpiGateUp ? 32 : EPI == kEpiRope ? 64 : 8;
+
+// Column pair e % 16 (< 8) and 8 further on of tile t, row m: `lo` and `hi` are the finished sums.
+template <typename T>
+__device__ __forceinline__ void store_rope_pair(const RopeEpilogue& rope, T* C, long ldc, int t, int m, int col, float lo_sum, float hi_sum) {
+    const int head = t >> 3, i = 8 * (t & 7) + col;
+    const int b = m / rope.S, tok = m - b * rope.S;
+    T* dst = head < rope.q_heads ? C + (long)m * ldc + (long)head * 128 + i
+                                 : static_cast<T*>(rope.kv_out) + b * rope.o_batch + tok * rope.o_row + (head - rope.q_heads) * rope.o_head + i;
+    T lo = (T)lo_sum, hi = (T)hi_sum;
+    if (head < rope.q_heads + rope.kv_heads) {
+        const int pos = min(max(rope.positions[b * rope.pos_batch + tok], 0), rope.n_pos - 1);
+        const float c = rope.cos_t[(long)pos * 64 + i], sn = rope.sin_t[(long)pos * 64 + i];
+        const float x = (float)lo, y = (float)hi;
+        lo = (T)(x * c - y * sn);
+        hi = (T)(y * c + x * sn);
+    }
+    dst[0] = lo;
+    dst[64] = hi;
+}
+
+// NORM = 1, 2, 4 or 8 (M <= NORM, K >= 1024 and a multiple of 512): A is the residual stream, and what is multiplied is its RMSNorm,
+// norm_weight * a * rsqrt(mean(a^2) + eps), rounded as rmsnorm_kernel (glue.hip) rounds it and with its order of summation. A
+// workgroup copies the rows and the norm weight into LDS in front of its first weights, normalises them there while those are
+// on their way, and reads its A fragments from there: the ring holds weights only. (The number of rows is a constant so that the rows'
+// reductions run side by side; rows behind M repeat the last one.)
+template <int NORM>
+constexpr int kSmallMNtStage = NORM > 0 ? 2 * 1024 : kSmallMNtStageBytes;
+constexpr int kNormRowPad = 64;   // bytes behind a row in LDS: the 64 bytes that four rows read together lie in different banks
+constexpr int kNormLdsMax = 80 * 1024;   // two workgroups to a CU
+static int smallm_nt_norm_rows(int M) { return M <= 2 ? M : M <= 4 ? 4 : 8; }
+static int smallm_nt_norm_lds(int M, int K) { return kSmallMNtWaves * kSmallMNtStages * kSmallMNtStage<1> + (smallm_nt_norm_rows(M) + 1) * (2 * K + kNormRowPad); }
+
+template <typename T, bool HALF_A, int EPI, int NORM = 0>
 __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(const T* __restrict__ A, const T* __restrict__ B,
                                                               T* C, const T* R, int M, int N, int K, long lda,
-                                                              long ldb, long ldc, long ldr, int n_tiles) {
+                                                              long ldb, long ldc, long ldr, int n_tiles, EpilogueArgs<EPI> epi,
+                                                              const T* __restrict__ norm_weight, float eps) {
+    constexpr bool GATE_UP = EPI == kEpiGateUp;
+    constexpr int kStageBytes = kSmallMNtStage<NORM>;
     using V8 = typename Elem<T>::v8;
     using V4 = typename Elem<T>::v4;
     using V2 = typename Elem<T>::v2;
@@ -1216,14 +1267,14 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
     const int ksteps = K / 64;
     const int s_begin = (int)((long)wave * ksteps / kSmallMNtWaves);
     const int s_end = (int)((long)(wave + 1) * ksteps / kSmallMNtWaves);
-    MI355_LDS char* wbase = smem + wave * kSmallMNtWaveBytes;
+    MI355_LDS char* wbase = smem + wave * kSmallMNtStages * kStageBytes;
 
     // slab = 16 rows x 128 bytes; a copy instruction covers 8 rows (row lane/8, chunk position lane%8);
     // chunk c of row r is stored at position c ^ (r & 7)
     const int c_row = lane >> 3;  // + 8*i
     const int c_chunk = (lane & 7) ^ (c_row & 7);
-    const int b_row0 = GATE_UP ? 64 * (tile >> 2) + 8 * (tile & 3) + c_row : n0 + c_row;
-    const int b_row1 = GATE_UP ? b_row0 + 32 : b_row0 + 8;
+    const int b_row0 = smallm_nt_first_row<EPI>(tile) + c_row;
+    const int b_row1 = b_row0 + kSmallMNtSecondRows<EPI>;
     const T* b_src0 = B + (long)min(b_row0, N - 1) * ldb + (long)s_begin * 64 + c_chunk * 8;
     const T* b_src1 = B + (long)min(b_row1, N - 1) * ldb + (long)s_begin * 64 + c_chunk * 8;
     const T* a_src0 = A + (long)min(m0 + c_row, M - 1) * lda + (long)s_begin * 64 + c_chunk * 8;
@@ -1231,13 +1282,13 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
 
     // HALF_A (M <= 8): rows 8..15 of the A slab are not copied; the fragment rows read from there hold whatever the
     // memory held, and so do rows 8..15 of the product, which are never stored (an output row depends on its own A row only)
-    constexpr int kCopies = HALF_A ? 3 : 4;
+    constexpr int kCopies = NORM > 0 ? 2 : HALF_A ? 3 : 4;
     auto issue_stage = [&](int slot) {
-        MI355_LDS char* st = wbase + slot * kSmallMNtStageBytes;
+        MI355_LDS char* st = wbase + slot * kStageBytes;
         copy16_global_to_lds(b_src0, st);
         copy16_global_to_lds(b_src1, st + 1024);
-        copy16_global_to_lds(a_src0, st + 2048);
-        if constexpr (!HALF_A) copy16_global_to_lds(a_src1, st + 3072);
+        if constexpr (NORM == 0) copy16_global_to_lds(a_src0, st + 2048);
+        if constexpr (NORM == 0 && !HALF_A) copy16_global_to_lds(a_src1, st + 3072);
         b_src0 += 64;
         b_src1 += 64;
         a_src0 += 64;
@@ -1250,16 +1301,30 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) f_off[sub] = f_row * 128 + (((4 * sub + (lane >> 4)) ^ (f_row & 7)) << 4);
 
+    // NORM: the normalised rows lie behind the ring, one behind the other, then the norm weight
+    MI355_LDS char* const rows = smem + kSmallMNtWaves * kSmallMNtStages * kStageBytes;
+    const int row_bytes = 2 * K + kNormRowPad;
+    MI355_LDS const char* a_norm = rows + min(f_row, NORM - 1) * row_bytes + s_begin * 128 + ((lane >> 4) << 4);
+
     float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
     auto k_step = [&](MI355_LDS const char* st) {
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
             V8 bf = Elem<T>::frag(lds_read_b128(st + f_off[sub]));
-            V8 af = Elem<T>::frag(lds_read_b128(st + 2048 + f_off[sub]));
+            V8 af = Elem<T>::frag(lds_read_b128(NORM > 0 ? a_norm + 64 * sub : st + 2048 + f_off[sub]));
             acc = Elem<T>::mfma16(af, bf, acc);
         }
+        if constexpr (NORM > 0) a_norm += 128;
     };
 
+    // in pieces of 512 values, piece p of each by wave p % 4
+    const int pieces = K / 512;
+    if constexpr (NORM > 0) {
+        for (int p = wave; p < pieces; p += kSmallMNtWaves)
+#pragma unroll
+            for (int r = 0; r <= NORM; ++r)
+                copy16_global_to_lds((r < NORM ? A + (long)min(r, M - 1) * lda : norm_weight) + lane * 8 + p * 512, rows + r * row_bytes + p * 1024);
+    }
     int issued = s_begin;
 #pragma unroll
     for (int i = 0; i < kSmallMNtStages - 1; ++i)
@@ -1267,6 +1332,60 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
             issue_stage(i);
             ++issued;
         }
+    if constexpr (NORM > 0) {
+        // a wave has at least four steps (K >= 1024), so exactly the copies of three stages were issued behind its own pieces
+        wait_vmcnt<kCopies * (kSmallMNtStages - 1)>();
+        asm volatile("" ::: "memory");
+        MI355_LDS char* const mine = rows + wave * 1024 + lane * 16;
+        float ss[NORM];
+#pragma unroll
+        for (int r = 0; r < NORM; ++r) ss[r] = 0.f;
+        for (int p = 0; p * kSmallMNtWaves + wave < pieces; ++p) {
+            V8 v[NORM];
+#pragma unroll
+            for (int r = 0; r < NORM; ++r) v[r] = Elem<T>::frag(lds_read_b128(mine + r * row_bytes + p * (kSmallMNtWaves * 1024)));
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int r = 0; r < NORM; ++r) ss[r] += (float)v[r][j] * (float)v[r][j];
+        }
+        __shared__ float scratch[NORM][kSmallMNtWaves];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+            for (int r = 0; r < NORM; ++r) ss[r] += __shfl_xor(ss[r], off, 64);
+        if (lane == 0)
+#pragma unroll
+            for (int r = 0; r < NORM; ++r) scratch[r][wave] = ss[r];
+        // (the barriers are written out: __syncthreads() may wait for the weights in flight)
+        asm volatile("" ::: "memory");
+        wait_lgkmcnt<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int r = 0; r < NORM; ++r) {
+            const float total = scratch[r][0] + scratch[r][1] + scratch[r][2] + scratch[r][3];
+            ss[r] = __builtin_amdgcn_rsqf(total / (float)K + eps);
+        }
+        for (int p = 0; p * kSmallMNtWaves + wave < pieces; ++p) {
+            V8 v[NORM + 1];
+#pragma unroll
+            for (int r = 0; r <= NORM; ++r) v[r] = Elem<T>::frag(lds_read_b128(mine + r * row_bytes + p * (kSmallMNtWaves * 1024)));
+#pragma unroll
+            for (int r = 0; r < NORM; ++r) {
+                V8 o;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) o[j] = (T)((float)v[NORM][j] * ((float)v[r][j] * ss[r]));
+                *(MI355_LDS V8*)(mine + r * row_bytes + p * (kSmallMNtWaves * 1024)) = o;
+            }
+        }
+        asm volatile("" ::: "memory");
+        wait_lgkmcnt<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
     int slot = 0, fill = kSmallMNtStages - 1;
     for (int s = s_begin; s < s_end; ++s) {
         if (issued < s_end) {
@@ -1277,11 +1396,11 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
         } else {
             wait_vmcnt<0>();
         }
-        k_step(wbase + slot * kSmallMNtStageBytes);
+        k_step(wbase + slot * kStageBytes);
         slot = (slot + 1 == kSmallMNtStages) ? 0 : slot + 1;
         wait_lgkmcnt<0>();  // the reads of this slot are complete before a later copy refills it
     }
-    if (const int k0 = ksteps * 64; k0 < K && wave == kSmallMNtWaves - 1) {
+    if (const int k0 = ksteps * 64; NORM == 0 && k0 < K && wave == kSmallMNtWaves - 1) {
         // the last K % 64 columns, by the last wave, whose copies have all landed: zeros behind K
         const int left = K - k0 - 8 * c_chunk;
         const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -1320,6 +1439,15 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
             }
             continue;
         }
+        if constexpr (EPI == kEpiRope) {
+            if ((o & 15) < 8 && m < M) {
+                float hi = 0.f;
+#pragma unroll
+                for (int w = 0; w < kSmallMNtWaves; ++w) hi += red[w * 256 + o + 8];
+                store_rope_pair(epi, C, ldc, tile, m, o & 15, sum, hi);
+            }
+            continue;
+        }
         const int n = n0 + (o & 15);
         if (m < M && n < N) {
             T v = (T)sum;
@@ -1336,11 +1464,12 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_kernel(co
 // the CU's memory pipeline as the weights themselves). The stream over (tile, k-step) is unrolled completely: every LDS
 // offset, copy destination and wait count is an immediate, a k-step is ~18 instructions. The partial
 // tiles of the four waves meet in LDS once, behind the stream (no barrier inside it).
-template <typename T, bool HALF_A, bool GATE_UP, int STEPS, int TPW>
+template <typename T, bool HALF_A, int EPI, int STEPS, int TPW>
 __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_rega_kernel(const T* __restrict__ A, const T* __restrict__ B,
                                                                    T* C, const T* R, int M, int N, long lda, long ldb,
-                                                                   long ldc, long ldr, int n_groups) {
+                                                                   long ldc, long ldr, int n_groups, EpilogueArgs<EPI> epi) {
     using V8 = typename Elem<T>::v8;
+    constexpr bool GATE_UP = EPI == kEpiGateUp;
     constexpr int NST = kSmallMNtStages, TOTAL = TPW * STEPS;
     constexpr int kCopiesA = HALF_A ? 1 : 2;
     extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
@@ -1359,16 +1488,15 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_rega_kern
     const int c_row = lane >> 3;
     const int c_chunk = (lane & 7) ^ (c_row & 7);
     const uint32_t b_voff0 = (uint32_t)((long)c_row * ldb * 2 + c_chunk * 16);
-    const uint32_t b_voff1 = (uint32_t)((long)(c_row + (GATE_UP ? 32 : 8)) * ldb * 2 + c_chunk * 16);
+    const uint32_t b_voff1 = (uint32_t)((long)(c_row + kSmallMNtSecondRows<EPI>) * ldb * 2 + c_chunk * 16);
     const uint32_t a_voff0 = (uint32_t)((long)min(c_row, M - 1) * lda * 2 + c_chunk * 16);
     const uint32_t a_voff1 = (uint32_t)((long)min(c_row + 8, M - 1) * lda * 2 + c_chunk * 16);
     const T* a_base = A + kbase;
-    // first weight row of tile t (GATE_UP: 8 gate rows there, their 8 up rows 32 further on)
     const T* b_base[TPW];
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
         const int t = tile0 + i;
-        b_base[i] = B + (long)(GATE_UP ? 64 * (t >> 2) + 8 * (t & 3) : t * 16) * ldb + kbase;
+        b_base[i] = B + (long)smallm_nt_first_row<EPI>(t) * ldb + kbase;
     }
     const uint32_t wave_lds = (uint32_t)(uintptr_t)(smem + wave * kSmallMNtWaveBytes);
 
@@ -1431,6 +1559,13 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_rega_kern
                 const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-sum * 1.4426950408889634f));
                 C[(long)m * ldc + 32 * (tile >> 2) + 8 * (tile & 3) + (e & 15)] = (T)(sum * sig * up);
             }
+        } else if constexpr (EPI == kEpiRope) {
+            if ((e & 15) < 8 && m < M) {
+                float hi = 0.f;
+#pragma unroll
+                for (int w = 0; w < kSmallMNtWaves; ++w) hi += rt[w * 256 + e + 8];
+                store_rope_pair(epi, C, ldc, tile, m, e & 15, sum, hi);
+            }
         } else {
             const int n = tile * 16 + (e & 15);
             if (m < M && n < N) {
@@ -1442,65 +1577,66 @@ __global__ __launch_bounds__(kSmallMNtWaves * 64) void hgemm_smallm_nt_rega_kern
     }
 }
 
-template <typename T, bool HALF_A, bool GATE_UP>
+template <typename T, bool HALF_A, int EPI>
 static hipError_t launch_smallm_nt_rega(const T* A, const T* B, T* C, const T* R, int M, int N, long lda, long ldb, long ldc,
-                                        long ldr, int n_tiles, int tpw, hipStream_t stream) {
+                                        long ldr, int n_tiles, int tpw, const EpilogueArgs<EPI>& epi, hipStream_t stream) {
     static DynamicLdsOnce once4, once2;
     const int groups = n_tiles / tpw;
     if (tpw == 4) {
         constexpr int lds = kSmallMNtLdsBytes + 4 * kSmallMNtWaves * 1024;
-        auto kern = hgemm_smallm_nt_rega_kernel<T, HALF_A, GATE_UP, 16, 4>;
+        auto kern = hgemm_smallm_nt_rega_kernel<T, HALF_A, EPI, 16, 4>;
         if (hipError_t e = once4.ensure(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
-        kern<<<dim3(groups), dim3(kSmallMNtWaves * 64), lds, stream>>>(A, B, C, R, M, N, lda, ldb, ldc, ldr, groups);
+        kern<<<dim3(groups), dim3(kSmallMNtWaves * 64), lds, stream>>>(A, B, C, R, M, N, lda, ldb, ldc, ldr, groups, epi);
     } else {
         constexpr int lds = kSmallMNtLdsBytes + 2 * kSmallMNtWaves * 1024;
-        auto kern = hgemm_smallm_nt_rega_kernel<T, HALF_A, GATE_UP, 16, 2>;
+        auto kern = hgemm_smallm_nt_rega_kernel<T, HALF_A, EPI, 16, 2>;
         if (hipError_t e = once2.ensure(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
-        kern<<<dim3(groups), dim3(kSmallMNtWaves * 64), lds, stream>>>(A, B, C, R, M, N, lda, ldb, ldc, ldr, groups);
+        kern<<<dim3(groups), dim3(kSmallMNtWaves * 64), lds, stream>>>(A, B, C, R, M, N, lda, ldb, ldc, ldr, groups, epi);
     }
     return hipGetLastError();
 }
 
-template <typename T>
-static hipError_t launch_smallm_nt(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
-                                   long ldc, long ldr, hipStream_t stream) {
-    static DynamicLdsOnce lds_once, lds_once_half;
+template <typename T, bool HALF_A, int EPI>
+static hipError_t launch_smallm_nt_half(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb, long ldc,
+                                        long ldr, int tpw, const EpilogueArgs<EPI>& epi, hipStream_t stream) {
+    static DynamicLdsOnce once;
     const int n_tiles = (N + 15) / 16;
-    if (const int tpw = N % 16 == 0 ? smallm_nt_rega_tpw(M, n_tiles, K, lda, ldb) : 0; tpw > 0) {
-        if (M <= 8) return launch_smallm_nt_rega<T, true, false>(A, B, C, R, M, N, lda, ldb, ldc, ldr, n_tiles, tpw, stream);
-        return launch_smallm_nt_rega<T, false, false>(A, B, C, R, M, N, lda, ldb, ldc, ldr, n_tiles, tpw, stream);
-    }
-    dim3 grid(n_tiles, (M + 15) / 16);
-    if (M <= 8) {
-        if (hipError_t e = lds_once_half.ensure(reinterpret_cast<const void*>(hgemm_smallm_nt_kernel<T, true, false>), kSmallMNtLdsBytes); e != hipSuccess) return e;
-        hgemm_smallm_nt_kernel<T, true, false><<<grid, dim3(kSmallMNtWaves * 64), kSmallMNtLdsBytes, stream>>>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, n_tiles);
-    } else {
-        if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(hgemm_smallm_nt_kernel<T, false, false>), kSmallMNtLdsBytes); e != hipSuccess) return e;
-        hgemm_smallm_nt_kernel<T, false, false><<<grid, dim3(kSmallMNtWaves * 64), kSmallMNtLdsBytes, stream>>>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, n_tiles);
-    }
+    if (tpw > 0) return launch_smallm_nt_rega<T, HALF_A, EPI>(A, B, C, R, M, N, lda, ldb, ldc, ldr, n_tiles, tpw, epi, stream);
+    auto kern = hgemm_smallm_nt_kernel<T, HALF_A, EPI>;
+    if (hipError_t e = once.ensure(reinterpret_cast<const void*>(kern), kSmallMNtLdsBytes); e != hipSuccess) return e;
+    kern<<<dim3(n_tiles, (M + 15) / 16), dim3(kSmallMNtWaves * 64), kSmallMNtLdsBytes, stream>>>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, n_tiles, epi,
+                                                                                                 nullptr, 0.f);
     return hipGetLastError();
 }
 
-// silu(A gate^T) * (A up^T) for up to 16 rows: N counts the rows of B ([32 gate | 32 up] groups, a multiple of 64), C is
-// [M, N / 2].
-template <typename T>
-static hipError_t launch_smallm_nt_gate_up(const T* A, const T* B, T* C, int M, int N, int K, long lda, long ldb, long ldc,
-                                           hipStream_t stream) {
-    static DynamicLdsOnce lds_once, lds_once_half;
+// EPI kEpiGateUp: silu(A gate^T) * (A up^T) for up to 16 rows: N counts the rows of B ([32 gate | 32 up] groups, a multiple of
+// 64), C is [M, N / 2]. kEpiRope: up to 64 rows, N whole heads.
+template <typename T, int EPI = kEpiPlain>
+static hipError_t launch_smallm_nt(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
+                                   long ldc, long ldr, hipStream_t stream, const EpilogueArgs<EPI>& epi = {}) {
+    const int tpw = N % 16 == 0 ? smallm_nt_rega_tpw(M, N / 16, K, lda, ldb) : 0;
+    if (M <= 8) return launch_smallm_nt_half<T, true, EPI>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, tpw, epi, stream);
+    return launch_smallm_nt_half<T, false, EPI>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, tpw, epi, stream);
+}
+
+template <typename T, int EPI>
+static hipError_t launch_smallm_nt_norm(const T* A, const T* norm_weight, float eps, const T* B, T* C, int M, int N, int K, long lda, long ldb,
+                                        long ldc, hipStream_t stream, const EpilogueArgs<EPI>& epi) {
     const int n_tiles = N / 16;
-    if (const int tpw = smallm_nt_rega_tpw(M, n_tiles, K, lda, ldb); tpw > 0) {
-        if (M <= 8) return launch_smallm_nt_rega<T, true, true>(A, B, C, nullptr, M, N, lda, ldb, ldc, 0, n_tiles, tpw, stream);
-        return launch_smallm_nt_rega<T, false, true>(A, B, C, nullptr, M, N, lda, ldb, ldc, 0, n_tiles, tpw, stream);
+    const auto launch = [&](auto rows) -> hipError_t {
+        static DynamicLdsOnce once;
+        auto kern = hgemm_smallm_nt_kernel<T, true, EPI, decltype(rows)::value>;
+        if (hipError_t e = once.ensure(reinterpret_cast<const void*>(kern), kNormLdsMax); e != hipSuccess) return e;
+        kern<<<dim3(n_tiles), dim3(kSmallMNtWaves * 64), smallm_nt_norm_lds(M, K), stream>>>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, n_tiles, epi,
+                                                                                              norm_weight, eps);
+        return hipGetLastError();
+    };
+    switch (smallm_nt_norm_rows(M)) {
+        case 1: return launch(std::integral_constant<int, 1>{});
+        case 2: return launch(std::integral_constant<int, 2>{});
+        case 4: return launch(std::integral_constant<int, 4>{});
+        default: return launch(std::integral_constant<int, 8>{});
     }
-    dim3 grid(n_tiles, 1);
-    if (M <= 8) {
-        if (hipError_t e = lds_once_half.ensure(reinterpret_cast<const void*>(hgemm_smallm_nt_kernel<T, true, true>), kSmallMNtLdsBytes); e != hipSuccess) return e;
-        hgemm_smallm_nt_kernel<T, true, true><<<grid, dim3(kSmallMNtWaves * 64), kSmallMNtLdsBytes, stream>>>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, n_tiles);
-    } else {
-        if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(hgemm_smallm_nt_kernel<T, false, true>), kSmallMNtLdsBytes); e != hipSuccess) return e;
-        hgemm_smallm_nt_kernel<T, false, true><<<grid, dim3(kSmallMNtWaves * 64), kSmallMNtLdsBytes, stream>>>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, n_tiles);
-    }
-    return hipGetLastError();
 }
 
 template <typename T, bool A_KC, bool B_KC, int BM, int BN, int WM, int WN, int EPI = 0, bool RAGGED = false, int STAGES = 0, int PER_CU = 1>
@@ -1659,7 +1795,7 @@ static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, in
     // N = columns of op(B); gate/up pairs are 64 columns wide. Few rows are better served by the small-M product.
     if (!aligned || K % 64 != 0 || K < 64 || N % 64 != 0 || lda >= (1L << 22) || ldb >= (1L << 22)) return hipErrorNotSupported;
     if constexpr (A_KC && B_KC) {   // generation step: the split-K small-M kernel with the same epilogue
-        if (M <= 16 && (variant == 0 || variant == kSmallM)) return launch_smallm_nt_gate_up<T>(A, B, C, M, N, K, lda, ldb, ldc, stream);
+        if (M <= 16 && (variant == 0 || variant == kSmallM)) return launch_smallm_nt<T, kEpiGateUp>(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 0, stream);
     }
     // More rows: the tile shape by the same model as the plain product's. On 64x64 tiles four waves lie side by side along M,
     // so that every wave holds the gate and the up columns of its rows.
@@ -1677,6 +1813,42 @@ static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, in
             return launch_main<T, A_KC, B_KC, 128, 128, 2, 2, 1, true>(MI355_ARGS, stream);
     }
 #undef MI355_ARGS
+}
+
+// The first two products of a generation step's layer, few enough rows for the small-M kernel of layout NT, with what stands
+// around them: the RMSNorm of their rows in front (norm.weight != nullptr), rotary embedding and the way into the KV cache behind
+// the QKV projection. hipErrorNotSupported: no such kernel for this call, nothing was launched.
+// Every workgroup normalises the rows for itself (~0.2 us a row, hidden behind the first weights in part), which is repaid as long
+// as two workgroups with their rows fit a CU's LDS. us per pass of a layer, norms on their own / in the products: 1024 wide, 8 rows
+// 27.4 / 26.7, 1 row 27.2 / 22.1; 2048 wide, 8 rows 47.1 / 45.1, 4 rows 45.7 / 41.0; 4096 wide, 4 rows 92.7 / 92.2, 1 row 92 / 87.2.
+static bool norm_fits(const NormPrologue& norm, int M, int K) {
+    return M <= 8 && K >= 1024 && K % 512 == 0 && smallm_nt_norm_lds(M, K) <= kNormLdsMax - 1024 &&
+           reinterpret_cast<uintptr_t>(norm.weight) % 16 == 0;
+}
+
+template <typename T>
+hipError_t gemm_step_qkv(const void* x, const NormPrologue& norm, const void* w, void* qkv, int M, int N, int K, long ldx, long ldb, long ldc,
+                         const RopeEpilogue& rope, hipStream_t stream) {
+    const T *A = static_cast<const T*>(x), *B = static_cast<const T*>(w);
+    T* C = static_cast<T*>(qkv);
+    const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 && ldx % 8 == 0 && ldb % 8 == 0;
+    if (!aligned || M > 64 || N % 128 != 0 || ldx >= (1L << 22) || ldb >= (1L << 22)) return hipErrorNotSupported;
+    if (norm.weight != nullptr) {
+        if (!norm_fits(norm, M, K)) return hipErrorNotSupported;
+        return launch_smallm_nt_norm<T, kEpiRope>(A, static_cast<const T*>(norm.weight), norm.eps, B, C, M, N, K, ldx, ldb, ldc, stream, rope);
+    }
+    if (choose_kernel(M, N, K, true, true, true, true, ldb % 64 == 0).shape != kSmallM) return hipErrorNotSupported;
+    return launch_smallm_nt<T, kEpiRope>(A, B, C, nullptr, M, N, K, ldx, ldb, ldc, 0, stream, rope);
+}
+
+template <typename T>
+hipError_t gemm_step_gate_up(const void* x, const NormPrologue& norm, const void* w, void* out, int M, int N, int K, long ldx, long ldb, long ldc,
+                             hipStream_t stream) {
+    const T *A = static_cast<const T*>(x), *B = static_cast<const T*>(w);
+    const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 && ldx % 8 == 0 && ldb % 8 == 0;
+    if (!aligned || N % 64 != 0 || !norm_fits(norm, M, K)) return hipErrorNotSupported;
+    return launch_smallm_nt_norm<T, kEpiGateUp>(A, static_cast<const T*>(norm.weight), norm.eps, B, static_cast<T*>(out), M, N, K, ldx, ldb, ldc,
+                                                stream, {});
 }
 
 // One translation unit per element type and layout (the build compiles the six side by side): MI355_HGEMM_T and
@@ -1699,9 +1871,18 @@ hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, in
     template hipError_t gemm_layout<T, LAYOUT>(const void*, const void*, void*, const void*, int, int, int, long, long, long,  \
                                                long, int, hipStream_t);                                                        \
     template hipError_t gemm_silu_mul_layout<T, LAYOUT>(const void*, const void*, void*, int, int, int, long, long, long, int, hipStream_t);
+#define MI355_HGEMM_INSTANTIATE_STEP(T)                                                                                        \
+    template hipError_t gemm_step_qkv<T>(const void*, const NormPrologue&, const void*, void*, int, int, int, long, long, long, \
+                                         const RopeEpilogue&, hipStream_t);                                                    \
+    template hipError_t gemm_step_gate_up<T>(const void*, const NormPrologue&, const void*, void*, int, int, int, long, long, long, hipStream_t);
 #ifdef MI355_HGEMM_T
 MI355_HGEMM_INSTANTIATE(MI355_HGEMM_T, MI355_HGEMM_LAYOUT)
+#ifdef MI355_HGEMM_STEP
+MI355_HGEMM_INSTANTIATE_STEP(MI355_HGEMM_T)
+#endif
 #else
+MI355_HGEMM_INSTANTIATE_STEP(half_t)
+MI355_HGEMM_INSTANTIATE_STEP(bf16_t)
 MI355_HGEMM_INSTANTIATE(half_t, MI355_GEMM_NN)
 MI355_HGEMM_INSTANTIATE(half_t, MI355_GEMM_NT)
 MI355_HGEMM_INSTANTIATE(half_t, MI355_GEMM_TN)

@@ -122,6 +122,18 @@ hipError_t hgemm_silu_mul_dispatch(const void* A, const void* B, void* C, int M,
     return entry(A, B, C, M, N2, K, lda, ldb, ldc, variant, stream);
 }
 
+hipError_t gemm_step_qkv_dispatch(const void* x, const NormPrologue& norm, const void* w, void* qkv, int M, int N, int K, const RopeEpilogue& rope,
+                                  int dtype, hipStream_t stream) {
+    const auto entry = dtype == MI355_DTYPE_BF16 ? &gemm_step_qkv<bf16_t> : &gemm_step_qkv<half_t>;
+    return entry(x, norm, w, qkv, M, N, K, K, K, N, rope, stream);
+}
+
+hipError_t gemm_step_gate_up_dispatch(const void* x, const NormPrologue& norm, const void* w, void* out, int M, int N, int K, int dtype,
+                                      hipStream_t stream) {
+    const auto entry = dtype == MI355_DTYPE_BF16 ? &gemm_step_gate_up<bf16_t> : &gemm_step_gate_up<half_t>;
+    return entry(x, norm, w, out, M, N, K, K, K, N / 2, stream);
+}
+
 #ifdef MI355_TIMELINE
 hipError_t (*timeline_hgemm_reader)(void*, size_t) = nullptr;
 #endif

@@ -40,6 +40,30 @@ template <typename T, int LAYOUT>
 hipError_t gemm_silu_mul_layout(const void* A, const void* B, void* C, int M, int N2, int K, long lda, long ldb, long ldc,
                                 int variant, hipStream_t stream);
 
+// The first two products of a layer's generation step (layout NT, few rows) with what stands around them.
+struct RopeEpilogue {   // behind the QKV projection, as mi355_rope_qkv takes it
+    void* kv_out;
+    long o_batch, o_row, o_head;
+    const float *cos_t, *sin_t;
+    const int* positions;
+    long pos_batch;
+    int n_pos, S, q_heads, kv_heads;
+};
+struct NormPrologue {   // RMSNorm of the rows; weight == nullptr: none
+    const void* weight;
+    float eps;
+};
+template <typename T>
+hipError_t gemm_step_qkv(const void* x, const NormPrologue& norm, const void* w, void* qkv, int M, int N, int K, long ldx, long ldb, long ldc,
+                         const RopeEpilogue& rope, hipStream_t stream);
+template <typename T>
+hipError_t gemm_step_gate_up(const void* x, const NormPrologue& norm, const void* w, void* out, int M, int N, int K, long ldx, long ldb, long ldc,
+                             hipStream_t stream);
+hipError_t gemm_step_qkv_dispatch(const void* x, const NormPrologue& norm, const void* w, void* qkv, int M, int N, int K, const RopeEpilogue& rope,
+                                  int dtype, hipStream_t stream);   // rows side by side
+hipError_t gemm_step_gate_up_dispatch(const void* x, const NormPrologue& norm, const void* w, void* out, int M, int N, int K, int dtype,
+                                      hipStream_t stream);
+
 // The kernel of a product (hgemm_choice.hip); the shapes' numbers are those of mi355_internal_hgemm_variant below.
 enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile128x256, kTile256x128, kTile32x64, kSmallM, kDeepRing };
 struct KernelChoice {
@@ -173,6 +197,15 @@ int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C,
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                     int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides,
                                     int dtype, int variant, void* stream);
+// The QKV projection of a generation step's layer with the RMSNorm of its rows (norm_weight null: none) and mi355_rope_qkv in one
+// launch: qkv = rope(rmsnorm(x) w_qkv^T), rotated keys and values into kv_out; x is [B, S, hidden], qkv [B, S, (q_heads + 2 kv_heads)
+// * 128]. And silu(gate) * up of the normalised rows (w_gu in groups of 32 gate and 32 up rows). MI355_ERR_UNSUPPORTED: nothing
+// was launched, take the single calls.
+int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, const void* w_qkv, void* qkv, void* kv_out, int B, int S, int q_heads,
+                            int kv_heads, int hidden, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
+                            const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions, int dtype, void* stream);
+int mi355_internal_step_gate_up(const void* x, const void* norm_weight, float eps, const void* w_gu, void* out, int rows, int inter, int hidden,
+                                int dtype, void* stream);
 // how few queries over `kv_valid_len` keys are cut: key ranges per (batch, kv head), 0 = by the prefill kernel; waves per workgroup
 int mi355_internal_fmha_decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves);
 }

@@ -23,7 +23,7 @@ EXPORTED_SYMBOLS = ("mi355_hgemm", "mi355_fmha_fwd", "mi355_fmha_fwd_strided", "
 # exported for tests and tuning runs, declared in csrc/mi355_serving_internal.h and not in the public header
 INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_add_variant", "mi355_internal_hgemm_choice",
                     "mi355_internal_hgemm_silu_mul_variant", "mi355_internal_fmha_fwd_variant",
-                    "mi355_internal_fmha_decode_plan")
+                    "mi355_internal_fmha_decode_plan", "mi355_internal_step_qkv", "mi355_internal_step_gate_up")
 
 _lib = None
 
@@ -97,6 +97,10 @@ def load():
     lib.mi355_internal_hgemm_choice.restype = i32
     lib.mi355_internal_hgemm_silu_mul_variant.argtypes = lib.mi355_internal_hgemm_variant.argtypes
     lib.mi355_internal_hgemm_silu_mul_variant.restype = i32
+    lib.mi355_internal_step_qkv.argtypes = [vp, vp, f32, vp, vp, vp, i32, i32, i32, i32, i32, i64, i64, i64, vp, vp, vp, i64, i32, i32, vp]
+    lib.mi355_internal_step_qkv.restype = i32
+    lib.mi355_internal_step_gate_up.argtypes = [vp, vp, f32, vp, vp, i32, i32, i32, i32, vp]
+    lib.mi355_internal_step_gate_up.restype = i32
     lib.mi355_internal_fmha_decode_plan.argtypes = [i32] * 5 + [ctypes.POINTER(i32)] * 2
     lib.mi355_internal_fmha_decode_plan.restype = i32
     lib.mi355_internal_fmha_fwd_variant.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, f32, i32, i32,

@@ -1,9 +1,9 @@
-// One call per forward pass of llama_layer.FineLlamaDecoderLayer: the eight launches of the layer issued back to back from
-// C++ through the C ABI of libmi355_serving.so. Issued one by one from Python (ctypes calls, tensor views, one allocation per
-// intermediate) they take the host ~85-95 us per layer, longer than a generation step keeps the GPU busy on any layer
-// narrower than ~4096; from here ~25 us, with one block of torch's allocator for the intermediates: a step of one
+// One call per forward pass of llama_layer.FineLlamaDecoderLayer: the eight launches of the layer (five for up to 8 rows) issued
+// back to back from C++ through the C ABI of libmi355_serving.so. Issued one by one from Python (ctypes calls, tensor views, one
+// allocation per intermediate) eight take the host ~85-95 us per layer, longer than a generation step keeps the GPU busy on any
+// layer narrower than ~4096; from here ~25 us, with one block of torch's allocator for the intermediates: a step of one
 // sequence through a layer 1024 wide 81 -> 29 us, 4 sequences through one 2048 wide 87 -> 45, first pass on new
-// tensors 132 -> 61.
+// tensors 132 -> 61. With five launches the first of these takes 23 us, the second 41.
 //
 // Stateless: every tensor is an argument of the call, nothing is kept between calls.
 #include <torch/extension.h>
@@ -15,6 +15,14 @@
 #include <vector>
 
 #include "mi355_serving.h"
+
+// of the same library (csrc/mi355_serving_internal.h)
+extern "C" int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, const void* w_qkv, void* qkv, void* kv_out, int B, int S,
+                                       int q_heads, int kv_heads, int hidden, int64_t out_batch, int64_t out_row, int64_t out_head,
+                                       const float* cos_table, const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions,
+                                       int dtype, void* stream);
+extern "C" int mi355_internal_step_gate_up(const void* x, const void* norm_weight, float eps, const void* w_gu, void* out, int rows, int inter,
+                                           int hidden, int dtype, void* stream);
 
 namespace {
 
@@ -114,15 +122,6 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
         const auto entry = bf16 ? &mi355_rmsnorm_bf16 : &mi355_rmsnorm;
         check(entry(in, nullptr, nullptr, w.data_ptr(), h, rows, (int)H, H, 0, 0, H, (float)eps, stream), "mi355_rmsnorm");
     };
-    norm(x.data_ptr(), ln1);
-    Events ev;
-    if (timed) {
-        CHECK_HIP(hipEventCreate(&ev.begin));
-        CHECK_HIP(hipEventCreate(&ev.end));
-        CHECK_HIP(hipDeviceSynchronize());
-        CHECK_HIP(hipEventRecord(ev.begin, stream));
-    }
-    linear(h, w_qkv, nullptr, qkv, rows, dtype, stream);
     // attention operands read where they lie: q in the fused projection, k and v there or in the cache (batch, head, row strides)
     const int64_t row = heads * D;
     struct Rows {   // where a [B, tokens, heads, 128] operand lies: bytes are 2 per element
@@ -130,13 +129,10 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
         int64_t batch, row, head;
     };
     int64_t keys = S;
+    // of the new tokens, keys in front of values; without a cache they stay where the projection puts them
+    Rows fresh = {qkv + 2 * n_q * D, S * row, row, D};
     Rows k = {qkv + 2 * n_q * D, S * row, row, D}, v = {k.ptr + 2 * n_kv * D, S * row, row, D};
-    if (kv.empty()) {
-        const auto entry = bf16 ? &mi355_rope_bf16 : &mi355_rope;
-        check(entry(qkv, qkv, (int)B, (int)S, (int)(n_q + n_kv), 0, (int)D, S * row, row, S * row, row, cos_p, sin_p, pos, pos_batch, n_pos, stream),
-              "mi355_rope");
-    } else {
-        Rows fresh;   // of the new tokens, keys in front of values
+    if (!kv.empty()) {
         keys = past + S;
         if (kv.size() == 1) {
             const at::Tensor& t = kv[0];
@@ -158,9 +154,37 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
             k = view(kv[1], keys, n_kv, "keys");
             v = view(kv[2], keys, n_kv, "values");
         }
-        const auto entry = bf16 ? &mi355_rope_qkv_bf16 : &mi355_rope_qkv;
-        check(entry(qkv, fresh.ptr, (int)B, (int)S, (int)n_q, (int)n_kv, (int)D, S * row, row, fresh.batch, fresh.row, fresh.head, cos_p, sin_p, pos,
-                    pos_batch, n_pos, stream), "mi355_rope_qkv");
+    }
+    // Norm, projection and rotary embedding of a few rows are one launch (two with the norm on its own where the attention block
+    // is timed, which begins behind it), of more rows three.
+    const auto step_qkv = [&](const void* in, const void* norm_weight) {
+        if (rows > 64) return false;
+        const int rc = mi355_internal_step_qkv(in, norm_weight, (float)eps, w_qkv.data_ptr(), qkv, fresh.ptr, (int)B, (int)S, (int)n_q, (int)n_kv, (int)H,
+                                               fresh.batch, fresh.row, fresh.head, cos_p, sin_p, pos, pos_batch, n_pos, dtype, stream);
+        if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_rope_qkv");
+        return rc == 0;
+    };
+    Events ev;
+    if (timed || !step_qkv(x.data_ptr(), ln1.data_ptr())) {
+        norm(x.data_ptr(), ln1);
+        if (timed) {
+            CHECK_HIP(hipEventCreate(&ev.begin));
+            CHECK_HIP(hipEventCreate(&ev.end));
+            CHECK_HIP(hipDeviceSynchronize());
+            CHECK_HIP(hipEventRecord(ev.begin, stream));
+        }
+        if (!step_qkv(h, nullptr)) {
+            linear(h, w_qkv, nullptr, qkv, rows, dtype, stream);
+            if (kv.empty()) {
+                const auto entry = bf16 ? &mi355_rope_bf16 : &mi355_rope;
+                check(entry(qkv, qkv, (int)B, (int)S, (int)(n_q + n_kv), 0, (int)D, S * row, row, S * row, row, cos_p, sin_p, pos, pos_batch, n_pos,
+                            stream), "mi355_rope");
+            } else {
+                const auto entry = bf16 ? &mi355_rope_qkv_bf16 : &mi355_rope_qkv;
+                check(entry(qkv, fresh.ptr, (int)B, (int)S, (int)n_q, (int)n_kv, (int)D, S * row, row, fresh.batch, fresh.row, fresh.head, cos_p,
+                            sin_p, pos, pos_batch, n_pos, stream), "mi355_rope_qkv");
+            }
+        }
     }
     {
         const int64_t strides[12] = {S * row, D, row, k.batch, k.head, k.row, v.batch, v.head, v.row, S * n_q * D, D, n_q * D};
@@ -177,9 +201,14 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
         CHECK_HIP(hipEventElapsedTime(&elapsed, ev.begin, ev.end));
         ms = elapsed;
     }
-    norm(out.data_ptr(), ln2);
     int rc = MI355_ERR_UNSUPPORTED;
-    if (gate_up_block > 0) {
+    if (gate_up_block > 0 && rows <= 16) {
+        rc = mi355_internal_step_gate_up(out.data_ptr(), ln2.data_ptr(), (float)eps, w_gu.data_ptr(), act, (int)rows, (int)F, (int)H, dtype, stream);
+        if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_hgemm_silu_mul");
+    }
+    const bool normalised = rc == 0;
+    if (!normalised) norm(out.data_ptr(), ln2);
+    if (!normalised && gate_up_block > 0) {
         const auto entry = bf16 ? &mi355_gemm_silu_mul_bf16 : &mi355_hgemm_silu_mul;
         rc = entry(h, w_gu.data_ptr(), act, (int)rows, (int)F, (int)H, H, H, F, MI355_GEMM_NT, stream);
         if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_hgemm_silu_mul");
