@@ -928,3 +928,30 @@ def test_k_walked_from_different_places_on_each_xcd(lib, gpu, variant, M, tiles)
     for K in (64 * tiles, 64 * tiles - 8):
         a, b = operands(M, 1096, K, "NT", seed=tiles + M)
         check(lib, gpu, a, b, "NT", K, variant=variant)
+
+
+def test_another_stream_gets_the_chip_before_a_large_product_is_done(lib, gpu):
+    """A product of several rounds of tiles gives its CUs back tile by tile: an RMSNorm of 8 rows, enqueued on another stream while the
+    product runs, takes its turn between them. Workgroups that walked the tiles kept it waiting to the end (791 of 812 us; 83
+    with one per tile). Several streams, of which the soonest counts, since two streams may share a hardware queue."""
+    M = N = K = 8192
+    a, b = (torch.randn(M, K, device=gpu, dtype=torch.float16) * 0.05 for _ in range(2))
+    c = torch.empty(M, N, device=gpu, dtype=torch.float16)
+    x, w = torch.randn(8, 4096, device=gpu, dtype=torch.float16), torch.ones(4096, device=gpu, dtype=torch.float16)
+    product, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(4)]
+    shares = []
+    for _ in range(6):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        small = [torch.cuda.Event(enable_timing=True) for _ in others]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(product):
+            begin.record()
+            lib.hgemm(a, b, "NN", out=c, variant=1)
+            end.record()
+        for s, done in zip(others, small):
+            with torch.cuda.stream(s):
+                lib.rmsnorm(x, w, 1e-5)
+                done.record()
+        torch.cuda.synchronize()
+        shares.append(min(begin.elapsed_time(e) for e in small) / begin.elapsed_time(end))
+    assert sorted(shares)[2] < 0.6, shares

@@ -42,7 +42,7 @@
 
 namespace mi355 {
 
-// profiling build: per tile of hgemm_main_kernel [wall: entry, loop start, loop end, exit; cycles: loop start, loop
+// profiling build: per workgroup of hgemm_main_kernel [wall: entry, loop start, loop end, exit; cycles: loop start, loop
 // end; K tiles; 0]
 MI355_TL(static __device__ unsigned long long hgemm_stamps[timeline::kMaxWorkgroups * timeline::kSlots];
          static hipError_t read_hgemm_stamps(void* dst, size_t bytes) {   // of this translation unit's kernels
@@ -243,34 +243,24 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
 // XOR-swizzled by row) and then stores whole rows: every store instruction writes complete 128-byte lines.
 // EPI == 1: the wave's columns come in groups of [32 gate | 32 up]; output block jo takes its gate from block
 // 4 (jo / 2) + jo % 2 and its up from two blocks further.
-// PASS_TM: blocks of 16 rows parked at a time. The wave's slice of LDS is made of pieces of 1 KiB, PIECE_STRIDE bytes apart.
-template <typename T, int TM, int TN, int EPI, bool RAGGED, int PASS_TM, int PIECE_STRIDE>
+template <typename T, int TM, int TN, int EPI, bool RAGGED>
 __device__ __forceinline__ void store_wave_tile(const float4v (&acc)[TM][TN], MI355_LDS char* cst, T* C, const T* R, long row0,
                                                 long col0, int M, int NC, long ldc, long ldr, int lane) {
     using V8 = typename Elem<T>::v8;
     using V4 = typename Elem<T>::v4;
     static_assert(EPI == 0 || TN % 4 == 0, "the gate/up epilogue pairs column blocks 32 columns apart");
-    static_assert(TM % PASS_TM == 0, "whole passes");
     constexpr int TNO = EPI == 1 ? TN / 2 : TN;   // column blocks a wave stores
     constexpr int kRowHalfs = TNO * 16;           // width of the stored wave sub-tile
     constexpr int kRowBytesC = kRowHalfs * 2;
     constexpr int kChunksC = kRowBytesC / 16;     // 16-byte chunks per row (4, 8 or 16)
-    constexpr int kRowsPerStore = 64 / kChunksC;  // rows covered by one store instruction, a piece of LDS
+    constexpr int kRowsPerStore = 64 / kChunksC;  // rows covered by one store instruction
     constexpr int kSwzC = kChunksC < 8 ? kChunksC - 1 : 7;
-    const int r = lane & 15;
-    const int g = lane >> 4;
-    const int rr = lane / kChunksC;
-    const int cc = lane % kChunksC;
-    T* cbase = C + row0 * ldc + col0 + cc * 8;
-    const long rows_left = M - row0;   // RAGGED: rows and columns that exist
-    const long cols_left = NC - (col0 + cc * 8);   // of this lane's 8
-    const T* rbase = R + row0 * ldr + col0 + cc * 8;
+    {
+        const int r = lane & 15;
+        const int g = lane >> 4;
 #pragma unroll
-    for (int pass = 0; pass < TM; pass += PASS_TM) {
-#pragma unroll
-        for (int i = 0; i < PASS_TM; ++i) {
+        for (int i = 0; i < TM; ++i) {
             const int row = i * 16 + r;
-            MI355_LDS char* row_ptr = cst + row / kRowsPerStore * PIECE_STRIDE + row % kRowsPerStore * kRowBytesC;
 #pragma unroll
             for (int jo = 0; jo < TNO; ++jo) {
                 V4 v;
@@ -278,22 +268,30 @@ __device__ __forceinline__ void store_wave_tile(const float4v (&acc)[TM][TN], MI
                 for (int q = 0; q < 4; ++q) {
                     if constexpr (EPI == 1) {
                         const int gj = (jo / 2) * 4 + (jo % 2);
-                        const float gt = acc[pass + i][gj][q];
+                        const float gt = acc[i][gj][q];
                         const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-gt * 1.4426950408889634f));
-                        v[q] = (T)(gt * sig * acc[pass + i][gj + 2][q]);
+                        v[q] = (T)(gt * sig * acc[i][gj + 2][q]);
                     } else {
-                        v[q] = (T)acc[pass + i][jo][q];
+                        v[q] = (T)acc[i][jo][q];
                     }
                 }
                 const int chunk = (2 * jo + (g >> 1)) ^ (row & kSwzC);
-                *(MI355_LDS V4*)(row_ptr + chunk * 16 + (g & 1) * 8) = v;
+                *(MI355_LDS V4*)(cst + row * kRowBytesC + chunk * 16 + (g & 1) * 8) = v;
             }
         }
-        // only this wave reads what it wrote: no workgroup barrier needed, the LDS operations of a wave complete in order
+    }
+    // only this wave reads what it wrote: no workgroup barrier needed, the LDS operations of a wave complete in order
+    {
+        const int rr = lane / kChunksC;
+        const int cc = lane % kChunksC;
+        T* cbase = C + row0 * ldc + col0 + cc * 8;
+        const long rows_left = M - row0;   // RAGGED: rows and columns that exist
+        const long cols_left = NC - (col0 + cc * 8);   // of this lane's 8
+        const T* rbase = R + row0 * ldr + col0 + cc * 8;
 #pragma unroll
-        for (int it = 0; it < PASS_TM * 16 / kRowsPerStore; ++it) {
-            const int in_pass = it * kRowsPerStore + rr, row = pass * 16 + in_pass;
-            V8 v = *(MI355_LDS const V8*)(cst + it * PIECE_STRIDE + rr * kRowBytesC + ((cc ^ (in_pass & kSwzC)) << 4));
+        for (int it = 0; it < TM * 16 / kRowsPerStore; ++it) {
+            const int row = it * kRowsPerStore + rr;
+            V8 v = *(MI355_LDS const V8*)(cst + row * kRowBytesC + ((cc ^ (row & kSwzC)) << 4));
             if constexpr (!RAGGED) {
                 if (R != nullptr) {
                     const V8 r = *(const V8*)(rbase + (long)row * ldr);
@@ -349,14 +347,8 @@ __device__ __forceinline__ void store_wave_tile(const float4v (&acc)[TM][TN], MI
 // (the 256x256 tiles are always merged by a kernel of their own: a workgroup alone would read 256 KiB per range, which no choice takes)
 template <int BM, int BN>
 constexpr bool kOwnMergeOnly = BM * BN == 256 * 256;
-// PERSIST (256x256 tiles, the whole of K): at most one workgroup per CU, which takes tiles blockIdx.x, + gridDim.x, .. and requests
-// the next tile's first K tiles before it stores the one it has finished. A workgroup per tile leaves a CU without loads in
-// flight from its last K tile to the first copy of its successor, once a round. us, one tile per workgroup / this: 8192 x 28672 x 4096
-// NT gate/up (14 rounds) 1328 / 1307, NN 1356 / 1339, 16384 x 8192 x 4096 NT (8) 777 / 766, 8192^3 NN (4) 761 / 748, one round the same.
-// What is worked out per lane between two tiles is kept from being carried through the K loop (lane_here): otherwise 50-90
-// registers were spilled, some inside the loop, and it lost 2-20 %.
 template <typename T, bool A_KC, bool B_KC, int BM, int BN, int WM, int WN, int EPI = 0, bool RAGGED = false, int STAGES = 0, int PER_CU = 1,
-          bool SPLIT_K = false, bool PERSIST = false>
+          bool SPLIT_K = false>
 __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WM * WN / 4, PER_CU * WM * WN / 4)))
 void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
                                                          T* C, const T* R, int M, int N, int K, long lda,
@@ -381,8 +373,10 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     const int wm = wave / Cfg::WN;
     const int wn = wave % Cfg::WN;
 
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    long m0, n0;   // origin of the tile being computed
+    int tile_m, tile_n;
+    tile_of_block(blockIdx.x, (M + Cfg::BM - 1) / Cfg::BM, (N + Cfg::BN - 1) / Cfg::BN, tile_m, tile_n);
+    const long m0 = (long)tile_m * Cfg::BM;
+    const long n0 = (long)tile_n * Cfg::BN;
     if constexpr (SPLIT_K) {   // this workgroup's range of K: whole K tiles, the last range ends with K
         const int all = (K + BK - 1) / BK;
         const int t0 = (int)((long)blockIdx.y * all / splits), t1 = (int)((long)(blockIdx.y + 1) * all / splits);
@@ -396,22 +390,28 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // A copy reads (tile base, kept in scalar registers and advanced per K tile) + (this lane's byte offset inside the
     // tile, a loop-invariant 32-bit VGPR) + (copy index * uniform step). Offsets inside a tile fit 32 bits because the
     // launcher only takes leading dimensions below 2^22 elements.
+    const char* a_base;
+    const char* b_base;
     uint32_t a_lane_off, b_lane_off, a_copy_step, b_copy_step;
     long a_k_step, b_k_step;
     if constexpr (A_KC) {  // A stored [M,K]
+        a_base = (const char*)(A + m0 * lda);
         a_lane_off = (uint32_t)(ATK::first_copy_offset(wave, lane, lda) * 2);
         a_copy_step = (uint32_t)(ATK::copy_stride(lda) * 2);
         a_k_step = ATK::ktile_stride(lda) * 2;
     } else {  // A stored [K,M]
+        a_base = (const char*)(A + m0);
         a_lane_off = (uint32_t)(ATM::first_copy_offset(wave, lane, lda) * 2);
         a_copy_step = (uint32_t)(ATM::copy_stride(lda) * 2);
         a_k_step = ATM::ktile_stride(lda) * 2;
     }
     if constexpr (B_KC) {  // B stored [N,K]
+        b_base = (const char*)(B + n0 * ldb);
         b_lane_off = (uint32_t)(BTK::first_copy_offset(wave, lane, ldb) * 2);
         b_copy_step = (uint32_t)(BTK::copy_stride(ldb) * 2);
         b_k_step = BTK::ktile_stride(ldb) * 2;
     } else {  // B stored [K,N]
+        b_base = (const char*)(B + n0);
         b_lane_off = (uint32_t)(BTN::first_copy_offset(wave, lane, ldb) * 2);
         b_copy_step = (uint32_t)(BTN::copy_stride(ldb) * 2);
         b_k_step = BTN::ktile_stride(ldb) * 2;
@@ -421,46 +421,36 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // front of the tile origin: the tile exists, so its first row and its first 8 columns do)
     uint32_t a_voff[RAGGED ? Cfg::A_INSTS : 1];
     uint32_t b_voff[RAGGED ? Cfg::B_INSTS : 1];
-    // The lane index as a value the compiler knows nothing about: what is worked out from it between two tiles is worked out
-    // there, and does not take a register all through the K loop.
-    auto lane_here = [&]() {
-        int l = lane;
-        if constexpr (PERSIST) asm volatile("" : "+v"(l));
-        return l;
-    };
-    auto fold_offsets = [&]() {
-        if constexpr (RAGGED) {
-            const int lane = lane_here();
-            // byte offset from the tile base of copy i of this lane; origin / extent along the tile's M (or N) axis
-            auto clamped = [&](long ld, bool k_contig, int rows_per_inst, int chunks_per_row, int rows_per_pass, int i,
-                               long origin, long extent, int swz) {
-                const int row = wave * rows_per_inst + lane / chunks_per_row + i * rows_per_pass;
-                const int chunk = (lane % chunks_per_row) ^ swz;
-                if (k_contig) return (uint32_t)(((min(origin + row, extent - 1) - origin) * ld + chunk * 8) * 2);   // row = M/N index
-                return (uint32_t)(((long)row * ld + min(origin + chunk * 8, extent - 8) - origin) * 2);              // row = K index
-            };
+    if constexpr (RAGGED) {
+        // byte offset from the tile base of copy i of this lane; origin / extent along the tile's M (or N) axis
+        auto clamped = [&](long ld, bool k_contig, int rows_per_inst, int chunks_per_row, int rows_per_pass, int i,
+                           long origin, long extent, int swz) {
+            const int row = wave * rows_per_inst + lane / chunks_per_row + i * rows_per_pass;
+            const int chunk = (lane % chunks_per_row) ^ swz;
+            if (k_contig) return (uint32_t)(((min(origin + row, extent - 1) - origin) * ld + chunk * 8) * 2);   // row = M/N index
+            return (uint32_t)(((long)row * ld + min(origin + chunk * 8, extent - 8) - origin) * 2);              // row = K index
+        };
 #pragma unroll
-            for (int i = 0; i < Cfg::A_INSTS; ++i) {
-                if constexpr (A_KC) {
-                    const int row = wave * ATK::kRowsPerInst + lane / ATK::kChunksPerRow;
-                    a_voff[i] = clamped(lda, true, ATK::kRowsPerInst, ATK::kChunksPerRow, ATK::kRowsPerPass, i, m0, M, ATK::swz(row));
-                } else {
-                    const int row = wave * ATM::kRowsPerInst + lane / ATM::kChunksPerRow + i * ATM::kRowsPerPass;
-                    a_voff[i] = clamped(lda, false, ATM::kRowsPerInst, ATM::kChunksPerRow, ATM::kRowsPerPass, i, m0, (M + 7) & ~7, ATM::swz(row));
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < Cfg::B_INSTS; ++i) {
-                if constexpr (B_KC) {
-                    const int row = wave * BTK::kRowsPerInst + lane / BTK::kChunksPerRow;
-                    b_voff[i] = clamped(ldb, true, BTK::kRowsPerInst, BTK::kChunksPerRow, BTK::kRowsPerPass, i, n0, N, BTK::swz(row));
-                } else {
-                    const int row = wave * BTN::kRowsPerInst + lane / BTN::kChunksPerRow + i * BTN::kRowsPerPass;
-                    b_voff[i] = clamped(ldb, false, BTN::kRowsPerInst, BTN::kChunksPerRow, BTN::kRowsPerPass, i, n0, (N + 7) & ~7, BTN::swz(row));
-                }
+        for (int i = 0; i < Cfg::A_INSTS; ++i) {
+            if constexpr (A_KC) {
+                const int row = wave * ATK::kRowsPerInst + lane / ATK::kChunksPerRow;
+                a_voff[i] = clamped(lda, true, ATK::kRowsPerInst, ATK::kChunksPerRow, ATK::kRowsPerPass, i, m0, M, ATK::swz(row));
+            } else {
+                const int row = wave * ATM::kRowsPerInst + lane / ATM::kChunksPerRow + i * ATM::kRowsPerPass;
+                a_voff[i] = clamped(lda, false, ATM::kRowsPerInst, ATM::kChunksPerRow, ATM::kRowsPerPass, i, m0, (M + 7) & ~7, ATM::swz(row));
             }
         }
-    };
+#pragma unroll
+        for (int i = 0; i < Cfg::B_INSTS; ++i) {
+            if constexpr (B_KC) {
+                const int row = wave * BTK::kRowsPerInst + lane / BTK::kChunksPerRow;
+                b_voff[i] = clamped(ldb, true, BTK::kRowsPerInst, BTK::kChunksPerRow, BTK::kRowsPerPass, i, n0, N, BTK::swz(row));
+            } else {
+                const int row = wave * BTN::kRowsPerInst + lane / BTN::kChunksPerRow + i * BTN::kRowsPerPass;
+                b_voff[i] = clamped(ldb, false, BTN::kRowsPerInst, BTN::kChunksPerRow, BTN::kRowsPerPass, i, n0, (N + 7) & ~7, BTN::swz(row));
+            }
+        }
+    }
     // K need not be a multiple of the tile depth: the last K tile, which then holds K % 64 columns (rows) of the
     // operands, is taken FIRST, by the prologue, with copies of its own (below); the loop never sees it.
     const int ktiles = (K + BK - 1) / BK;
@@ -471,15 +461,16 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // this: 128 x 28672 x 4096 NT 54.3 / 47.7, 64 rows 52.0 / 47.9, 32 rows 49.5 / 43.5, 33 x 50257 85.7 / 82.0, 256 rows 84.6 / 81.8,
     // 128 x 6144 and 64 x 4096 x 14336 the same; more rows of tiles, and weights stored [K,N], whose rows lie side by side,
     // gain nothing or lose 1-4 %.
-    constexpr bool kStagger = A_KC && B_KC && !SPLIT_K && !PERSIST && BM <= 128 && BN <= 128;
+    constexpr bool kStagger = A_KC && B_KC && !SPLIT_K && BM <= 128 && BN <= 128;
     int before_wrap = ktiles;   // K tiles in front of the one at k = 0 that follows the last
-    if (kStagger && tiles_m <= 2 && k_first == BK) {
+    if (kStagger && M <= 2 * BM && k_first == BK) {
         static_assert(!kStagger || Cfg::NSTAGE_A == Cfg::NSTAGE_B, "whole turns of both rings in front of the wrap");
         const int whole = (ktiles - ktiles * (int)(blockIdx.x & 7) / 8) / Cfg::NSTAGE_A * Cfg::NSTAGE_A;
         if (whole > 0) before_wrap = whole;
     }
     const long first_tile = k_first < BK ? ktiles - 1 : ktiles - before_wrap;   // position along K, in tiles, of the tile taken first
-    int4v a_res, b_res;
+    int4v a_res = make_buffer_resource(a_base + first_tile * a_k_step);
+    int4v b_res = make_buffer_resource(b_base + first_tile * b_k_step);
 
     // ---- LDS fragment read offsets (bytes inside one stage) -------------------------------------------
     // A fragments: TM blocks of 16 rows; B fragments: TN blocks of 16 columns; a K tile is two 32-deep substeps.
@@ -522,22 +513,10 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     }
 
     float4v acc[TM][TN];
-    MI355_TL(auto record = [&](int tile) {   // of the tile just stored
-        wait_vmcnt<0>();   // the stores of this wave have been accepted
-        tl_w[3] = timeline::wall_clock();
-        if (tid == 0 && tile < timeline::kMaxWorkgroups) {
-            unsigned long long* rec = hgemm_stamps + (long)tile * timeline::kSlots;
-            rec[0] = tl_w[0]; rec[1] = tl_w[1]; rec[2] = tl_w[2]; rec[3] = tl_w[3];
-            rec[4] = tl_c[0]; rec[5] = tl_c[1]; rec[6] = (unsigned long long)((K + BK - 1) / BK); rec[7] = 0;
-        }
-    };)
-    auto clear_acc = [&]() {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
-    };
-    clear_acc();
+        for (int j = 0; j < TN; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
 
     // Software pipeline, pinned slot by slot (a slot = one MFMA 16x16x32 and what is issued in its shadow;
     // sched_barrier keeps the compiler from moving anything between slots):
@@ -668,8 +647,7 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // of the range of the resource (2 GiB for these copies; offsets inside a tile stay below that), and a copy that is
     // out of range writes zeros to LDS. Then the bases go back to k = 0 (with K a multiple of 64 the first tile is the
     // one at k = 0 and the bases move on to the next: the tiles are then walked in memory order).
-    auto fetch_first = [&]() {
-        const int lane = lane_here();
+    {
         constexpr uint32_t kOutOfRange = 0x80000000u;   // with any uniform offset added it stays at or above the range, without wrapping
         a_res[2] = (int)0x80000000u;
         b_res[2] = (int)0x80000000u;
@@ -696,9 +674,8 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
         });
         advance_base(a_res, k_first < BK ? -first_tile * a_k_step : a_k_step);
         advance_base(b_res, k_first < BK ? -first_tile * b_k_step : b_k_step);
-    };
-    // the copies of K tile sc, where A's (B's) ring has a stage for it
-    auto fetch_stage = [&](auto sc) {
+    }
+    static_for<1, NSB>([&](auto sc) {
         constexpr int t = decltype(sc)::value;
         const int records = sign_mask_scalar(t - ktiles);
         a_res[2] = records;
@@ -708,178 +685,142 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
         });
         if constexpr (t < NSA) advance_base(a_res, a_k_step);
         advance_base(b_res, b_k_step);
-    };
-    auto start_tile = [&](int id) {
-        int tile_m, tile_n;
-        tile_of_block(id, tiles_m, tiles_n, tile_m, tile_n);
-        m0 = (long)tile_m * BM;
-        n0 = (long)tile_n * BN;
-        a_res = make_buffer_resource((const char*)(A + (A_KC ? m0 * lda : m0)) + first_tile * a_k_step);
-        b_res = make_buffer_resource((const char*)(B + (B_KC ? n0 * ldb : n0)) + first_tile * b_k_step);
-        if constexpr (RAGGED) fold_offsets();
-        fetch_first();
-        static_for<1, NSA>(fetch_stage);
-    };
-    constexpr int TNO = EPI == 1 ? TN / 2 : TN;   // column blocks a wave stores
-    int id = blockIdx.x;
-    start_tile(id);
-    static_for<NSA, NSB>(fetch_stage);
+    });
     wait_vmcnt<Cfg::A_INSTS * (NSA - 1) + Cfg::B_INSTS * (NSB - 1)>();
-    for (;;) {
-        __syncthreads();
-        if constexpr (RAGGED && (A_KC || B_KC)) {
-            if ((k_first & 7) != 0) {   // K ends inside a 16-byte chunk of the rows: zeros for what its copy brought from behind K
-                const int chunk = k_first >> 3;
-                auto clear = [&](auto tk, MI355_LDS char* stage, int rows) {
-                    using TK = decltype(tk);
-                    for (int row = wave * 64 + lane_here(); row < rows; row += Cfg::NTHREADS) {
-                        MI355_LDS uint16_t* c = (MI355_LDS uint16_t*)(stage + row * TK::kRowBytes + ((chunk ^ TK::swz(row)) << 4));
-                        for (int e = k_first & 7; e < 8; ++e) c[e] = 0;
-                    }
-                };
-                if constexpr (A_KC) clear(ATK{}, smem, BM);
-                if constexpr (B_KC) clear(BTK{}, smem + kBRegion, BN);
-                __syncthreads();
-            }
-        }
-        load_frags(Sub0{}, Sub0{}, af[0], bf[0]);
-
-        // One K tile in stage sc (a compile-time constant: the loop below is unrolled over the ring). Every tile issues the
-        // same instructions, so the count the waits rely on never changes: once no tile is left to fetch, the copies run on
-        // an empty buffer (num_records = 0: out of range, nothing is fetched).
-        auto tile = [&](auto sc, int kt) {
-            using Next = std::integral_constant<int, (decltype(sc)::value + 1) % kUnroll>;
-            substep(af[0], bf[0], [&](auto mc) { frags_of_slot(sc, Sub1{}, mc, af[1], bf[1]); });
-            // my copies of the next tile have landed and my reads of this stage are complete; after the barrier that holds
-            // for every wave, so this stage may be refilled and the next one may be read
-            wait_vmcnt<Cfg::A_INSTS * (NSA - 2) + Cfg::B_INSTS * (NSB - 2)>();
-            __syncthreads();
-            a_res[2] = sign_mask_scalar(kt + NSA - ktiles);   // -1 while a tile is left to fetch, else 0
-            b_res[2] = NSA == NSB ? a_res[2] : sign_mask_scalar(kt + NSB - ktiles);
-            substep(af[1], bf[1], [&](auto mc) {
-                frags_of_slot(Next{}, Sub0{}, mc, af[0], bf[0]);
-                copies_of_slot(sc, mc);   // tiles kt + NSA of A, kt + NSB of B
-            });
-            advance_base(a_res, a_k_step);
-            advance_base(b_res, b_k_step);
-        };
-        int kt = 0;
-        MI355_TL(tl_w[1] = timeline::wall_clock(); tl_c[0] = timeline::shader_cycles();)
-        // (the copies run NSA tiles ahead: they go back to k = 0 when the tile NSA in front of the wrap is next)
-        for (int stop = before_wrap < ktiles ? before_wrap - NSA : ktiles;; stop = ktiles) {
-            for (; kt < stop; kt += kUnroll)
-                static_for<0, kUnroll>([&](auto sc) {
-                    if (kt + decltype(sc)::value < ktiles) tile(sc, kt + decltype(sc)::value);
-                });
-            if (!kStagger || stop == ktiles) break;
-            advance_base(a_res, -ktiles * a_k_step);
-            advance_base(b_res, -ktiles * b_k_step);
-        }
-        MI355_TL(tl_w[2] = timeline::wall_clock(); tl_c[1] = timeline::shader_cycles();)
-
-        // ---- epilogue ------------------------------------------------------------------------------------------------
-        static_assert(Cfg::NWAVES * TM * 16 * TNO * 32 <= Cfg::LDS_BYTES, "epilogue staging does not fit in LDS");
-        wait_vmcnt<0>();  // the last tiles' copies (on the empty buffer) have written their zeros
-        __syncthreads();  // every wave has finished reading the operand stages
-        const int lane = lane_here();
-        if constexpr (SPLIT_K) {
-            if (kOwnMergeOnly<BM, BN> || counters == nullptr) {   // the partial tiles are merged by a kernel of their own: [range][padded M][padded N]
-                const long np = (long)((N + BN - 1) / BN) * BN, mp = (long)((M + BM - 1) / BM) * BM;
-                float* dst = part + ((long)blockIdx.y * mp + m0 + wm * TM * 16 + (lane & 15)) * np + n0 + wn * TN * 16 + 4 * (lane >> 4);
-#pragma unroll
-                for (int b = 0; b < TM * TN; ++b) *(float4v*)(dst + (long)(b / TN) * 16 * np + (b % TN) * 16) = acc[b / TN][b % TN];
-                return;
-            }
-            if constexpr (!kOwnMergeOnly<BM, BN>) {
-                // partial tile (tile, range): pair p (two floats) of lane t's accumulator block b at pair (b * 2 + p) * NTHREADS + t,
-                // so that every store and load instruction of a wave covers 512 contiguous bytes
-                constexpr int NB = TM * TN;
-                constexpr long kTilePairs = (long)Cfg::NTHREADS * NB * 2;
-                uint64_t* const tile_part = reinterpret_cast<uint64_t*>(part) + (long)blockIdx.x * splits * kTilePairs + tid;
-                uint64_t* const mine = tile_part + (long)blockIdx.y * kTilePairs;
-                // (device-scope atomic stores, i.e. `global_store_dwordx2 .. sc1`, written as such so that the compiler places the
-                // wait states between the last matrix instructions and the first memory instruction that reads their result: a
-                // wave that arrives last at the barrier above is only a few cycles behind its last MFMA)
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-#pragma unroll
-                    for (int p = 0; p < 2; ++p) {
-                        const float4v v = acc[b / TN][b % TN];
-                        const uint64_t w = (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2 * p]) | (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2 * p + 1]) << 32;
-                        __hip_atomic_store(mine + (long)(b * 2 + p) * Cfg::NTHREADS, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    }
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's part has reached memory before the ticket is drawn
-                __syncthreads();
-                MI355_LDS unsigned* ticket_sh = (MI355_LDS unsigned*)smem;
-                if (tid == 0) *ticket_sh = __hip_atomic_fetch_add(&counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __syncthreads();
-                const unsigned ticket = *ticket_sh;
-                __syncthreads();   // the epilogue below reuses that LDS
-                if (ticket != (unsigned)(splits - 1)) return;
-                // The last one: every other workgroup of this tile drew its ticket after its part had reached memory. The parts
-                // are read with device-coherent loads and added in the order of the ranges, this workgroup's own part too (it is
-                // what the registers hold, but a fixed place for it would cost more registers than the load costs time). A batch
-                // of loads is a round trip to memory of ~1 us whatever its size, so a batch is as large as the registers allow:
-                // 64 registers of a lane, all blocks of one to four ranges.
-                constexpr int kChunk = NB < 16 ? NB : 16, kBatch = 16 / kChunk < 4 ? 16 / kChunk : 4;
-                static_assert(NB % kChunk == 0, "whole chunks of blocks");
-#pragma unroll
-                for (int b0 = 0; b0 < NB; b0 += kChunk) {
-                    float4v sum[kChunk];
-#pragma unroll
-                    for (int b = 0; b < kChunk; ++b) sum[b] = float4v{0.f, 0.f, 0.f, 0.f};
-                    for (int r0 = 0; r0 < splits; r0 += kBatch) {
-                        uint64_t v[kBatch][kChunk][2];
-#pragma unroll
-                        for (int u = 0; u < kBatch; ++u) {
-                            const uint64_t* pa = tile_part + (long)min(r0 + u, splits - 1) * kTilePairs + (long)b0 * 2 * Cfg::NTHREADS;
-#pragma unroll
-                            for (int b = 0; b < kChunk * 2; ++b)
-                                v[u][b / 2][b % 2] = __hip_atomic_load(pa + (long)b * Cfg::NTHREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);   // all loads of the batch are issued before the first is waited for
-#pragma unroll
-                        for (int u = 0; u < kBatch; ++u)
-                            if (r0 + u < splits)
-#pragma unroll
-                                for (int b = 0; b < kChunk; ++b)
-#pragma unroll
-                                    for (int q = 0; q < 4; ++q) sum[b][q] += __builtin_bit_cast(float, (uint32_t)(v[u][b][q / 2] >> (32 * (q & 1))));
-                    }
-#pragma unroll
-                    for (int b = 0; b < kChunk; ++b) acc[(b0 + b) / TN][(b0 + b) % TN] = sum[b];
+    __syncthreads();
+    if constexpr (RAGGED && (A_KC || B_KC)) {
+        if ((k_first & 7) != 0) {   // K ends inside a 16-byte chunk of the rows: zeros for what its copy brought from behind K
+            const int chunk = k_first >> 3;
+            auto clear = [&](auto tk, MI355_LDS char* stage, int rows) {
+                using TK = decltype(tk);
+                for (int row = tid; row < rows; row += Cfg::NTHREADS) {
+                    MI355_LDS uint16_t* c = (MI355_LDS uint16_t*)(stage + row * TK::kRowBytes + ((chunk ^ TK::swz(row)) << 4));
+                    for (int e = k_first & 7; e < 8; ++e) c[e] = 0;
                 }
-                if (tid == 0) __hip_atomic_store(&counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        const long row0 = m0 + wm * TM * 16, col0 = (EPI == 1 ? n0 / 2 : n0) + wn * TNO * 16;
-        const int NC = EPI == 1 ? N / 2 : N;   // columns of C
-        if constexpr (!PERSIST) {
-            store_wave_tile<T, TM, TN, EPI, RAGGED, TM, 1024>(acc, smem + wave * (TM * 16 * TNO * 32), C, R, row0, col0, M, NC, ldc, ldr, lane);
-            MI355_TL(record(id);)
-            break;
-        } else {
-            // The next tile's copies go out in front of this tile's stores, into every stage but B's last: that one is where the
-            // waves park 32 rows of C at a time, each in the four pieces of 1 KiB that its own copies into that stage will fill,
-            // so that no wave waits for another here.
-            const int done = id;
-            id += gridDim.x;
-            const bool more = id < tiles_m * tiles_n;
-            if (more) start_tile(id);
-            static_assert(NSB == NSA + 1 && Cfg::B_INSTS * 1024 >= 2 * 16 * TNO * 32, "B's last stage holds 32 rows of every wave");
-            store_wave_tile<T, TM, TN, EPI, RAGGED, 2, Cfg::NWAVES * 1024>(acc, smem + kBRegion + (NSB - 1) * Cfg::B_BYTES + wave * 1024, C, R, row0,
-                                                                           col0, M, NC, ldc, ldr, lane);
-            MI355_TL(record(done); tl_w[0] = tl_w[3];)
-            if (!more) break;
-            wait_lgkmcnt<0>();   // what this wave parked has been read
-            static_for<NSA, NSB>(fetch_stage);
-            // the tile's first stages have landed: behind them went the other copies and, counted only where their number is
-            // fixed, the stores (the counter is in the order of issue)
-            constexpr int kStores = RAGGED ? 0 : TM * 16 * TNO * 32 / 1024;
-            wait_vmcnt<Cfg::A_INSTS * (NSA - 1) + Cfg::B_INSTS * (NSB - 1) + kStores>();
-            clear_acc();
+            };
+            if constexpr (A_KC) clear(ATK{}, smem, BM);
+            if constexpr (B_KC) clear(BTK{}, smem + kBRegion, BN);
+            __syncthreads();
         }
     }
+    load_frags(Sub0{}, Sub0{}, af[0], bf[0]);
+
+    // One K tile in stage sc (a compile-time constant: the loop below is unrolled over the ring). Every tile issues the
+    // same instructions, so the count the waits rely on never changes: once no tile is left to fetch, the copies run on
+    // an empty buffer (num_records = 0: out of range, nothing is fetched).
+    auto tile = [&](auto sc, int kt) {
+        using Next = std::integral_constant<int, (decltype(sc)::value + 1) % kUnroll>;
+        substep(af[0], bf[0], [&](auto mc) { frags_of_slot(sc, Sub1{}, mc, af[1], bf[1]); });
+        // my copies of the next tile have landed and my reads of this stage are complete; after the barrier that holds
+        // for every wave, so this stage may be refilled and the next one may be read
+        wait_vmcnt<Cfg::A_INSTS * (NSA - 2) + Cfg::B_INSTS * (NSB - 2)>();
+        __syncthreads();
+        a_res[2] = sign_mask_scalar(kt + NSA - ktiles);   // -1 while a tile is left to fetch, else 0
+        b_res[2] = NSA == NSB ? a_res[2] : sign_mask_scalar(kt + NSB - ktiles);
+        substep(af[1], bf[1], [&](auto mc) {
+            frags_of_slot(Next{}, Sub0{}, mc, af[0], bf[0]);
+            copies_of_slot(sc, mc);   // tiles kt + NSA of A, kt + NSB of B
+        });
+        advance_base(a_res, a_k_step);
+        advance_base(b_res, b_k_step);
+    };
+    int kt = 0;
+    MI355_TL(tl_w[1] = timeline::wall_clock(); tl_c[0] = timeline::shader_cycles();)
+    // (the copies run NSA tiles ahead: they go back to k = 0 when the tile NSA in front of the wrap is next)
+    for (int stop = before_wrap < ktiles ? before_wrap - NSA : ktiles;; stop = ktiles) {
+        for (; kt < stop; kt += kUnroll)
+            static_for<0, kUnroll>([&](auto sc) {
+                if (kt + decltype(sc)::value < ktiles) tile(sc, kt + decltype(sc)::value);
+            });
+        if (!kStagger || stop == ktiles) break;
+        advance_base(a_res, -ktiles * a_k_step);
+        advance_base(b_res, -ktiles * b_k_step);
+    }
+    MI355_TL(tl_w[2] = timeline::wall_clock(); tl_c[1] = timeline::shader_cycles();)
+
+    // ---- epilogue ------------------------------------------------------------------------------------------------
+    constexpr int TNO = EPI == 1 ? TN / 2 : TN;   // column blocks a wave stores
+    static_assert(Cfg::NWAVES * TM * 16 * TNO * 32 <= Cfg::LDS_BYTES, "epilogue staging does not fit in LDS");
+    wait_vmcnt<0>();  // the last tiles' copies (on the empty buffer) have written their zeros
+    __syncthreads();  // every wave has finished reading the operand stages
+    if constexpr (SPLIT_K) {
+        if (kOwnMergeOnly<BM, BN> || counters == nullptr) {   // the partial tiles are merged by a kernel of their own: [range][padded M][padded N]
+            const long np = (long)((N + BN - 1) / BN) * BN, mp = (long)((M + BM - 1) / BM) * BM;
+            float* dst = part + ((long)blockIdx.y * mp + m0 + wm * TM * 16 + (lane & 15)) * np + n0 + wn * TN * 16 + 4 * (lane >> 4);
+#pragma unroll
+            for (int b = 0; b < TM * TN; ++b) *(float4v*)(dst + (long)(b / TN) * 16 * np + (b % TN) * 16) = acc[b / TN][b % TN];
+            return;
+        }
+        // partial tile (tile, range): pair p (two floats) of lane t's accumulator block b at pair (b * 2 + p) * NTHREADS + t,
+        // so that every store and load instruction of a wave covers 512 contiguous bytes
+        constexpr int NB = TM * TN;
+        constexpr long kTilePairs = (long)Cfg::NTHREADS * NB * 2;
+        uint64_t* const tile_part = reinterpret_cast<uint64_t*>(part) + (long)blockIdx.x * splits * kTilePairs + tid;
+        uint64_t* const mine = tile_part + (long)blockIdx.y * kTilePairs;
+        // (device-scope atomic stores, i.e. `global_store_dwordx2 .. sc1`, written as such so that the compiler places the
+        // wait states between the last matrix instructions and the first memory instruction that reads their result: a
+        // wave that arrives last at the barrier above is only a few cycles behind its last MFMA)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const float4v v = acc[b / TN][b % TN];
+                const uint64_t w = (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2 * p]) | (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2 * p + 1]) << 32;
+                __hip_atomic_store(mine + (long)(b * 2 + p) * Cfg::NTHREADS, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's part has reached memory before the ticket is drawn
+        __syncthreads();
+        MI355_LDS unsigned* ticket_sh = (MI355_LDS unsigned*)smem;
+        if (tid == 0) *ticket_sh = __hip_atomic_fetch_add(&counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const unsigned ticket = *ticket_sh;
+        __syncthreads();   // the epilogue below reuses that LDS
+        if (ticket != (unsigned)(splits - 1)) return;
+        // The last one: every other workgroup of this tile drew its ticket after its part had reached memory. The parts
+        // are read with device-coherent loads and added in the order of the ranges, this workgroup's own part too (it is
+        // what the registers hold, but a fixed place for it would cost more registers than the load costs time). A batch
+        // of loads is a round trip to memory of ~1 us whatever its size, so a batch is as large as the registers allow:
+        // 64 registers of a lane, all blocks of one to four ranges.
+        constexpr int kChunk = NB < 16 ? NB : 16, kBatch = 16 / kChunk < 4 ? 16 / kChunk : 4;
+        static_assert(NB % kChunk == 0, "whole chunks of blocks");
+#pragma unroll
+        for (int b0 = 0; b0 < NB; b0 += kChunk) {
+            float4v sum[kChunk];
+#pragma unroll
+            for (int b = 0; b < kChunk; ++b) sum[b] = float4v{0.f, 0.f, 0.f, 0.f};
+            for (int r0 = 0; r0 < splits; r0 += kBatch) {
+                uint64_t v[kBatch][kChunk][2];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    const uint64_t* pa = tile_part + (long)min(r0 + u, splits - 1) * kTilePairs + (long)b0 * 2 * Cfg::NTHREADS;
+#pragma unroll
+                    for (int b = 0; b < kChunk * 2; ++b)
+                        v[u][b / 2][b % 2] = __hip_atomic_load(pa + (long)b * Cfg::NTHREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                __builtin_amdgcn_sched_barrier(0);   // all loads of the batch are issued before the first is waited for
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u)
+                    if (r0 + u < splits)
+#pragma unroll
+                        for (int b = 0; b < kChunk; ++b)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) sum[b][q] += __builtin_bit_cast(float, (uint32_t)(v[u][b][q / 2] >> (32 * (q & 1))));
+            }
+#pragma unroll
+            for (int b = 0; b < kChunk; ++b) acc[(b0 + b) / TN][(b0 + b) % TN] = sum[b];
+        }
+        if (tid == 0) __hip_atomic_store(&counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    store_wave_tile<T, TM, TN, EPI, RAGGED>(acc, smem + wave * (TM * 16 * TNO * 32), C, R, m0 + wm * TM * 16,
+                                            (EPI == 1 ? n0 / 2 : n0) + wn * TNO * 16, M, EPI == 1 ? N / 2 : N, ldc, ldr, lane);
+    MI355_TL(
+        wait_vmcnt<0>();   // the stores of this wave have been accepted
+        tl_w[3] = timeline::wall_clock();
+        if (tid == 0 && blockIdx.x < timeline::kMaxWorkgroups) {
+            unsigned long long* rec = hgemm_stamps + (long)blockIdx.x * timeline::kSlots;
+            rec[0] = tl_w[0]; rec[1] = tl_w[1]; rec[2] = tl_w[2]; rec[3] = tl_w[3];
+            rec[4] = tl_c[0]; rec[5] = tl_c[1]; rec[6] = (unsigned long long)ktiles; rec[7] = 0;
+        })
 }
 
 // Merges the partial tiles of a split-K launch without counters: C = sum over the ranges, in their order (+ R after the
@@ -1639,17 +1580,21 @@ static hipError_t launch_smallm_nt_norm(const T* A, const T* norm_weight, float 
     }
 }
 
+// One workgroup per tile, so that a CU is given back after every tile. (256 workgroups that walk the tiles, and request the next
+// tile's operands in front of the stores of the last, gain 0.1-0.4 % of a product alone: 8192^3 NN 805.2 us against 805.8. With one CU held by
+// a kernel of another stream the workgroup left over begins its walk when the others end theirs, 8192^3 1.66 times its time alone
+// against 1.10, 8192 x 28672 x 4096 gate/up 1.80 against 1.02; an RMSNorm of 8 rows on another stream waits for the whole product, 791 us
+// against 83.)
 template <typename T, bool A_KC, bool B_KC, int BM, int BN, int WM, int WN, int EPI = 0, bool RAGGED = false, int STAGES = 0, int PER_CU = 1>
 static hipError_t launch_main(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
                               long ldc, long ldr, hipStream_t stream) {
     using Cfg = MainCfg<A_KC, B_KC, BM, BN, WM, WN, STAGES>;
-    constexpr bool kPersist = BM == 256 && BN == 256;
-    auto kern = hgemm_main_kernel<T, A_KC, B_KC, BM, BN, WM, WN, EPI, RAGGED, STAGES, PER_CU, false, kPersist>;
+    auto kern = hgemm_main_kernel<T, A_KC, B_KC, BM, BN, WM, WN, EPI, RAGGED, STAGES, PER_CU>;
     static DynamicLdsOnce lds_once;
     if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES); e != hipSuccess) return e;
     const long nblocks = (long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
-    int blocks = kPersist && nblocks > 256 ? 256 : (int)nblocks;
+    const int blocks = (int)nblocks;
     MI355_TL(timeline_hgemm_reader = &read_hgemm_stamps;)
     kern<<<dim3(blocks), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, stream>>>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, nullptr, nullptr, 1);
     return hipGetLastError();
