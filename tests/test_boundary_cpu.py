@@ -48,6 +48,25 @@ def test_profiling_twin_exports_the_library_plus_its_readers(lib):
     assert twin.mi355_timeline_stream_read(None, ctypes.c_size_t(64), None, None) != 0   # null pointers: refused, nothing launched
 
 
+def test_a_refused_step_kernel_leaves_no_error_text(lib):
+    """The decoder layer offers its first two products to the step's kernels and goes on with the single calls where they refuse:
+    a forward pass that succeeds leaves the text of the caller's last failure as it was. (Refused before anything is launched.)"""
+    cdll = lib.load()
+    p = ctypes.c_void_p(0x1000)
+
+    def qkv(B, S, hidden, norm=p):
+        return cdll.mi355_internal_step_qkv(p, norm, 1e-5, p, p, p, B, S, 8, 2, hidden, S * 1536, 1536, 128, p, p, p, 0, 16, 0, None)
+
+    assert cdll.mi355_hgemm(None, None, None, 4, 4, 4, 4, 4, 4, 0, None) == lib.ERR_BAD_ARGUMENT
+    text = cdll.mi355_last_error()
+    for rows, hidden in ((65, 1024), (9, 1024), (8, 4096), (1, 1000), (1, 512)):     # beyond 64 rows, 8, a CU's LDS; widths
+        assert qkv(rows, 1, hidden) == qkv(1, rows, hidden) == lib.ERR_UNSUPPORTED
+    for rows, hidden in ((9, 1024), (8, 4096), (1, 1000), (1, 512)):
+        assert cdll.mi355_internal_step_gate_up(p, p, 1e-5, p, p, rows, 2816, hidden, 0, None) == lib.ERR_UNSUPPORTED
+    assert cdll.mi355_last_error() == text
+    assert qkv(0, 1, 1024) == lib.ERR_BAD_ARGUMENT and b"step_qkv" in cdll.mi355_last_error()
+
+
 def test_capi_rejects_bad_arguments_without_a_gpu(lib):
     cdll = lib.load()
     assert cdll.mi355_hgemm(None, None, None, 4, 4, 4, 4, 4, 4, 0, None) == 10001

@@ -385,13 +385,15 @@ int mi355_silu_mul_bf16(const void* gate_up, void* out, int64_t rows, int inter,
 }
 
 
-// Used by the decoder layer only (declared in mi355_serving_internal.h).
+// Used by the decoder layer only (declared in mi355_serving_internal.h). A refusal (MI355_ERR_UNSUPPORTED) is no failure, its caller goes
+// on with the single calls: it writes no text.
 int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, const void* w_qkv, void* qkv, void* kv_out, int B, int S, int q_heads,
                             int kv_heads, int hidden, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
                             const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions, int dtype, void* stream) {
     const char* fn = "mi355_internal_step_qkv";
     if (!x || !w_qkv || hidden < 1) return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer or no columns", fn);
-    if (B < 1 || S < 1 || (int64_t)B * S > 64) return fail(MI355_ERR_UNSUPPORTED, "%s: at most 64 rows", fn);
+    if (B < 1 || S < 1) return fail(MI355_ERR_BAD_ARGUMENT, "%s: no rows", fn);
+    if ((int64_t)B * S > 64) return MI355_ERR_UNSUPPORTED;
     if (q_heads < 1 || kv_heads < 1 || q_heads > (1 << 20) || kv_heads > (1 << 20))
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: q_heads and kv_heads must be >= 1", fn);
     const int64_t width = ((int64_t)q_heads + 2 * (int64_t)kv_heads) * 128;
@@ -401,7 +403,7 @@ int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, c
                                       n_positions, S, q_heads, kv_heads};
     const hipError_t e = mi355::gemm_step_qkv_dispatch(x, {norm_weight, eps}, w_qkv, qkv, B * S, (int)width, hidden, rope, dtype,
                                                        static_cast<hipStream_t>(stream));
-    if (e == hipErrorNotSupported) return fail(MI355_ERR_UNSUPPORTED, "%s: no such kernel for these sizes", fn);
+    if (e == hipErrorNotSupported) return MI355_ERR_UNSUPPORTED;
     return e == hipSuccess ? 0 : hip_fail(e, fn);
 }
 
@@ -412,7 +414,7 @@ int mi355_internal_step_gate_up(const void* x, const void* norm_weight, float ep
         return fail(MI355_ERR_BAD_ARGUMENT, "%s: null pointer or empty operand", fn);
     const hipError_t e = mi355::gemm_step_gate_up_dispatch(x, {norm_weight, eps}, w_gu, out, rows, 2 * inter, hidden, dtype,
                                                            static_cast<hipStream_t>(stream));
-    if (e == hipErrorNotSupported) return fail(MI355_ERR_UNSUPPORTED, "%s: no such kernel for these sizes", fn);
+    if (e == hipErrorNotSupported) return MI355_ERR_UNSUPPORTED;
     return e == hipSuccess ? 0 : hip_fail(e, fn);
 }
 

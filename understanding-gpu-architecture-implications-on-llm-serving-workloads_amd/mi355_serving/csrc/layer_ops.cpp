@@ -1,4 +1,4 @@
-// One call per forward pass of llama_layer.FineLlamaDecoderLayer: the eight launches of the layer (five for up to 8 rows) issued
+// One call per forward pass of llama_layer.FineLlamaDecoderLayer: the eight launches of the layer (down to five for up to 8 rows) issued
 // back to back from C++ through the C ABI of libmi355_serving.so. Issued one by one from Python (ctypes calls, tensor views, one
 // allocation per intermediate) eight take the host ~85-95 us per layer, longer than a generation step keeps the GPU busy on any
 // layer narrower than ~4096; from here ~25 us, with one block of torch's allocator for the intermediates: a step of one
@@ -155,17 +155,18 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
             v = view(kv[2], keys, n_kv, "values");
         }
     }
-    // Norm, projection and rotary embedding of a few rows are one launch (two with the norm on its own where the attention block
-    // is timed, which begins behind it), of more rows three.
+    // Norm, projection and rotary embedding of up to 8 rows are one launch where their norm pays inside the product (norm_fits in
+    // hgemm.hip), two where it does not, where the attention block is timed, which begins behind it, and of up to 64 rows whose
+    // projection is the small-M kernel's; three otherwise.
     const auto step_qkv = [&](const void* in, const void* norm_weight) {
         if (rows > 64) return false;
         const int rc = mi355_internal_step_qkv(in, norm_weight, (float)eps, w_qkv.data_ptr(), qkv, fresh.ptr, (int)B, (int)S, (int)n_q, (int)n_kv, (int)H,
                                                fresh.batch, fresh.row, fresh.head, cos_p, sin_p, pos, pos_batch, n_pos, dtype, stream);
-        if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_rope_qkv");
+        if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_internal_step_qkv");
         return rc == 0;
     };
     Events ev;
-    if (timed || !step_qkv(x.data_ptr(), ln1.data_ptr())) {
+    if (timed || rows > 8 || !step_qkv(x.data_ptr(), ln1.data_ptr())) {
         norm(x.data_ptr(), ln1);
         if (timed) {
             CHECK_HIP(hipEventCreate(&ev.begin));
@@ -202,9 +203,9 @@ std::tuple<at::Tensor, double> layer_forward(const at::Tensor& hidden_states, co
         ms = elapsed;
     }
     int rc = MI355_ERR_UNSUPPORTED;
-    if (gate_up_block > 0 && rows <= 16) {
+    if (gate_up_block > 0 && rows <= 8) {
         rc = mi355_internal_step_gate_up(out.data_ptr(), ln2.data_ptr(), (float)eps, w_gu.data_ptr(), act, (int)rows, (int)F, (int)H, dtype, stream);
-        if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_hgemm_silu_mul");
+        if (rc != MI355_ERR_UNSUPPORTED) check(rc, "mi355_internal_step_gate_up");
     }
     const bool normalised = rc == 0;
     if (!normalised) norm(out.data_ptr(), ln2);
