@@ -267,6 +267,48 @@ def test_step_gate_up_equals_the_launches_it_replaces(lib, gpu, dtype, rows, F, 
     assert torch.equal(out[:rows], ref) and bool((out[rows:] == 3.0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [8192, 8704, 11776])
+def test_step_kernels_at_the_widest_rows_they_take(lib, gpu, dtype, hidden):
+    """One row up to 11776 wide (RMSNorm keeps up to 4096 and 8192 in registers, walks wider ones twice): the single launches' bits,
+    the projection's on the small-M kernel."""
+    test_step_qkv_equals_the_launches_it_replaces(lib, gpu, dtype, True, 1, 1, 3, 1, hidden, True)
+    test_step_gate_up_equals_the_launches_it_replaces(lib, gpu, dtype, 1, 96, hidden)
+
+
+@pytest.mark.parametrize("rows,F,hidden,taken", [
+    (8, 7168, 2048, True), (8, 8192, 2048, True), (8, 8224, 2048, False),          # two rounds of 512 workgroups, three
+    (5, 4096, 2560, True), (8, 4128, 2560, False), (8, 8960, 1536, False), (8, 8960, 1024, True),
+    (4, 14336, 3072, True), (4, 14336, 4096, False), (3, 18944, 3584, False), (4, 8192, 4096, False),   # last: the rows-in-registers kernel applies
+    (4, 11008, 4096, True), (2, 14336, 4096, True), (1, 8192, 4096, False), (1, 4096, 4096, True), (2, 18944, 3584, True)])
+def test_norm_is_part_of_the_gate_up_product_only_where_it_pays(lib, gpu, rows, F, hidden, taken):
+    x, ln = torch.randn(rows, hidden, device=gpu).half(), torch.ones(hidden, device=gpu, dtype=torch.float16)
+    w, out = torch.zeros(2 * F, hidden, device=gpu, dtype=torch.float16), torch.empty(rows, F, device=gpu, dtype=torch.float16)
+    rc = lib.load().mi355_internal_step_gate_up(x.data_ptr(), ln.data_ptr(), 1e-5, w.data_ptr(), out.data_ptr(), rows, F, hidden, 0, 0)
+    torch.cuda.synchronize()
+    assert rc == (0 if taken else lib.ERR_UNSUPPORTED)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [3, 4, 8])
+def test_step_gate_up_of_rows_without_finite_values(lib, gpu, dtype, rows):
+    """A row of zeros, one with an infinity, one with a NaN, one whose squares overflow nothing but fp16: the single launches' results,
+    and each row's its own (the rows share LDS and the reductions)."""
+    hidden, F = 1536, 160
+    x = (3 * so.randn_fp16((rows, hidden), 1)).to(dtype).to(gpu)
+    x[0], x[1, 700], x[2, 1535] = 0, float("inf"), float("nan")
+    x[-1, 5] = 60000.0
+    ln, w = (1 + so.randn_fp16((hidden,), 2, 0.1)).to(dtype).to(gpu), so.randn_fp16((2 * F, hidden), 3, 0.05).to(dtype).to(gpu)
+    ref = lib.hgemm_silu_mul(lib.rmsnorm(x, ln, 1e-5), w, "NT")
+    out = torch.empty_like(ref)
+    assert lib.load().mi355_internal_step_gate_up(x.data_ptr(), ln.data_ptr(), 1e-5, w.data_ptr(), out.data_ptr(), rows, F, hidden,
+                                                  lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, 0) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.nan_to_num(), ref.nan_to_num())
+    assert bool((out[0] == 0).all()) and bool(out[1].isnan().all()) and bool(out[2].isnan().all())
+    assert rows == 3 or not bool(out[3:].isnan().any())
+
+
 def layer_weights(H, n_q, n_kv, F, seed=0):
     D = 128
     g = lambda shape, s, std: so.randn_fp16(shape, seed + s, std)
@@ -322,6 +364,25 @@ def test_decoder_layer_positions_of_each_row_and_strided_hidden_states(lib, gpu,
     for bad in (rows[:, :, None].expand(B, S, 2), rows.repeat(2, 1)):
         with pytest.raises((AssertionError, RuntimeError)):
             layer(xg, bad.to(gpu))
+
+
+@pytest.mark.parametrize("B", [2, 3, 4, 5, 8, 9])
+def test_decoder_layer_step_4096_wide_on_both_sides_of_the_fused_norm(lib, gpu, B):
+    """Up to 4 rows of 4096 fit a CU's LDS beside the weights, 5 to 8 take the norm as a launch of its own."""
+    from llama_layer import FineKVCache, FineLlamaDecoderLayer
+    H, n_q, n_kv, F, past = 4096, 4, 1, 1024, 40
+    w = layer_weights(H, n_q, n_kv, F, seed=70)
+    layer = FineLlamaDecoderLayer({k: v.to(gpu) for k, v in w.items()}, n_q, n_kv, max_positions=64)
+    cache = FineKVCache(B, past + 1, n_kv, device=gpu)
+    k_past, v_past = (so.randn_fp16((B, n_kv, past, 128), 80 + i) for i in range(2))
+    cache.k[:, :past], cache.v[:, :past] = k_past.transpose(1, 2).to(gpu), v_past.transpose(1, 2).to(gpu)
+    cache.length = past
+    x = so.randn_fp16((B, 1, H), 90 + B)
+    out = layer(x.to(gpu), kv_cache=cache)
+    ref, k_ref, v_ref = so.llama_decoder_layer_ref(x, w, torch.full((B, 1), past), n_q, n_kv, past_k=k_past, past_v=v_past)
+    ok, st = layer_close(out, ref)
+    assert ok, st
+    assert (cache.k.transpose(1, 2).float().cpu() - k_ref).abs().max() <= 2e-2 and (cache.v.transpose(1, 2).float().cpu() - v_ref).abs().max() <= 2e-2
 
 
 def test_decoder_layer_generation_steps_with_cache(lib, gpu):

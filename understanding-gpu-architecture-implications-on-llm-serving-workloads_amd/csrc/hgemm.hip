@@ -1763,12 +1763,23 @@ static hipError_t launch_silu_mul(const T* A, const T* B, T* C, int M, int N, in
 // The first two products of a generation step's layer, few enough rows for the small-M kernel of layout NT, with what stands
 // around them: the RMSNorm of their rows in front (norm.weight != nullptr), rotary embedding and the way into the KV cache behind
 // the QKV projection. hipErrorNotSupported: no such kernel for this call, nothing was launched.
-// Every workgroup normalises the rows for itself (~0.2 us a row, hidden behind the first weights in part), which is repaid as long
-// as two workgroups with their rows fit a CU's LDS. us per pass of a layer, norms on their own / in the products: 1024 wide, 8 rows
-// 27.4 / 26.7, 1 row 27.2 / 22.1; 2048 wide, 8 rows 47.1 / 45.1, 4 rows 45.7 / 41.0; 4096 wide, 4 rows 92.7 / 92.2, 1 row 92 / 87.2.
-static bool norm_fits(const NormPrologue& norm, int M, int K) {
-    return M <= 8 && K >= 1024 && K % 512 == 0 && smallm_nt_norm_lds(M, K) <= kNormLdsMax - 1024 &&
-           reinterpret_cast<uintptr_t>(norm.weight) % 16 == 0;
+// Every workgroup normalises the rows for itself (~0.2 us a row, hidden behind the first weights in part), with two workgroups and
+// their rows on a CU at most, so a product of many workgroups pays for it once per round of 512, and for more than two rows that
+// exceeds the launch it saves where the rows are long. us, weights from HBM, norm on its own / in the product: gate/up 8 rows 1536 x
+// 4096 9.7 / 8.7 (1 round), x 8960 15.6 / 18.2 (3), 2048 x 7168 16.2 / 15.5 (2), x 16384 28.8 / 31.0 (4), 2560 x 4096 12.8 / 11.6 (1), x 6912
+// 19.1 / 19.5 (2); 4 rows 2560 x 10240 23.1 / 22.2 (3), 3072 x 16384 38.1 / 37.3 (4), 3584 x 18944 48.7 / 48.8 (5), 4096 x 11008 35.1 / 34.0
+// (3), x 14336 41.7 / 43.2 (4); 1 and 2 rows gain 0 - 3 us at any width (4096 x 14336 41.6 / 41.7, 6144 x 24576 100.6 / 98.8, 8192 x 28672,
+// one row, 152.4 / 151.0). Over more than one round the kernel that keeps the rows in registers is the better one where it
+// applies (4096 x 8192, 4 rows, 27.6 / 28.4, 1 row 27.3 / 27.6). QKV projections are one or two rounds: 4096 x 6144 4 rows 14.1 / 12.5, 1024 x
+// 1536 8 rows 6.0 / 5.5, also where the choice by shape would take another kernel than the small-M one: 1024 x 16384 8 rows 14.3 / 14.0,
+// 1 row 13.8 / 8.2, 11264 x 1280 20.9 / 13.1.
+static bool norm_fits(const NormPrologue& norm, int M, int N, int K) {
+    if (M > 8 || K < 1024 || K % 512 != 0 || smallm_nt_norm_lds(M, K) > kNormLdsMax - 1024 || reinterpret_cast<uintptr_t>(norm.weight) % 16 != 0)
+        return false;
+    const int rows = smallm_nt_norm_rows(M);
+    const long rounds = (N / 16 + 511) / 512;
+    if (rounds > 1 && smallm_nt_rega_tpw(M, N / 16, K, K, K) > 0) return false;
+    return rows <= 2 || rounds * K <= (rows == 4 ? 12288 : 4096);
 }
 
 template <typename T>
@@ -1779,7 +1790,7 @@ hipError_t gemm_step_qkv(const void* x, const NormPrologue& norm, const void* w,
     const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 && ldx % 8 == 0 && ldb % 8 == 0;
     if (!aligned || M > 64 || N % 128 != 0 || ldx >= (1L << 22) || ldb >= (1L << 22)) return hipErrorNotSupported;
     if (norm.weight != nullptr) {
-        if (!norm_fits(norm, M, K)) return hipErrorNotSupported;
+        if (!norm_fits(norm, M, N, K)) return hipErrorNotSupported;
         return launch_smallm_nt_norm<T, kEpiRope>(A, static_cast<const T*>(norm.weight), norm.eps, B, C, M, N, K, ldx, ldb, ldc, stream, rope);
     }
     if (choose_kernel(M, N, K, true, true, true, true, ldb % 64 == 0).shape != kSmallM) return hipErrorNotSupported;
@@ -1791,7 +1802,7 @@ hipError_t gemm_step_gate_up(const void* x, const NormPrologue& norm, const void
                              hipStream_t stream) {
     const T *A = static_cast<const T*>(x), *B = static_cast<const T*>(w);
     const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 && ldx % 8 == 0 && ldb % 8 == 0;
-    if (!aligned || N % 64 != 0 || !norm_fits(norm, M, K)) return hipErrorNotSupported;
+    if (!aligned || N % 64 != 0 || !norm_fits(norm, M, N, K)) return hipErrorNotSupported;
     return launch_smallm_nt_norm<T, kEpiGateUp>(A, static_cast<const T*>(norm.weight), norm.eps, B, static_cast<T*>(out), M, N, K, ldx, ldb, ldc,
                                                 stream, {});
 }

@@ -199,8 +199,8 @@ int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V,
                                     int dtype, int variant, void* stream);
 // The QKV projection of a generation step's layer with the RMSNorm of its rows (norm_weight null: none) and mi355_rope_qkv in one
 // launch: qkv = rope(rmsnorm(x) w_qkv^T), rotated keys and values into kv_out; x is [B, S, hidden], qkv [B, S, (q_heads + 2 kv_heads)
-// * 128]. And silu(gate) * up of the normalised rows (w_gu in groups of 32 gate and 32 up rows). MI355_ERR_UNSUPPORTED: nothing
-// was launched, take the single calls.
+// * 128]. And silu(gate) * up of the normalised rows (w_gu in groups of 32 gate and 32 up rows). The bits of the single launches on
+// the small-M kernel. MI355_ERR_UNSUPPORTED (no error text): nothing was launched, take the single calls.
 int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, const void* w_qkv, void* qkv, void* kv_out, int B, int S, int q_heads,
                             int kv_heads, int hidden, int64_t out_batch, int64_t out_row, int64_t out_head, const float* cos_table,
                             const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions, int dtype, void* stream);

@@ -13,7 +13,8 @@ the gate/up epilogue does not apply, an MLP width that is no multiple of 32, and
     (strided operands, GQA inside the kernel, output written as [B, S, Hq*D]) -> O projection with the residual
     added in its epilogue -> rmsnorm -> gate/up GEMM with SiLU(gate)*up applied in its epilogue -> down GEMM with the
     residual added in its epilogue.
-With up to 8 rows (a generation step) each norm is part of the product behind it and RoPE of the QKV product: five launches.
+With up to 8 rows (a generation step) RoPE is part of the QKV product, and each norm of the product behind it where that pays (1 or 2 rows
+up to 7680 wide, 4 up to 4608, 8 up to 2560, fewer in front of a wide MLP: `norm_fits` in csrc/hgemm.hip): five to seven launches.
 Weights keep the nn.Linear layout ([out_features, in_features]); nothing is transposed or repacked beyond
 concatenating q/k/v and interleaving gate/up along the output dimension once at construction.
 """
