@@ -662,7 +662,7 @@ def test_operands_with_unaligned_rows_through_aligned_copies(lib, gpu, dtype, la
                                                     (33, 391, 136, 2, True), (70, 72, 2112, 16, False), (1, 8, 192, 3, True)])
 def test_ranges_of_k_of_any_length_on_every_tile_shape(lib, gpu, layout, shape, M, N, K, splits, own_merge):
     # ranges that are no equal shares of K, the last one with a K tail; merged by the last workgroup of a tile or by a kernel of
-    # their own: the same bits on every launch, since the ranges are added in their order either way
+    # their own (256x256 tiles by the latter whichever is asked for): the same bits on every launch, since the ranges are added in their order either way
     if shape == 7 and layout == "TN":
         pytest.skip("32-row tiles exist for layouts with a K-contiguous A")
     a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
@@ -834,7 +834,8 @@ def test_more_ranges_pinned_than_k_has_tiles(lib, gpu, layout, K, splits, shape,
 @pytest.mark.parametrize("own_merge", [False, True])
 @pytest.mark.parametrize("M,N,ldc_pad", [(150, 264, 0), (131, 203, 2)])      # aligned rows of C; odd width, unaligned rows
 def test_residual_behind_the_merge_of_ranges_of_k(lib, gpu, dtype, layout, shape, own_merge, M, N, ldc_pad):
-    # the merge of the partial tiles adds the residual to the rounded sum, in the last workgroup of a tile or in the merge kernel:
+    # the merge of the partial tiles adds the residual to the rounded sum, in the last workgroup of a tile or in the merge kernel (which
+    # 256x256 tiles take whichever is asked for):
     # bit for bit the same kernel's product plus the residual, for a residual of its own and in place
     if shape == 7 and layout == "TN":
         pytest.skip("32-row tiles exist for layouts with a K-contiguous A")

@@ -103,7 +103,8 @@ static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, b
             const float us = fmaxf(loop_us(s, c.per_cu), floor_us), tile_kib = (float)(bm * bn) / 256.f;
             const float part_mb = (float)(tiles * s) * tile_kib / 1024.f;
             if (part_mb > 64.f) break;
-            consider(us + 1.17f + s * tile_kib * (2.f / 64.f) + part_mb * .267f, c.shape, s, false);
+            if (c.shape != kTile256x256)   // (those have the merge kernel only)
+                consider(us + 1.17f + s * tile_kib * (2.f / 64.f) + part_mb * .267f, c.shape, s, false);
             consider(us + 3.91f + part_mb * .418f, c.shape, s, true);
         }
     }

@@ -85,7 +85,7 @@ KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles
 // the activation slab is half as large to begin with: 8 x 14336 x 4096 22.3 -> 20.5 us with two tiles (21.2 with four),
 // 8 x 28672 x 4096 39.1 -> 39.4-39.9 either way, so the widest products keep one tile per workgroup there.
 inline int smallm_nt_rega_tpw(int M, int n_tiles, int K, long lda, long ldb) {
-    if (M > 16 || K != 4096 || lda >= (1L << 22) || ldb >= (1L << 22)) return 0;   // lane offsets of up to 40 rows in 32 bits
+    if (M > 16 || K != 4096 || lda >= (1L << 22) || ldb >= (1L << 22)) return 0;   // lane offsets of up to 72 rows in 32 bits
     if (M <= 8) return n_tiles % 2 == 0 && n_tiles / 2 >= 192 && n_tiles / 2 <= 512 ? 2 : 0;
     for (int tpw : {4, 2})
         if (n_tiles % tpw == 0 && n_tiles / tpw >= 192) return tpw;
@@ -180,7 +180,7 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 //   gemm: 0 = by shape; 1 = 256x256 tiles, 2 = 128x128, 3 = 64x128 (layout NT: 128x64), 4 = 64x64 with a ring of four
 //         stages, 5 = 128x256, 6 = 256x128, 7 = 32x64 (layouts NN and NT), 8 = the small-M kernels (up to 64 rows), 9 = 64x64 with
 //         a ring of eight; shapes 1 .. 7 take s ranges of K with variant + 16 s, merged by a kernel of their own (instead of
-//         the last workgroup of a tile) with variant + 16 s + 4096. The gate/up product: 1, 2, 4, 5, 6, 8, 9
+//         the last workgroup of a tile) with variant + 16 s + 4096, shape 1 always. The gate/up product: 1, 2, 4, 5, 6, 8, 9
 //   fmha: 0 = by shape, 1 = 128-query workgroups, 2 = 256-query workgroups (1 and 2 also keep generation-step shapes off
 //         the split-KV path), 3 = keys cut into ranges and merged (an error where the choice by shape would not do that)
 extern "C" {

@@ -31,7 +31,7 @@ def variants(M, N, K, layout):
         for s in RANGES:
             if shape == 9 or tiles > 400 or tiles * s > 1200 or -(-K // 64) < 2 * s or tiles * s * bm * bn > 16 << 20:
                 break
-            out += [shape + 16 * s, shape + 16 * s + 4096]
+            out += [shape + 16 * s + 4096] + [shape + 16 * s] * (shape != 1)      # 256x256 tiles have the merge kernel only
     return out
 
 
