@@ -883,19 +883,34 @@ def test_256x256_tiles_with_few_k_tiles(lib, gpu, layout, K):
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
 @pytest.mark.parametrize("M,N,K,residual", [(4352, 4096, 64, True), (4200, 4104, 200, True), (4200, 4104, 72, False), (8448, 4352, 128, False)])
 def test_256x256_tiles_over_several_rounds(lib, gpu, dtype, layout, M, N, K, residual):
-    """More 256x256 tiles than CUs, so that a workgroup takes two or three of them: 272, 289 and 561 tiles, whole and ragged, K of
-    one to four tiles. Expected: the same kernel on row blocks of the product that are one round each, bit for bit."""
-    a, b = operands(M, N, K, layout, seed=M + K)
-    ag, bg = a.to(gpu, dtype), b.to(gpu, dtype)
+    """More 256x256 tiles than CUs: 272, 289 and 561 tiles, whole and ragged, K of one to four tiles. Expected: the same kernel on
+    row blocks of the product that are one round each, bit for bit."""
+    a, b = (t.to(dtype) for t in operands(M, N, K, layout, seed=M + K))
+    ag, bg = a.to(gpu), b.to(gpu)
     r = torch.randn(M, N, generator=torch.Generator().manual_seed(9)).to(gpu, dtype) if residual else None
     c = lib.hgemm(ag, bg, layout, residual=r, variant=1)
     for i in range(0, M, 3584):
         rows = slice(i, min(i + 3584, M))
         part = ag[:, rows].contiguous() if layout == "TN" else ag[rows]
         assert torch.equal(c[rows], lib.hgemm(part, bg, layout, residual=r[rows] if residual else None, variant=1))
-    ok, st = so.gemm_tolerance_ok(c[:64].cpu() if not residual else (c[:64].float() - r[:64].float()).cpu(),
-                                  so.gemm_ref(a[:, :64].contiguous() if layout == "TN" else a[:64], b, layout), K)
-    assert dtype != torch.float16 or ok, st
+    ref, out = so.gemm_ref(a[:, :64].contiguous() if layout == "TN" else a[:64], b, layout), c[:64].float().cpu()
+    if residual:
+        out -= r[:64].float().cpu()
+    if dtype == torch.float16:
+        ok, st = so.gemm_tolerance_ok(out, ref, K)
+        assert ok, st
+    else:   # sums of K products of about 1 in 32 bits, rounded to 8 significand bits, and once more behind the residual
+        bound = K * K * 2.0 ** -24 + 2.0 ** -8 * 1.01 * ref.abs()
+        if residual:
+            bound += 2.0 ** -8 * c[:64].float().cpu().abs()
+        assert bool(((out - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("K", [67, 203])
+def test_256x256_tiles_over_several_rounds_of_k_that_ends_inside_a_chunk(lib, gpu, dtype, layout, K):
+    test_k_that_ends_inside_a_chunk_of_padded_rows(lib, gpu, dtype, layout, 1, 4200, 4104, K)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -929,6 +944,35 @@ def test_k_walked_from_different_places_on_each_xcd(lib, gpu, variant, M, tiles)
     for K in (64 * tiles, 64 * tiles - 8):
         a, b = operands(M, 1096, K, "NT", seed=tiles + M)
         check(lib, gpu, a, b, "NT", K, variant=variant)
+
+
+@pytest.mark.parametrize("variant,rows", [(2, (128, 256)), (3, (128, 256)), (4, (64, 128)), (7, (32, 64)), (9, (64,))])
+@pytest.mark.parametrize("tiles", [2, 3, 4, 5, 8, 9, 16, 23])
+def test_k_walked_from_different_places_by_whole_tiles(lib, gpu, variant, rows, tiles):
+    """The same where nothing is ragged, which has kernels of its own. Every weight row is there 16 times, on columns of all XCDs:
+    their sums differ by the order of the K tiles only, one rounding to fp16 apart at most."""
+    for M in rows:
+        a, b = operands(M, 64, 64 * tiles, "NT", seed=tiles + M)
+        b = b.repeat(16, 1)
+        c = check(lib, gpu, a, b, "NT", 64 * tiles, variant=variant).float().view(M, 16, 64)
+        spread = c.amax(1) - c.amin(1)
+        assert bool((spread <= 2.0 ** -10 * c.abs().amax(1) + (64 * tiles) ** 2 * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("variant,M,F", [(2, 128, 512), (2, 256, 512), (2, 200, 480), (4, 33, 544), (4, 128, 512), (9, 64, 512), (9, 40, 544)])
+def test_gate_up_with_k_walked_from_different_places(lib, gpu, dtype, variant, M, F):
+    cdll, st = lib.load(), torch.cuda.current_stream().cuda_stream
+    for K in [64 * t for t in (2, 3, 5, 8, 9, 17)]:
+        g = torch.Generator().manual_seed(M + K)
+        x, w = torch.randn(M, K, generator=g).to(dtype), (torch.randn(2 * F, K, generator=g) * 0.05).to(dtype)
+        xg, wg = x.to(gpu), w.to(gpu)
+        out = torch.full((M, F), float("nan"), device=gpu, dtype=dtype)
+        code = lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16
+        assert cdll.mi355_internal_hgemm_silu_mul_variant(xg.data_ptr(), wg.data_ptr(), out.data_ptr(), M, F, K, K, K, F, lib.LAYOUTS["NT"], code,
+                                                          variant, st) == 0
+        ref = so.silu_mul_ref(x.float() @ w.view(-1, 2, 32, K).transpose(0, 1).reshape(2 * F, K).float().t()).float()
+        assert (out.cpu().float() - ref).norm() <= (2e-3 if dtype == torch.float16 else 1.6e-2) * ref.norm()
 
 
 def test_another_stream_gets_the_chip_before_a_large_product_is_done(lib, gpu):
