@@ -78,6 +78,8 @@ extern "C" {
  * dimension, a multiple of 8, leaves behind M, N or K; what is read there does not reach C). C (and
  * a residual) may have any row stride and alignment (global memory takes 16-byte accesses at any element; only the
  * last N % 8 columns of a row are stored element by element).
+ * Sums over K are formed in 32 bits, in an order that depends on the sizes and, in layout NT with up to 256 rows, on the
+ * column too: the same call gives the same bits every time, but equal rows of B may give results one rounding apart.
  */
 int mi355_hgemm(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                 int64_t ldc, int layout, void* stream);

@@ -161,9 +161,11 @@ struct MainCfg {
     static constexpr int NSTAGE = STAGES > 0 ? STAGES : STAGE_BYTES > 48 * 1024 ? 2 : STAGE_BYTES > 24 * 1024 ? 3 : STAGE_BYTES > 16 * 1024 ? 5 : 8;
     // The 256x256 tiles fill the 160 KiB: 2 x 32 KiB of A, 3 x 32 KiB of B. A copy of B then has two K tiles to land instead of
     // one, and A's, which most workgroups find in L2, wait behind less. Where B (a weight) comes from HBM a K tile takes ~1.1 us to
-    // arrive, longer than its matrix instructions (us, 2 stages of both / 3 of B; operands from HBM): 500 x 28672 x 4096 NT
-    // gate/up 109 / 100, 500 x 6144 x 4096 92 / 77, 8192 x 4096 x 14336 717 / 666, 8192 x 28672 x 4096 gate/up 1405 / 1335, 8192^3 NN
-    // 774 / 757, NT 787 / 751, TN 772 / 772. The third stage to A instead: 104, 88, 653, 1335, 754, 749, 769. (A deeper ring does
+    // arrive, longer than its matrix instructions (us, 2 stages of both / 3 of B, operands from HBM, in turn on one card): 500 x 28672 x
+    // 4096 NT gate/up 110 / 103, 500 x 6144 x 4096 93 / 77, 2048 x 28672 x 4096 gate/up 403 / 376, 8192 x 4096 x 14336 731 / 681, 8192 x 28672
+    // x 4096 gate/up 1428 / 1377, 8192^3 NN 798 / 787, NT 807 / 775, TN 803 / 801. The third stage to A instead, on another card, 3 of B / 3
+    // of A: 100 / 104, 77 / 88, 8192 x 4096 x 14336 666 / 653, gate/up 1335 / 1335, 8192^3 757 / 749, 751 / 754, 772 / 769: up to 2 % more where
+    // the grid is full, 4 - 14 % less under a few rows of tiles; one rule for all sizes takes B. (A deeper ring does
     // nothing for the smaller tiles, which already have two or more K tiles in flight: 128x128 tiles with four or five stages, 64x128
     // with six, and 128x256 and 256x128 tiles with a fourth stage of either operand are within 1 % of what they are.)
     static constexpr int NSTAGE_A = NSTAGE, NSTAGE_B = NSTAGE + (STAGE_BYTES > 48 * 1024 ? 1 : 0);
@@ -458,9 +460,12 @@ void hgemm_main_kernel(const T* __restrict__ A, const T* __restrict__ B,
     // A weight stored [N,K] under one or two rows of tiles: every workgroup streams 128-byte pieces of its own rows, a row apart,
     // and all of them the same columns at the same time, which keeps part of the memory channels busy and the others waiting.
     // The XCDs therefore start an eighth of K apart from each other and go on at k = 0 behind the last tile. us, in step /
-    // this: 128 x 28672 x 4096 NT 54.3 / 47.7, 64 rows 52.0 / 47.9, 32 rows 49.5 / 43.5, 33 x 50257 85.7 / 82.0, 256 rows 84.6 / 81.8,
-    // 128 x 6144 and 64 x 4096 x 14336 the same; more rows of tiles, and weights stored [K,N], whose rows lie side by side,
-    // gain nothing or lose 1-4 %.
+    // this, weights from HBM: 128 x 28672 x 4096 gate/up 53.9 / 48.1, 64 rows 51.7 / 48.2, 32 rows 46.6 / 43.6, 33 x 50257 bf16 87.1 / 82.2, 128 x
+    // 18432 45.9 / 43.2, 128 x 8192 x 8192 42.4 / 39.5, 256 x 28672 84.1 / 82.7, 128 x 6144 and 64 x 4096 x 14336 the same; more rows of tiles, and
+    // weights stored [K,N], whose rows lie side by side, gain nothing or lose 1-4 %.
+    // The order of the 32-bit sums so depends on the XCD a column's tile falls on (a call repeats itself bit for bit): equal weight
+    // rows may come out one rounding apart. Against float64 nothing changes (32 products of 17 - 256 rows, fp16 and bf16): relative errors
+    // are equal to 5e-7 of themselves, 0.5 % fewer results are other than the exact one rounded.
     constexpr bool kStagger = A_KC && B_KC && !SPLIT_K && BM <= 128 && BN <= 128;
     int before_wrap = ktiles;   // K tiles in front of the one at k = 0 that follows the last
     if (kStagger && M <= 2 * BM && k_first == BK) {

@@ -3,7 +3,11 @@
 // The constants (microseconds) were fitted to timings of the pinned kernels over 3788 products (1 .. 8192 rows, 128 .. 262144
 // columns, K 128 .. 14336, all layouts, round and ragged sizes) and 700 products with the gate/up epilogue, weights from HBM: a
 // coordinate search for the least regret, the time of the chosen kernel over that of the fastest one. Over those products
-// the choice takes 1.6 % longer than the fastest kernel on average (gate/up 0.5 %). perf/gemm_choice.py measures that.
+// the choice took 1.6 % longer than the fastest kernel on average (gate/up 0.5 %). perf/gemm_choice.py measures that. Two changes
+// since, a third stage of B on the 256x256 tiles and the staggered walk of K under one or two rows of tiles (NT), made kernels 2 - 20 %
+// faster without moving the lines between them: over 400 products of one seed 2.0 % before and 2.1 % after, over 3000 of another
+// 2.2 % (0.3 % where 256x256 tiles are chosen, NT 17 - 64 rows 1.7 %, 65 - 256 1.2 %, NN and TN up to 16 rows 4.3 %), over 800 drawn
+// gate/up products 3.0 %.
 //   * A tiled kernel runs in rounds of one workgroup per CU (two for the small tiles) of `K tiles * step + fixed`. The step
 //     is set by the CU's intake of 64 bytes per cycle as much as by the matrix instructions (see the tile shapes' rings at
 //     MainCfg), and is a sixth (256x128) to twice (32x64) longer where the second operand is too large to stay in the
