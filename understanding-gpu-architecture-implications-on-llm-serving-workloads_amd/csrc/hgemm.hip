@@ -165,7 +165,9 @@ struct MainCfg {
     // 4096 NT gate/up 110 / 103, 500 x 6144 x 4096 93 / 77, 2048 x 28672 x 4096 gate/up 403 / 376, 8192 x 4096 x 14336 731 / 681, 8192 x 28672
     // x 4096 gate/up 1428 / 1377, 8192^3 NN 798 / 787, NT 807 / 775, TN 803 / 801. The third stage to A instead, on another card, 3 of B / 3
     // of A: 100 / 104, 77 / 88, 8192 x 4096 x 14336 666 / 653, gate/up 1335 / 1335, 8192^3 757 / 749, 751 / 754, 772 / 769: up to 2 % more where
-    // the grid is full, 4 - 14 % less under a few rows of tiles; one rule for all sizes takes B. (A deeper ring does
+    // the grid is full, 4 - 14 % less under a few rows of tiles; one rule for all sizes takes B. The price: no LDS is left on the CU, so a
+    // kernel of another stream that uses any waits for a tile to end (an RMSNorm of 8 rows beside 8192^3 35 us with 128 KiB, 220 now; kernels
+    // of over 32 KiB always did, those without LDS do not). (A deeper ring does
     // nothing for the smaller tiles, which already have two or more K tiles in flight: 128x128 tiles with four or five stages, 64x128
     // with six, and 128x256 and 256x128 tiles with a fourth stage of either operand are within 1 % of what they are.)
     static constexpr int NSTAGE_A = NSTAGE, NSTAGE_B = NSTAGE + (STAGE_BYTES > 48 * 1024 ? 1 : 0);
