@@ -1588,10 +1588,10 @@ static hipError_t launch_smallm_nt_norm(const T* A, const T* norm_weight, float 
 }
 
 // One workgroup per tile, so that a CU is given back after every tile. (256 workgroups that walk the tiles, and request the next
-// tile's operands in front of the stores of the last, gain 0.1-0.4 % of a product alone: 8192^3 NN 805.2 us against 805.8. With one CU held by
-// a kernel of another stream the workgroup left over begins its walk when the others end theirs, 8192^3 1.66 times its time alone
-// against 1.10, 8192 x 28672 x 4096 gate/up 1.80 against 1.02; an RMSNorm of 8 rows on another stream waits for the whole product, 791 us
-// against 83.)
+// tile's operands in front of the stores of the last, gain 0-1 % of a product alone: 8192^3 NN 805.2 us against 805.8 on one card, 781
+// against 787 on another. With one CU held by a kernel of another stream the workgroup left over begins its walk when the others end
+// theirs, 8192^3 1.66 times its time alone against 1.10, 8192 x 28672 x 4096 gate/up 1.80 against 1.02; an RMSNorm of 8 rows on another
+// stream waits for the whole product, 831 us against 220.)
 template <typename T, bool A_KC, bool B_KC, int BM, int BN, int WM, int WN, int EPI = 0, bool RAGGED = false, int STAGES = 0, int PER_CU = 1>
 static hipError_t launch_main(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
                               long ldc, long ldr, hipStream_t stream) {
