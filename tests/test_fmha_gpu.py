@@ -729,3 +729,35 @@ def test_two_threads_whose_first_generation_step_is_on_one_stream(lib, gpu):
             t.join()
         stream.synchronize()
         assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("variant,B,Hq,Hkv,Sq,Sk,causal", [
+    (1, 5, 64, 8, 40, 64, False), (1, 5, 64, 8, 100, 128, False), (1, 6, 64, 16, 130, 130, True), (1, 9, 32, 8, 300, 300, True),
+    (1, 9, 32, 4, 50, 400, True), (1, 3, 48, 8, 300, 129, True),     # the last: items that see no key between items that do
+    (2, 9, 32, 8, 257, 257, True), (2, 5, 32, 32, 512, 513, False), (2, 4, 40, 8, 600, 1100, True), (2, 6, 32, 8, 700, 190, True),
+])
+def test_items_of_a_long_list_equal_the_same_items_on_their_own(lib, gpu, dtype, variant, B, Hq, Hkv, Sq, Sk, causal):
+    """Several work items per workgroup, 1 .. 18 key tiles each: one item's tiles follow the last one's in the ring, whatever slot that
+    leaves them in. A batch row alone is one item per workgroup; the arithmetic is the same, so are the bits."""
+    q, k, v = (x.to(gpu, dtype) for x in so.fmha_inputs(B, Hq, Hkv, Sq, Sk, seed=Sq + Sk))
+    o, lse = lib.fmha_fwd(q, k, v, causal=causal, variant=variant)
+    for b in range(B):
+        o1, lse1 = lib.fmha_fwd(q[b:b + 1], k[b:b + 1], v[b:b + 1], causal=causal, variant=variant)
+        assert torch.equal(o[b], o1[0]) and torch.equal(lse[b], lse1[0]), b
+    o_ref, lse_ref = so.attention_ref(q[-1:].cpu().float(), k[-1:].cpu().float(), v[-1:].cpu().float(), causal=causal)
+    tol = (2e-3, 1e-3) if dtype == torch.float16 else (1.6e-2, 1e-3)
+    assert (o[-1:].cpu().float() - o_ref.float()).abs().max() <= tol[0]
+    seen = torch.isfinite(lse_ref)
+    assert (lse[-1:].cpu() - lse_ref)[seen].abs().max() <= tol[1] and torch.equal(torch.isfinite(lse[-1:].cpu()), seen)
+
+
+def test_more_items_than_a_workgroup_lists_at_once(lib, gpu):
+    """Items are listed 64 at a time per workgroup: 70 x 256 heads are 70 for each of 256."""
+    B, H, Sq, Sk = 70, 256, 16, 70
+    g = torch.Generator(device=gpu).manual_seed(3)
+    q, k, v = (torch.randn(B, h, s, 128, generator=g, device=gpu, dtype=torch.float16) for h, s in ((H, Sq), (8, Sk), (8, Sk)))
+    o, lse = lib.fmha_fwd(q, k, v, causal=True, variant=1)
+    for b in (0, 13, 34, 69):
+        o1, lse1 = lib.fmha_fwd(q[b:b + 1], k[b:b + 1], v[b:b + 1], causal=True, variant=1)
+        assert torch.equal(o[b], o1[0]) and torch.equal(lse[b], lse1[0]), b

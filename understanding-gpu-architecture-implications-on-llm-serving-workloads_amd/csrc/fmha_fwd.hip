@@ -79,7 +79,7 @@ __device__ __forceinline__ float max3v(float a, float b, float c) {
 // with the q tiles that see the most keys (causal) first and dealt out in rounds that run forwards and backwards in turn:
 // the workgroup that got the heaviest item of one round gets the lightest of the next.
 __device__ __forceinline__ bool fmha_work_item(int wg, int n_wg, int round, int q_tiles, int group, int Hkv, int B, int& b,
-                                               int& hq, int& q_tile) {
+                                               int& hkv, int& hq, int& q_tile) {
     const int kv_groups = Hkv * B;
     int x = 0, n_x = 1;
     if (kv_groups % 8 == 0 && n_wg % 8 == 0) {
@@ -96,7 +96,8 @@ __device__ __forceinline__ bool fmha_work_item(int wg, int n_wg, int round, int 
     q_tile = q_tiles - 1 - rank;
     const int kvg = x * gpx + gl;
     b = kvg / Hkv;
-    hq = (kvg - b * Hkv) * group + hin;
+    hkv = kvg - b * Hkv;
+    hq = hkv * group + hin;
     return true;
 }
 
@@ -186,51 +187,77 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     const int g = lane >> 4;
     const int c16 = lane & 15;
 
-    // ---- the work item this workgroup is on (set_item) --------------------------------------------------------------
+    // ---- work items -------------------------------------------------------------------------------------------------
     const int group = Hq / Hkv;
-    int shift = Sk - Sq;
-    const int kv_valid_all = kv_valid;
-    long o_row = sd.o_row;
-    int b = 0, hq = 0, q_wave0 = 0, n_tiles = 0, n_full = 0, last_tile = 0;
-    const T* Qh = Q;
-    const T* Kh = K;
-    const T* Vh = V;
-    T* Oh = O;
-    auto set_item = [&](int round) -> bool {
-        int q_tile;
-        if (!fmha_work_item(blockIdx.x, gridDim.x, round, q_tiles, group, Hkv, SEG ? B * segments : B, b, hq, q_tile)) return false;
-        const int hkv = hq / group;
-        const int q_block0 = q_tile * BM;
-        q_wave0 = q_block0 + wave * WQ;
+    struct Item {
+        const T *Qh, *Kh, *Vh;
+        T* Oh;
+        int lse_row;             // (batch, q head), of a range too: row of LSE / Sq
+        int q_block0;            // first query
+        int kv_valid, shift;     // valid keys; key j is visible to query i iff j <= i + shift (causal)
+        int n_tiles;             // key tiles; may be <= 0: no visible key for the whole work item
+        int exists;              // 0: no such item, nothing else is set
+    };
+    const long o_row = SEG ? (long)D : sd.o_row;
+    auto item_of = [&](int round) -> Item {
+        // (opaque copies: the compiler would work out reciprocals and products of these once and keep them in vector registers through the
+        // loop over the keys, which has none to spare)
+        int q_tiles_ = q_tiles, group_ = group, Hkv_ = Hkv, batches = SEG ? B * segments : B;
+        asm volatile("" : "+s"(q_tiles_), "+s"(group_), "+s"(Hkv_), "+s"(batches));
+        Item it;
+        int b, hkv, hq, q_tile;
+        it.n_tiles = 0;
+        it.exists = fmha_work_item(blockIdx.x, gridDim.x, round, q_tiles_, group_, Hkv_, batches, b, hkv, hq, q_tile);
+        if (!it.exists) return it;
+        it.q_block0 = q_tile * BM;
+        long k0 = 0;
         if constexpr (SEG) {   // b counts (batch, range) pairs
             const int seg = b % segments;
             b /= segments;
-            const long k0 = (long)seg * seg_len;
-            Qh = Q + b * sd.q_batch + hq * sd.q_head;
-            Kh = K + b * sd.k_batch + hkv * sd.k_head + k0 * sd.k_row;
-            Vh = V + b * sd.v_batch + hkv * sd.v_head + k0 * sd.v_row;
-            Oh = O + (((long)seg * B + b) * Hq + hq) * (long)Sq * D;
-            o_row = D;
-            kv_valid = min(max(kv_valid_all - (int)k0, 0), seg_len);
-            shift = Sk - Sq - (int)k0;
-            b = seg * B + b;   // the LSE row of this item, below
+            k0 = (long)seg * seg_len;
+            it.lse_row = (seg * B + b) * Hq + hq;
+            it.Oh = O + (long)it.lse_row * Sq * D;
+            it.kv_valid = min(max(kv_valid - (int)k0, 0), seg_len);
         } else {
-        Qh = Q + b * sd.q_batch + hq * sd.q_head;
-        Kh = K + b * sd.k_batch + hkv * sd.k_head;
-        Vh = V + b * sd.v_batch + hkv * sd.v_head;
-        Oh = O + b * sd.o_batch + hq * sd.o_head;
+            it.lse_row = b * Hq + hq;
+            it.Oh = O + b * sd.o_batch + hq * sd.o_head;
+            it.kv_valid = kv_valid;
         }
-        int k_end = kv_valid;
-        if (causal) k_end = min(k_end, min(q_block0 + BM, Sq) - 1 + shift + 1);
-        n_tiles = (k_end + BN - 1) / BN;            // may be <= 0: no visible key for the whole work item
-        n_full = min(n_tiles, kv_valid / BN);       // tiles 0 .. n_full-1 have all 64 rows
-        last_tile = n_tiles - 1;
-        return true;
+        it.shift = Sk - Sq - (int)k0;
+        it.Qh = Q + b * sd.q_batch + hq * sd.q_head;
+        it.Kh = K + b * sd.k_batch + hkv * sd.k_head + k0 * sd.k_row;
+        it.Vh = V + b * sd.v_batch + hkv * sd.v_head + k0 * sd.v_row;
+        int k_end = it.kv_valid;
+        if (causal) k_end = min(k_end, min(it.q_block0 + BM, Sq) - 1 + it.shift + 1);
+        it.n_tiles = (k_end + BN - 1) / BN;
+        return it;
     };
+    // The items to come are worked out 64 at a time, one per lane of the last wave, while the workgroup waits for its first loads, and
+    // kept in LDS: the scalar registers have no room for two items, and the divisions would take a wave ~1900 cycles at every change.
+    constexpr int kListed = 64;
+    __shared__ Item listed[kListed];
+    const auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    const auto uniform_ptr = [](auto* p) {
+        const uint64_t u = reinterpret_cast<uint64_t>(p);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)u), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+        return reinterpret_cast<decltype(p)>((uint64_t)hi << 32 | lo);
+    };
+    auto item_listed = [&](int round) -> Item {
+        const Item& l = listed[(round - 1) % kListed];
+        Item it;
+        it.Qh = uniform_ptr(l.Qh); it.Kh = uniform_ptr(l.Kh); it.Vh = uniform_ptr(l.Vh); it.Oh = uniform_ptr(l.Oh);
+        it.lse_row = uniform(l.lse_row); it.q_block0 = uniform(l.q_block0); it.kv_valid = uniform(l.kv_valid);
+        it.shift = uniform(l.shift); it.n_tiles = uniform(l.n_tiles); it.exists = uniform(l.exists);
+        return it;
+    };
+    // steps of an item in which the pair that is copied (tiles j + 3 of K, j + 2 of V) is made of full tiles
+    auto fast_steps = [](int n_tiles, int kv_valid) { return min(min(n_tiles, kv_valid / BN) - 3, n_tiles - 1); };
+    Item cur = item_of(0);   // a launch has no more workgroups than items
+    int q_wave0 = cur.q_block0 + wave * WQ;
 
     // Q fragments (B operand of the first product): lane holds Q[16 qb + c][32 ks + 8 g .. +7]
     V8 qf[QB][4];
-    auto load_q = [&]() {
+    auto load_q = [&](const T* Qh, int q_wave0) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
             const int qrow = min(q_wave0 + qb * 16 + c16, Sq - 1);
@@ -242,45 +269,47 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
 
     // copy i of this wave covers tile rows 32 i + 4 wave + lane/16, 16-byte chunk position lane%16
     const int copy_row0 = wave * 4 + (lane >> 4);
-    const uint32_t copy_kcol = ((lane & 15) ^ swz_k(copy_row0)) * 16;
-    const uint32_t copy_vcol = ((lane & 15) ^ swz_v16(copy_row0)) * 16;
     const uint32_t k_row_bytes = (uint32_t)sd.k_row * 2, v_row_bytes = (uint32_t)sd.v_row * 2;
     const long k_tile_bytes = (long)BN * sd.k_row * 2, v_tile_bytes = (long)BN * sd.v_row * 2;
     const uint32_t lds_wave = (uint32_t)(uintptr_t)smem + (uint32_t)wave * 1024u;
-    // general copies: the tile index is clamped to the last tile (past the end a copy re-reads that tile into a slot nobody
-    // reads any more) and rows past the last valid key onto it (masked later, but V must not feed NaNs into 0 * V)
-    auto issue_k1 = [&](int q, int i) {   // half i of K(q) into slot q % NBUF
-        const int tile = min(q, last_tile);
-        const int last = kv_valid - 1 - tile * BN;
-        copy16_global_to_lds((const char*)Kh + tile * k_tile_bytes, (uint32_t)min(copy_row0 + 32 * i, last) * k_row_bytes + copy_kcol,
-                             smem + (q & (NBUF - 1)) * TILE_BYTES + (i * NWAVES + wave) * 1024);
-    };
-    auto issue_v1 = [&](int q, int i) {   // half i of V(q - 1) into slot q % NBUF
-        const int tile = max(min(q - 1, last_tile), 0);
-        const int last = kv_valid - 1 - tile * BN;
-        copy16_global_to_lds((const char*)Vh + tile * v_tile_bytes, (uint32_t)min(copy_row0 + 32 * i, last) * v_row_bytes + copy_vcol,
-                             smem + VBUF0 + (q & (NBUF - 1)) * TILE_BYTES + (i * NWAVES + wave) * 1024);
-    };
-    // copies of the unrolled loop: tile base pointers of K(j + 3) and V(j + 2), advanced once per tile step
-    uint32_t k_lane_off[2], v_lane_off[2];
+    uint32_t k_lane_off[2], v_lane_off[2];   // of a tile with all 64 rows
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        k_lane_off[i] = (uint32_t)(copy_row0 + 32 * i) * k_row_bytes + copy_kcol;
-        v_lane_off[i] = (uint32_t)(copy_row0 + 32 * i) * v_row_bytes + copy_vcol;
+        k_lane_off[i] = (uint32_t)(copy_row0 + 32 * i) * k_row_bytes + ((lane & 15) ^ swz_k(copy_row0)) * 16;
+        v_lane_off[i] = (uint32_t)(copy_row0 + 32 * i) * v_row_bytes + ((lane & 15) ^ swz_v16(copy_row0)) * 16;
     }
+    // The ring runs on from one item to the next: pair q of an item whose pair 0 lies in slot `ring` is in slot (ring + q) % NBUF, and
+    // what its last pair, n_tiles, leaves free (it has no K) is K(0) of the next item: pair n_tiles + q of this item is pair q of the next.
+    // General copies, each operand from the item whose pair 0 is pair `first` of the current one: the tile index is clamped to that
+    // item's last tile (past the end, where no next item follows, a copy re-reads that tile into a slot nobody reads any more) and rows
+    // past the last valid key onto it (masked later, but V must not feed NaNs into 0 * V).
+    struct Source {
+        const T* base;
+        int first, last_tile, valid;
+    };
+    int ring = 0;
+    Source src_k = {cur.Kh, 0, cur.n_tiles - 1, cur.kv_valid}, src_v = {cur.Vh, 0, cur.n_tiles - 1, cur.kv_valid};
+    auto issue_k1 = [&](int q, int i) {   // half i of K(q)
+        const int tile = min(q - src_k.first, src_k.last_tile);
+        const int last = src_k.valid - 1 - tile * BN;
+        copy16_global_to_lds((const char*)src_k.base + tile * k_tile_bytes, k_lane_off[i] - (uint32_t)max(copy_row0 + 32 * i - last, 0) * k_row_bytes,
+                             smem + ((ring + q) & (NBUF - 1)) * TILE_BYTES + (i * NWAVES + wave) * 1024);
+    };
+    auto issue_v1 = [&](int q, int i) {   // half i of V(q - 1)
+        const int tile = max(min(q - 1 - src_v.first, src_v.last_tile), 0);
+        const int last = src_v.valid - 1 - tile * BN;
+        copy16_global_to_lds((const char*)src_v.base + tile * v_tile_bytes, v_lane_off[i] - (uint32_t)max(copy_row0 + 32 * i - last, 0) * v_row_bytes,
+                             smem + VBUF0 + ((ring + q) & (NBUF - 1)) * TILE_BYTES + (i * NWAVES + wave) * 1024);
+    };
+    auto issue_first_pairs = [&]() {
+        for (int q = 0; q < 3; ++q) {
+            issue_k1(q, 0); issue_k1(q, 1);
+            if (q > 0) { issue_v1(q, 0); issue_v1(q, 1); }
+        }
+    };
+    // copies of the unrolled loop: tile base pointers of K(j + 3) and V(j + 2), advanced once per tile step
     const char* k_next = nullptr;
     const char* v_next = nullptr;
-    // the first pairs of the current item: K(0), K(1), V(0), K(2), V(1)
-    auto issue_first_pairs = [&]() {
-        issue_k1(0, 0); issue_k1(0, 1);
-        issue_k1(1, 0); issue_k1(1, 1);
-        issue_v1(1, 0); issue_v1(1, 1);
-        issue_k1(2, 0); issue_k1(2, 1);
-        issue_v1(2, 0); issue_v1(2, 1);
-        k_next = (const char*)Kh + 3 * k_tile_bytes;
-        v_next = (const char*)Vh + 2 * v_tile_bytes;
-    };
-
     // fragment addresses: loop-invariant registers, the slot and the block inside the tile are immediate offsets
     //   K fragment (key block kb, d step ks): row 16 kb + c, chunk (4 ks + g) ^ (row & 15)
     //   V^T fragment (key step j, d block db), transposing read t: key row 32 j + 16 t + 4 g + c / 4, d 16 db + 4 (c % 4) .. +3
@@ -404,27 +433,28 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     using Dyn = std::integral_constant<int, -1>;
 
     // softmax of tile `tile`. CSLOT >= 0: the four copies of the pair in ring slot CSLOT ride along, full tiles from the
-    // running pointers; CSLOT == -1: general copies of pair cq; CSLOT == -2: none.
-    auto softmax_tile = [&](float4v(&s)[4][QB], int tile, V8(&pf)[2][QB], auto cslot_c, int cq) {
+    // running pointers; CSLOT == -1: general copies of pair tile + 3; CSLOT == -2: the same where that is a pair of the next item, none
+    // otherwise.
+    auto softmax_tile = [&](float4v(&s)[4][QB], int tile, V8(&pf)[2][QB], auto cslot_c) {
         constexpr int CSLOT = decltype(cslot_c)::value;
         auto copy = [&](auto which_c) {
             constexpr int W = decltype(which_c)::value;   // 0, 1: halves of K; 2, 3: halves of V
             if constexpr (CSLOT >= 0) {
                 if constexpr (W < 2) copy16_global_to_lds_at<CSLOT * TILE_BYTES + W * NWAVES * 1024>(k_next, k_lane_off[W], lds_wave);
                 else copy16_global_to_lds_at<VBUF0 + CSLOT * TILE_BYTES + (W - 2) * NWAVES * 1024>(v_next, v_lane_off[W - 2], lds_wave);
-            } else if constexpr (CSLOT == -1) {
-                if constexpr (W < 2) issue_k1(cq, W);
-                else issue_v1(cq, W - 2);
+            } else if (CSLOT == -1 || src_v.first > 0) {
+                if constexpr (W < 2) issue_k1(tile + 3, W);
+                else issue_v1(tile + 3, W - 2);
             }
         };
         const int key0 = tile * BN;
-        const bool need_mask = (key0 + BN > kv_valid) || (causal && (key0 + BN - 1 > q_wave0 + shift));
+        const bool need_mask = (key0 + BN > cur.kv_valid) || (causal && (key0 + BN - 1 > q_wave0 + cur.shift));
         copy(std::integral_constant<int, 0>{});
         if (need_mask) {
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) {
                 const int qi = q_wave0 + qb * 16 + c16;
-                const int lim = causal ? min(kv_valid - 1, qi + shift) : kv_valid - 1;  // last visible key
+                const int lim = causal ? min(cur.kv_valid - 1, qi + cur.shift) : cur.kv_valid - 1;  // last visible key
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
@@ -525,14 +555,20 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     };
 
     // ---- persistent loop over the work items of this workgroup ----------------------------------------------------------
-    // The first pairs and the Q fragments of the NEXT item are requested as soon as the last barrier of the current one is
-    // passed (every wave has finished reading LDS, and the Q registers are free), in front of the current item's epilogue:
-    // normalising and storing O runs while those loads are on their way, and the workgroup never goes back to the
-    // dispatcher between items.
+    // The first pairs of the next item ride in the last softmax phases of the current one and its Q fragments are loaded behind the last
+    // use of the current ones, so that the next item starts, when O has been normalised and stored (nothing waits for the stores), on
+    // operands that are there. Requested together behind the last barrier, these 144 KiB and the 64 KiB of O took the CU, whose share of
+    // memory's rate is ~56 GB/s from HBM, 17200 cycles from the last barrier of an item to the first of the next (4 x 32/32 x 1001, not
+    // causal; 128-query items of 13 x 64/8 x 353, causal, 8400); so they take 5700 (3200). us, before / now: 16 x 32/8 x 512 causal
+    // 86 / 76, 13 x 64/8 x 353 128-query items 102 / 83, 16 x 64/8 x 200 70 / 60, 8 x 32/8 x 1000 106 / 96, 1 x 32/8 x 4844 181 / 177, not causal
+    // 4 x 32/32 x 1001 74.9 / 73.1, 5 x 32/8 x 1328 160 / 152. The unrolled loop wants pair 0 in slot 0: an item that has steps for it
+    // starts there, also where that means that its first pairs can only leave behind the last barrier of the item in front (a second copy
+    // of the general step in front of the loop makes the 256-query instantiation spill 400 bytes a lane).
     MI355_TL(unsigned long long tl_tiles = 0;)
-    set_item(0);   // a launch has no more workgroups than items
-    load_q();
-    if (n_tiles > 0) issue_first_pairs();
+    load_q(cur.Qh, q_wave0);
+    if (cur.n_tiles > 0) issue_first_pairs();
+    const bool more_items = (long)q_tiles * Hq * B * (SEG ? segments : 1) > gridDim.x;   // of the launch, than it has workgroups
+    bool landed = false;   // the current item's first pairs and Q fragments have been waited for
     for (int round = 0;;) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
@@ -543,88 +579,139 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
 #pragma unroll
             for (int db = 0; db < 8; ++db) o[db][qb] = float4v{0.f, 0.f, 0.f, 0.f};
         }
-        if (n_tiles > 0) {
-            // pairs 0, 1, 2 and Q have landed (and the stores of the previous item's epilogue have been accepted)
-            wait_vmcnt<0>();
-            __syncthreads();
-            if (late) end_phase();   // waves 4..7 idle during P0
+        ++round;
+        bool more = false;   // this workgroup has another item
+        int n_next = 0;      // its key tiles, if its first pairs are copied while the current item is worked on
+        if (more_items && (round - 1) % kListed == 0 && wave == NWAVES - 1) listed[lane] = item_of(round + lane);
+        if (cur.n_tiles > 0) {
+            const int n_tiles = cur.n_tiles;
+            if (!landed) wait_vmcnt<0>();
+            wait_lgkmcnt<0>();
+            phase_barrier();
+            if (late) phase_barrier();   // waves 4..7 idle during P0
 
             float4v s[4][QB];
             V8 pf[2][QB];
             V8 fr[AHEAD];
-            MI355_TL(if (round == 0) tl_w[1] = timeline::wall_clock(); const unsigned long long tl_c0 = timeline::shader_cycles();)
-            preload(I0{}, std::integral_constant<int, 0>{}, 0, fr);
+            MI355_TL(if (round == 1) tl_w[1] = timeline::wall_clock(); const unsigned long long tl_c0 = timeline::shader_cycles();)
+            preload(I0{}, Dyn{}, ring & (NBUF - 1), fr);
             __builtin_amdgcn_s_setprio(1);
-            mfma_phase(I0{}, I16{}, std::integral_constant<int, 0>{}, 0, s, pf, fr);               // S(0) alone
+            mfma_phase(I0{}, I16{}, Dyn{}, ring & (NBUF - 1), s, pf, fr);               // S(0) alone
             __builtin_amdgcn_s_setprio(0);
             pin_s(s);
-            end_phase();
+            phase_barrier();   // (pairs 1 and 2 are there: nothing to wait for)
             // tile step j: softmax(j) (with the copies of pair j + 3), then S(j+1) and O += V(j)^T P(j) on pair j + 1
             auto step = [&](auto u_c, int j) {
-                constexpr int U = decltype(u_c)::value;   // j % NBUF in the unrolled loop, -1 in the general one
+                constexpr int U = decltype(u_c)::value;   // (ring + j) % NBUF in the unrolled loop, -1 in the general one
                 using CopySlot = std::integral_constant<int, (U >= 0 ? (U + 3) % NBUF : -1)>;
                 using ReadSlot = std::integral_constant<int, (U >= 0 ? (U + 1) % NBUF : -1)>;
-                softmax_tile(s, j, pf, CopySlot{}, j + 3);
+                softmax_tile(s, j, pf, CopySlot{});
                 pin_p(pf);
-                preload(I0{}, ReadSlot{}, (j + 1) & (NBUF - 1), fr);
+                preload(I0{}, ReadSlot{}, (ring + j + 1) & (NBUF - 1), fr);
                 end_phase();
                 __builtin_amdgcn_s_setprio(1);
-                mfma_phase(I0{}, I32{}, ReadSlot{}, (j + 1) & (NBUF - 1), s, pf, fr);
+                mfma_phase(I0{}, I32{}, ReadSlot{}, (ring + j + 1) & (NBUF - 1), s, pf, fr);
                 __builtin_amdgcn_s_setprio(0);
                 pin_s(s);
                 pin_o();
                 end_phase();
             };
             // unrolled loop: while the pair copied in step j (tiles j + 3 and j + 2) is made of full tiles
-            const int j_fast = max(0, min(n_full - 3, n_tiles - 1)) & ~(NBUF - 1);
+            const int j_fast = (ring & (NBUF - 1)) == 0 ? max(0, fast_steps(n_tiles, cur.kv_valid)) & ~(NBUF - 1) : 0;
             int j = 0;
+            k_next = (const char*)cur.Kh + 3 * k_tile_bytes;
+            v_next = (const char*)cur.Vh + 2 * v_tile_bytes;
             for (; j < j_fast; j += NBUF) {
                 step(std::integral_constant<int, 0>{}, j);
                 step(std::integral_constant<int, 1>{}, j + 1);
                 step(std::integral_constant<int, 2>{}, j + 2);
                 step(std::integral_constant<int, 3>{}, j + 3);
             }
-            for (; j + 1 < n_tiles; ++j) step(Dyn{}, j);
-            softmax_tile(s, n_tiles - 1, pf, std::integral_constant<int, -2>{}, 0);
+            for (; j + 1 < n_tiles; ++j) {
+                if (more_items && j + 3 >= n_tiles) {   // the copies go on to the next item: K with pair n_tiles, V with the one behind
+                    const Item& next = listed[(round - 1) % kListed];
+                    const int n = uniform(next.n_tiles), valid = uniform(next.kv_valid);
+                    if (n > 0 && (((ring + n_tiles) & (NBUF - 1)) == 0 || fast_steps(n, valid) < NBUF)) {
+                        n_next = n;
+                        src_k = {uniform_ptr(next.Kh), n_tiles, n - 1, valid};
+                        if (j + 2 == n_tiles) src_v = {uniform_ptr(next.Vh), n_tiles, n - 1, valid};
+                    }
+                }
+                step(Dyn{}, j);
+            }
+            if (more_items) more = uniform(listed[(round - 1) % kListed].exists);
+            if (more) load_q(uniform_ptr(listed[(round - 1) % kListed].Qh), uniform(listed[(round - 1) % kListed].q_block0) + wave * WQ);
+            softmax_tile(s, n_tiles - 1, pf, std::integral_constant<int, -2>{});
+            if (n_tiles == 2 && n_next > 0) {   // two tiles have no step that copies pair n_tiles: K(0) of the next item
+                issue_k1(2, 0);
+                issue_k1(2, 1);
+            }
             pin_p(pf);
-            preload(I16{}, Dyn{}, n_tiles & (NBUF - 1), fr);
-            end_phase();
-            mfma_phase(I16{}, I32{}, Dyn{}, n_tiles & (NBUF - 1), s, pf, fr);     // O += V(last)^T P(last) alone
-            end_phase();
-            if (!late) end_phase();  // waves 0..3 idle while waves 4..7 finish
-            // behind this barrier no wave reads LDS any more; the copies past the end of the item that are still on their
-            // way must land before the next item's pairs are sent into the same slots (or the workgroup ends)
+            preload(I16{}, Dyn{}, (ring + n_tiles) & (NBUF - 1), fr);
+            phase_barrier();
+            mfma_phase(I16{}, I32{}, Dyn{}, (ring + n_tiles) & (NBUF - 1), s, pf, fr);     // O += V(last)^T P(last) alone
+            phase_barrier();
+            if (!late) phase_barrier();  // waves 0..3 idle while waves 4..7 finish
+            // Behind this barrier no wave reads LDS any more. This wave's copies have landed, past the end of the item or of the
+            // next one, and so have the next Q fragments: used here, in front of the stores of the epilogue, which the compiler would
+            // otherwise wait for as well where it waits for the fragments.
             wait_vmcnt<0>();
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) asm volatile("" : "+v"(qf[qb][0]), "+v"(qf[qb][1]), "+v"(qf[qb][2]), "+v"(qf[qb][3]));
             MI355_TL(tl_w[2] = timeline::wall_clock(); tl_c[1] += timeline::shader_cycles() - tl_c0; tl_tiles += (unsigned long long)n_tiles;)
+        } else {
+            wait_lgkmcnt<0>();
+            phase_barrier();
+            if (more_items) more = uniform(listed[(round - 1) % kListed].exists);
+            if (more) load_q(uniform_ptr(listed[(round - 1) % kListed].Qh), uniform(listed[(round - 1) % kListed].q_block0) + wave * WQ);
         }
 
         // what the epilogue needs of the item just finished, then on to the next one
-        T* const o_item = Oh;
+        T* const o_item = cur.Oh;
         const int q_item0 = q_wave0;
-        float* const lse_item = LSE == nullptr ? nullptr : LSE + ((long)b * Hq + hq) * (long)Sq;
-        const bool more = set_item(++round);
+        float* const lse_item = LSE == nullptr ? nullptr : LSE + (long)cur.lse_row * Sq;
         if (more) {
-            load_q();
-            if (n_tiles > 0) issue_first_pairs();
+            landed = n_next > 0;
+            ring = landed ? ring + cur.n_tiles : 0;
+            cur = item_listed(round);
+            q_wave0 = cur.q_block0 + wave * WQ;
+            src_k = {cur.Kh, 0, cur.n_tiles - 1, cur.kv_valid};
+            src_v = {cur.Vh, 0, cur.n_tiles - 1, cur.kv_valid};
+            if (cur.n_tiles > 0 && !landed) issue_first_pairs();
         }
         // ---- finalize: O / l, LSE: lane holds O[query 16 qb + c][d = 16 db + 4 g + 0..3] --------------------------------
+        // 16 rows at a time go through this wave's 4 KiB of the slot in front of pair 0, which nobody reads or fills before the wave's own
+        // copies of pair 3, so that a store instruction writes four whole rows (as they lie in the accumulators it would write 32 bytes
+        // of each of 16 rows, four times as many lines for the CU's memory pipeline). Chunk k of row r lies at k ^ r.
+        int lane_ = lane;
+        asm volatile("" : "+v"(lane_));   // or the compiler keeps these addresses in vector registers through the loop over the keys
+        const int r16 = lane_ & 15, r4 = lane_ >> 4;
+        MI355_LDS char* const park = smem + ((ring - 1) & (NBUF - 1)) * TILE_BYTES + wave * 1024;
+        auto park_row = [&](int row) -> MI355_LDS char* {   // rows 4 a .. 4 a + 3 in the wave's quarter a: halves of K, halves of V
+            const int a = row >> 2;
+            return park + (a >> 1) * VBUF0 + (a & 1) * (NWAVES * 1024) + (row & 3) * ROW_BYTES;
+        };
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
             const float l_tot = kSumOnMatrixPipe ? l_acc[qb][0] : quad_sum(l_acc[qb][0]);
             const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
-            const int qi = q_item0 + qb * 16 + c16;
-            if (qi < Sq) {
-                T* orow = o_item + qi * o_row + 4 * g;
+            MI355_LDS char* const mine = park_row(r16);
 #pragma unroll
-                for (int db = 0; db < 8; ++db) {
-                    V4 v;
+            for (int db = 0; db < 8; ++db) {
+                V4 v;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (T)(o[db][qb][e] * inv);
-                    *(V4*)(orow + db * 16) = v;
-                }
-                if (lse_item != nullptr && g == 0)
-                    lse_item[qi] = (l_tot > 0.f) ? (m_run[qb] * scale_log2 + __builtin_log2f(l_tot)) * 0.69314718055994531f : -INFINITY;
+                for (int e = 0; e < 4; ++e) v[e] = (T)(o[db][qb][e] * inv);
+                *(MI355_LDS V4*)(mine + (((2 * db + (r4 >> 1)) ^ r16) << 4) + (r4 & 1) * 8) = v;
             }
+            const int q_first = q_item0 + qb * 16;
+            if (lse_item != nullptr && r4 == 0 && q_first + r16 < Sq)
+                lse_item[q_first + r16] = (l_tot > 0.f) ? (m_run[qb] * scale_log2 + __builtin_log2f(l_tot)) * 0.69314718055994531f : -INFINITY;
+            V8 row[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) row[a] = *(MI355_LDS const V8*)(park_row(4 * a + r4) + ((r16 ^ (4 * a + r4)) << 4));
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                if (q_first + 4 * a + r4 < Sq) *(V8*)(o_item + (q_first + 4 * a + r4) * o_row + 8 * r16) = row[a];
         }
         if (!more) break;
     }
