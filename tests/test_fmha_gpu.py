@@ -761,3 +761,16 @@ def test_more_items_than_a_workgroup_lists_at_once(lib, gpu):
     for b in (0, 13, 34, 69):
         o1, lse1 = lib.fmha_fwd(q[b:b + 1], k[b:b + 1], v[b:b + 1], causal=True, variant=1)
         assert torch.equal(o[b], o1[0]) and torch.equal(lse[b], lse1[0]), b
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,causal", [
+    (4, 64, 8, 152, False), (5, 16, 4, 405, False), (1, 8, 2, 1331, False),      # 256-query items, also fewer of them than CUs
+    (6, 64, 8, 270, True), (3, 64, 8, 638, True),                               # 128-query items, also more 256-query items than CUs
+])
+def test_either_kind_of_item_by_expected_time(lib, gpu, B, Hq, Hkv, S, causal):
+    """The choice by expected time gives the bits of one of the two pinned kernels, and those are right."""
+    q, k, v = so.fmha_inputs(B, Hq, Hkv, S, S, seed=S)
+    o, lse = run(lib, gpu, q, k, v, causal)
+    pinned = [run(lib, gpu, q, k, v, causal, variant=n) for n in (1, 2)]
+    assert any(torch.equal(o, po) and torch.equal(lse, pl) for po, pl in pinned)
+    check(lib, gpu, q[-1:], k[-1:], v[-1:], causal)

@@ -17,6 +17,7 @@
 //                      ds_read_b64_tr_b16 in that same key order.
 // K and V tiles (64 keys x 128 d) are copied global -> LDS with 16-byte direct-to-LDS copies into a ring of four slots
 // per operand, 16-byte chunks XOR-swizzled so that both the b128 reads (K) and the transposing reads (V) are conflict free.
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -934,6 +935,35 @@ static hipError_t launch_fmha_segmented(const T* Q, const T* K, const T* V, T* O
     return hipGetLastError();
 }
 
+// Expected time of a call on work items of 128 `qb` queries, beside what both kinds have in common: that of the workgroup with the most
+// to do, as fmha_work_item deals the items out. An item takes 2.2 us and 1.25 us per key tile (256 queries, every K / V fragment feeding
+// two MFMAs: 4.6 and 1.75). That weighs the queries a tile is padded by, the last round of items and, causal, the length of the
+// heaviest item against the better kernel. Over 170 drawn calls (1 .. 16 sequences, 64 .. 8192 queries, 8 .. 64 heads, causal or not, and
+// chunks over a cache) the choice is within 0.2 % of the faster one on average; a rule on the number of 256-query items that preceded it, 1.7 %. us,
+// 128- / 256-query items: 13 x 64/8 x 353 causal 83 / 99, 9 x 32/32 x 317 causal 34 / 42, 16 x 32/8 x 512 causal 85 / 76, 4 x 64/8 x 152 17.0 / 13.7,
+// 3 x 16/4 x 917 36.6 / 29.1, 1 x 8/2 x 7441 228 / 183, 1 x 32/8 x 1331 44.7 / 35.6, 10 x 40/8 x 255 34.1 / 28.6, 8 x 64/8 x 638 causal 104 / 115.
+static float one_walk_us(int qb, int cus, int B, int Hq, int Sq, int Sk, int causal, int kv_valid) {
+    const float item = qb == 2 ? 4.6f : 2.2f, tile = qb == 2 ? 1.75f : 1.25f;
+    const long bm = 128 * qb, q_tiles = (Sq + bm - 1) / bm, per_rank = (long)Hq * B, items = q_tiles * per_rank;
+    const long wgs = std::min<long>(items, cus), rounds = (items + wgs - 1) / wgs;
+    const auto rank_us = [&](long rank) {   // rank 0: the q tile that sees the most keys
+        long keys = kv_valid;
+        if (causal) keys = std::min<long>(keys, std::min((q_tiles - rank) * bm, (long)Sq) + Sk - Sq);
+        return item + tile * (float)std::max(0L, (keys + 63) / 64);
+    };
+    if (rounds > 64) return (rank_us(0) + rank_us(q_tiles - 1)) * .5f * (float)items / (float)wgs;
+    // the first, the last and the middle one, and the last one that has an item in the last round
+    const long rest = items - (rounds - 1) * wgs, probes[4] = {0, wgs - 1, wgs / 2, (rounds - 1) % 2 == 0 ? rest - 1 : wgs - rest};
+    float most = 0.f;
+    for (const long w : probes) {
+        float sum = 0.f;
+        for (long r = 0; r < rounds; ++r)
+            if (const long u = r * wgs + (r % 2 ? wgs - 1 - w : w); u < items) sum += rank_us(u / per_rank);
+        most = std::max(most, sum);
+    }
+    return most;
+}
+
 template <typename T>
 static hipError_t fmha_fwd_dispatch_t(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                       int Sq, int Sk, float scale, int causal, int kv_valid_len, const FmhaStrides& sd,
@@ -961,24 +991,9 @@ static hipError_t fmha_fwd_dispatch_t(const void* Q, const void* K, const void* 
     }
     if (variant == 3) return hipErrorInvalidConfiguration;   // the test hook asked for key ranges where they do not apply
     if (variant == 0) {
-        // 256-query workgroups (every K / V fragment feeds two MFMAs) once their work items fill the machine: clearly more
-        // of them than CUs for a causal problem (with about one per CU it runs as long as its heaviest item, and 128-query
-        // items balance better), one per CU otherwise. Measured (b x heads q/kv x s, 128- / 256-query items, us): causal
-        // 1 x 32/8 x 1024 20 / 30, 1 x 32/8 x 2048 45 / 51, 2 x 32/8 x 1024 30 / 32, 1 x 16/16 x 4096 76 / 88,
-        // 1 x 8/8 x 8192 139 / 163, 2 x 8/2 x 4096 76 / 88, but 32 x 32/8 x 256 68 / 64, 8 x 32/8 x 512 42 / 39,
-        // 1 x 32/8 x 3000 92 / 78, 2 x 32/8 x 1536 56 / 50, 4 x 32/8 x 1024 57 / 50, 1 x 32/8 x 4096 149 / 126,
-        // 16 x 32/8 x 768 148 / 128, 4 x 32/8 x 2048 170 / 147; not causal 2 x 32/8 x 1024 42 / 36, 1 x 32/8 x 2048 73 / 62,
-        // 4 x 32/32 x 1024 89 / 71. A problem that is not causal and has a few more 256-query items than CUs runs as long
-        // as two of them, on a quarter of the machine at the end; twice as many 128-query items are three to a CU then,
-        // each a little more than half as long (1 x H/1 x 2048 with H = 33 .. 44, i.e. 264 .. 352 items: 94.5 - 97.6 us
-        // against 99.9; 368 items 99.6 / 100.0; 384 items 102.6 / 100.1).
-        // (A causal problem whose queries are the last of at least twice as many keys - a chunk of new tokens against a
-        // cache - has items of nearly equal length, like a problem that is not causal: 1 x 32/8 x 2048 queries over 8192
-        // keys 223 / 200.)
-        const long wg256 = (long)((Sq + 255) / 256) * Hq * B;
-        const bool uneven = causal && Sk < 2 * (long)Sq;
-        variant = (Sq >= 256 && wg256 >= (uneven ? 320 : 256)) ? 2 : 1;
-        if (!causal && wg256 > 256 && wg256 <= 352) variant = 1;
+        int cus = 0;
+        if (hipError_t e = compute_units(cus); e != hipSuccess) return e;
+        variant = one_walk_us(2, cus, B, Hq, Sq, Sk, causal, kv_valid_len) < one_walk_us(1, cus, B, Hq, Sq, Sk, causal, kv_valid_len) ? 2 : 1;
     }
     if (variant == 2) return launch_fmha_pingpong<T, 2>(q, k, v, o, LSE, B, Hq, Hkv, Sq, Sk, scale, causal, kv_valid_len, sd, stream);
     return launch_fmha_pingpong<T, 1>(q, k, v, o, LSE, B, Hq, Hkv, Sq, Sk, scale, causal, kv_valid_len, sd, stream);
