@@ -11,6 +11,9 @@ from torch import Tensor
 
 __all__ = ["fine_fmha", "fine_fmha_with_lse"]
 
+# the operators of all indices, looked up by name once
+_KERNELS = {i: getattr(torch.ops.fmha_unified, f"finefmha_{i}").default for i in range(8)}
+
 
 def fine_fmha(q: Tensor, k: Tensor, v: Tensor, causal: bool, is_decode, kernel_index: int) -> Tensor:
     """softmax(q k^T / sqrt(d) + mask) v for q [B,Hq,Sq,128], k, v [B,Hkv,Sk,128] (fp16, GPU).
@@ -23,9 +26,11 @@ def fine_fmha(q: Tensor, k: Tensor, v: Tensor, causal: bool, is_decode, kernel_i
     are the same mask when ``Sq == Sk``, the only causal case the reference's tests and drivers use. A query row with no
     visible key (``Sq > Sk`` only) gives zeros. The result is a new contiguous [B, Hq, Sq, 128] tensor.
     """
-    kernel = getattr(torch.ops.fmha_unified, f"finefmha_{int(kernel_index)}")
+    kernel = _KERNELS.get(kernel_index) if type(kernel_index) is int else None
+    if kernel is None:
+        kernel = getattr(torch.ops.fmha_unified, f"finefmha_{int(kernel_index)}").default
     decode_length = k.size(2)
-    return kernel.default(q, k, v, bool(causal), bool(is_decode), decode_length)
+    return kernel(q, k, v, bool(causal), bool(is_decode), decode_length)
 
 
 def fine_fmha_with_lse(q: Tensor, k: Tensor, v: Tensor, causal: bool, is_decode=False) -> Tuple[Tensor, Tensor]:

@@ -13,6 +13,7 @@
 // non-square operands work, the output is allocated with empty() instead of zeros(), the launch goes to the
 // current stream, and every argument is validated before the device is touched.
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
@@ -24,6 +25,11 @@ namespace gemm_unified {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {}
 
 namespace {
+
+// an uninitialised GPU tensor, without a trip through the dispatcher (0.4 us)
+at::Tensor gpu_empty(at::IntArrayRef size, at::ScalarType type, const at::Tensor& like) {
+    return at::Tensor(at::detail::empty_cuda(size, type, like.device(), std::nullopt));
+}
 
 at::Tensor run_gemm(const at::Tensor& a, const at::Tensor& b, int layout, const char* name) {
     TORCH_CHECK(a.dim() == 2 && b.dim() == 2, name, ": a and b must be 2-D, got ", a.dim(), "-D and ", b.dim(), "-D");
@@ -51,7 +57,7 @@ at::Tensor run_gemm(const at::Tensor& a, const at::Tensor& b, int layout, const 
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
     at::Tensor ac = a.contiguous();
     at::Tensor bc = b.contiguous();
-    at::Tensor c = at::empty({M, N}, a.options());
+    at::Tensor c = gpu_empty({M, N}, a.scalar_type(), a);
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
     // Leading dimensions are the logical row lengths of the contiguous operands, not stride(0): torch ignores the stride of
     // a size-1 dimension when it decides contiguity, so a [1, K] operand may carry any stride(0).
@@ -62,7 +68,7 @@ at::Tensor run_gemm(const at::Tensor& a, const at::Tensor& b, int layout, const 
     at::Tensor ws;
     if (need > 0) {
         try {
-            ws = at::empty({static_cast<int64_t>(need)}, a.options().dtype(at::kByte));
+            ws = gpu_empty({static_cast<int64_t>(need)}, at::kByte, a);
         } catch (const c10::OutOfMemoryError&) {
             need = 0;
         }
