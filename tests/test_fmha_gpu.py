@@ -774,3 +774,52 @@ def test_either_kind_of_item_by_expected_time(lib, gpu, B, Hq, Hkv, S, causal):
     pinned = [run(lib, gpu, q, k, v, causal, variant=n) for n in (1, 2)]
     assert any(torch.equal(o, po) and torch.equal(lse, pl) for po, pl in pinned)
     check(lib, gpu, q[-1:], k[-1:], v[-1:], causal)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal,kvv", [
+    (1, 32, 8, 58, 2068, True, None),      # 7 ranges of 5 key tiles
+    (1, 8, 2, 36, 2386, True, 2350),       # 13 ranges, the last a short one
+    (1, 4, 4, 128, 1217, False, 1217),     # one valid key in the last tile
+    (2, 4, 2, 130, 1030, True, 1000),      # two q tiles
+    (1, 2, 1, 1500, 1400, True, None),     # causal: ranges that early q tiles do not see, rows that see no key
+])
+def test_key_ranges_over_shorter_caches(lib, gpu, dtype, B, Hq, Hkv, Sq, Sk, causal, kvv):
+    """Partial results in 32 bits: no further from attention over the same inputs in float32 than one walk over all keys."""
+    q, k, v = (x.to(dtype) for x in so.fmha_inputs(B, Hq, Hkv, Sq, Sk, seed=Sq + Sk + Hq))
+    tol = 2e-3 if dtype == torch.float16 else 1.6e-2
+    o4, l4 = run(lib, gpu, q, k, v, causal, kvv, variant=4)
+    o0, l0 = run(lib, gpu, q, k, v, causal, kvv)                  # the choice by shape takes the same path
+    assert torch.equal(o0, o4) and torch.equal(l0, l4)
+    o1, l1 = run(lib, gpu, q, k, v, causal, kvv, variant=1)
+    o_ref, l_ref = so.attention_ref(q.float(), k.float(), v.float(), causal=causal, kv_valid_len=kvv)
+    seen = torch.isfinite(l_ref)
+    assert torch.equal(torch.isfinite(l4), seen) and bool((o4[~seen] == 0).all())
+    assert (o4.float() - o_ref).abs().max() <= tol and (l4 - l_ref)[seen].abs().max() <= 1e-3
+    far = lambda o: (o.double() - o_ref.double()).norm()
+    assert far(o4) <= 1.02 * far(o1)       # (both are one rounding of O and of the probabilities away)
+    if kvv is not None and kvv < Sk:       # keys past the valid length may hold anything
+        k, v = k.clone(), v.clone()
+        k[:, :, kvv:] = float("nan")
+        v[:, :, kvv:] = float("inf")
+        o_p, l_p = run(lib, gpu, q, k, v, causal, kvv)
+        assert torch.equal(o4, o_p) and torch.equal(l4, l_p)
+
+
+def test_shorter_caches_without_the_librarys_workspace(lib, gpu):
+    """Where the library's buffer may not be made (a capture on a fresh stream) or is not to be used, the keys are walked in one go."""
+    q, k, v = (t.to(gpu) for t in so.fmha_inputs(1, 8, 2, 64, 1900, seed=4))
+    whole = lib.fmha_fwd(q, k, v, causal=True, variant=1)[0]
+    assert not torch.equal(lib.fmha_fwd(q, k, v, causal=True)[0], torch.zeros_like(whole))
+    assert lib.fmha_workspace_bytes(1, 8, 2, 64, 1900) == 0
+    out = torch.zeros_like(q)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        lib.fmha_fwd(q, k, v, causal=True, return_lse=False, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, whole) or torch.equal(out, lib.fmha_fwd(q, k, v, causal=True)[0])

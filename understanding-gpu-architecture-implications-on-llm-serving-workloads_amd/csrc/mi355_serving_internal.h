@@ -182,7 +182,8 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 //         a ring of eight; shapes 1 .. 7 take s ranges of K with variant + 16 s, merged by a kernel of their own (instead of
 //         the last workgroup of a tile) with variant + 16 s + 4096, shape 1 always. The gate/up product: 1, 2, 4, 5, 6, 8, 9
 //   fmha: 0 = by shape, 1 = 128-query workgroups, 2 = 256-query workgroups (1 and 2 also keep generation-step shapes off
-//         the split-KV path), 3 = keys cut into ranges and merged (an error where the choice by shape would not do that)
+//         the split-KV path), 3 = keys of a long cache cut into ranges and merged, 4 = those of a shorter one, partial results in 32 bits
+//         (an error where the choice by shape would not do that)
 extern "C" {
 int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int layout, int dtype, int variant, void* stream);
