@@ -989,14 +989,15 @@ static hipError_t launch_fmha_segmented(const T* Q, const T* K, const T* V, T* O
 }
 
 // Expected time of a call on work items of 128 `qb` queries, beside what both kinds have in common: that of the workgroup with the most
-// to do, as fmha_work_item deals the items out. An item takes 2.2 us and 1.25 us per key tile (256 queries, every K / V fragment feeding
-// two MFMAs: 4.6 and 1.75). That weighs the queries a tile is padded by, the last round of items and, causal, the length of the
+// to do, as fmha_work_item deals the items out. An item takes 2.6 us and 1.2 us per key tile (256 queries, every K / V fragment feeding
+// two MFMAs: 4.6 and 1.75); a last round of 128-query items up to a quarter less, the emptier it is (the clock rises; 528 .. 768 items over
+// 2048 keys 94.5 .. 102.6 us, as 256-query items 99.9 .. 100.1). That weighs the queries a tile is padded by, the last round of items and, causal, the length of the
 // heaviest item against the better kernel. Over 170 drawn calls (1 .. 16 sequences, 64 .. 8192 queries, 8 .. 64 heads, causal or not, and
 // chunks over a cache) the choice is within 0.2 % of the faster one on average; a rule on the number of 256-query items that preceded it, 1.7 %. us,
 // 128- / 256-query items: 13 x 64/8 x 353 causal 83 / 99, 9 x 32/32 x 317 causal 34 / 42, 16 x 32/8 x 512 causal 85 / 76, 4 x 64/8 x 152 17.0 / 13.7,
 // 3 x 16/4 x 917 36.6 / 29.1, 1 x 8/2 x 7441 228 / 183, 1 x 32/8 x 1331 44.7 / 35.6, 10 x 40/8 x 255 34.1 / 28.6, 8 x 64/8 x 638 causal 104 / 115.
 static float one_walk_us(int qb, int cus, int B, int Hq, int Sq, int Sk, int causal, int kv_valid) {
-    const float item = qb == 2 ? 4.6f : 2.2f, tile = qb == 2 ? 1.75f : 1.25f;
+    const float item = qb == 2 ? 4.6f : 2.6f, tile = qb == 2 ? 1.75f : 1.2f;
     const long bm = 128 * qb, q_tiles = (Sq + bm - 1) / bm, per_rank = (long)Hq * B, items = q_tiles * per_rank;
     const long wgs = std::min<long>(items, cus), rounds = (items + wgs - 1) / wgs;
     const auto rank_us = [&](long rank) {   // rank 0: the q tile that sees the most keys
@@ -1007,11 +1008,12 @@ static float one_walk_us(int qb, int cus, int B, int Hq, int Sq, int Sk, int cau
     if (rounds > 64) return (rank_us(0) + rank_us(q_tiles - 1)) * .5f * (float)items / (float)wgs;
     // the first, the last and the middle one, and the last one that has an item in the last round
     const long rest = items - (rounds - 1) * wgs, probes[4] = {0, wgs - 1, wgs / 2, (rounds - 1) % 2 == 0 ? rest - 1 : wgs - rest};
+    const float last = qb == 2 ? 1.f : .76f + .24f * (float)rest / (float)wgs;
     float most = 0.f;
     for (const long w : probes) {
         float sum = 0.f;
         for (long r = 0; r < rounds; ++r)
-            if (const long u = r * wgs + (r % 2 ? wgs - 1 - w : w); u < items) sum += rank_us(u / per_rank);
+            if (const long u = r * wgs + (r % 2 ? wgs - 1 - w : w); u < items) sum += rank_us(u / per_rank) * (r > 0 && r == rounds - 1 ? last : 1.f);
         most = std::max(most, sum);
     }
     return most;
