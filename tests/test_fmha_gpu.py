@@ -823,3 +823,21 @@ def test_shorter_caches_without_the_librarys_workspace(lib, gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, whole) or torch.equal(out, lib.fmha_fwd(q, k, v, causal=True)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal", [
+    (1, 16, 1, 1, 300, False), (1, 17, 1, 1, 300, False), (2, 32, 1, 1, 77, False),                # one and two blocks of 16 columns
+    (1, 1, 1, 1, 9000, False), (1, 2, 1, 1, 9000, False), (1, 3, 1, 1, 5000, False), (1, 4, 1, 1, 700, False), (1, 5, 1, 1, 20000, False),
+    (1, 8, 1, 4, 3000, True), (2, 6, 2, 3, 2100, True), (300, 2, 1, 1, 64, False), (1, 16, 4, 4, 200, True),
+])
+def test_generation_step_columns_and_shares_of_the_merge(lib, gpu, dtype, B, Hq, Hkv, Sq, Sk, causal):
+    """Columns at the edge of a block of 16; merges whose outputs are a quarter, a half and more of the threads, with a last share of
+    fewer key ranges, or none."""
+    q, k, v = (x.to(dtype) for x in so.fmha_inputs(B, Hq, Hkv, Sq, Sk, seed=Hq + Sk))
+    o, lse = lib.fmha_fwd(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal)
+    o2, lse2 = lib.fmha_fwd(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal)
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+    o_ref, lse_ref = so.attention_ref(q.float(), k.float(), v.float(), causal=causal)
+    assert (o.cpu().float() - o_ref).abs().max() <= (2e-3 if dtype == torch.float16 else 1.6e-2)
+    assert (lse.cpu() - lse_ref).abs().max() <= 1e-3

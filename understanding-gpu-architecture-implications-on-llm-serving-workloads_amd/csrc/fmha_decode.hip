@@ -59,20 +59,29 @@ constexpr int kMaxSplitPairs = 255;
 constexpr size_t kCounterBytes = size_t(kMaxSplitPairs + 1) * kCounterStride * sizeof(unsigned);   // 64 KiB
 
 __device__ __forceinline__ int swz_k(int row) { return row & 15; }
-__device__ __forceinline__ int swz_v(int row) {
-    int r = row & 3;
-    return (r << 1) | ((r & 1) << 3);
+__device__ __forceinline__ int swz_v(int row) { return (row & 7) << 1; }
+// maximum / sum over the four lanes that hold a column
+__device__ __forceinline__ float quad_max(float x) {
+    x = fmaxf(x, __shfl_xor(x, 16, 64));
+    return fmaxf(x, __shfl_xor(x, 32, 64));
 }
-__device__ __forceinline__ float other_half(float x) {
-    int idx = ((int)(threadIdx.x & 63) ^ 32) << 2;
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(idx, __builtin_bit_cast(int, x)));
+__device__ __forceinline__ float quad_sum(float x) {
+    x += __shfl_xor(x, 16, 64);
+    return x + __shfl_xor(x, 32, 64);
 }
 }  // namespace dec
 
 // Workgroup wg = (b * Hkv + hkv) * splits + s covers key tiles [s * tiles_per_split, (s + 1) * tiles_per_split).
 // WAVES waves with NSTAGE pipeline stages of 16 KiB each (two waves: a single key range only). <4, 2> (one wave per SIMD, one tile in flight behind the one
 // being consumed, 128 KiB of LDS) measured better than <3, 3> for short and for long key ranges alike.
-template <typename T, int WAVES, int NSTAGE>
+// NB: blocks of 16 columns. Both products are MFMA 16x16x32, laid out as in the prefill kernel (fmha_fwd.hip): S^T[kb] (16 keys x 16 columns)
+// = K[kb] Q^T, O^T[db] (16 d x 16 columns) += V^T[db] P^T; a lane holds 4 keys of a key block, or 4 d of a d block, of one column, the statistics
+// of a column live in four lanes, which only talk to each other when the exponent reference moves. A wave is alone on its SIMD and a tile a
+// chain of dependent steps: with 32x32x16 instructions, eight of them one behind the other for S^T, half of their columns empty where a kv
+// head has up to 16 query rows, and a cross-lane maximum in every tile, 301 keys (three tiles a wave) of 1 x 8/2 heads took 7.2 us, now 5.9;
+// the combine of the waves, then one output and two exponentials per thread and column, is part of that (1.4 -> 0.9 us). 1 x 32/8 heads over 256
+// keys 6.3 -> 5.1, 500 8.5 -> 7.0, 8191 12.8 -> 12.2, 64 x 64/8 over 300 19.8 -> 16.9; 8 x 32/8 over 8192, bound by HBM, 50.6 either way.
+template <typename T, int WAVES, int NSTAGE, int NB>
 __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, T* __restrict__ O, float* __restrict__ LSE,
     float* part, unsigned* counters, int B, int Hq, int Hkv, int Sq, int Sk, float scale_log2, int causal, int kv_valid,
@@ -92,14 +101,14 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     MI355_LDS char* wbase = (MI355_LDS char*)smem_raw + wave * WAVE_BYTES;
 
-    const int h = lane >> 5;
-    const int l32 = lane & 31;
+    const int g = lane >> 4;
+    const int c16 = lane & 15;
     const int s_idx = blockIdx.x % splits;
     const int bh = blockIdx.x / splits;
     const int hkv = bh % Hkv;
     const int b = bh / Hkv;
     const int group = Hq / Hkv;
-    const int ncols = group * Sq;  // <= 32
+    const int ncols = group * Sq;  // <= 16 NB
     const int shift = Sk - Sq;
 
     const T* Kh = K + b * sd.k_batch + hkv * sd.k_head;
@@ -138,17 +147,19 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
         }
     };
 
-    const int k_base = l32 * ROW_BYTES + ((h ^ (lane & 15)) << 4);  // xor (ks << 5)
-    const int v_row = 4 * h + ((lane & 15) >> 2);
-    const int v_clow = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-    const int v_base = TILE_BYTES + v_row * ROW_BYTES + ((v_clow ^ swz_v(v_row)) << 4) + (lane & 1) * 8;  // xor (db << 6)
+    const int k_base = c16 * ROW_BYTES + ((g ^ c16) << 4);   // xor (ks << 6), + kb * 16 rows
+    const int v_row = 4 * g + (c16 >> 2);
+    const int v_base = TILE_BYTES + v_row * ROW_BYTES + ((((c16 & 3) >> 1) ^ swz_v(v_row)) << 4) + (c16 & 1) * 8;  // xor (db << 5)
 
-    float16v o[4];
+    float4v o[NB][8];
+    float m_run[NB], l_run[NB];
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int nb = 0; nb < NB; ++nb) {
+        m_run[nb] = -INFINITY;
+        l_run[nb] = 0.f;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;
+        for (int db = 0; db < 8; ++db) o[nb][db] = float4v{0.f, 0.f, 0.f, 0.f};
+    }
 
     const int n_loc = t_end - t_begin;
     // each wave starts at a different tile of its piece and wraps around (the online softmax does not care about the
@@ -165,26 +176,31 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     // Everything about the queries comes behind the first key / value copies, so that those leave as early as possible
     // and the latency of the query fetch hides under theirs.
     // column c of the packed query block = (q head hkv*group + c / Sq, query row c % Sq)
-    const int col = min(l32, ncols - 1);
-    const int hq = hkv * group + col / Sq;
-    const int qi = col % Sq;
-    const T* qp = Q + b * sd.q_batch + hq * sd.q_head + qi * sd.q_row + 8 * h;
-    const int lim = causal ? min(kv_valid - 1, qi + shift) : kv_valid - 1;  // last visible key of this column
+    int lim[NB];      // last visible key of this lane's column(s)
+    V8 qf[NB][4];     // Q[column][32 ks + 8 g .. +7]
+    int lim_min = kv_valid - 1;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        const int col = min(16 * nb + c16, ncols - 1);
+        const int hq = hkv * group + col / Sq;
+        const int qi = col % Sq;
+        const T* qp = Q + b * sd.q_batch + hq * sd.q_head + qi * sd.q_row + 8 * g;
+        lim[nb] = causal ? min(kv_valid - 1, qi + shift) : kv_valid - 1;
+        lim_min = min(lim_min, lim[nb]);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) qf[nb][ks] = *(const V8*)(qp + ks * 32);
+    }
     // smallest such limit over the wave: tiles that end at or before it need no mask code
-    int lim_min = lim;
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) lim_min = min(lim_min, __shfl_xor(lim_min, off, 64));
+    for (int off = 8; off >= 1; off >>= 1) lim_min = min(lim_min, __shfl_xor(lim_min, off, 64));
     lim_min = __builtin_amdgcn_readfirstlane(lim_min);
-    V8 qf[8];
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = *(const V8*)(qp + ks * 16);
     // A use of the query fragments in front of the loop: the compiler waits for their loads where they are first used,
     // and it does not count the tile copies (inline assembly) among the loads in flight. With the first use inside the
     // loop that wait, "everything I know of has landed", came back on every iteration as vmcnt(0) in front of the S^T
     // products and held each tile's arithmetic until the NEXT tile's copies had landed too: no copy ever overlapped
     // arithmetic. Out here it waits once, for the first tile and the queries, which the first iteration needs anyway.
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));
+    for (int nb = 0; nb < NB; ++nb) asm volatile("" : "+v"(qf[nb][0]), "+v"(qf[nb][1]), "+v"(qf[nb][2]), "+v"(qf[nb][3]));
     int slot = 0, fill = NSTAGE - 1;
     for (int tt0 = t_begin; tt0 < t_end; ++tt0) {
         const int t = tile_of(tt0 - t_begin);
@@ -200,121 +216,139 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
         MI355_LDS char* st = wbase + slot * STAGE_BYTES;
         slot = (slot + 1 == NSTAGE) ? 0 : slot + 1;
 
-        // S^T = K Q^T : lane holds keys 8p + 4h + q of column l32
-        float16v s;
+        // S^T = K Q^T: lane holds keys 16 kb + 4 g + 0..3 of its column
+        float4v s[NB][2];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = 0.f;
+        for (int nb = 0; nb < NB; ++nb) s[nb][0] = s[nb][1] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            V8 kf = Elem<T>::frag(lds_read_b128(st + (k_base ^ (ks << 5))));
-            s = Elem<T>::mfma32(kf, qf[ks], s);
-        }
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                V8 kf = Elem<T>::frag(lds_read_b128(st + ((k_base ^ (ks << 6)) + kb * 16 * ROW_BYTES)));
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) s[nb][kb] = Elem<T>::mfma16(kf, qf[nb][ks], s[nb][kb]);
+            }
         const int key0 = t * TK;
         if (key0 + TK - 1 > lim_min) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                int key = key0 + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (key > lim) s[e] = -INFINITY;
-            }
-        }
-        float mx = s[0];
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
-        mx = fmaxf(mx, other_half(mx));
+                for (int e = 0; e < 8; ++e)
+                    if (key0 + 16 * (e >> 2) + 4 * g + (e & 3) > lim[nb]) s[nb][e >> 2][e & 3] = -INFINITY;
+        }
         // lazy rescaling as in the prefill kernel: m_run is the exponent reference of the running sums and only moves
-        // (with O and l rescaled) when some column exceeds it by more than 2^kLazyLog2
-        const bool raise = (mx - m_run) * scale_log2 > kLazyLog2;  // -inf - -inf = NaN compares false
+        // (with O and l rescaled) when some score exceeds it by more than 2^kLazyLog2
+        float mx[NB];
+        bool raise = false;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            mx[nb] = fmaxf(fmaxf(fmaxf(s[nb][0][0], s[nb][0][1]), fmaxf(s[nb][0][2], s[nb][0][3])),
+                           fmaxf(fmaxf(s[nb][1][0], s[nb][1][1]), fmaxf(s[nb][1][2], s[nb][1][3])));
+            raise = raise || (mx[nb] - m_run[nb]) * scale_log2 > kLazyLog2;  // -inf - -inf = NaN compares false
+        }
         if (__builtin_amdgcn_ballot_w64(raise) != 0) {
-            float m_new = fmaxf(m_run, mx);
-            float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-            float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * scale_log2);
-            m_run = m_new;
-            l_run *= alpha;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int nb = 0; nb < NB; ++nb) {
+                const float m_new = fmaxf(m_run[nb], quad_max(mx[nb]));
+                const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f((m_run[nb] - m_use) * scale_log2);
+                m_run[nb] = m_new;
+                l_run[nb] *= alpha;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
+                for (int db = 0; db < 8; ++db) o[nb][db] *= alpha;
+            }
         }
-        const float neg_ms = (m_run == -INFINITY) ? 0.f : -m_run * scale_log2;
-        float psum = 0.f;
-        V8 pf[2];
+        V8 pf[NB];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            V8 pk;
+        for (int nb = 0; nb < NB; ++nb) {
+            const float neg_ms = (m_run[nb] == -INFINITY) ? 0.f : -m_run[nb] * scale_log2;
+            float psum = 0.f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * tt + j], scale_log2, neg_ms));
+            for (int e = 0; e < 8; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[nb][e >> 2][e & 3], scale_log2, neg_ms));
                 psum += p;
-                pk[j] = (T)p;
+                pf[nb][e] = (T)p;
             }
-            pf[tt] = pk;
+            l_run[nb] += psum;
         }
-        l_run += psum;
-        // O^T += V^T P^T
+        // O^T += V^T P^T; the 8 keys of a lane of P are 4 g + 0..3 and 16 + 4 g + 0..3, V^T is gathered in that order
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int db = 0; db < 8; ++db) {
+            MI355_LDS char* vp = st + (v_base ^ (db << 5));
+            V8 vf = Elem<T>::frag(concat(lds_read_tr16_b64(vp), lds_read_tr16_b64(vp + 16 * ROW_BYTES)));
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                int off = (v_base ^ (db << 6)) + (16 * tt) * ROW_BYTES;
-                V8 vf = Elem<T>::frag(concat(lds_read_tr16_b64(st + off), lds_read_tr16_b64(st + off + 8 * ROW_BYTES)));
-                o[db] = Elem<T>::mfma32(vf, pf[tt], o[db]);
-            }
+            for (int nb = 0; nb < NB; ++nb) o[nb][db] = Elem<T>::mfma16(vf, pf[nb], o[nb][db]);
+        }
         wait_lgkmcnt<0>();  // the reads of this slot are complete before a later copy refills it
     }
 
     // ---- combine the waves of the workgroup through LDS (the pipelines are drained: their memory is free) ------------
     // per wave: O~ [ncols][128] floats, then m [32], l [32]
-    const float l_tot = l_run + other_half(l_run);
     MI355_TL(tl[2] = timeline::wall_clock();)
     __syncthreads();
     MI355_LDS float* cmb = (MI355_LDS float*)smem_raw;
     const int wave_floats = ncols * D + 64;
     {
         MI355_LDS float* mine = cmb + wave * wave_floats;
-        if (l32 < ncols) {
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+        for (int nb = 0; nb < NB; ++nb) {
+            const int col = 16 * nb + c16;
+            const float l_tot = quad_sum(l_run[nb]);
+            if (col < ncols) {
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    float4v v;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) v[q] = o[db][4 * p + q];
-                    *(MI355_LDS float4v*)(mine + l32 * D + db * 32 + 8 * p + 4 * h) = v;
+                for (int db = 0; db < 8; ++db) *(MI355_LDS float4v*)(mine + col * D + db * 16 + 4 * g) = o[nb][db];
+                if (g == 0) {
+                    mine[ncols * D + col] = m_run[nb];
+                    mine[ncols * D + 32 + col] = l_tot;
                 }
-            if (h == 0) {
-                mine[ncols * D + l32] = m_run;
-                mine[ncols * D + 32 + l32] = l_tot;
             }
         }
     }
     __syncthreads();
     const long row0 = ((long)b * Hq + (long)hkv * group) * Sq;   // LSE index of column 0 (columns are consecutive rows)
-    // element idx = (column, d) of the workgroup's result; weights 2^((m_w - m) c), 0 for waves without a visible key
-    auto combined = [&](int c, int d, float& m_out, float& l_out) {
-        float m = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) m = fmaxf(m, cmb[w * wave_floats + ncols * D + c]);
-        float acc = 0.f, l = 0.f;
+    const int n_out = ncols * (D / 4);   // output elements f = (column f / 32, d 4 (f % 32) .. +3)
+    // an output element over the workgroup's waves; weights 2^((m_w - m) c), 0 for waves without a visible key
+    auto combined = [&](int f, float& m_out, float& l_out) {
+        const int c = f >> 5;
+        float mw[WAVES], lw[WAVES];
+        float4v ow[WAVES];
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            const float mw = cmb[w * wave_floats + ncols * D + c];
-            const float wgt = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((mw - m) * scale_log2);
-            acc += wgt * cmb[w * wave_floats + c * D + d];
-            l += wgt * cmb[w * wave_floats + ncols * D + 32 + c];
+            mw[w] = cmb[w * wave_floats + ncols * D + c];
+            lw[w] = cmb[w * wave_floats + ncols * D + 32 + c];
+            ow[w] = *(MI355_LDS const float4v*)(cmb + w * wave_floats + 4 * f);
+        }
+        float m = -INFINITY, l = 0.f;
+        float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) m = fmaxf(m, mw[w]);
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float wgt = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((mw[w] - m) * scale_log2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += wgt * ow[w][e];
+            l += wgt * lw[w];
         }
         m_out = m;
         l_out = l;
         return acc;
     };
+    auto store_out = [&](int f, const float4v& acc, float m, float l) {
+        const int c = f >> 5, d = (f & 31) * 4;
+        const float inv = (l > 0.f) ? 1.f / l : 0.f;
+        const int chq = hkv * group + c / Sq, cqi = c % Sq;
+        typename Elem<T>::v4 ov;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[e] * inv);
+        *(typename Elem<T>::v4*)(O + b * sd.o_batch + chq * sd.o_head + cqi * sd.o_row + d) = ov;
+        if (LSE != nullptr && d == 0)
+            LSE[row0 + c] = (l > 0.f) ? (m * scale_log2 + __builtin_log2f(l)) * 0.69314718055994531f : -INFINITY;
+    };
     if (splits == 1) {   // the only key range of this (batch, kv head): the result is final
-        for (int idx = tid; idx < ncols * D; idx += NTHREADS) {
-            const int c = idx >> 7, d = idx & (D - 1);
+        for (int f = tid; f < n_out; f += NTHREADS) {
             float m, l;
-            const float acc = combined(c, d, m, l);
-            const int chq = hkv * group + c / Sq, cqi = c % Sq;
-            O[b * sd.o_batch + chq * sd.o_head + cqi * sd.o_row + d] = (T)((l > 0.f) ? acc / l : 0.f);
-            if (LSE != nullptr && d == 0)
-                LSE[row0 + c] = (l > 0.f) ? (m * scale_log2 + __builtin_log2f(l)) * 0.69314718055994531f : -INFINITY;
+            const float4v acc = combined(f, m, l);
+            store_out(f, acc, m, l);
         }
         MI355_TL(wait_vmcnt<0>(); tl[7] = timeline::wall_clock(); tl_dump();)
         return;
@@ -323,7 +357,7 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     // merges them is ordered by instructions, not by a release / acquire pair: a device-scope fence writes back and
     // invalidates a whole L2 here, and an acquire-release ticket costs 2.5-3 us per launch (b = 1 over 8192 keys: 13.8 us
     // against 11.0). What takes the fence's place, step by step:
-    //   1. every partial result is stored with a device-scope atomic store, i.e. `global_store_dword .. sc1`: written through
+    //   1. every partial result is stored with a device-scope atomic store, i.e. `global_store_dwordx2 .. sc1`: written through
     //      the XCD's L2 to memory, nothing of it stays dirty in a cache;
     //   2. `s_waitcnt vmcnt(0)` behind the stores: on gfx9-family parts a store leaves vmcnt only when the memory system has
     //      acknowledged it at the scope it was issued with. The wait is an assembly statement with a memory clobber, so the
@@ -337,14 +371,15 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     //      ticket's value, which the hardware cannot pass before the atomic has returned.
     // tests/test_inline_asm_loads_cpu.py checks 1, 2 and 5 in the generated code.
     float* mypart = part + (long)blockIdx.x * ncols * PART_STRIDE;
-    for (int idx = tid; idx < ncols * D; idx += NTHREADS) {
-        const int c = idx >> 7, d = idx & (D - 1);
+    for (int f = tid; f < n_out; f += NTHREADS) {
+        const int c = f >> 5, d = (f & 31) * 4;
         float m, l;
-        __hip_atomic_store(mypart + c * PART_STRIDE + d, combined(c, d, m, l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (d == 0) {
-            __hip_atomic_store(mypart + c * PART_STRIDE + D, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(mypart + c * PART_STRIDE + D + 1, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        const float4v acc = combined(f, m, l);
+        const auto pair = [](float x, float y) { return (uint64_t)__builtin_bit_cast(uint32_t, x) | (uint64_t)__builtin_bit_cast(uint32_t, y) << 32; };
+        uint64_t* dst = reinterpret_cast<uint64_t*>(mypart + c * PART_STRIDE + d);
+        __hip_atomic_store(dst, pair(acc[0], acc[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(dst + 1, pair(acc[2], acc[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (d == 0) __hip_atomic_store(reinterpret_cast<uint64_t*>(mypart + c * PART_STRIDE + D), pair(m, l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // ---- ticket: the workgroup that completes the set of key ranges of (b, hkv) merges them ----------------------------
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's partial results have reached memory before the ticket is drawn
@@ -369,13 +404,13 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     // BATCH loads of 16 bytes each: the outputs of key ranges sp0 .. sp0 + BATCH - 1 for 4 d of one column
     // (in groups of 8 key ranges, a group only when it holds a key range that exists: a call with 4 key ranges issues 8
     // loads per thread, not 32; within a group, key ranges past the last one repeat it and get weight zero)
-    auto load_batch = [&](float4v(&v)[BATCH], const float* pc, int sp0) {
+    auto load_batch = [&](float4v(&v)[BATCH], const float* pc, int sp0, int sp_end) {
 #pragma unroll
         for (int g8 = 0; g8 < BATCH; g8 += 8) {
-            if (sp0 + g8 < splits) {
+            if (sp0 + g8 < sp_end) {
 #pragma unroll
                 for (int u = g8; u < g8 + 8; ++u) {
-                    const float* pa = pc + (long)min(sp0 + u, splits - 1) * split_stride;
+                    const float* pa = pc + (long)min(sp0 + u, sp_end - 1) * split_stride;
                     asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v[u]) : "v"(pa) : "memory");
                 }
             }
@@ -392,8 +427,14 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
     // the first batch of this thread's first output element goes out before the statistics are fetched: one memory
     // round trip serves both
     float4v v[BATCH];
-    const int n_out = ncols * (D / 4);   // output elements f = (column, group of 4 d)
-    if (tid < n_out) load_batch(v, base + (tid >> 5) * PART_STRIDE + (tid & 31) * 4, 0);
+    // Where the outputs are a half or a quarter as many as the threads (or fewer), two or four threads share one and take a part of
+    // the key ranges each; their sums meet in LDS, in order.
+    const int parts = n_out * 4 <= NTHREADS ? 4 : n_out * 2 <= NTHREADS ? 2 : 1;
+    const int per_part = (splits + parts - 1) / parts;
+    const int my_part = parts == 1 ? 0 : tid / n_out;   // >= parts: an idle thread
+    const int first_sp = my_part * per_part, end_sp = my_part < parts ? min(first_sp + per_part, splits) : first_sp;
+    const int first_f = parts == 1 ? tid : tid - my_part * n_out;
+    if (first_f < n_out && first_sp < end_sp) load_batch(v, base + (first_f >> 5) * PART_STRIDE + (first_f & 31) * 4, first_sp, end_sp);
     for (int i = tid; i < splits * ncols; i += NTHREADS) {
         const float* ps = base + (long)(i / ncols) * split_stride + (i % ncols) * PART_STRIDE + D;
         float ms, ls;
@@ -425,28 +466,29 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
         if (i < ncols) st_mc[c] = m;
     }
     __syncthreads();
-    for (int f = tid; f < n_out; f += NTHREADS) {
-        const int c = f >> 5, d = (f & 31) * 4;
-        const float* pc = base + c * PART_STRIDE + d;
+    MI355_LDS float* st_acc = cmb + ((3 * splits * ncols + ncols + 3) & ~3);   // [parts - 1][n_out][4], then [parts - 1][n_out]: their sums of l
+    for (int f = first_f; f < n_out; f += NTHREADS) {   // (more than one part: every thread, once)
+        const int c = f >> 5;
+        const float* pc = base + c * PART_STRIDE + (f & 31) * 4;
         float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
         float l = 0.f;
-        for (int sp0 = 0; sp0 < splits; sp0 += BATCH) {
-            if (f != tid || sp0 != 0) load_batch(v, pc, sp0);
+        for (int sp0 = first_sp; sp0 < end_sp; sp0 += BATCH) {
+            if (f != first_f || sp0 != first_sp) load_batch(v, pc, sp0, end_sp);
             // the weights of this batch, while its loads are in flight (all LDS reads first, so they overlap each other);
             // key ranges past the last one repeat it with weight zero
             float wgt[BATCH], ls[BATCH];
 #pragma unroll
             for (int g8 = 0; g8 < BATCH; g8 += 8) {
-                if (sp0 + g8 < splits) {
+                if (sp0 + g8 < end_sp) {
 #pragma unroll
                     for (int u = g8; u < g8 + 8; ++u) {
-                        const int sp = min(sp0 + u, splits - 1);
+                        const int sp = min(sp0 + u, end_sp - 1);
                         wgt[u] = st_w[sp * ncols + c];
                         ls[u] = st_l[sp * ncols + c];
                     }
 #pragma unroll
                     for (int u = g8; u < g8 + 8; ++u) {
-                        if (sp0 + u >= splits) wgt[u] = ls[u] = 0.f;
+                        if (sp0 + u >= end_sp) wgt[u] = ls[u] = 0.f;
                         l += ls[u];
                     }
                 }
@@ -454,7 +496,7 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
             wait_batch(v);
 #pragma unroll
             for (int g8 = 0; g8 < BATCH; g8 += 8) {
-                if (sp0 + g8 < splits) {
+                if (sp0 + g8 < end_sp) {
 #pragma unroll
                     for (int u = g8; u < g8 + 8; ++u)
 #pragma unroll
@@ -462,15 +504,20 @@ __global__ __launch_bounds__(WAVES * 64) void fmha_decode_kernel(
                 }
             }
         }
+        if (parts > 1) {
+            if (my_part > 0 && my_part < parts) {
+                *(MI355_LDS float4v*)(st_acc + 4 * ((my_part - 1) * n_out + f)) = acc;
+                st_acc[4 * (parts - 1) * n_out + (my_part - 1) * n_out + f] = l;
+            }
+            __syncthreads();
+            if (my_part > 0) break;
+            for (int p = 1; p < parts; ++p) {
+                acc += *(MI355_LDS const float4v*)(st_acc + 4 * ((p - 1) * n_out + f));
+                l += st_acc[4 * (parts - 1) * n_out + (p - 1) * n_out + f];
+            }
+        }
         MI355_TL(tl[6] = timeline::wall_clock();)
-        const float inv = (l > 0.f) ? 1.f / l : 0.f;
-        const int chq = hkv * group + c / Sq, cqi = c % Sq;
-        typename Elem<T>::v4 ov;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[e] * inv);
-        *(typename Elem<T>::v4*)(O + b * sd.o_batch + chq * sd.o_head + cqi * sd.o_row + d) = ov;
-        if (LSE != nullptr && d == 0)
-            LSE[row0 + c] = (l > 0.f) ? (st_mc[c] * scale_log2 + __builtin_log2f(l)) * 0.69314718055994531f : -INFINITY;
+        store_out(f, acc, st_mc[c], l);
     }
     // ready for the next call that uses this workspace (a device-scope store like the tickets, which are the only other
     // accesses to the counter; the next launch on the stream starts after this one has ended)
@@ -493,8 +540,10 @@ static hipError_t clear_counters(void* counters, long n, hipStream_t stream) {
 // longer than a short walk over the keys; the prefill kernel pads every head's queries to 128 rows, but has a workgroup per
 // query head, and pays only from 256 of those on. us, prefill kernel / this one: 1 x 32/8 heads, 8 queries over 64 keys 5.6 / 11.6,
 // over 300 9.2 / 13.8; 4 x 32/32, 20 queries over 128 keys 7.1 / 10.0; 1 x 32/8, one query over 300 keys 9.1 / 7.9; 64 x 32/8,
-// one query over 300 keys 65 / 17, 5 queries 65 / 23. The model is within 4 % of the faster one on average over 24 head
-// configurations, 1 .. 32 queries and 32 .. 511 keys (0.66 of the prefill kernel's time, nowhere more than 1.09).
+// one query over 300 keys 65 / 17, 5 queries 65 / 23. The model was within 4 % of the faster one on average over 24 head
+// configurations, 1 .. 32 queries and 32 .. 511 keys (0.66 of the prefill kernel's time, nowhere more than 1.09); with up to 16 columns this
+// kernel has since become faster (one block of matrix instructions 16 columns wide): 2 x 16/4, 4 queries over 112 keys 7.4 / 6.1, 1 x 32/8, 4
+// over 300 9.3 / 7.1.
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
     const long cols = (long)(Hq / Hkv) * Sq;
     if (cols > 32 || Sk < kv_valid_len || B < 1) return false;
@@ -504,6 +553,8 @@ bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid
     const float prefill_us = 4.9f + .78f * tiles64 + (float)((items + 255) / 256 - 1) * (2.4f + 1.09f * tiles64);
     const float step_us = kv_valid_len <= 64 && wgs > 256   // two waves, two workgroups to a CU
                               ? (float)((wgs + 511) / 512) * (2.8f + .34f * (float)cols + .0403f * (float)kv_valid_len)
+                          : cols <= 16 && kv_valid_len > 64
+                              ? (float)((wgs + 255) / 256) * (3.f + .13f * (float)cols + .6f * ceilf(tiles32 / 4.f))
                               : (float)((wgs + 255) / 256) * (3.5f + .225f * (float)cols + 1.1f * ceilf(tiles32 / 4.f));
     return step_us <= 1.03f * prefill_us;
 }
@@ -682,14 +733,14 @@ static hipError_t static_scratch_ptr(char** out) {
     return hipSuccess;
 }
 
-template <typename T, int WAVES, int NSTAGE>
+template <typename T, int WAVES, int NSTAGE, int NB>
 static hipError_t launch_decode(const T* Q, const T* K, const T* V, T* O, float* LSE, float* part, unsigned* counters, int B,
                                 int Hq, int Hkv, int Sq, int Sk, float scale_log2, int causal, int kv_valid, int splits,
                                 int tiles_per_split, long workgroups, const FmhaStrides& sd, hipStream_t stream) {
     constexpr int LDS = WAVES * NSTAGE * dec::STAGE_BYTES;
     static_assert(LDS >= WAVES * (32 * dec::D + 64) * 4 + 64, "the combine step reuses the pipeline memory");
-    static_assert(WAVES < 4 || LDS >= (3 * dec::kMaxSplits * 32 + 32 + 64) * 4, "so does the merge of the key ranges");
-    auto kern = fmha_decode_kernel<T, WAVES, NSTAGE>;
+    static_assert(WAVES < 4 || LDS >= (3 * dec::kMaxSplits * 32 + 32 + 64 + 5 * WAVES * 64) * 4, "so does the merge of the key ranges");
+    auto kern = fmha_decode_kernel<T, WAVES, NSTAGE, NB>;
     static DynamicLdsOnce lds_once;
     if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(kern), LDS); e != hipSuccess) return e;
     if (workgroups > 0x7fffffffL) return hipErrorInvalidValue;
@@ -730,11 +781,10 @@ hipError_t fmha_decode_dispatch(const T* Q, const T* K, const T* V, T* O, float*
     float* part = reinterpret_cast<float*>(wsp + plan.counter_bytes);
     unsigned* counters = reinterpret_cast<unsigned*>(wsp);
     const float scale_log2 = scale * 1.4426950408889634f;
-    if (plan.waves == 2)
-        return launch_decode<T, 2, 2>(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits,
-                                      plan.tiles_per_split, plan.workgroups, sd, stream);
-    return launch_decode<T, 4, 2>(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits,
-                                  plan.tiles_per_split, plan.workgroups, sd, stream);
+    const bool wide = (Hq / Hkv) * Sq > 16;   // two blocks of 16 columns
+    const auto launch = plan.waves == 2 ? (wide ? &launch_decode<T, 2, 2, 2> : &launch_decode<T, 2, 2, 1>) : (wide ? &launch_decode<T, 4, 2, 2> : &launch_decode<T, 4, 2, 1>);
+    return launch(Q, K, V, O, LSE, part, counters, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid, plan.splits, plan.tiles_per_split,
+                  plan.workgroups, sd, stream);
 }
 
 template hipError_t fmha_decode_dispatch<half_t>(const half_t*, const half_t*, const half_t*, half_t*, float*, int, int, int, int,

@@ -696,6 +696,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         };
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
+            if (q_item0 + qb * 16 >= Sq) break;   // no such rows (a few queries are done 0.5 us sooner for it)
             const float l_tot = kSumOnMatrixPipe ? l_acc[qb][0] : quad_sum(l_acc[qb][0]);
             const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
             if constexpr (SEG == kRangesF32) {   // 64 bytes of a row as they lie
