@@ -116,8 +116,8 @@ int mi355_hgemm_add(const void* A, const void* B, const void* R, void* C, int M,
  * length is not a multiple of 8, a view that starts at an odd element). mi355_gemm_workspace_bytes says how many bytes the
  * copies of a call may take (0: none are made). With that much `workspace` (16-byte aligned, contents irrelevant before and
  * after the call) such operands are copied first and the product runs on the fast paths, where that is expected to be done
- * sooner (1999 x 3001 x 2503 NN: 712 us without, 43 with; one row against a wide operand, or a short K, is not); with
- * less, or NULL, the call runs without copies, like the entry points above.
+ * sooner (1999 x 3001 x 2503 NN: 59 us without, 43 with; up to a few hundred rows, or with a short K, it is not); with
+ * less, or NULL, the call reads them where they lie, like the entry points above.
  * Calls that share a workspace must be ordered on one stream. The operators of gemm_unified pass memory of torch's
  * allocator; the reference's kernels take none of these shapes.
  */

@@ -656,6 +656,42 @@ def test_operands_with_unaligned_rows_through_aligned_copies(lib, gpu, dtype, la
     assert bool((c[M:] == 5.0).all()) and bool((c[:, N:] == 5.0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("variant", [10, 11, 10 + 16 * 3, 11 + 16 * 7])
+@pytest.mark.parametrize("M,N,K,off_a,off_b,residual", [
+    (1, 1, 1, 0, 0, False), (3, 2, 2, 1, 3, True), (2, 300, 3, 0, 1, False), (8, 1, 71, 7, 0, False), (64, 64, 64, 0, 0, False), (64, 128, 320, 1, 2, True),
+    (65, 63, 191, 0, 0, False), (127, 129, 257, 3, 5, True), (128, 256, 513, 0, 1, False), (5, 1031, 449, 0, 0, True), (257, 7, 640, 2, 0, False)])
+def test_operands_read_where_they_lie(lib, gpu, dtype, layout, variant, M, N, K, off_a, off_b, residual):
+    # the direct kernel: K and C that end anywhere, operands of fewer than 8 elements, fewer K tiles than loads in flight, empty ranges. What
+    # surrounds the operands holds NaNs, what surrounds C comes back untouched. One rounding of the product, one of the sum with a residual.
+    a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
+    a, b = a.to(dtype), b.to(dtype)
+    raw = lambda t, off: torch.cat((torch.full((off,), float("nan"), dtype=dtype), t.reshape(-1),
+                                    torch.full((9,), float("nan"), dtype=dtype))).to(gpu)
+    ag, bg = raw(a, off_a), raw(b, off_b)
+    c = torch.full((M + 1, N + 3), 5.0, dtype=dtype, device=gpu)
+    r = (torch.randn(M, N, generator=torch.Generator().manual_seed(7)) * 2).to(dtype)
+    rg = r.to(gpu)
+    tail = (lib.LAYOUTS[layout], lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, variant, torch.cuda.current_stream(gpu).cuda_stream)
+    pa, pb = ag.data_ptr() + 2 * off_a, bg.data_ptr() + 2 * off_b
+    if residual:
+        rc = lib.load().mi355_internal_hgemm_add_variant(pa, pb, rg.data_ptr(), c.data_ptr(), M, N, K, a.shape[1], b.shape[1], N, N + 3, *tail)
+    else:
+        rc = lib.load().mi355_internal_hgemm_variant(pa, pb, c.data_ptr(), M, N, K, a.shape[1], b.shape[1], N + 3, *tail)
+    assert rc == 0
+    torch.cuda.synchronize()
+    ref = so.gemm_ref(a, b, layout)
+    got = c[:M, :N].cpu().float()
+    err = (got - (r.float() if residual else 0.0) - ref).abs()
+    # fp32 sums in two orders: K 2^-23 of the sum of magnitudes at most; one rounding of the product, one of the sum
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    sums = K * 2.0 ** -23 * so.gemm_ref(a.abs(), b.abs(), layout)
+    bound = (1 + eps) * (eps * ref.abs() + sums) + (eps * got.abs() * 1.01 if residual else 0.0) + 2.0 ** -24
+    assert bool((err <= bound).all()), float((err - bound).max())
+    assert bool((c[M:] == 5.0).all()) and bool((c[:, N:] == 5.0).all())
+
+
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
 @pytest.mark.parametrize("shape", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("M,N,K,splits,own_merge", [(150, 200, 1000, 3, False), (150, 203, 1000, 3, True), (257, 64, 712, 5, False),

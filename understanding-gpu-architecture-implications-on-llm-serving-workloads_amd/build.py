@@ -34,7 +34,7 @@ DEVICE_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wno-inline-asm", "-Wno-unused-command-line-argument",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/hgemm_dispatch.hip", "csrc/hgemm_choice.hip", "csrc/gemm_pack.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip", "csrc/glue.hip", "csrc/capi.hip"]
+KERNEL_SOURCES = ["csrc/hgemm.hip", "csrc/hgemm_direct.hip", "csrc/hgemm_dispatch.hip", "csrc/hgemm_choice.hip", "csrc/gemm_pack.hip", "csrc/fmha_fwd.hip", "csrc/fmha_decode.hip", "csrc/glue.hip", "csrc/capi.hip"]
 # A source listed here is compiled once per entry, each time with that entry's defines, into objects of its own (side by
 # side with the others): the GEMM source holds every tile shape for two element types and three layouts, and one
 # compiler process each cuts the time the build waits for it to a third of what one per element type takes.
@@ -43,7 +43,7 @@ SOURCE_PARTS = {"csrc/hgemm.hip": [(t + "." + l.lower(), ["-DMI355_HGEMM_T=%s_t"
                                    for t in ("fp16", "bf16") for l in ("NN", "NT", "TN")]}
 # Per-source additions. The GEMM keeps its MFMA accumulators in ordinary VGPRs: left to itself the compiler moves part of
 # them to AGPRs in the 4-wave kernels and then shuffles them back and forth inside the K loop.
-SOURCE_FLAGS = {"csrc/hgemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+SOURCE_FLAGS = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for src in ("csrc/hgemm.hip", "csrc/hgemm_direct.hip")}
 
 
 def check_archs():

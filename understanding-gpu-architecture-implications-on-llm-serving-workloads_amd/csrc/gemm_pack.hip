@@ -1,8 +1,7 @@
 // Aligned copies of GEMM operands whose rows are not 16-byte aligned (a dense matrix whose row length is not a multiple of
-// 8, a view that starts at an odd element). The GEMM's global -> LDS copies move 16 aligned bytes; without this pass such products
-// run the bounds-checked kernel (and some still do: copies_pay in hgemm_dispatch.hip), which gathers its operands element by element, one memory round trip (~0.85 us) per 16 columns of K. Measured without / with the copies:
-// 1999 x 3001 x 2503 NN 712 / 43 us, 3789 x 8336 x 5632 TN 2555 / 309, 998 x 12720 x 6719 NN 4231 / 163, 2 x 13248 x 5824 TN
-// 318 / 32, 5 x 744 x 11040 TN 502 / 38, 88 x 384 x 1020 TN 38 / 6.
+// 8, a view that starts at an odd element). The tiled kernels' global -> LDS copies move 16 aligned bytes; the direct kernel
+// (hgemm_direct.hip) reads such operands where they lie, at about half the tiled kernels' rate on large products. Which of the two a
+// product takes: copies_pay in hgemm_dispatch.hip, with both sides measured.
 #include "mi355_common.h"
 #include "mi355_serving_internal.h"
 

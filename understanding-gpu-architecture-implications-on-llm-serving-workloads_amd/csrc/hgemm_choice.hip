@@ -133,4 +133,39 @@ KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles
     return e.choice;
 }
 
+// The direct kernel (hgemm_direct.hip) for a product: tiles and ranges of K. A K tile costs a CU .37 us on 64x64 tiles however many of
+// them share it (its LDS is busy: every operand byte is written once and read twice), .94 us on one 128x128 tile and 1.54 on two.
+// Fitted to 1460 timings of 230 products (1 .. 2600 rows, 64 .. 20000 columns, K 40 .. 9000, all layouts, weights from HBM): the
+// choice among these kernels and the aligned copies, copies_pay, takes 1.9 % longer than the fastest of them on average; copies and
+// the gather that they were weighed against before, 33 %.
+KernelChoice choose_direct(int M, int N, int K, int layout, bool split_ok) {
+    static const int ranges[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    const int ktiles = (K + 63) / 64;
+    const float b_bytes = 2.f * (float)N * (float)K, out_mb = 2e-6f * (float)M * (float)N, mb = b_bytes * 1e-6f + 2e-6f * (float)M * (float)K + out_mb;
+    const float hbm = b_bytes > 20e6f ? 1.f : 0.f, floor_us = mb / 3.6f + 4.06f;
+    KernelChoice best;
+    best.us = 1e30f;
+    for (const int shape : {(int)kDirect64x64, (int)kDirect128x128}) {
+        const bool large = shape == kDirect128x128;
+        const int bm = large ? 128 : 64;
+        if (large && M <= 32) break;
+        const long tiles = (long)((M + bm - 1) / bm) * ((N + bm - 1) / bm);
+        const float factor = (layout == MI355_GEMM_NT ? 1.045f : layout == MI355_GEMM_TN ? .95f : 1.f) * (1.f + hbm * (large ? .066f : .276f));
+        for (const int s : ranges) {
+            const long wgs = tiles * s;
+            const float part_mb = 4e-6f * (float)wgs * (float)(bm * bm);
+            if (s > 1 && (!split_ok || ktiles < 2 * s || part_mb > 48.f)) break;
+            const float per_cu = (float)((wgs + 255) / 256);
+            const float step = large ? std::fmax(.943f * (float)((wgs + 511) / 512), .769f * per_cu) : .367f * per_cu;
+            float us = std::fmax((large ? 5.31f : 4.23f) + (float)((ktiles + s - 1) / s) * step * factor, floor_us) + out_mb * (large ? .223f : .561f);
+            if (s > 1) us += 1.84f + .413f * part_mb + .116f * (float)s;
+            if (us >= best.us) continue;
+            best.us = us;
+            best.shape = shape;
+            best.splits = s;
+        }
+    }
+    return best;
+}
+
 }  // namespace mi355

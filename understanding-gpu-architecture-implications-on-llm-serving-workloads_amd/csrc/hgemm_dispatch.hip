@@ -60,27 +60,37 @@ hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, std::
     return hipSuccess;
 }
 
-// Whether the copies of a plan are repaid: a launch, each copied operand read and written once, and the product on the fast
-// kernels, against the bounds-checked kernel, whose workgroups of 64 x 64 take 16 columns of K per memory round trip (0.85 us)
-// until more of them than fit wait for each other, longer with more rows and by layout. Constants fitted to 379 products with and
-// without copies (1 .. 512 rows, 64 .. 262144 columns, K 66 .. 8192): over those the rule is 0.4 % off the faster one on average,
-// copying always 7 %. us, without / with copies: 1 x 128257 x 512 NN 49 / 83, 1 x 256001 x 1024 212 / 309, 16 x 128256 x 131 19 / 26,
-// 2 x 300 x 77 4.7 / 7.9; 64 x 50257 x 4096 1071 / 236, 16 x 14337 x 4096 220 / 69, 1 x 1001 x 513 24 / 9.
+// Whether the copies of a plan are repaid: a launch, each copied operand read and written once, and the product on the kernels for
+// aligned rows, against the direct kernel, which reads the operands where they lie. us, copies / direct: 2169 x 2399 x 1727 NT
+// 34.5 / 47.7, 475 x 7131 x 4859 TN 64 / 77, 1999 x 3001 x 2503 NN 43 / 59; 99 x 9001 x 3021 NT 43 / 30, 8 x 6407 x 983 NN 19.2 / 10.5,
+// 1 x 591 x 391 NN 9.9 / 7.9, 62 x 19578 x 5867 NT 168 / 78.
 static bool copies_pay(const GemmPackPlan& plan, int M, int N, int K, int layout) {
-    const float wgs = (float)((M + 63) / 64) * (float)((N + 63) / 64), rows = (float)(M < 64 ? M : 64);
-    const float per_wg = layout == MI355_GEMM_NT ? 1.94e-4f * (1.f + .0144f * rows) : 4.04e-5f * (1.f + (layout == MI355_GEMM_TN ? .0103f : .0559f) * rows);
-    const float without_us = 2.32f + (float)K * fmaxf(.0533f, per_wg * wgs);
     const KernelChoice fast = choose_kernel(M, N, K, layout != MI355_GEMM_TN, layout == MI355_GEMM_NT, true, true, plan.b.ld % 64 == 0);
-    return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < without_us;
+    return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < choose_direct(M, N, K, layout, true).us;
 }
 
-// Below a few K steps the bounds-checked kernel is done before a second launch would start. Where the copies are not repaid the
-// product runs without them whatever memory there is; large ones are not asked for either.
+// What callers are asked for, by sizes and alignment: room for small copies always, for large ones where copying them takes less time than
+// a workgroup per 64 x 64 outputs that gathers its operands 16 columns of K at a time (.0533 us per column of K, more where such
+// workgroups wait for each other). An upper bound: what a call uses is hgemm_copy_bytes.
 size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
     if (K <= 64) return 0;
     const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
     if (!plan.a.pack && !plan.b.pack) return 0;
-    return plan.bytes() <= (size_t(1) << 20) || copies_pay(plan, M, N, K, layout) ? plan.bytes() : 0;
+    if (plan.bytes() <= (size_t(1) << 20)) return plan.bytes();
+    const float wgs = (float)((M + 63) / 64) * (float)((N + 63) / 64), rows = (float)(M < 64 ? M : 64);
+    const float per_wg = layout == MI355_GEMM_NT ? 1.94e-4f * (1.f + .0144f * rows) : 4.04e-5f * (1.f + (layout == MI355_GEMM_TN ? .0103f : .0559f) * rows);
+    const float gather_us = 2.32f + (float)K * fmaxf(.0533f, per_wg * wgs);
+    const KernelChoice fast = choose_kernel(M, N, K, layout != MI355_GEMM_TN, layout == MI355_GEMM_NT, true, true, plan.b.ld % 64 == 0);
+    return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < gather_us ? plan.bytes() : 0;
+}
+
+// At most what hgemm_workspace_bytes asks for.
+size_t hgemm_copy_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
+    if (K <= 64) return 0;
+    const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
+    if (!plan.a.pack && !plan.b.pack) return 0;
+    if (!copies_pay(plan, M, N, K, layout)) return 0;
+    return hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout);
 }
 
 template <typename T>
@@ -97,17 +107,17 @@ static hipError_t gemm_of_type(const void* A, const void* B, void* C, const void
 hipError_t hgemm_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb,
                           long ldc, long ldr, int layout, int dtype, int variant, void* workspace, size_t workspace_bytes,
                           hipStream_t stream) {
-    if (const size_t need = workspace ? hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout) : 0; need > 0 && need <= workspace_bytes) {
+    if ((variant & 15) == kDirect64x64 || (variant & 15) == kDirect128x128)
+        return gemm_direct_dispatch(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, dtype, variant, stream);
+    if (const size_t need = workspace ? hgemm_copy_bytes(A, B, M, N, K, lda, ldb, layout) : 0; need > 0 && need <= workspace_bytes) {
         const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
-        if (copies_pay(plan, M, N, K, layout)) {
-            char* a_copy = static_cast<char*>(workspace);
-            char* b_copy = a_copy + plan.b_offset();
-            if (hipError_t e = gemm_pack_launch(plan, A, B, lda, ldb, a_copy, b_copy, stream); e != hipSuccess) return e;
-            if (plan.a.pack) A = a_copy;
-            if (plan.b.pack) B = b_copy;
-            lda = plan.a.ld;
-            ldb = plan.b.ld;
-        }
+        char* a_copy = static_cast<char*>(workspace);
+        char* b_copy = a_copy + plan.b_offset();
+        if (hipError_t e = gemm_pack_launch(plan, A, B, lda, ldb, a_copy, b_copy, stream); e != hipSuccess) return e;
+        if (plan.a.pack) A = a_copy;
+        if (plan.b.pack) B = b_copy;
+        lda = plan.a.ld;
+        ldb = plan.b.ld;
     }
     if (dtype == MI355_DTYPE_BF16) return gemm_of_type<bf16_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);
     return gemm_of_type<half_t>(A, B, C, R, M, N, K, lda, ldb, ldc, ldr, layout, variant, stream);

@@ -65,7 +65,7 @@ hipError_t gemm_step_gate_up_dispatch(const void* x, const NormPrologue& norm, c
                                       hipStream_t stream);
 
 // The kernel of a product (hgemm_choice.hip); the shapes' numbers are those of mi355_internal_hgemm_variant below.
-enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile128x256, kTile256x128, kTile32x64, kSmallM, kDeepRing };
+enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile128x256, kTile256x128, kTile32x64, kSmallM, kDeepRing, kDirect64x64, kDirect128x128 };
 struct KernelChoice {
     int shape = kTile128x128;
     int splits = 1;           // ranges of K
@@ -115,8 +115,14 @@ struct GemmPackPlan {
 GemmPackPlan gemm_pack_plan(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
 hipError_t gemm_pack_launch(const GemmPackPlan& plan, const void* A, const void* B, long lda, long ldb, void* a_copy, void* b_copy,
                             hipStream_t stream);
-// Bytes of workspace a product can use (0: none, nothing to copy or not worth it).
+// The product of operands of any alignment and stride (hgemm_direct.hip): by shape (variant 0), or a pinned kernel. And the tiles and
+// ranges of K that it takes by shape.
+KernelChoice choose_direct(int M, int N, int K, int layout, bool split_ok);
+hipError_t gemm_direct_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc, long ldr,
+                                int layout, int dtype, int variant, hipStream_t stream);
+// Bytes of workspace a caller is asked for (0: none, nothing to copy or not worth it), and those that the call then uses.
 size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
+size_t hgemm_copy_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
 
 // Element strides of the attention operands: tensor[b][h][s][d] lives at b*batch + h*head + s*row + d (d contiguous).
 struct FmhaStrides {
@@ -175,12 +181,13 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 }  // namespace mi355
 
 // Test and tuning hooks: exported from the shared library but not part of its public header. They take the kernel
-// variant as an argument (no process-wide state). Where a layout lacks a pinned kernel the choice by shape or the bounds-checked
-// kernel takes its place; of more ranges than K has tiles as many are taken as it has.
+// variant as an argument (no process-wide state). Where a layout lacks a pinned kernel, or the operands' rows are not aligned, the
+// choice by shape takes its place; of more ranges than K has tiles as many are taken as it has.
 //   gemm: 0 = by shape; 1 = 256x256 tiles, 2 = 128x128, 3 = 64x128 (layout NT: 128x64), 4 = 64x64 with a ring of four
 //         stages, 5 = 128x256, 6 = 256x128, 7 = 32x64 (layouts NN and NT), 8 = the small-M kernels (up to 64 rows), 9 = 64x64 with
 //         a ring of eight; shapes 1 .. 7 take s ranges of K with variant + 16 s, merged by a kernel of their own (instead of
-//         the last workgroup of a tile) with variant + 16 s + 4096, shape 1 always. The gate/up product: 1, 2, 4, 5, 6, 8, 9
+//         the last workgroup of a tile) with variant + 16 s + 4096, shape 1 always. 10, 11 = the direct kernel for operands of any
+//         alignment on 64x64 and 128x128 tiles, s ranges of K with + 16 s. The gate/up product: 1, 2, 4, 5, 6, 8, 9
 //   fmha: 0 = by shape, 1 = 128-query workgroups, 2 = 256-query workgroups (1 and 2 also keep generation-step shapes off
 //         the split-KV path), 3 = keys of a long cache cut into ranges and merged, 4 = those of a shorter one, partial results in 32 bits
 //         (an error where the choice by shape would not do that)
