@@ -804,6 +804,45 @@ def test_k_that_ends_inside_a_chunk_of_padded_rows(lib, gpu, dtype, layout, vari
     assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["NN", "TN"])
+@pytest.mark.parametrize("M,N,K,ranges,residual", [(16, 128, 512, 2, False), (1, 24, 9, 2, False), (16, 77, 1063, 3, True), (7, 300, 1016, 8, False),
+                                                   (33, 200, 1003, 5, True), (64, 129, 520, 8, False), (16, 4096, 4096, 0, False), (5, 4160, 4100, 0, True)])
+def test_few_rows_in_128_columns_and_ranges_of_k(lib, gpu, dtype, layout, M, N, K, ranges, residual):
+    # more ranges than k-steps, more waves than k-steps of a range, K that ends inside a step or a chunk (NaNs behind it), several row
+    # blocks, C of any alignment; ranges 0: by shape. Called three times: the tickets are back at zero. One rounding of the product, one of the sum.
+    a, b = operands(M, N, K, layout, seed=M + N + K, b_std=0.05)
+    a, b = a.to(dtype), b.to(dtype)
+    pad = lambda t: torch.cat((t, torch.full((t.shape[0], -t.shape[1] % 8), float("nan"), dtype=t.dtype)), 1).to(gpu)
+    ag, bg = pad(a), pad(b)
+    r = (torch.randn(M, N, generator=torch.Generator().manual_seed(7)) * 2).to(dtype)
+    rg = r.to(gpu)
+    ldc = N + 3 if N % 2 else N + 4
+    tail = (lib.LAYOUTS[layout], lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, 8 + 16 * ranges if ranges else 0, torch.cuda.current_stream(gpu).cuda_stream)
+    if not ranges:
+        assert lib.load().mi355_internal_hgemm_choice(M, N, K, bg.shape[1], lib.LAYOUTS[layout], None) == 8
+    ref = so.gemm_ref(a, b, layout)
+    # fp32 sums in two orders: K 2^-23 of the sum of magnitudes at most; one rounding of the product, one of the sum
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    sums = K * 2.0 ** -23 * so.gemm_ref(a.abs(), b.abs(), layout)
+    first = None
+    for _ in range(3):
+        c = torch.full((M + 1, ldc), 4.0, dtype=dtype, device=gpu)
+        if residual:
+            rc = lib.load().mi355_internal_hgemm_add_variant(ag.data_ptr(), bg.data_ptr(), rg.data_ptr(), c.data_ptr(), M, N, K, ag.shape[1], bg.shape[1], N, ldc, *tail)
+        else:
+            rc = lib.load().mi355_internal_hgemm_variant(ag.data_ptr(), bg.data_ptr(), c.data_ptr(), M, N, K, ag.shape[1], bg.shape[1], ldc, *tail)
+        assert rc == 0
+        torch.cuda.synchronize()
+        got = c[:M, :N].cpu().float()
+        err = (got - (r.float() if residual else 0.0) - ref).abs()
+        bound = (1 + eps) * (eps * ref.abs() + sums) + (eps * got.abs() * 1.01 if residual else 0.0) + 2.0 ** -24
+        assert bool((err <= bound).all()), float((err - bound).max())
+        assert bool((c[M:] == 4.0).all()) and bool((c[:, N:] == 4.0).all())
+        assert first is None or torch.equal(first, got)
+        first = got
+
+
 def test_products_of_unaligned_operands_run_when_no_memory_for_copies_is_left(lib, gpu):
     # torch's allocator is limited to a little more than it holds: the outputs fit, aligned copies of the second operand
     # (117 MB, the layer's weight 67 MB) do not. The operator, the ctypes wrapper and the decoder layer run the product without copies.

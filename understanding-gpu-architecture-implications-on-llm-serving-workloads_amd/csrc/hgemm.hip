@@ -825,6 +825,204 @@ __global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_nn_kernel(cons
     }
 }
 
+// The same for a longer K and up to 16384 columns: rows of 256 bytes, which the memory system delivers faster than rows of 128, the
+// waves taking k-steps in turn, so that the workgroup reads 256 consecutive rows at a time, and ranges of K (blockIdx.z, at least two) in the
+// place of more workgroups side by side. HBM-bound; the ranges are merged by the last workgroup of a tile, in their order (`part` and
+// `counters` as in the tiled kernels), which costs ~2 us. us, weights from HBM, what was taken before (this kernel's 64 columns or split
+// tiles) / now: 16 x 14336 x 4096 25.5 / 24.5, 16 x 12288 x 4096 25.4 / 22.3, 16 x 6144 x 4096 15.6 / 14.0, 16 x 4096 x 4096 12.4 / 10.9, 16 x 4096 x 14336
+// 28.7 / 25.1, 16 x 1024 x 4096 8.9 / 8.1; with K = 1024 the merge costs more than it gives: 16 x 8192 x 1024 7.5 / 8.1.
+constexpr int kWideCols = 128;
+constexpr int kWideStages = 2;
+constexpr int kWideStageBytes = 9 * 1024;   // 8 KiB of B + 1 KiB of A
+constexpr int kWideLdsBytes = kSmallMWaves * kWideStages * kWideStageBytes;
+constexpr int kWideRed = kWideCols + 4;     // floats between the rows of a wave's partial tile: its four rows of a store lie on different banks
+constexpr int kWideRanges = 8;              // at most
+static_assert(kWideLdsBytes >= kSmallMWaves * 16 * kWideRed * 4, "the reduction reuses the pipeline memory");
+static_assert(kSmallMWaves * 64 * 4 == 16 * kWideCols, "a thread merges and stores four columns of a row");
+
+template <typename T, bool A_KC>
+__global__ __launch_bounds__(kSmallMWaves * 64) void hgemm_smallm_wide_kernel(const T* __restrict__ A, const T* __restrict__ B, T* C, const T* R, int M,
+                                                                int N, int K, long lda, long ldb, long ldc, long ldr, float* part, unsigned* counters) {
+    using V8 = typename Elem<T>::v8;
+    using V4 = typename Elem<T>::v4;
+    extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
+    MI355_LDS char* smem = (MI355_LDS char*)smem_raw;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = blockIdx.x * kWideCols;
+    const int m0 = blockIdx.y * 16;
+    const int splits = gridDim.z;
+    const int ksteps = K / 32;
+    const int r_begin = (int)((long)blockIdx.z * ksteps / splits);
+    const int r_end = (int)((long)(blockIdx.z + 1) * ksteps / splits);
+    const int first = r_begin + wave, steps = (r_end - first + kSmallMWaves - 1) / kSmallMWaves;   // (no step left: 0, or a quotient rounded up to 0)
+    MI355_LDS char* wbase = smem + wave * (kWideStages * kWideStageBytes);
+
+    // B slab: 32 rows (k) x 256 bytes; copy i covers rows 4i .. 4i+3, chunk c of row r at c ^ 2 * (r % 4 + 4 * (r / 8 % 2)): the eight rows
+    // and chunk pairs that lanes 0..31 of a transposing read touch lie on distinct banks. A slab as in the kernel above.
+    const int b_row = lane >> 4;
+    const int n_chunk_max = (N + 7) / 8 - 1;
+    const int b_col[2] = {min(n0 / 8 + ((lane & 15) ^ (2 * b_row)), n_chunk_max) * 8, min(n0 / 8 + ((lane & 15) ^ (2 * b_row) ^ 8), n_chunk_max) * 8};
+    const int a_row = lane >> 2;
+    const int a_chunk = (lane & 3) ^ ((a_row >> 1) & 3);
+    const int at_slot = lane >> 1;
+    const int at_k = (at_slot & ~12) | ((at_slot & 4) << 1) | ((at_slot & 8) >> 1);
+    const auto b_at = [&](int step, int i) { return B + ((long)step * 32 + 4 * i + b_row) * ldb + b_col[(i >> 1) & 1]; };
+    const auto a_at = [&](int step) {
+        return A_KC ? A + (long)min(m0 + a_row, M - 1) * lda + (long)step * 32 + a_chunk * 8
+                    : A + ((long)step * 32 + at_k) * lda + min(m0 + 8 * (lane & 1), ((M + 7) & ~7) - 8);
+    };
+    const auto issue = [&](int i, int slot) {
+        const int step = first + i * kSmallMWaves;
+        MI355_LDS char* st = wbase + slot * kWideStageBytes;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) copy16_global_to_lds(b_at(step, c), st + c * 1024);
+        copy16_global_to_lds(a_at(step), st + 8192);
+    };
+
+    const int at_read_k = 8 * (lane >> 4) + ((lane & 15) >> 2);
+    const int at_read_slot = (at_read_k & ~12) | ((at_read_k & 4) << 1) | ((at_read_k & 8) >> 1);
+    const int a_off = A_KC ? 8192 + (lane & 15) * 64 + (((lane >> 4) ^ (((lane & 15) >> 1) & 3)) << 4)
+                           : 8192 + at_read_slot * 32 + (lane & 3) * 8;
+    const int bt_row = at_read_k;
+    const int bt_swz = 2 * ((bt_row & 3) | (((bt_row >> 3) & 1) << 2));
+    float4v acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = float4v{0.f, 0.f, 0.f, 0.f};
+    const auto k_step = [&](MI355_LDS const char* st) {
+        V8 af;
+        if constexpr (A_KC) af = Elem<T>::frag(lds_read_b128(st + a_off));
+        else af = Elem<T>::frag(concat(lds_read_tr16_b64(st + a_off), lds_read_tr16_b64(st + a_off + 256)));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            MI355_LDS const char* const p = st + bt_row * 256 + (((2 * j + ((lane & 3) >> 1)) ^ bt_swz) << 4) + (lane & 1) * 8;
+            const half4 lo = lds_read_tr16_b64(p), hi = lds_read_tr16_b64(p + 4 * 256);
+            acc[j] = Elem<T>::mfma16(af, Elem<T>::frag(concat(lo, hi)), acc[j]);
+        }
+    };
+
+    // the last K % 32 rows of B (columns of A) go through registers of one wave, zeros behind K: requested in front of its steps, as waiting
+    // for them behind the steps costs 2.5 us (2 x 4736 x 3480 13.2)
+    const int k0 = ksteps * 32;
+    const bool tail = k0 < K && wave == kSmallMWaves - 1 && blockIdx.z == splits - 1;
+    half8 tail_b[8] = {}, tail_a = {};
+    if (tail) {   // rows behind K: the last one again
+#pragma unroll
+        for (int c = 0; c < 8; ++c) tail_b[c] = *(const half8*)(B + (long)min(k0 + 4 * c + b_row, K - 1) * ldb + b_col[(c >> 1) & 1]);
+        tail_a = *(const half8*)(A_KC ? A + (long)min(m0 + a_row, M - 1) * lda + min(k0 + 8 * a_chunk, (K - 1) & ~7)
+                                      : A + (long)min(k0 + at_k, K - 1) * lda + min(m0 + 8 * (lane & 1), ((M + 7) & ~7) - 8));
+    }
+
+    static_assert(kWideStages == 2, "one step is in flight while one is worked on");
+    if (steps > 0) issue(0, 0);
+    for (int i = 0; i < steps; ++i) {
+        if (i + 1 < steps) {
+            issue(i + 1, (i + 1) & 1);
+            wait_vmcnt<9>();
+        } else {
+            wait_vmcnt<0>();
+        }
+        k_step(wbase + (i & 1) * kWideStageBytes);
+        wait_lgkmcnt<0>();   // the reads of this slot are complete before a later copy refills it
+    }
+    if (tail) {   // (its steps' copies have all landed)
+        const half8 zero = {};
+        const int a_left = K - k0 - (A_KC ? 8 * a_chunk : at_k);
+        if (A_KC) tail_a = first_of_chunk(tail_a, a_left);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) *(MI355_LDS half8*)(wbase + c * 1024 + lane * 16) = k0 + 4 * c + b_row < K ? tail_b[c] : zero;
+        *(MI355_LDS half8*)(wbase + 8192 + lane * 16) = a_left > 0 ? tail_a : zero;
+        wait_lgkmcnt<0>();
+        k_step(wbase);
+    }
+
+    // the 8 partial tiles through LDS: acc[j][q] is D[m = 4*(lane/16) + q][n = 16j + lane%16]; a thread adds four columns of row tid / 32
+    __syncthreads();   // every wave is done with its staging memory
+    MI355_LDS float* red = (MI355_LDS float*)smem;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[(wave * 16 + 4 * (lane >> 4) + q) * kWideRed + 16 * j + (lane & 15)] = acc[j][q];
+    __syncthreads();
+    float4v sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kSmallMWaves; ++w) sum += *(MI355_LDS const float4v*)(red + (w * 16 + tid / 32) * kWideRed + tid % 32 * 4);
+    {
+        // partial tile (tile, range): pair p of thread t at pair p * 512 + t; stores, ticket and loads as in hgemm_main_kernel
+        constexpr int kPairs = 16 * kWideCols / 2, kThreads = kSmallMWaves * 64;
+        const int tile = blockIdx.y * gridDim.x + blockIdx.x;
+        uint64_t* const tile_part = reinterpret_cast<uint64_t*>(part) + (long)tile * splits * kPairs + tid;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const uint64_t v = (uint64_t)__builtin_bit_cast(uint32_t, (float)sum[2 * p]) | (uint64_t)__builtin_bit_cast(uint32_t, (float)sum[2 * p + 1]) << 32;
+            __hip_atomic_store(tile_part + (long)blockIdx.z * kPairs + p * kThreads, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's part has reached memory before the ticket is drawn
+        __syncthreads();
+        MI355_LDS unsigned* ticket_sh = (MI355_LDS unsigned*)smem;
+        if (tid == 0) *ticket_sh = __hip_atomic_fetch_add(&counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*ticket_sh != (unsigned)(splits - 1)) return;
+        uint64_t v[kWideRanges][2];   // all ranges in flight together
+#pragma unroll
+        for (int r = 0; r < kWideRanges; ++r)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                v[r][p] = __hip_atomic_load(tile_part + (long)min(r, splits - 1) * kPairs + p * kThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_sched_barrier(0);
+        sum = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < kWideRanges; ++r)
+            if (r < splits)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sum[q] += __builtin_bit_cast(float, (uint32_t)(v[r][q / 2] >> (32 * (q & 1))));
+        if (tid == 0) __hip_atomic_store(&counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int m = m0 + tid / 32, n = n0 + tid % 32 * 4;
+    if (m >= M || n >= N) return;
+    T* const c = C + (long)m * ldc + n;
+    const T* const r = R + (long)m * ldr + n;
+    // four columns go out in one 8-byte store where the rows of C (and of the residual) allow it
+    if (n + 4 <= N && ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(R)) & 7) == 0 && ((ldc | ldr) & 3) == 0) {
+        V4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = (T)sum[q];
+        if (R != nullptr) {
+            const V4 x = *(const V4*)r;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = (T)((float)v[q] + (float)x[q]);
+        }
+        *(V4*)c = v;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (n + q < N) {
+                T v = (T)sum[q];
+                if (R != nullptr) v = (T)((float)v + (float)r[q]);
+                c[q] = v;
+            }
+    }
+}
+
+// hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: no workspace to be had, the caller takes another kernel.
+template <typename T, bool A_KC>
+static hipError_t launch_smallm_wide(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb, long ldc, long ldr, int ranges,
+                                     hipStream_t stream) {
+    static DynamicLdsOnce lds_once;
+    if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(hgemm_smallm_wide_kernel<T, A_KC>), kWideLdsBytes); e != hipSuccess) return e;
+    ranges = std::min(ranges, kWideRanges);
+    const unsigned tiles_n = (N + kWideCols - 1) / kWideCols, tiles_m = (M + 15) / 16;
+    const size_t tiles = (size_t)tiles_n * tiles_m;
+    if (tiles * sizeof(unsigned) > kSplitKCounterBytes) return hipErrorOutOfMemory;
+    char* ws = nullptr;
+    std::unique_lock<std::mutex> order;
+    if (hipError_t e = split_k_workspace(kSplitKCounterBytes + tiles * ranges * (16 * kWideCols * 4), stream, &ws, &order); e != hipSuccess) return e;
+    hgemm_smallm_wide_kernel<T, A_KC><<<dim3(tiles_n, tiles_m, ranges), dim3(kSmallMWaves * 64), kWideLdsBytes, stream>>>(
+        A, B, C, R, M, N, K, lda, ldb, ldc, ldr, reinterpret_cast<float*>(ws + kSplitKCounterBytes), reinterpret_cast<unsigned*>(ws));
+    return hipGetLastError();
+}
+
 template <typename T, bool A_KC>
 static hipError_t launch_smallm_nn(const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
                                    long ldc, long ldr, hipStream_t stream) {
@@ -1355,6 +1553,7 @@ static KernelChoice pinned_kernel(int variant, int K) {
     k.splits = std::min((variant >> 4) & 0xff, (K + 63) / 64);   // a range is at least one K tile: an empty one would copy a whole tile from behind K
     if (k.splits < 1) k.splits = 1;
     k.own_merge = (variant >> 12) != 0;
+    if (k.shape == kSmallM && k.splits > 1) std::swap(k.splits, k.wide_ranges);
     return k;
 }
 // hipErrorNotSupported: no such kernel for this layout
@@ -1362,6 +1561,8 @@ template <typename T, bool A_KC, bool B_KC>
 static hipError_t run_kernel(const KernelChoice& k, const T* A, const T* B, T* C, const T* R, int M, int N, int K, long lda, long ldb,
                              long ldc, long ldr, bool c_aligned, hipStream_t stream) {
 #define MI355_ARGS A, B, C, R, M, N, K, lda, ldb, ldc, ldr
+    if constexpr (!B_KC)
+        if (k.shape == kSmallM && k.wide_ranges > 1) return launch_smallm_wide<T, A_KC>(MI355_ARGS, k.wide_ranges, stream);
     if (k.splits > 1) {
         switch (k.shape) {
             case kTile128x128: return launch_split_k<T, A_KC, B_KC, 128, 128, 2, 2>(MI355_ARGS, k.splits, k.own_merge, stream);
@@ -1437,7 +1638,7 @@ static hipError_t launch_layout(const T* A, const T* B, T* C, const T* R, int M,
         for (;;) {
             const hipError_t e = run_kernel<T, A_KC, B_KC>(pick, A, B, C, R, M, N, K, lda, ldb, ldc, ldr, c_aligned, stream);
             // no workspace to be had (the stream is being captured and has none yet): the best kernel without split-K
-            if (pick.splits <= 1 || variant > 0 || (e != hipErrorStreamCaptureUnsupported && e != hipErrorOutOfMemory)) {
+            if ((pick.splits <= 1 && pick.wide_ranges <= 1) || variant > 0 || (e != hipErrorStreamCaptureUnsupported && e != hipErrorOutOfMemory)) {
                 if (e != hipErrorNotSupported) return e;
                 break;
             }

@@ -20,8 +20,10 @@
 //     decides between the small-M kernels and the 64x64 tiles for a few rows against a vocabulary: 8 x 50304 x 4096 NT
 //     68.7 us on the former, 80.2 on the latter; 8 x 28672 x 8192 80 / 90; 16 x 28672 x 4096, activation rows in registers,
 //     39.7 / 45.5. In layouts NN and TN the small-M kernel takes rounds of 256 workgroups of 64 columns, and the lines of rows
-//     that are no whole ones twice: 16 x 14336 x 4096 NN 23.0 us (64x64 tiles 24.1), 16 x 28672 x 4096 52 (64x128 tiles
-//     44), 16 x 50264 x 4096 123 (79).
+//     that are no whole ones twice: 16 x 28672 x 4096 NN 52 us (64x128 tiles 44), 16 x 50264 x 4096 123 (79); or, up to 16 rows and 16384
+//     columns, one round of 128 columns and ranges of K: 16 x 14336 x 4096 24.5 (25.7 without, 64x64 tiles 26), 16 x 4096 x 14336 25.1 (68, split
+//     tiles 28.7).
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include "mi355_common.h"
@@ -64,6 +66,7 @@ static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, b
         best.shape = shape;
         best.splits = splits;
         best.own_merge = own_merge;
+        best.wide_ranges = 0;
         best.us = us;
     };
     if (M <= 64 && !gate_up) {   // the small-M kernels: workgroups of 16 rows and 64 (layout NT: 16) columns, the whole of K
@@ -77,6 +80,16 @@ static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, b
         } else {
             const float stream = b_bytes * (1.f + (float)(row_blocks - 1) * .1f) * (from_hbm && !whole_lines ? 2.04f : 1.f) / 5.7e6f;
             consider(fmaxf(1.67f + ceilf(wgs / 256.f) * (k * (from_hbm ? 1.38f : 1.f) * .169f + .565f), stream + 2.56f), kSmallM, 1, false);
+            // 128 columns and as many ranges of K as CUs are left: 1.4 us for a step of 256 rows, 6.1 TB/s, 1.3 times the bytes where rows are no
+            // whole lines, 5.4 us beside them (within 0.6 us of 12 products timed, 8.1 .. 28.2 us); times .92 (TN: .88), as the other kernels' times
+            // here come out against those of the same measurement
+            if (const int n_wide = (N + 127) / 128, ranges = std::min(8, std::min(256 / n_wide, K / 256)); M <= 16 && split_ok && ranges > 1) {
+                const float steps = ceilf((float)K / (256.f * (float)ranges)), wide_us = (a_kc ? .92f : .88f) * (5.4f + fmaxf(1.4f * steps, b_bytes * (whole_lines ? 1.f : 1.3f) / 6.1e6f));
+                if (wide_us < best_us) {
+                    consider(wide_us, kSmallM, 1, false);
+                    best.wide_ranges = ranges;
+                }
+            }
         }
     }
     if (!tiles_ok) return best;

@@ -69,6 +69,7 @@ enum KernelShape { kTile256x256 = 1, kTile128x128, kTileHalf, kTile64x64, kTile1
 struct KernelChoice {
     int shape = kTile128x128;
     int splits = 1;           // ranges of K
+    int wide_ranges = 0;      // kSmallM, layouts NN and TN: ranges of K of hgemm_smallm_wide_kernel, 0 = the kernel of 64 columns
     bool own_merge = false;   // their partial tiles are merged by a kernel of their own
     float us = 0.f;           // expected time
 };
@@ -186,7 +187,8 @@ hipError_t silu_mul_dispatch(const void* in, void* out, long rows, int inter, in
 //   gemm: 0 = by shape; 1 = 256x256 tiles, 2 = 128x128, 3 = 64x128 (layout NT: 128x64), 4 = 64x64 with a ring of four
 //         stages, 5 = 128x256, 6 = 256x128, 7 = 32x64 (layouts NN and NT), 8 = the small-M kernels (up to 64 rows), 9 = 64x64 with
 //         a ring of eight; shapes 1 .. 7 take s ranges of K with variant + 16 s, merged by a kernel of their own (instead of
-//         the last workgroup of a tile) with variant + 16 s + 4096, shape 1 always. 10, 11 = the direct kernel for operands of any
+//         the last workgroup of a tile) with variant + 16 s + 4096, shape 1 always; 8 + 16 s (layouts NN and TN, s > 1) = 128 columns and
+//         s ranges of K, merged by the last workgroup of a tile. 10, 11 = the direct kernel for operands of any
 //         alignment on 64x64 and 128x128 tiles, s ranges of K with + 16 s. The gate/up product: 1, 2, 4, 5, 6, 8, 9
 //   fmha: 0 = by shape, 1 = 128-query workgroups, 2 = 256-query workgroups (1 and 2 also keep generation-step shapes off
 //         the split-KV path), 3 = keys of a long cache cut into ranges and merged, 4 = those of a shorter one, partial results in 32 bits
