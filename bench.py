@@ -32,11 +32,11 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # HBM bytes per launch from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (KiB per dispatch), each scaled by what the same
 # counter reads for a 1 GiB device-to-device copy (FETCH_SIZE x2.0, WRITE_SIZE x1.0); see profiles/.
 MEASURED_TRAFFIC_BYTES = (790997 * 2.0 + 131072 * 1.0) * 1024        # hgemm_main_kernel, 8192^3 NN
-MEASURED_TRAFFIC_BYTES_G2C = (57882 * 2.0 + 448 * 1.0) * 1024          # hgemm_smallm_nn_kernel, 16 x 14336 x 4096
+MEASURED_TRAFFIC_BYTES_G2C = (58812 * 2.0 + 2251 * 1.0) * 1024         # hgemm_smallm_wide_kernel, 16 x 14336 x 4096
 MEASURED_TRAFFIC_BYTES_FMHA = (26670 * 2.0 + 33280 * 1.0) * 1024     # fmha_fwd_pingpong_kernel, F4
 # the figures above are constants copied from these counter summaries (they are not read at run time)
 TRAFFIC_SOURCE = {"gemm": "constant from profiles/hgemm_main_kernel_256x256_8192_nn.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)",
-                  "g2c": "constant from profiles/hgemm_smallm_nn_kernel_g2c_16x14336x4096_nn.md",
+                  "g2c": "constant from profiles/hgemm_smallm_wide_kernel_g2c_16x14336x4096_nn.md",
                   "fmha": "constant from profiles/fmha_fwd_pingpong_kernel_f4_causal_gqa.md"}
 
 
@@ -319,7 +319,7 @@ def main():
         g2c = other["G2c_gemm_decode_16x14336x4096"]
         # achieved = the rate with a weight that is in no cache (a different copy per launch); launches that reuse one
         # 117 MB weight find part of it in the 256 MB memory-side cache and read faster than the HBM figure they are held against
-        roofline_g2c = {"kernel": "hgemm_smallm_nn_kernel (G2c: 16 x 14336 x 4096, NN)", "bound": "hbm",
+        roofline_g2c = {"kernel": "hgemm_smallm_wide_kernel (G2c: 16 x 14336 x 4096, NN)", "bound": "hbm",
                         "achieved": g2c["gbs_weights_not_cached"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
                         "frac": g2c["gbs_weights_not_cached"] / PEAK_HBM_GBS, "achieved_same_weight_every_launch": g2c["gbs"],
                         "traffic": MEASURED_TRAFFIC_BYTES_G2C, "traffic_source": TRAFFIC_SOURCE["g2c"]}
