@@ -752,6 +752,21 @@ def test_items_of_a_long_list_equal_the_same_items_on_their_own(lib, gpu, dtype,
     assert (lse[-1:].cpu() - lse_ref)[seen].abs().max() <= tol[1] and torch.equal(torch.isfinite(lse[-1:].cpu()), seen)
 
 
+@pytest.mark.parametrize("variant", [1, 2])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq", [(1, 7, 7, 300), (3, 15, 5, 520), (2, 9, 3, 130), (13, 6, 2, 700), (5, 24, 8, 33), (1, 1, 1, 1), (31, 21, 3, 260)])
+def test_every_item_of_odd_counts_of_heads_and_batches(lib, gpu, variant, B, Hq, Hkv, Sq):
+    """Items are found by products with reciprocals of the head, group and rank counts: each (batch, head, q tile) is done once. The bits of a head
+    alone, and the oracle for the last one."""
+    q, k, v = (x.to(gpu) for x in so.fmha_inputs(B, Hq, Hkv, Sq, Sq, seed=Sq + B))
+    o, lse = lib.fmha_fwd(q, k, v, causal=True, variant=variant)
+    for b, h in [(b, (5 * b + 3) % Hq) for b in range(B)] + [(0, h) for h in range(Hq)]:
+        kv = h // (Hq // Hkv)
+        o1, lse1 = lib.fmha_fwd(q[b:b + 1, h:h + 1].contiguous(), k[b:b + 1, kv:kv + 1].contiguous(), v[b:b + 1, kv:kv + 1].contiguous(), causal=True, variant=variant)
+        assert torch.equal(o[b, h], o1[0, 0]) and torch.equal(lse[b, h], lse1[0, 0]), (b, h)
+    o_ref, lse_ref = so.attention_ref(q[-1:].cpu().float(), k[-1:].cpu().float(), v[-1:].cpu().float(), causal=True)
+    assert (o[-1:].cpu().float() - o_ref.float()).abs().max() <= 2e-3 and (lse[-1:].cpu() - lse_ref).abs().max() <= 1e-3
+
+
 def test_more_items_than_a_workgroup_lists_at_once(lib, gpu):
     """Items are listed 64 at a time per workgroup: 70 x 256 heads are 70 for each of 256."""
     B, H, Sq, Sk = 70, 256, 16, 70

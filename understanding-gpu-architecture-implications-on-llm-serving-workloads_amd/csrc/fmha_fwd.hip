@@ -73,32 +73,59 @@ __device__ __forceinline__ float max3v(float a, float b, float c) {
 
 }  // namespace fmha
 
-// Work item `round` of workgroup `wg` out of `n_wg`: a (batch, q head, q tile), or false when the workgroup has none left.
+// n / d for 0 <= n < 2^31, as a product: with 2^(s-1) < d <= 2^s, mul = ceil(2^(31+s) / d) is at most (d - 1) / d above the quotient, so
+// n * mul is less than 2^(31+s) above n * 2^(31+s) / d. On the device three scalar instructions, where a division is ~35, most of
+// them vector ones: those that a workgroup needs to find its first item took ~0.5 us in front of its first load (us, divisions / products: 1 x
+// 8/2 heads, 45 queries 6.4 / 5.8, 1 x 32/8, 128 8.1 / 7.6, 8 x 32/8, 128 10.4 / 9.9, 1 x 8/2, 300 over 600 keys 13.3 / 12.8).
+struct Divisor {
+    uint32_t mul;
+    int shift;   // 31 + s
+};
+static Divisor divisor_of(long d) {
+    int s = 0;
+    while ((1L << s) < d) ++s;
+    return {(uint32_t)(((1ULL << (31 + s)) + (uint64_t)d - 1) / (uint64_t)d), 31 + s};
+}
+__device__ __forceinline__ int divide(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.mul) >> d.shift); }
+
+// How the items of a launch are dealt out (see fmha_work_item)
+struct ItemMap {
+    int group, Hkv, per_rank, groups_per_xcd, xcd_shift, wgs;   // wgs: workgroups per XCD; xcd_shift 0: the launch is not cut by XCD
+    Divisor by_group, by_hkv, by_rank, by_segments;
+};
+static ItemMap item_map(int B, int Hq, int Hkv, int segments, long blocks) {
+    ItemMap m;
+    const long kv_groups = (long)Hkv * B * segments;
+    m.group = Hq / Hkv;
+    m.Hkv = Hkv;
+    m.xcd_shift = kv_groups % 8 == 0 && blocks % 8 == 0 ? 3 : 0;
+    m.wgs = (int)(blocks >> m.xcd_shift);
+    m.groups_per_xcd = (int)(kv_groups >> m.xcd_shift);
+    m.per_rank = m.groups_per_xcd * m.group;
+    m.by_group = divisor_of(m.group);
+    m.by_hkv = divisor_of(Hkv);
+    m.by_rank = divisor_of(m.per_rank);
+    m.by_segments = divisor_of(segments);
+    return m;
+}
+
+// Work item `round` of workgroup `wg`: a (batch, q head, q tile), or false when the workgroup has none left.
 // A launch has at most one workgroup per CU; each walks its own list of items (no global counter: nothing to reset, nothing
 // two launches could share). Workgroups with ids congruent mod 8 share an XCD (and its L2): when the (batch, kv head)
 // groups divide evenly every XCD gets whole groups, so K and V are fetched from HBM once. On an XCD the items are ranked
 // with the q tiles that see the most keys (causal) first and dealt out in rounds that run forwards and backwards in turn:
 // the workgroup that got the heaviest item of one round gets the lightest of the next.
-__device__ __forceinline__ bool fmha_work_item(int wg, int n_wg, int round, int q_tiles, int group, int Hkv, int B, int& b,
-                                               int& hkv, int& hq, int& q_tile) {
-    const int kv_groups = Hkv * B;
-    int x = 0, n_x = 1;
-    if (kv_groups % 8 == 0 && n_wg % 8 == 0) {
-        x = wg % 8;
-        n_x = 8;
-    }
-    const int wl = wg / n_x, wgs = n_wg / n_x;   // workgroup index on its XCD, workgroups per XCD
-    const int gpx = kv_groups / n_x;             // (batch, kv head) groups per XCD
-    const int per_rank = gpx * group;            // items of one q tile on this XCD
-    const int u = round * wgs + ((round & 1) ? wgs - 1 - wl : wl);
-    if (u >= per_rank * q_tiles) return false;
-    const int rank = u / per_rank, rem = u - rank * per_rank;
-    const int gl = rem / group, hin = rem - gl * group;
+__device__ __forceinline__ bool fmha_work_item(int wg, int round, int q_tiles, const ItemMap& m, int& b, int& hkv, int& hq, int& q_tile) {
+    const int x = wg & ((1 << m.xcd_shift) - 1), wl = wg >> m.xcd_shift;   // XCD, workgroup index on it
+    const int u = round * m.wgs + ((round & 1) ? m.wgs - 1 - wl : wl);
+    if (u >= m.per_rank * q_tiles) return false;
+    const int rank = divide(u, m.by_rank), rem = u - rank * m.per_rank;   // per_rank: items of one q tile on this XCD
+    const int gl = divide(rem, m.by_group), hin = rem - gl * m.group;
     q_tile = q_tiles - 1 - rank;
-    const int kvg = x * gpx + gl;
-    b = kvg / Hkv;
-    hkv = kvg - b * Hkv;
-    hq = hkv * group + hin;
+    const int kvg = x * m.groups_per_xcd + gl;
+    b = divide(kvg, m.by_hkv);
+    hkv = kvg - b * m.Hkv;
+    hq = hkv * m.group + hin;
     return true;
 }
 
@@ -168,7 +195,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
                                                                const T* __restrict__ V, T* __restrict__ O,
                                                                float* __restrict__ LSE, int B, int Hq, int Hkv, int Sq,
                                                                int Sk, float scale_log2, int causal, int kv_valid,
-                                                               int q_tiles, FmhaStrides sd, int segments, int seg_len) {
+                                                               int q_tiles, FmhaStrides sd, int segments, int seg_len, ItemMap map) {
     using namespace fmha;
     using V8 = typename Elem<T>::v8;
     using V4 = typename Elem<T>::v4;
@@ -191,7 +218,6 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     const int c16 = lane & 15;
 
     // ---- work items -------------------------------------------------------------------------------------------------
-    const int group = Hq / Hkv;
     struct Item {
         const T *Qh, *Kh, *Vh;
         T* Oh;
@@ -203,20 +229,22 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     };
     const long o_row = SEG ? (long)D : sd.o_row;
     auto item_of = [&](int round) -> Item {
-        // (opaque copies: the compiler would work out reciprocals and products of these once and keep them in vector registers through the
-        // loop over the keys, which has none to spare)
-        int q_tiles_ = q_tiles, group_ = group, Hkv_ = Hkv, batches = SEG ? B * segments : B;
-        asm volatile("" : "+s"(q_tiles_), "+s"(group_), "+s"(Hkv_), "+s"(batches));
+        // (opaque copies: the compiler would form products of these once and keep them in registers through the loop over the keys, which
+        // has none to spare)
+        int q_tiles_ = q_tiles;
+        ItemMap map_ = map;
+        asm volatile("" : "+s"(q_tiles_), "+s"(map_.per_rank), "+s"(map_.group), "+s"(map_.Hkv));
         Item it;
         int b, hkv, hq, q_tile;
         it.n_tiles = 0;
-        it.exists = fmha_work_item(blockIdx.x, gridDim.x, round, q_tiles_, group_, Hkv_, batches, b, hkv, hq, q_tile);
+        it.exists = fmha_work_item(blockIdx.x, round, q_tiles_, map_, b, hkv, hq, q_tile);
         if (!it.exists) return it;
         it.q_block0 = q_tile * BM;
         long k0 = 0;
         if constexpr (SEG != kOneWalk) {   // b counts (batch, range) pairs
-            const int seg = b % segments;
-            b /= segments;
+            const int pair = b;
+            b = divide(pair, map_.by_segments);
+            const int seg = pair - b * segments;
             k0 = (long)seg * seg_len;
             it.lse_row = (seg * B + b) * Hq + hq;
             it.Oh = O + (long)it.lse_row * Sq * (SEG == kRangesF32 ? D * (int)(sizeof(float) / sizeof(T)) : D);
@@ -771,7 +799,7 @@ static hipError_t launch_fmha_pingpong(const T* Q, const T* K, const T* V, T* O,
     if (((long)Hkv * B) % 8 == 0 && blocks >= 8) blocks &= ~7L;
     const float scale_log2 = scale * 1.4426950408889634f;
     kern<<<dim3((unsigned)blocks), dim3(512), LDS, stream>>>(Q, K, V, O, LSE, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid,
-                                                             q_tiles, sd, 1, 0);
+                                                             q_tiles, sd, 1, 0, item_map(B, Hq, Hkv, 1, blocks));
     return hipGetLastError();
 }
 
@@ -982,7 +1010,7 @@ static hipError_t launch_fmha_segmented(const T* Q, const T* K, const T* V, T* O
     if (((long)Hkv * B * segments) % 8 == 0 && blocks >= 8) blocks &= ~7L;
     const float scale_log2 = scale * 1.4426950408889634f;
     kern<<<dim3((unsigned)blocks), dim3(512), LDS, stream>>>(Q, K, V, reinterpret_cast<T*>(o_part), lse_part, B, Hq, Hkv, Sq, Sk, scale_log2, causal, kv_valid,
-                                                             q_tiles, sd, segments, seg_len);
+                                                             q_tiles, sd, segments, seg_len, item_map(B, Hq, Hkv, segments, blocks));
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     auto merge = fmha_merge_segments_kernel<T, P, SEG == kRangesF32 ? kMaxSegmentsF32 : kMaxSegments>;
     merge<<<dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream>>>(o_part, lse_part, O, LSE, B, Hq, Sq, segments, sd);
