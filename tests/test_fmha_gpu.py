@@ -778,6 +778,28 @@ def test_more_items_than_a_workgroup_lists_at_once(lib, gpu):
         assert torch.equal(o[b], o1[0]) and torch.equal(lse[b], lse1[0]), b
 
 
+@pytest.mark.parametrize("variant,B,Sq,Sk,causal", [
+    (1, 70, 16, 70, True),       # 70 items for each of 256 workgroups, waves without rows
+    (1, 140, 100, 200, False),   # 140: the list is written three times; four key tiles an item
+    (1, 24, 300, 20, True),      # 72, the 24 that see keys in front: items without a visible key where the list is written again
+    (1, 17, 520, 300, True),     # 85, those without a visible key at the end, items of different length around the 64th
+    (2, 70, 200, 70, False),     # 256-query items: 70
+    (2, 36, 300, 20, True),      # 72, the second half without a visible key
+])
+def test_every_item_of_lists_that_are_written_several_times(lib, gpu, variant, B, Sq, Sk, causal):
+    """All rows of calls with more than 64 items per workgroup, against calls of a few batch rows, whose lists are written once: the same bits."""
+    H, rows = 256, 64 // ((Sq + 128 * variant - 1) // (128 * variant)) // 2
+    g = torch.Generator(device=gpu).manual_seed(Sq + Sk)
+    q, k, v = (torch.randn(B, h, s, 128, generator=g, device=gpu, dtype=torch.float16) for h, s in ((H, Sq), (8, Sk), (8, Sk)))
+    o, lse = lib.fmha_fwd(q, k, v, causal=causal, variant=variant)
+    for b in range(0, B, rows):
+        part = slice(b, b + rows)
+        o1, lse1 = lib.fmha_fwd(q[part], k[part], v[part], causal=causal, variant=variant)
+        assert torch.equal(o[part], o1) and torch.equal(lse[part], lse1), b
+    if Sq > Sk and causal:
+        assert bool((o[:, :, :Sq - Sk] == 0).all()) and bool(torch.isinf(lse[:, :, :Sq - Sk]).all())
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,S,causal", [
     (4, 64, 8, 152, False), (5, 16, 4, 405, False), (1, 8, 2, 1331, False),      # 256-query items, also fewer of them than CUs
     (6, 64, 8, 270, True), (3, 64, 8, 638, True),                               # 128-query items, also more 256-query items than CUs

@@ -22,6 +22,7 @@
 #include <mutex>
 #include <type_traits>
 #include <utility>
+#include "fmha_items.h"
 #include "mi355_common.h"
 #include "mi355_serving_internal.h"
 #include "mi355_timeline.h"
@@ -249,9 +250,9 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         return it;
     };
     // The items to come are worked out 64 at a time, one per lane of the last wave, while the workgroup waits for its first loads, and
-    // kept in LDS: the scalar registers have no room for two items, and the divisions would take a wave ~1900 cycles at every change.
-    constexpr int kListed = 64;
-    __shared__ Item listed[kListed];
+    // kept in LDS (fmha_items.h: in two halves in turn): the scalar registers have no room for two items.
+    __shared__ Item listed_[ListedItems::kHeld];
+    const auto listed = [&](int round) -> Item& { return listed_[ListedItems::entry(round)]; };
     const auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
     const auto uniform_ptr = [](auto* p) {
         const uint64_t u = reinterpret_cast<uint64_t>(p);
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         return reinterpret_cast<decltype(p)>((uint64_t)hi << 32 | lo);
     };
     auto item_listed = [&](int round) -> Item {
-        const Item& l = listed[(round - 1) % kListed];
+        const Item& l = listed(round);
         Item it;
         it.Qh = uniform_ptr(l.Qh); it.Kh = uniform_ptr(l.Kh); it.Vh = uniform_ptr(l.Vh); it.Oh = uniform_ptr(l.Oh);
         it.lse_row = uniform(l.lse_row); it.q_block0 = uniform(l.q_block0); it.kv_valid = uniform(l.kv_valid);
@@ -598,7 +599,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         ++round;
         bool more = false;   // this workgroup has another item
         int n_next = 0;      // its key tiles, if its first pairs are copied while the current item is worked on
-        if (more_items && (round - 1) % kListed == 0 && wave == NWAVES - 1) listed[lane] = item_of(round + lane);
+        if (more_items && ListedItems::refill(round) && wave == NWAVES - 1) listed(round + lane) = item_of(round + lane);
         if (cur.n_tiles > 0) {
             const int n_tiles = cur.n_tiles;
             if (!landed) wait_vmcnt<0>();
@@ -645,7 +646,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
             }
             for (; j + 1 < n_tiles; ++j) {
                 if (more_items && j + 3 >= n_tiles) {   // the copies go on to the next item: K with pair n_tiles, V with the one behind
-                    const Item& next = listed[(round - 1) % kListed];
+                    const Item& next = listed(round);
                     const int n = uniform(next.n_tiles), valid = uniform(next.kv_valid);
                     if (n > 0 && (((ring + n_tiles) & (NBUF - 1)) == 0 || fast_steps(n, valid) < NBUF)) {
                         n_next = n;
@@ -655,8 +656,8 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
                 }
                 step(Dyn{}, j);
             }
-            if (more_items) more = uniform(listed[(round - 1) % kListed].exists);
-            if (more) load_q(uniform_ptr(listed[(round - 1) % kListed].Qh), uniform(listed[(round - 1) % kListed].q_block0) + wave * WQ);
+            if (more_items) more = uniform(listed(round).exists);
+            if (more) load_q(uniform_ptr(listed(round).Qh), uniform(listed(round).q_block0) + wave * WQ);
             softmax_tile(s, n_tiles - 1, pf, std::integral_constant<int, -2>{});
             if (n_tiles == 2 && n_next > 0) {   // two tiles have no step that copies pair n_tiles: K(0) of the next item
                 issue_k1(2, 0);
@@ -678,8 +679,8 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         } else {
             wait_lgkmcnt<0>();
             phase_barrier();
-            if (more_items) more = uniform(listed[(round - 1) % kListed].exists);
-            if (more) load_q(uniform_ptr(listed[(round - 1) % kListed].Qh), uniform(listed[(round - 1) % kListed].q_block0) + wave * WQ);
+            if (more_items) more = uniform(listed(round).exists);
+            if (more) load_q(uniform_ptr(listed(round).Qh), uniform(listed(round).q_block0) + wave * WQ);
         }
 
         // what the epilogue needs of the item just finished, then on to the next one
