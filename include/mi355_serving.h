@@ -15,9 +15,8 @@
  *     nothing and calls on different streams never share a buffer.
  *     A call that would have to allocate while its stream is being captured fails (hipErrorStreamCaptureUnsupported)
  *     and launches nothing: run the step once on that stream before capturing it, and replay the graph on the stream it
- *     was captured on (or use mi355_fmha_fwd_ws with memory of your own). Only the calling stream's capture state is
- *     visible to the library: a first (or growing) call made while ANOTHER stream captures in global capture mode is a
- *     hipMalloc inside that capture and invalidates it, so make such calls before any capture starts.
+ *     was captured on (or use mi355_fmha_fwd_ws with memory of your own). A first (or growing) call made while
+ *     ANOTHER stream is being captured, in any mode, leaves that capture alone (the hipMalloc is made in relaxed capture mode).
  *     The GEMM entry points keep a second buffer of the same kind per (device, stream) for the partial tiles of products
  *     that are cut into ranges of K because their tiles do not fill the machine (>= 8 MiB, up to 96 MiB); a GEMM call
  *     that cannot get it (its stream is being captured and has none yet, or hipMalloc fails) does not fail: it

@@ -862,6 +862,52 @@ def test_shorter_caches_without_the_librarys_workspace(lib, gpu):
         assert torch.equal(out, whole) or torch.equal(out, lib.fmha_fwd(q, k, v, causal=True)[0])
 
 
+def fresh_stream():
+    """A stream that the library has never seen (torch hands out its pooled ones again)."""
+    import ctypes
+    raw = ctypes.c_void_p()
+    assert ctypes.CDLL("libamdhip64.so").hipStreamCreate(ctypes.byref(raw)) == 0
+    return torch.cuda.ExternalStream(raw.value)
+
+
+@pytest.mark.parametrize("call", ["shorter cache", "long cache", "generation step", "product of few rows", "product of unaligned operands"])
+def test_a_first_call_on_one_stream_leaves_the_capture_of_another_alone(lib, gpu, call):
+    """Each kind of call that takes a workspace of the library, made for the first time on its stream in the middle of a capture (global
+    mode) of another stream: it gets its workspace, and the graph replays what was recorded."""
+    if "product" in call:
+        g = torch.Generator().manual_seed(5)
+        M, N, K = (16, 4096, 4096) if "few" in call else (9, 1001, 4097)
+        a, b = (torch.randn(s, generator=g).half().to(gpu) for s in ((M, K), (K, N)))
+        run_it = lambda out: lib.load().mi355_hgemm(a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, K, N, N, lib.LAYOUTS["NN"],
+                                                    torch.cuda.current_stream(gpu).cuda_stream)
+        out = torch.zeros(M, N, dtype=torch.float16, device=gpu)
+    else:
+        B, Hq, Hkv, Sq, Sk = {"shorter cache": (1, 8, 2, 64, 1900), "long cache": (1, 32, 8, 128, 4096), "generation step": (1, 32, 8, 1, 4096)}[call]
+        q, k, v = (t.to(gpu) for t in so.fmha_inputs(B, Hq, Hkv, Sq, Sk, seed=6))
+        run_it = lambda out: lib.fmha_fwd(q, k, v, causal=True, return_lse=False, out=out)
+        out = torch.zeros_like(q)
+    run_it(out)                        # with the workspace of the current stream
+    want = out.clone()
+    x, w, y = (torch.randn(s, device=gpu).half() for s in ((64, 128), (64, 128), (64, 64)))
+    lib.hgemm(x, w, "NT", out=y)
+    want_y = y.clone()
+    out.zero_()
+    captured, other = fresh_stream(), fresh_stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        lib.hgemm(x, w, "NT", out=y)
+        with torch.cuda.stream(other):
+            run_it(out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)      # on the same path as with a workspace
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want_y)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal", [
     (1, 16, 1, 1, 300, False), (1, 17, 1, 1, 300, False), (2, 32, 1, 1, 77, False),                # one and two blocks of 16 columns

@@ -666,9 +666,8 @@ size_t fmha_decode_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int k
 // mi355_fmha_fwd_ws). Calls on one stream are ordered, so they can share a buffer; calls on different streams get
 // different ones. Nothing can be allocated while the stream is capturing: such a call fails with
 // hipErrorStreamCaptureUnsupported unless an earlier call on the same stream already made the buffer large enough (run
-// the step once before capturing it, or hand in a workspace of your own). Only the calling stream's capture state can be
-// seen from here: while ANOTHER stream of the process captures in global capture mode, a first or growing call (a
-// hipMalloc) would invalidate that capture, so make those calls before any capture starts. The ticket
+// the step once before capturing it, or hand in a workspace of your own); a capture on another stream goes on undisturbed
+// (workspace_malloc). The ticket
 // counters of a new buffer are set to zero here, on the calling stream, in front of whatever uses it (no synchronous fill of the
 // whole buffer on the null stream). `order` comes back holding the lock of that (device, stream): the caller keeps it until
 // its kernel is issued, so that no call of another thread on the same stream, with a buffer that has grown meanwhile or not
@@ -698,7 +697,7 @@ static hipError_t decode_workspace(size_t bytes, hipStream_t stream, char** out,
         if (cap != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
         const size_t want = bytes < (size_t(4) << 20) ? (size_t(4) << 20) : bytes + bytes / 2;
         void* fresh = nullptr;
-        e = hipMalloc(&fresh, want);
+        e = workspace_malloc(&fresh, want);
         if (e != hipSuccess) return e;
         b.ptr = fresh;   // the previous buffer, if any, stays allocated (see above)
         b.size = want;

@@ -882,7 +882,7 @@ static hipError_t segment_workspace(size_t bytes, hipStream_t stream, char** out
         if (cap != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
         const size_t want = bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes + bytes / 2;
         void* fresh = nullptr;
-        e = hipMalloc(&fresh, want);
+        e = workspace_malloc(&fresh, want);
         if (e != hipSuccess) return e;
         b.ptr = fresh;   // the previous buffer, if any, stays allocated (see above)
         b.size = want;

@@ -13,6 +13,16 @@ static __global__ void hgemm_clear_kernel(unsigned* p, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
 }
 
+// hipMalloc in relaxed capture mode: in the thread's own (global) mode an allocation while any other stream is being captured fails and
+// invalidates that capture, and a first call on one stream would end what another one records.
+hipError_t workspace_malloc(void** out, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipError_t e = hipThreadExchangeStreamCaptureMode(&mode); e != hipSuccess) return e;
+    const hipError_t e = hipMalloc(out, bytes);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    return e != hipSuccess ? e : back;
+}
+
 // The workspace of the split-K path: one buffer per (device, stream), allocated at first use and replaced by a larger one when
 // a call needs more; a buffer that has been handed to a kernel is never freed (a HIP graph captured earlier may hold its
 // address). Nothing can be allocated while the stream is capturing: such a call (no buffer yet, or too small a one) fails
@@ -45,7 +55,7 @@ hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, std::
         if (cap != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
         const size_t want = bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes + bytes / 2;
         void* fresh_buf = nullptr;
-        e = hipMalloc(&fresh_buf, want);
+        e = workspace_malloc(&fresh_buf, want);
         if (e != hipSuccess) return e;
         b.ptr = fresh_buf;   // the previous buffer, if any, stays allocated (see above)
         b.size = want;

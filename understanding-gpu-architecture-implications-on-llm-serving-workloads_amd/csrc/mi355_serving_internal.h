@@ -93,6 +93,8 @@ inline int smallm_nt_rega_tpw(int M, int n_tiles, int K, long lda, long ldb) {
     return 0;
 }
 
+// Device memory for a workspace of the library; another stream's capture does not notice.
+hipError_t workspace_malloc(void** out, size_t bytes);
 // Workspace of the split-K path: ticket counters (one per tile, at zero between launches), then `bytes` minus those for
 // partial tiles. hipErrorStreamCaptureUnsupported / hipErrorOutOfMemory: none to be had.
 constexpr size_t kSplitKCounterBytes = 16 * 1024;   // up to 4096 tiles
