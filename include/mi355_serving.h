@@ -18,14 +18,19 @@
  *     was captured on (or use mi355_fmha_fwd_ws with memory of your own). A first (or growing) call made while
  *     ANOTHER stream is being captured, in any mode, leaves that capture alone (the hipMalloc is made in relaxed capture mode).
  *     The GEMM entry points keep a second buffer of the same kind per (device, stream) for the partial tiles of products
- *     that are cut into ranges of K because their tiles do not fill the machine (>= 8 MiB, up to 96 MiB); a GEMM call
+ *     that are cut into ranges of K because their tiles do not fill the machine (>= 8 MiB, up to 96 MiB), among them products of
+ *     up to 16 rows in layouts NN and TN and products of operands with unaligned rows; a GEMM call
  *     that cannot get it (its stream is being captured and has none yet, or hipMalloc fails) does not fail: it
- *     runs the kernels without ranges of K, so a captured call is faster when the step ran once on that stream before.
+ *     runs the kernels without ranges of K, so a captured call is faster when the step ran once on that stream before (and
+ *     its graph is then replayed on that stream, as above).
  *     The attention entry points other than mi355_fmha_fwd_ws (which takes the caller's) and mi355_fmha_fwd_noalloc
- *     (which walks all keys in one kernel) keep a third buffer of that kind
- *     for a chunk of queries against a long cache (at most 128 work items of 128 or 256 queries, kv_valid_len >= 2048: the keys
- *     are cut into up to 8 ranges and a second kernel merges the partial outputs, which take ranges * B * Hq * Sq * 260
- *     bytes; >= 8 MiB); a call that cannot get it walks all keys in one kernel instead of failing, like the GEMM;
+ *     (which walks all keys in one kernel) keep a third buffer of that kind (>= 8 MiB)
+ *     for a few queries against many keys (at most 128 work items of 128 or 256 queries), whose keys are cut into ranges, a second kernel
+ *     merging the partial outputs: for kv_valid_len >= 2048 up to 8 ranges, ranges * B * Hq * Sq * 260 bytes; where these do not
+ *     apply and kv_valid_len > 192, up to 16 ranges whose partial outputs stay in 32 bits, ranges * B * Hq * Sq * 516 bytes (less than
+ *     17 MB). A call that cannot get it walks all keys in one kernel instead of failing, like the GEMM; so does, of the second
+ *     kind, every call that is captured, so that its graph may be replayed on any stream, and one with memory of the caller.
+ *     The results of one walk and of ranges may differ in the last bits;
  *   - `stream` is a hipStream_t passed as void* (NULL = the null stream); calls are asynchronous;
  *   - fp16 data is IEEE binary16 (`_Float16` / `__half` / torch.float16);
  *   - return value 0 = launched; non-zero = a hipError_t value or MI355_ERR_* below, nothing was launched.
@@ -33,7 +38,7 @@
  *   - calls are re-entrant and thread-safe, with one exception: mi355_fmha_fwd_noalloc, whose calls share one fixed
  *     array per GPU and must not overlap on a GPU (see there). The only other mutable global state is one-time kernel
  *     attribute initialisation (atomic flags) and the mutex-protected table of those workspaces. Which kernel runs
- *     depends on the arguments alone.
+ *     depends on the arguments and, where ranges of K or of keys are concerned, on whether the call is captured and its workspace to be had.
  */
 #ifndef MI355_SERVING_H
 #define MI355_SERVING_H
@@ -258,7 +263,8 @@ int mi355_silu_mul_bf16(const void* gate_up, void* out, int64_t rows, int inter,
  * up to a tenth more); for a chunk of queries against a long cache (see the
  * conventions above) ranges * B * Hq * Sq * 260 bytes, which the call uses if `workspace_bytes` covers them and otherwise
  * does without (it then walks all keys in one kernel; a split-KV call with too small a workspace fails); 0 for every
- * other shape (then `workspace` may be NULL). mi355_fmha_fwd_ws is mi355_fmha_fwd_strided (strides == NULL:
+ * other shape (then `workspace` may be NULL), also where mi355_fmha_fwd_strided cuts a shorter cache into ranges: this entry
+ * point walks it in one go. mi355_fmha_fwd_ws is mi355_fmha_fwd_strided (strides == NULL:
  * contiguous [B, H, S, D] operands) for dtype MI355_DTYPE_FP16 or MI355_DTYPE_BF16 that keeps those partial results in
  * `workspace` (16-byte aligned, at least that many bytes, contents irrelevant before and after the call: a small kernel
  * clears the part that must start at zero) and never allocates. Calls that share a workspace must be ordered on one stream. No counterpart in the reference, whose
@@ -281,8 +287,9 @@ int mi355_fmha_fwd_ws(const void* Q, const void* K, const void* V, void* O, floa
  * zero when the library is loaded and every completed call leaves them at zero; a call that does not complete (an aborted
  * kernel, overlapping calls) can leave one that is not, and later calls for that (batch, kv head) then write no output
  * and report no error until the process ends (mi355_fmha_fwd_ws zeroes its counters on every call and has no such
- * memory). Shapes outside the split-KV path (prefill) do not touch the array and behave exactly like
- * mi355_fmha_fwd_strided.
+ * memory). Shapes outside the split-KV path (prefill) do not touch the array: they walk all keys in
+ * one kernel, like mi355_fmha_fwd_strided where that has no buffer for ranges of keys (bit for bit; where it has one and uses
+ * it, the last bits may differ).
  */
 int mi355_fmha_fwd_noalloc(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv, int Sq,
                            int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides, void* stream);

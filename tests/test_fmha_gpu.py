@@ -870,6 +870,46 @@ def fresh_stream():
     return torch.cuda.ExternalStream(raw.value)
 
 
+@pytest.mark.parametrize("entry", ["captured", "captured behind eager calls", "memory of the caller", "no allocation"])
+@pytest.mark.parametrize("Sq,Sk", [(64, 1900), (36, 2386)])
+def test_shorter_caches_are_walked_in_one_go_without_a_buffer_of_the_library(lib, gpu, entry, Sq, Sk):
+    """A captured call (also on a stream that has the buffer: its graph may be replayed on any stream, beside eager calls on the stream it was
+    captured on), a call with memory of the caller, and the entry point that allocates nothing give the bits of one walk over the keys."""
+    q, k, v = (t.to(gpu) for t in so.fmha_inputs(1, 8, 2, Sq, Sk, seed=4))
+    whole = lib.fmha_fwd(q, k, v, causal=True, variant=1)[0].clone()
+    ranges = lib.fmha_fwd(q, k, v, causal=True)[0].clone()
+    assert not torch.equal(ranges, whole) and torch.equal(ranges, lib.fmha_fwd(q, k, v, causal=True, variant=4)[0])
+    assert lib.fmha_workspace_bytes(1, 8, 2, Sq, Sk) == 0
+    out = torch.zeros_like(q)
+    if entry == "memory of the caller":
+        for room in (16, 64 << 20):     # none is asked for; more than the ranges would take
+            lib.fmha_fwd(q, k, v, causal=True, return_lse=False, out=out.zero_(), workspace=torch.empty(room, dtype=torch.uint8, device=gpu))
+            assert torch.equal(out, whole)
+        return
+    if entry == "no allocation":
+        assert torch.equal(lib.fmha_fwd_noalloc(q, k, v, out, causal=True), whole)
+        return
+    stream = fresh_stream()
+    other = torch.zeros_like(q)
+    torch.cuda.synchronize()
+    if entry == "captured behind eager calls":
+        with torch.cuda.stream(stream):
+            lib.fmha_fwd(q, k, v, causal=True, return_lse=False, out=other)
+        torch.cuda.synchronize()
+        assert torch.equal(other, ranges)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        lib.fmha_fwd(q, k, v, causal=True, return_lse=False, out=out)
+    for _ in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()                   # on the current stream, beside eager calls on the stream it was captured on
+        with torch.cuda.stream(stream):
+            lib.fmha_fwd(q, k, v, causal=True, return_lse=False, out=other)
+        torch.cuda.synchronize()
+        assert torch.equal(out, whole) and torch.equal(other, ranges)
+
+
 @pytest.mark.parametrize("call", ["shorter cache", "long cache", "generation step", "product of few rows", "product of unaligned operands"])
 def test_a_first_call_on_one_stream_leaves_the_capture_of_another_alone(lib, gpu, call):
     """Each kind of call that takes a workspace of the library, made for the first time on its stream in the middle of a capture (global

@@ -937,10 +937,18 @@ size_t fmha_key_range_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Sk, in
     return long_cache_plan(B, Hq, Sq, kv_valid_len).bytes((long)B * Hq * Sq);
 }
 
+static bool being_captured(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // the null stream while another one is captured
+    return true;
+}
+
 // Over shorter caches, and with a few items over any, the same where a small model expects it to be done sooner: a 128-query item takes
 // 6 us and 0.7 us per key tile on an empty machine (1.0 with a workgroup on every CU), the second kernel 4.2 us and its bytes. At most as many (item, range)
 // pairs as CUs, at least two key tiles per range, at most 16 ranges. What these calls held in 32 bits from end to end stays so: their
-// partial outputs are not rounded. In the library's own workspace only: a caller's is asked for, and used, for long caches. us, one walk
+// partial outputs are not rounded. In the library's own workspace only (a caller's is asked for, and used, for long caches), and not in a call
+// that is captured: such a graph holds no buffer of the library and may be replayed on any stream, as the header says of these sizes. us, one walk
 // / ranges, causal: 1 x 32/8 heads, 58 queries over 2068 keys 28.4 / 16.4, 1 x 8/2, 36 over 2386 31.7 / 12.9, 1 x 16/4, 88 over 1561 23.4 / 15.9,
 // 1 x 16/4, 229 over 1829 26.1 / 19.7, 1 x 64/8, 69 over 1500 22.5 / 19.3; but 1 x 32/8, 500 over 2000 28.6 / 33.2, 1 x 16/4, 882 over 1797 26.8 /
 // 29.1, 1 x 32/8, 254 over 1425 23.0 / 22.7.
@@ -1050,8 +1058,9 @@ static hipError_t fmha_fwd_dispatch_t(const void* Q, const void* K, const void* 
     KeyRangePlan plan;
     if (variant == 0 || variant == 3) plan = long_cache_plan(B, Hq, Sq, kv_valid_len);
     if ((variant == 0 && plan.segments == 0) || variant == 4) plan = short_cache_plan(B, Hq, Sq, kv_valid_len);
+    if (plan.f32 && variant == 0 && (ws.kind != FmhaWorkspace::kLibrary || being_captured(stream))) plan = {};
     const size_t range_bytes = plan.bytes((long)B * Hq * Sq);
-    const bool caller_ws = !plan.f32 && ws.kind == FmhaWorkspace::kCaller && ws.ptr != nullptr && ws.bytes >= range_bytes &&
+    const bool caller_ws = ws.kind == FmhaWorkspace::kCaller && ws.ptr != nullptr && ws.bytes >= range_bytes &&
                            reinterpret_cast<uintptr_t>(ws.ptr) % 16 == 0;
     if (range_bytes > 0 && (ws.kind == FmhaWorkspace::kLibrary || caller_ws)) {
         char* const mem = caller_ws ? static_cast<char*>(ws.ptr) : nullptr;
