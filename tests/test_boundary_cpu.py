@@ -271,6 +271,15 @@ def test_short_caches_take_the_kernel_that_is_done_first(lib):
         assert decode_plan(lib, B, Hq, Hkv, Sq, kv)[0] > 0, (B, Hq, Hkv, Sq, kv)
 
 
+def test_short_caches_of_many_sequences_take_the_generation_step_kernel(lib):
+    # 17 to 32 columns, or up to 64 keys of more (sequence, kv head) pairs than CUs, where the prefill kernel's items need several rounds
+    for B, Hq, Hkv, Sq, kv in ((16, 32, 1, 1, 100), (32, 16, 2, 4, 65), (16, 32, 8, 8, 65), (16, 32, 8, 8, 128), (8, 64, 8, 4, 128), (20, 32, 32, 12, 8),
+                               (64, 32, 32, 12, 33), (32, 32, 32, 16, 8)):
+        assert decode_plan(lib, B, Hq, Hkv, Sq, kv) == (1, 2 if kv <= 64 else 4), (B, Hq, Hkv, Sq, kv)
+    for B, Hq, Hkv, Sq, kv in ((1, 32, 8, 8, 300), (8, 32, 32, 17, 128), (4, 32, 8, 5, 64), (1, 32, 1, 1, 480), (2, 32, 32, 28, 448)):
+        assert decode_plan(lib, B, Hq, Hkv, Sq, kv)[0] == 0, (B, Hq, Hkv, Sq, kv)
+
+
 @pytest.mark.parametrize("layout,few_rows,shapes", [
     # up to 16 rows against an nn.Linear weight: the small-M kernels, which stream it fastest, also beyond a layer's widths
     ("NT", (1, 4, 8), [(50304, 4096), (50257, 4096), (128256, 2048), (28672, 8192), (14336, 14336), (14336, 4096), (4096, 14336), (4096, 4096)]),

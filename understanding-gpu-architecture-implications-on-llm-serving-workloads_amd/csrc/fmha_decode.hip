@@ -546,12 +546,12 @@ static hipError_t clear_counters(void* counters, long n, hipStream_t stream) {
 // Few query rows per kv head: this kernel, except over a short cache where the prefill kernel is expected to be done first. It
 // walks up to 32 columns of queries side by side and combines its waves column by column, which with many columns takes
 // longer than a short walk over the keys; the prefill kernel pads every head's queries to 128 rows, but has a workgroup per
-// query head, and pays only from 256 of those on. us, prefill kernel / this one: 1 x 32/8 heads, 8 queries over 64 keys 5.6 / 11.6,
-// over 300 9.2 / 13.8; 4 x 32/32, 20 queries over 128 keys 7.1 / 10.0; 1 x 32/8, one query over 300 keys 9.1 / 7.9; 64 x 32/8,
-// one query over 300 keys 65 / 17, 5 queries 65 / 23. The model was within 4 % of the faster one on average over 24 head
-// configurations, 1 .. 32 queries and 32 .. 511 keys (0.66 of the prefill kernel's time, nowhere more than 1.09); with up to 16 columns this
-// kernel has since become faster (one block of matrix instructions 16 columns wide): 2 x 16/4, 4 queries over 112 keys 7.4 / 6.1, 1 x 32/8, 4
-// over 300 9.3 / 7.1.
+// query head, and pays only from 256 of those on. us from the operators, operands from HBM, prefill kernel / this one: 1 x 32/8 heads, 8 queries over
+// 300 keys 9.3 / 11; 8 x 32/32, 17 queries over 128 9.0 / 9.6; 16 x 32/1, 1 over 100 12.5 / 8.4; 16 x 32/8, 8 over 65 12.7 / 8.8; 8 x 64/8,
+// 4 over 128 12.3 / 8.7; 20 x 32/32, 12 over 8 14.1 / 8.3; 64 x 32/32, 12 over 33 34.7 / 20.0. Over 420 calls of 17 .. 32 columns (2 .. 512 workgroups,
+// 40 .. 511 keys) the model takes .6 % longer than the faster kernel on average, 1.36 times at worst (8 x 32/32, 20 over 256 16.3 / 12.0); over 80
+// of up to 16 columns over up to 64 keys .2 % and 1.35 times. The constants of the kernel's 32-column instructions that it had before took 2.4 % and
+// 5.2 % longer; up to 16 columns over more keys: 2 x 16/4, 4 queries over 112 keys 7.4 / 6.1, 1 x 32/8, 4 over 300 9.3 / 7.1.
 bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid_len) {
     const long cols = (long)(Hq / Hkv) * Sq;
     if (cols > 32 || Sk < kv_valid_len || B < 1) return false;
@@ -560,10 +560,12 @@ bool fmha_decode_applicable(int B, int Hq, int Hkv, int Sq, int Sk, int kv_valid
     const long items = (long)B * Hq, wgs = (long)B * Hkv;
     const float prefill_us = 4.9f + .78f * tiles64 + (float)((items + 255) / 256 - 1) * (2.4f + 1.09f * tiles64);
     const float step_us = kv_valid_len <= 64 && wgs > 256   // two waves, two workgroups to a CU
-                              ? (float)((wgs + 511) / 512) * (2.8f + .34f * (float)cols + .0403f * (float)kv_valid_len)
-                          : cols <= 16 && kv_valid_len > 64
+                              ? (float)((wgs + 511) / 512) * (3.5f + .11f * (float)cols + .033f * (float)kv_valid_len)
+                          : cols > 16
+                              ? (float)((wgs + 255) / 256) * (4.2f + .1f * (float)cols + 1.05f * ceilf(tiles32 / 4.f))
+                          : kv_valid_len > 64
                               ? (float)((wgs + 255) / 256) * (3.f + .13f * (float)cols + .6f * ceilf(tiles32 / 4.f))
-                              : (float)((wgs + 255) / 256) * (3.5f + .225f * (float)cols + 1.1f * ceilf(tiles32 / 4.f));
+                              : (float)((wgs + 255) / 256) * (3.5f + .225f * (float)cols + 1.1f);
     return step_us <= 1.03f * prefill_us;
 }
 
