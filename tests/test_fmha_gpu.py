@@ -800,6 +800,29 @@ def test_every_item_of_lists_that_are_written_several_times(lib, gpu, variant, B
         assert bool((o[:, :, :Sq - Sk] == 0).all()) and bool(torch.isinf(lse[:, :, :Sq - Sk]).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal", [
+    (1, 3, 1, 16, 16, True), (2, 16, 2, 9, 64, True), (12, 32, 8, 16, 128, True), (24, 32, 8, 15, 65, False), (9, 32, 8, 17, 70, True),
+    (1, 4, 1, 16, 700, False), (9, 32, 8, 11, 5, True), (1, 1, 1, 1, 1, False), (20, 32, 8, 10, 200, True),
+])
+def test_up_to_16_queries_are_stored_as_they_lie(lib, gpu, dtype, B, Hq, Hkv, Sq, Sk, causal):
+    """The kernel for up to 16 queries (and 17 beside it), one item per workgroup and several: O as a contiguous tensor and as a
+    [B, S, H, D] view between rows that stay untouched, LSE, queries that see no key; items alone have the same bits."""
+    q, k, v = (x.to(dtype) for x in so.fmha_inputs(B, Hq, Hkv, Sq, Sk, seed=Sq + Sk))
+    o, lse = run(lib, gpu, q, k, v, causal, variant=1)
+    o_ref, lse_ref = so.attention_ref(q.float(), k.float(), v.float(), causal=causal)
+    assert (o.float() - o_ref).abs().max() <= (2e-3 if dtype == torch.float16 else 1.6e-2)
+    seen = torch.isfinite(lse_ref)
+    assert torch.equal(torch.isfinite(lse), seen) and (lse - lse_ref)[seen].abs().max() <= 1e-3 and bool((o[~seen] == 0).all())
+    rows = torch.full((B, Sq + 2, Hq, 128), 7.0, dtype=dtype, device=gpu)
+    view = rows[:, 1:-1].transpose(1, 2)
+    lib.fmha_fwd(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal, return_lse=False, out=view, variant=1)
+    assert torch.equal(view.cpu(), o) and bool((rows[:, 0] == 7).all()) and bool((rows[:, -1] == 7).all())
+    for b in {0, B // 2, B - 1}:
+        o1, lse1 = run(lib, gpu, q[b:b + 1], k[b:b + 1], v[b:b + 1], causal, variant=1)
+        assert torch.equal(o[b], o1[0]) and torch.equal(lse[b], lse1[0])
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,S,causal", [
     (4, 64, 8, 152, False), (5, 16, 4, 405, False), (1, 8, 2, 1331, False),      # 256-query items, also fewer of them than CUs
     (6, 64, 8, 270, True), (3, 64, 8, 638, True),                               # 128-query items, also more 256-query items than CUs

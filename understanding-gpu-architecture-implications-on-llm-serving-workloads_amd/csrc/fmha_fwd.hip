@@ -169,20 +169,25 @@ __device__ __forceinline__ void copy16_global_to_lds_at(const void* uniform_base
         : "memory", "m0", "scc");
 }
 
-// SEG: the keys are cut into `segments` ranges of seg_len keys (a multiple of 64) and a work item is (batch, range, head, q
+// kRanges, kRangesF32: the keys are cut into `segments` ranges of seg_len keys (a multiple of 64) and a work item is (batch, range, head, q
 // tile): it attends to its range only (K and V start seg * seg_len rows further on, the valid length and the causal limit
 // are counted from there) and writes its O, normalised over its range, and its LSE to the partial buffers
 // O [segments][B][Hq][Sq][128] and LSE [segments][B][Hq][Sq]; fmha_merge_segments_kernel combines them. For a few queries
 // against a long cache, where one item per (head, q tile) would leave most CUs idle behind a long walk over the keys.
-// kRanges: the partial outputs are of type T; kRangesF32: they are kept in 32 bits.
-enum { kOneWalk = 0, kRanges = 1, kRangesF32 = 2 };
-template <typename T, int QB, int SEG = kOneWalk>
+// MODE: kRanges: the partial outputs are of type T; kRangesF32: they are kept in 32 bits. kFewRows: one walk over all keys, for up to 16
+// queries, which are a single block of rows of the first wave and are stored as they lie: through LDS they are a chain of its own behind the
+// item, and a branch in the other kernels costs those up to 2 %. us, through LDS / as they lie: 64 x 16/2 heads, 9 queries over 64 keys 17.1 /
+// 15.9, 24 x 32/8, 16 over 64 13.8 / 13.1, 12 x 64/8, 16 over 128 18.2 / 17.6.
+enum { kOneWalk = 0, kRanges = 1, kRangesF32 = 2, kFewRows = 3 };
+constexpr int kFewRowsMax = 16;
+template <typename T, int QB, int MODE = kOneWalk>
 __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __restrict__ Q, const T* __restrict__ K,
                                                                const T* __restrict__ V, T* __restrict__ O,
                                                                float* __restrict__ LSE, int B, int Hq, int Hkv, int Sq,
                                                                int Sk, float scale_log2, int causal, int kv_valid,
                                                                int q_tiles, FmhaStrides sd, int segments, int seg_len, ItemMap map) {
     using namespace fmha;
+    constexpr bool SEG = MODE == kRanges || MODE == kRangesF32;
     using V8 = typename Elem<T>::v8;
     using V4 = typename Elem<T>::v4;
     constexpr int NWAVES = 8;
@@ -227,13 +232,13 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         if (!it.exists) return it;
         it.q_block0 = q_tile * BM;
         long k0 = 0;
-        if constexpr (SEG != kOneWalk) {   // b counts (batch, range) pairs
+        if constexpr (SEG) {   // b counts (batch, range) pairs
             const int pair = b;
             b = divide(pair, map_.by_segments);
             const int seg = pair - b * segments;
             k0 = (long)seg * seg_len;
             it.lse_row = (seg * B + b) * Hq + hq;
-            it.Oh = O + (long)it.lse_row * Sq * (SEG == kRangesF32 ? D * (int)(sizeof(float) / sizeof(T)) : D);
+            it.Oh = O + (long)it.lse_row * Sq * (MODE == kRangesF32 ? D * (int)(sizeof(float) / sizeof(T)) : D);
             it.kv_valid = min(max(kv_valid - (int)k0, 0), seg_len);
         } else {
             it.lse_row = b * Hq + hq;
@@ -717,7 +722,21 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
             if (q_item0 + qb * 16 >= Sq) break;   // no such rows (a few queries are done 0.5 us sooner for it)
             const float l_tot = kSumOnMatrixPipe ? l_acc[qb][0] : quad_sum(l_acc[qb][0]);
             const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
-            if constexpr (SEG == kRangesF32) {   // 64 bytes of a row as they lie
+            if constexpr (MODE == kFewRows) {
+                if (r16 < Sq) {
+                    T* const row = o_item + r16 * o_row + 4 * r4;
+#pragma unroll
+                    for (int db = 0; db < 8; ++db) {
+                        V4 v;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = (T)(o[db][qb][e] * inv);
+                        *(V4*)(row + db * 16) = v;
+                    }
+                    if (lse_item != nullptr && r4 == 0) lse_item[r16] = (l_tot > 0.f) ? (m_run[qb] * scale_log2 + __builtin_log2f(l_tot)) * 0.69314718055994531f : -INFINITY;
+                }
+                break;
+            }
+            if constexpr (MODE == kRangesF32) {   // 64 bytes of a row as they lie
                 float* const row = reinterpret_cast<float*>(o_item) + (long)(q_item0 + qb * 16 + r16) * D + 4 * r4;
                 if (q_item0 + qb * 16 + r16 < Sq) {
 #pragma unroll
@@ -769,13 +788,13 @@ static hipError_t compute_units(int& cus) {
     return hipSuccess;
 }
 
-template <typename T, int QB>
+template <typename T, int QB, int MODE = kOneWalk>
 static hipError_t launch_fmha_pingpong(const T* Q, const T* K, const T* V, T* O, float* LSE, int B, int Hq,
                                    int Hkv, int Sq, int Sk, float scale, int causal, int kv_valid, const FmhaStrides& sd,
                                    hipStream_t stream) {
     constexpr int BM = 128 * QB;
     constexpr int LDS = 8 * fmha::TILE_BYTES;
-    auto kern = fmha_fwd_pingpong_kernel<T, QB>;
+    auto kern = fmha_fwd_pingpong_kernel<T, QB, MODE>;
     static DynamicLdsOnce lds_once;
     if (hipError_t e = lds_once.ensure(reinterpret_cast<const void*>(kern), LDS); e != hipSuccess) return e;
     const int q_tiles = (Sq + BM - 1) / BM;
@@ -796,7 +815,7 @@ static hipError_t launch_fmha_pingpong(const T* Q, const T* K, const T* V, T* O,
 // ---------------------------------------------------------------------------------------------------------------
 // A few queries against a long cache (a chunk of a prompt appended to earlier chunks): one work item per (head, q tile)
 // would leave most CUs idle behind a walk over all keys, so the keys are cut into ranges, every (range, head, q tile) is
-// a work item of the same kernel (SEG) and a second kernel merges the ranges:
+// a work item of the same kernel (MODE) and a second kernel merges the ranges:
 //   O = sum_s w_s O_s / sum_s w_s,  w_s = exp(LSE_s - max_s LSE_s),  LSE = max_s LSE_s + log(sum_s w_s)
 // (a range without a visible key has LSE_s = -inf and weight 0; a row without any visible key gets O = 0, LSE = -inf).
 // The partial results live in a workspace of the library's own, one buffer per (device, stream), allocated at first use
@@ -1081,6 +1100,7 @@ static hipError_t fmha_fwd_dispatch_t(const void* Q, const void* K, const void* 
         variant = one_walk_us(2, cus, B, Hq, Sq, Sk, causal, kv_valid_len) < one_walk_us(1, cus, B, Hq, Sq, Sk, causal, kv_valid_len) ? 2 : 1;
     }
     if (variant == 2) return launch_fmha_pingpong<T, 2>(q, k, v, o, LSE, B, Hq, Hkv, Sq, Sk, scale, causal, kv_valid_len, sd, stream);
+    if (Sq <= kFewRowsMax) return launch_fmha_pingpong<T, 1, kFewRows>(q, k, v, o, LSE, B, Hq, Hkv, Sq, Sk, scale, causal, kv_valid_len, sd, stream);
     return launch_fmha_pingpong<T, 1>(q, k, v, o, LSE, B, Hq, Hkv, Sq, Sk, scale, causal, kv_valid_len, sd, stream);
 }
 
