@@ -118,7 +118,8 @@ int mi355_hgemm_add(const void* A, const void* B, const void* R, void* C, int M,
  * mi355_hgemm / mi355_hgemm_add (R may be NULL) for dtype MI355_DTYPE_FP16 or MI355_DTYPE_BF16, with memory of the caller for
  * aligned copies of operands the fast paths cannot read: rows that are not 16-byte aligned (a dense matrix whose row
  * length is not a multiple of 8, a view that starts at an odd element). mi355_gemm_workspace_bytes says how many bytes the
- * copies of a call may take (0: none are made). With that much `workspace` (16-byte aligned, contents irrelevant before and
+ * copies of a call may take at most (0: none are made; most products of up to a few hundred rows need none either, whatever it answers,
+ * and leave the workspace untouched). With that much `workspace` (16-byte aligned, contents irrelevant before and
  * after the call) such operands are copied first and the product runs on the fast paths, where that is expected to be done
  * sooner (1999 x 3001 x 2503 NN: 59 us without, 43 with; up to a few hundred rows, or with a short K, it is not); with
  * less, or NULL, the call reads them where they lie, like the entry points above.

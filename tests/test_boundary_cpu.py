@@ -308,3 +308,19 @@ def test_aligned_copies_of_large_operands_are_asked_for_only_where_they_are_repa
         assert ask(M, N, K, lay) == 0, (M, N, K, lay)
     for M, N, K, lay in ((64, 50257, 4096, "NN"), (16, 14337, 4096, "NN"), (16, 128256, 4099, "NT"), (1999, 3001, 2503, "NN"), (256, 4097, 4096, "TN")):
         assert ask(M, N, K, lay) >= N * K * 2 * (lay != "TN" or N % 8 != 0), (M, N, K, lay)
+
+
+def test_the_copies_of_a_call_never_take_more_than_is_asked_for_and_often_nothing(lib):
+    # what the operators allocate (the bytes that the call uses) against what the public query asks for
+    import random
+    args = lambda M, N, K, lay: (4096, 1 << 40, M, N, K, M if lay == "TN" else K, K if lay == "NT" else N, lib.LAYOUTS[lay])
+    ask = lambda *c: lib.load().mi355_gemm_workspace_bytes(*args(*c))
+    use = lambda *c: lib.load().mi355_internal_gemm_copy_bytes(*args(*c))
+    for c in ((8, 50257, 4096, "NN"), (64, 50257, 4096, "NN"), (62, 19578, 5867, "NT"), (16, 14337, 4096, "NN")):
+        assert use(*c) == 0 and ask(*c) > 100 << 20, c       # read where they lie
+    for c in ((1999, 3001, 2503, "NN"), (2169, 2399, 1727, "NT"), (4097, 4097, 4097, "TN")):
+        assert use(*c) == ask(*c) > 0, c
+    rng = random.Random(1)
+    for _ in range(3000):
+        c = tuple(int(lo * (hi / lo) ** rng.random()) for lo, hi in ((1, 8192), (16, 100000), (8, 16384))) + (rng.choice(("NN", "NT", "TN")),)
+        assert use(*c) in (0, ask(*c)), c

@@ -884,6 +884,42 @@ def test_products_of_unaligned_operands_run_when_no_memory_for_copies_is_left(li
     assert float((got.float() - want).norm() / want.norm()) < 2.0 ** -10      # one more rounding of the last product
 
 
+def test_unaligned_operands_take_memory_only_where_they_are_copied(lib, gpu):
+    # the operator and the binding allocate the result, and room for copies where the call makes some; where there is no room for those left
+    # (torch's allocator limited to a little more than it holds) the product is made without them
+    import gemm_unified
+    for M, N, K in ((64, 14337, 4096), (1999, 3001, 2503)):
+        a, b = operands(M, N, K, "NN", seed=M, b_std=0.05)
+        ag, bg = a.to(gpu), b.to(gpu)
+        copies = lib.load().mi355_internal_gemm_copy_bytes(ag.data_ptr(), bg.data_ptr(), M, N, K, K, N, 0)
+        assert (copies > 0) == (M > 64)
+        ref = so.gemm_ref(a, b, "NN")
+        for product in (lambda: gemm_unified.ops.fine_gemm(ag, bg, 0), lambda: lib.hgemm(ag, bg, "NN")):
+            product()
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            c = product()
+            assert torch.cuda.max_memory_allocated() - before <= 2 * M * N + copies + 4096
+            ok, st = so.gemm_tolerance_ok(c.cpu(), ref, K)
+            assert ok, st
+        if copies:
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            try:
+                torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 * M * N + (4 << 20)) / torch.cuda.get_device_properties(gpu).total_memory)
+                filler = []
+                with pytest.raises(torch.OutOfMemoryError):
+                    while True:
+                        filler.append(torch.empty(copies, dtype=torch.uint8, device=gpu))
+                c = gemm_unified.ops.fine_gemm(ag, bg, 0)
+                torch.cuda.synchronize()
+            finally:
+                torch.cuda.set_per_process_memory_fraction(1.0)
+            ok, st = so.gemm_tolerance_ok(c.cpu(), ref, K)
+            assert ok, st
+
+
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
 @pytest.mark.parametrize("K,splits", [(40, 3), (64, 2), (130, 16), (200, 255)])
 @pytest.mark.parametrize("shape,own_merge", [(2, False), (4, True), (1, False)])

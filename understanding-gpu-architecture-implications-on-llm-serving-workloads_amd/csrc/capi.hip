@@ -83,6 +83,11 @@ size_t mi355_gemm_workspace_bytes(const void* A, const void* B, int M, int N, in
     return mi355::hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout);
 }
 
+size_t mi355_internal_gemm_copy_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout) {
+    if (!A || !B || M < 1 || N < 1 || K < 1 || layout < MI355_GEMM_NN || layout > MI355_GEMM_TN) return 0;
+    return mi355::hgemm_copy_bytes(A, B, M, N, K, lda, ldb, layout);
+}
+
 int mi355_gemm_ws(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldr,
                   int64_t ldc, int layout, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
     if (dtype != MI355_DTYPE_FP16 && dtype != MI355_DTYPE_BF16) return fail(MI355_ERR_BAD_ARGUMENT, "mi355_gemm_ws: unknown dtype %d", dtype);

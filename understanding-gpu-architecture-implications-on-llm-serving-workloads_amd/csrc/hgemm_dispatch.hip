@@ -79,28 +79,27 @@ static bool copies_pay(const GemmPackPlan& plan, int M, int N, int K, int layout
     return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < choose_direct(M, N, K, layout, true).us;
 }
 
-// What callers are asked for, by sizes and alignment: room for small copies always, for large ones where copying them takes less time than
-// a workgroup per 64 x 64 outputs that gathers its operands 16 columns of K at a time (.0533 us per column of K, more where such
-// workgroups wait for each other). An upper bound: what a call uses is hgemm_copy_bytes.
+size_t hgemm_copy_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
+    if (K <= 64) return 0;
+    const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
+    if (!plan.a.pack && !plan.b.pack) return 0;
+    return copies_pay(plan, M, N, K, layout) ? plan.bytes() : 0;
+}
+
+// The public query answers as it did when a workgroup per 64 x 64 outputs that gathers its operands 16 columns of K at a time (.0533 us per
+// column of K, more where such workgroups wait for each other) was what such products ran on without copies: never less than the copies
+// of the call take, and often more, as the direct kernel needs none for most of these products (hgemm_copy_bytes: 0 where this asks for
+// 412 MB, 8 x 50257 x 4096 NN).
 size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
     if (K <= 64) return 0;
     const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
     if (!plan.a.pack && !plan.b.pack) return 0;
-    if (plan.bytes() <= (size_t(1) << 20)) return plan.bytes();
+    if (plan.bytes() <= (size_t(1) << 20) || copies_pay(plan, M, N, K, layout)) return plan.bytes();
     const float wgs = (float)((M + 63) / 64) * (float)((N + 63) / 64), rows = (float)(M < 64 ? M : 64);
     const float per_wg = layout == MI355_GEMM_NT ? 1.94e-4f * (1.f + .0144f * rows) : 4.04e-5f * (1.f + (layout == MI355_GEMM_TN ? .0103f : .0559f) * rows);
     const float gather_us = 2.32f + (float)K * fmaxf(.0533f, per_wg * wgs);
     const KernelChoice fast = choose_kernel(M, N, K, layout != MI355_GEMM_TN, layout == MI355_GEMM_NT, true, true, plan.b.ld % 64 == 0);
     return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < gather_us ? plan.bytes() : 0;
-}
-
-// At most what hgemm_workspace_bytes asks for.
-size_t hgemm_copy_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {
-    if (K <= 64) return 0;
-    const GemmPackPlan plan = gemm_pack_plan(A, B, M, N, K, lda, ldb, layout);
-    if (!plan.a.pack && !plan.b.pack) return 0;
-    if (!copies_pay(plan, M, N, K, layout)) return 0;
-    return hgemm_workspace_bytes(A, B, M, N, K, lda, ldb, layout);
 }
 
 template <typename T>

@@ -123,7 +123,7 @@ hipError_t gemm_pack_launch(const GemmPackPlan& plan, const void* A, const void*
 KernelChoice choose_direct(int M, int N, int K, int layout, bool split_ok);
 hipError_t gemm_direct_dispatch(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda, long ldb, long ldc, long ldr,
                                 int layout, int dtype, int variant, hipStream_t stream);
-// Bytes of workspace a caller is asked for (0: none, nothing to copy or not worth it), and those that the call then uses.
+// Bytes of workspace the public query asks for (0: none, nothing to copy or not worth it), and those that the copies of a call take.
 size_t hgemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
 size_t hgemm_copy_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout);
 
@@ -209,6 +209,9 @@ int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C,
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                     int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides,
                                     int dtype, int variant, void* stream);
+// bytes of workspace that mi355_gemm_ws uses for a call (0: it makes no copies): what the operators, the Python binding and the decoder layer
+// allocate, where mi355_gemm_workspace_bytes may ask for more
+size_t mi355_internal_gemm_copy_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout);
 // The QKV projection of a generation step's layer with the RMSNorm of its rows (norm_weight null: none) and mi355_rope_qkv in one
 // launch: qkv = rope(rmsnorm(x) w_qkv^T), rotated keys and values into kv_out; x is [B, S, hidden], qkv [B, S, (q_heads + 2 kv_heads)
 // * 128]. And silu(gate) * up of the normalised rows (w_gu in groups of 32 gate and 32 up rows). The bits of the single launches on

@@ -19,6 +19,9 @@
 
 #include "mi355_serving.h"
 
+// of the same library (csrc/mi355_serving_internal.h)
+extern "C" size_t mi355_internal_gemm_copy_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout);
+
 namespace gemm_unified {
 
 // Registers _C as a Python extension module.
@@ -62,9 +65,9 @@ at::Tensor run_gemm(const at::Tensor& a, const at::Tensor& b, int layout, const 
     // Leading dimensions are the logical row lengths of the contiguous operands, not stride(0): torch ignores the stride of
     // a size-1 dimension when it decides contiguity, so a [1, K] operand may carry any stride(0).
     const int64_t lda = ac.size(1), ldb = bc.size(1);
-    // operands with unaligned rows: room for aligned copies, from torch's allocator (reused in the stream's order); where there is
-    // none left the product runs without copies
-    size_t need = mi355_gemm_workspace_bytes(ac.data_ptr(), bc.data_ptr(), (int)M, (int)N, (int)K, lda, ldb, layout);
+    // operands with unaligned rows: room for aligned copies where the call makes some, from torch's allocator (reused in the stream's
+    // order); where there is none left the product runs without copies
+    size_t need = mi355_internal_gemm_copy_bytes(ac.data_ptr(), bc.data_ptr(), (int)M, (int)N, (int)K, lda, ldb, layout);
     at::Tensor ws;
     if (need > 0) {
         try {

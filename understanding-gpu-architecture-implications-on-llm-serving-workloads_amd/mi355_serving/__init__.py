@@ -21,7 +21,7 @@ EXPORTED_SYMBOLS = ("mi355_hgemm", "mi355_fmha_fwd", "mi355_fmha_fwd_strided", "
                     "mi355_fmha_fwd_workspace_bytes", "mi355_fmha_fwd_ws", "mi355_fmha_fwd_noalloc",
                     "mi355_last_error", "mi355_serving_version")
 # exported for tests and tuning runs, declared in csrc/mi355_serving_internal.h and not in the public header
-INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_add_variant", "mi355_internal_hgemm_choice",
+INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_add_variant", "mi355_internal_hgemm_choice", "mi355_internal_gemm_copy_bytes",
                     "mi355_internal_hgemm_silu_mul_variant", "mi355_internal_fmha_fwd_variant",
                     "mi355_internal_fmha_decode_plan", "mi355_internal_step_qkv", "mi355_internal_step_gate_up")
 
@@ -80,6 +80,8 @@ def load():
     lib.mi355_serving_version.restype = i32
     lib.mi355_gemm_workspace_bytes.argtypes = [vp, vp, i32, i32, i32, i64, i64, i32]
     lib.mi355_gemm_workspace_bytes.restype = ctypes.c_size_t
+    lib.mi355_internal_gemm_copy_bytes.argtypes = lib.mi355_gemm_workspace_bytes.argtypes
+    lib.mi355_internal_gemm_copy_bytes.restype = ctypes.c_size_t
     lib.mi355_gemm_ws.argtypes = [vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i64, i32, i32, vp, ctypes.c_size_t, vp]
     lib.mi355_gemm_ws.restype = i32
     lib.mi355_fmha_fwd_workspace_bytes.argtypes = [i32] * 6
@@ -171,10 +173,10 @@ def hgemm(a, b, layout="NN", out=None, residual=None, variant=0):
             _check(load().mi355_internal_hgemm_add_variant(_ptr(a), _ptr(b), _ptr(residual), _ptr(out), M, N, K, lda, ldb,
                                                            max(residual.stride(0), N), max(out.stride(0), N), *tail))
         return out
-    # operands with unaligned rows: room for aligned copies of them, if there is any
+    # operands with unaligned rows: room for aligned copies where the call makes some, if there is any
     need = 0
     if (lda | ldb) & 7 or (_ptr(a) | _ptr(b)) & 15:
-        need = load().mi355_gemm_workspace_bytes(_ptr(a), _ptr(b), M, N, K, lda, ldb, lay)
+        need = load().mi355_internal_gemm_copy_bytes(_ptr(a), _ptr(b), M, N, K, lda, ldb, lay)
     ws = None
     if need:
         try:

@@ -17,6 +17,7 @@
 #include "mi355_serving.h"
 
 // of the same library (csrc/mi355_serving_internal.h)
+extern "C" size_t mi355_internal_gemm_copy_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout);
 extern "C" int mi355_internal_step_qkv(const void* x, const void* norm_weight, float eps, const void* w_qkv, void* qkv, void* kv_out, int B, int S,
                                        int q_heads, int kv_heads, int hidden, int64_t out_batch, int64_t out_row, int64_t out_head,
                                        const float* cos_table, const float* sin_table, const int32_t* positions, int64_t pos_batch, int n_positions,
@@ -47,7 +48,7 @@ struct Events {   // the pair of events around the attention block when it is ti
 // C = A W^T (+ R) for activations [M, K] and an nn.Linear weight [N, K], both with rows side by side
 void linear(const void* a, const at::Tensor& w, const void* r, void* c, int64_t M, int dtype, hipStream_t stream) {
     const int64_t N = w.size(0), K = w.size(1);
-    size_t need = mi355_gemm_workspace_bytes(a, w.data_ptr(), (int)M, (int)N, (int)K, K, K, MI355_GEMM_NT);
+    size_t need = mi355_internal_gemm_copy_bytes(a, w.data_ptr(), (int)M, (int)N, (int)K, K, K, MI355_GEMM_NT);
     at::Tensor ws;
     if (need > 0) {
         try {
