@@ -900,7 +900,8 @@ def test_unaligned_operands_take_memory_only_where_they_are_copied(lib, gpu):
             torch.cuda.reset_peak_memory_stats()
             before = torch.cuda.memory_allocated()
             c = product()
-            assert torch.cuda.max_memory_allocated() - before <= 2 * M * N + copies + 4096
+            # (of a block that is up to 1 MiB too large torch's allocator hands out the whole; copies of the second operand are 117 and 15 MB)
+            assert torch.cuda.max_memory_allocated() - before <= 2 * M * N + copies + (2 << 20)
             ok, st = so.gemm_tolerance_ok(c.cpu(), ref, K)
             assert ok, st
         if copies:
