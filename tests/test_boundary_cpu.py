@@ -318,7 +318,9 @@ def test_the_copies_of_a_call_never_take_more_than_is_asked_for_and_often_nothin
     use = lambda *c: lib.load().mi355_internal_gemm_copy_bytes(*args(*c))
     for c in ((8, 50257, 4096, "NN"), (64, 50257, 4096, "NN"), (62, 19578, 5867, "NT"), (16, 14337, 4096, "NN")):
         assert use(*c) == 0 and ask(*c) > 100 << 20, c       # read where they lie
-    for c in ((1999, 3001, 2503, "NN"), (2169, 2399, 1727, "NT"), (4097, 4097, 4097, "TN")):
+    # large products, and a long K whose ranges leave one CU of an XCD with twice the work of the others (3 ranges of 84 tiles: 33 workgroups)
+    for c in ((1999, 3001, 2503, "NN"), (2169, 2399, 1727, "NT"), (4097, 4097, 4097, "TN"), (751, 385, 8595, "NN"), (1029, 261, 6005, "NN"),
+              (561, 551, 5443, "NT"), (1287, 221, 5129, "NT"), (2439, 321, 3389, "NN")):
         assert use(*c) == ask(*c) > 0, c
     rng = random.Random(1)
     for _ in range(3000):

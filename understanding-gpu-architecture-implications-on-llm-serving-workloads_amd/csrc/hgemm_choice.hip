@@ -146,16 +146,19 @@ KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles
     return e.choice;
 }
 
-// The direct kernel (hgemm_direct.hip) for a product: tiles and ranges of K. A K tile costs a CU .37 us on 64x64 tiles however many of
-// them share it (its LDS is busy: every operand byte is written once and read twice), .94 us on one 128x128 tile and 1.54 on two.
-// Fitted to 1460 timings of 230 products (1 .. 2600 rows, 64 .. 20000 columns, K 40 .. 9000, all layouts, weights from HBM): the
-// choice among these kernels and the aligned copies, copies_pay, takes 1.9 % longer than the fastest of them on average; copies and
-// the gather that they were weighed against before, 33 %.
+// The direct kernel (hgemm_direct.hip) for a product: tiles and ranges of K. A K tile costs a CU .41 us on 64x64 tiles however many of
+// them share it (its LDS is busy: every operand byte is written once and read twice), .99 us on one 128x128 tile and 1.65 on two. An XCD's
+// 32 CUs take an eighth of the tiles, of every range, rounded up: 84 tiles in 3 ranges are 252 workgroups, but 33 on most XCDs, and one CU
+// of each walks K for two of them (751 x 385 x 8595 NN 42.6 us, copies 32.3; counted over 256 CUs this was expected to take 25).
+// Fitted to 2027 timings of 190 products (1 .. 2600 rows, 64 .. 20000 columns, K 40 .. 9000, all layouts, both operands from HBM; rms 6.6 %). The
+// choice among these kernels and the aligned copies, copies_pay, takes .80 of the time of copies and of the gather that these kernels
+// replaced on average, and 4.6 % more than the fastest of them; slower than those: 3 x 17073 x 65 NN 7.2 us (gathered 5.9), 1 x 73 x 1439 NT 9.1
+// (8.2), 191 x 8893 x 1763 TN 29.6 (27.7), and with K up to 64 some by up to 8 % (441 x 6011 x 41 TN 7.4, 6.9).
 KernelChoice choose_direct(int M, int N, int K, int layout, bool split_ok) {
     static const int ranges[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int ktiles = (K + 63) / 64;
-    const float b_bytes = 2.f * (float)N * (float)K, out_mb = 2e-6f * (float)M * (float)N, mb = b_bytes * 1e-6f + 2e-6f * (float)M * (float)K + out_mb;
-    const float hbm = b_bytes > 20e6f ? 1.f : 0.f, floor_us = mb / 3.6f + 4.06f;
+    const float in_mb = 2e-6f * ((float)M + (float)N) * (float)K, out_mb = 2e-6f * (float)M * (float)N, floor_us = (in_mb + out_mb) / 3.48f + 4.34f;
+    const float factor = (layout == MI355_GEMM_TN ? .92f : 1.f) * (in_mb > 20.f ? 1.05f : 1.f);
     KernelChoice best;
     best.us = 1e30f;
     for (const int shape : {(int)kDirect64x64, (int)kDirect128x128}) {
@@ -163,15 +166,14 @@ KernelChoice choose_direct(int M, int N, int K, int layout, bool split_ok) {
         const int bm = large ? 128 : 64;
         if (large && M <= 32) break;
         const long tiles = (long)((M + bm - 1) / bm) * ((N + bm - 1) / bm);
-        const float factor = (layout == MI355_GEMM_NT ? 1.045f : layout == MI355_GEMM_TN ? .95f : 1.f) * (1.f + hbm * (large ? .066f : .276f));
         for (const int s : ranges) {
-            const long wgs = tiles * s;
-            const float part_mb = 4e-6f * (float)wgs * (float)(bm * bm);
+            const float part_mb = 4e-6f * (float)(tiles * s) * (float)(bm * bm);
             if (s > 1 && (!split_ok || ktiles < 2 * s || part_mb > 48.f)) break;
-            const float per_cu = (float)((wgs + 255) / 256);
-            const float step = large ? std::fmax(.943f * (float)((wgs + 511) / 512), .769f * per_cu) : .367f * per_cu;
-            float us = std::fmax((large ? 5.31f : 4.23f) + (float)((ktiles + s - 1) / s) * step * factor, floor_us) + out_mb * (large ? .223f : .561f);
-            if (s > 1) us += 1.84f + .413f * part_mb + .116f * (float)s;
+            const long on_xcd = (tiles + 7) / 8 * s;
+            const float per_cu = (float)((on_xcd + 31) / 32);
+            const float step = large ? std::fmax(.994f * (float)((on_xcd + 63) / 64), .826f * per_cu) : .41f * per_cu;
+            float us = std::fmax((large ? 5.23f : 4.34f) + (float)((ktiles + s - 1) / s) * step * factor, floor_us) + out_mb * (large ? .222f : .522f);
+            if (s > 1) us += 1.8f + .38f * part_mb + .11f * (float)s;
             if (us >= best.us) continue;
             best.us = us;
             best.shape = shape;
