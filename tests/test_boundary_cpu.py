@@ -300,6 +300,16 @@ def test_products_of_few_rows_that_the_tiles_finish_first(lib, M, N, K, layout):
     assert lib.load().mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout], None) != 8
 
 
+def test_128_columns_and_ranges_of_k_are_taken_where_they_are_done_first(lib):
+    ranges = lambda M, N, K, layout: lib.load().mi355_internal_hgemm_wide_ranges(M, N, K, N, lib.LAYOUTS[layout])
+    for M, N, K, layout, want in ((16, 14336, 4096, "NN", 2), (16, 4096, 4096, "NN", 8), (8, 6144, 4096, "TN", 5), (16, 4096, 14336, "NN", 8),
+                                  (1, 1024, 4096, "NN", 8), (16, 12288, 4096, "TN", 2)):
+        assert ranges(M, N, K, layout) == want, (M, N, K, layout)
+    # a short K, where the merge costs more than it gives; more rows or columns; an nn.Linear weight
+    for M, N, K, layout in ((16, 8192, 1024, "NN"), (16, 4096, 512, "TN"), (17, 4096, 4096, "NN"), (16, 28672, 4096, "NN"), (16, 4096, 4096, "NT")):
+        assert ranges(M, N, K, layout) == 0, (M, N, K, layout)
+
+
 def test_aligned_copies_of_large_operands_are_asked_for_only_where_they_are_repaid(lib):
     # unaligned dense operands, bytes of the copies asked for: nothing where reading and writing a large operand takes longer than
     # the bounds-checked kernel takes for the product

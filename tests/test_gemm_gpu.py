@@ -821,6 +821,7 @@ def test_few_rows_in_128_columns_and_ranges_of_k(lib, gpu, dtype, layout, M, N, 
     tail = (lib.LAYOUTS[layout], lib.DTYPE_BF16 if dtype == torch.bfloat16 else lib.DTYPE_FP16, 8 + 16 * ranges if ranges else 0, torch.cuda.current_stream(gpu).cuda_stream)
     if not ranges:
         assert lib.load().mi355_internal_hgemm_choice(M, N, K, bg.shape[1], lib.LAYOUTS[layout], None) == 8
+        assert lib.load().mi355_internal_hgemm_wide_ranges(M, N, K, bg.shape[1], lib.LAYOUTS[layout]) > 1
     ref = so.gemm_ref(a, b, layout)
     # fp32 sums in two orders: K 2^-23 of the sum of magnitudes at most; one rounding of the product, one of the sum
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11

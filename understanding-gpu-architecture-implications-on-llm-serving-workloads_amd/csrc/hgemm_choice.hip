@@ -81,13 +81,19 @@ static KernelChoice cheapest_kernel(int M, int N, int K, bool a_kc, bool b_kc, b
             const float stream = b_bytes * (1.f + (float)(row_blocks - 1) * .1f) * (from_hbm && !whole_lines ? 2.04f : 1.f) / 5.7e6f;
             consider(fmaxf(1.67f + ceilf(wgs / 256.f) * (k * (from_hbm ? 1.38f : 1.f) * .169f + .565f), stream + 2.56f), kSmallM, 1, false);
             // 128 columns and as many ranges of K as CUs are left: 1.4 us for a step of 256 rows, 6.1 TB/s, 1.3 times the bytes where rows are no
-            // whole lines, 5.4 us beside them (within 0.6 us of 12 products timed, 8.1 .. 28.2 us); times .92 (TN: .88), as the other kernels' times
-            // here come out against those of the same measurement
-            if (const int n_wide = (N + 127) / 128, ranges = std::min(8, std::min(256 / n_wide, K / 256)); M <= 16 && split_ok && ranges > 1) {
-                const float steps = ceilf((float)K / (256.f * (float)ranges)), wide_us = (a_kc ? .92f : .88f) * (5.4f + fmaxf(1.4f * steps, b_bytes * (whole_lines ? 1.f : 1.3f) / 6.1e6f));
+            // whole lines, 5.4 us beside them; times .92 (TN: .88), as the other kernels' times here come out against those of the same measurement.
+            // Of the time without this kernel the choice takes .906 over 165 products of layers' widths (1, 8, 16 rows, 256 .. 16384 columns, K 1024 ..
+            // 14336, weights from HBM; at worst 1.067, 1 x 3072 x 2048 NN 7.7 / 8.2) and .969 over 330 drawn ones (at worst 1.18, 16 x 1536 x 10176 NN
+            // 12.1 / 14.2, 16 x 1280 x 1536 TN 5.8 / 6.9); .962 where the weight lies in the memory-side cache, which delivers it faster to more
+            // workgroups side by side: there 16 x 14336 x 4096 NN takes 21.3 us, 19.4 on 64 columns (from HBM 24.4, 25.6), 16 x 8192 x 2048 TN 8.2, 6.6
+            // (from HBM 11.4, 11.4). Where a weight lies is not known here.
+            const int n_wide = (N + 127) / 128, ranges_wide = M <= 16 && split_ok ? std::min(8, std::min(256 / n_wide, K / 256)) : 0;
+            if (ranges_wide > 1) {
+                const float steps = ceilf((float)K / (256.f * (float)ranges_wide));
+                const float wide_us = (a_kc ? .92f : .88f) * (5.4f + fmaxf(1.4f * steps, b_bytes * (whole_lines ? 1.f : 1.3f) / 6.1e6f));
                 if (wide_us < best_us) {
                     consider(wide_us, kSmallM, 1, false);
-                    best.wide_ranges = ranges;
+                    best.wide_ranges = ranges_wide;
                 }
             }
         }

@@ -202,8 +202,10 @@ int mi355_internal_hgemm_variant(const void* A, const void* B, void* C, int M, i
 int mi355_internal_hgemm_add_variant(const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                      int64_t ldr, int64_t ldc, int layout, int dtype, int variant, void* stream);
 // the variant that the choice by shape takes for a product of 16-byte aligned operands (ldb: row stride of the second one), and the
-// time it expects (us may be null)
+// time it expects (us may be null); for the small-M kernels (8) in layouts NN and TN the second says which: ranges of K of the 128-column
+// kernel, to be pinned with 8 + 16 ranges, or 0, the 64-column kernel
 int mi355_internal_hgemm_choice(int M, int N, int K, int64_t ldb, int layout, float* us);
+int mi355_internal_hgemm_wide_ranges(int M, int N, int K, int64_t ldb, int layout);
 int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                                           int64_t ldc, int layout, int dtype, int variant, void* stream);
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,

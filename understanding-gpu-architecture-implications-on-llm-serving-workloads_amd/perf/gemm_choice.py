@@ -22,6 +22,8 @@ RANGES = (2, 3, 4, 5, 6, 8, 10, 12, 16)
 def variants(M, N, K, layout):
     """The pinned kernels that fit a product, ranges of K included."""
     out = [8] if M <= 64 else []
+    if M <= 16 and layout != "NT":      # 128 columns and ranges of K
+        out += [8 + 16 * s for s in (2, 4, 6, 8) if s * 256 <= K]
     for shape, (bm, bn) in TILE.items():
         if (shape == 7 and layout == "TN") or (shape == 9 and M > 64) or (bm > 64 and bm >= 2 * M):
             continue
@@ -77,6 +79,8 @@ def main():
     for i in range(args.products):
         M, N, K, layout = draw(rng, args.rows)
         chosen = cdll.mi355_internal_hgemm_choice(M, N, K, K if layout == "NT" else N, lib.LAYOUTS[layout], None)
+        if chosen == 8 and layout != "NT":
+            chosen += 16 * cdll.mi355_internal_hgemm_wide_ranges(M, N, K, N, lib.LAYOUTS[layout])
         todo = sorted(set(variants(M, N, K, layout)) | {chosen})
         best = {v: time_us(M, N, K, layout, v, 4) for v in todo}
         for _ in range(3):
