@@ -312,7 +312,7 @@ def test_128_columns_and_ranges_of_k_are_taken_where_they_are_done_first(lib):
 
 def test_aligned_copies_of_large_operands_are_asked_for_only_where_they_are_repaid(lib):
     # unaligned dense operands, bytes of the copies asked for: nothing where reading and writing a large operand takes longer than
-    # the bounds-checked kernel takes for the product
+    # the product takes without copies
     ask = lambda M, N, K, lay: lib.load().mi355_gemm_workspace_bytes(4096, 1 << 40, M, N, K, M if lay == "TN" else K, K if lay == "NT" else N, lib.LAYOUTS[lay])
     for M, N, K, lay in ((1, 128257, 512, "NN"), (1, 256001, 1024, "TN"), (4, 128257, 512, "NN"), (2, 53001, 102, "NN")):
         assert ask(M, N, K, lay) == 0, (M, N, K, lay)

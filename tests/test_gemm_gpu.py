@@ -294,7 +294,7 @@ def test_grids_walked_in_super_blocks(lib, gpu, variant, tile_m, tile_n, layout,
 def _seeded_shapes(n, seed):
     """n products drawn with a fixed seed: row counts from one to a few thousand, widths and depths on and off the tile grid
     (multiples of 8, sometimes odd), every layout. The library picks the kernel (variant 0): small-M, one of the four tile
-    shapes (with or without a K tail or ranges of K), behind aligned copies of unaligned operands, or the bounds-checked kernel."""
+    shapes (with or without a K tail or ranges of K), behind aligned copies of unaligned operands, or on the direct kernel."""
     rng = np.random.default_rng(seed)
     out = []
     for _ in range(n):
@@ -442,7 +442,7 @@ def test_strided_leading_dimensions(lib, gpu):
 @pytest.mark.parametrize("layout", ["NN", "NT"])
 def test_leading_dimension_beyond_the_tiled_kernels_reach(lib, gpu, layout):
     """The tiled kernels address a tile with 32-bit byte offsets and take leading dimensions below 2^22 elements; a wider
-    operand must take the bounds-checked kernel and still be right (A is a 128 x 64 corner of a 128 x 2^22 buffer)."""
+    operand must take the direct kernel and still be right (A is a 128 x 64 corner of a 128 x 2^22 buffer)."""
     M, N, K, lda = 128, 64, 64, 1 << 22
     abig = torch.zeros((M, lda), dtype=torch.float16, device=gpu)
     a = so.randn_fp16((M, K), 3)
@@ -578,7 +578,7 @@ def test_bfloat16_gemm_exact_cases_and_torch_operator(lib, gpu):
                                    (16, 4096, 1024),     # small-M kernels (NN, NT)
                                    (12, 6144, 4096),     # NT: several row tiles per workgroup, A kept in registers
                                    (8, 72, 192),
-                                   (100, 70, 50)])       # bounds-checked kernel
+                                   (100, 70, 50)])       # direct kernel
 def test_residual_epilogue_equals_product_then_add(lib, gpu, dtype, layout, M, N, K):
     """residual + proj(x) (modeling_llama.py:776,781): the fused form must give, bit for bit, what the product followed by
     an elementwise add in the same type gives, for a separate output, for a residual with a row stride, and in place."""

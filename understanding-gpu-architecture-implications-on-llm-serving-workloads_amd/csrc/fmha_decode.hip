@@ -605,7 +605,9 @@ static DecodePlan decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid) {
     // memory's rate: 0.32 us while up to 64 of them run, 0.38 with 128, 0.69 with all 256 (measured over 8192 keys); then
     // the merge. Below 512 keys one workgroup walks them all: no workspace is needed, and the merge would take as long as
     // the walk. us, with the even cut / by this rule: 8 pairs over 1000 keys 9.1 / 8.0, 52 pairs over 8191 keys (five ranges are
-    // 260 workgroups) 56.8 / 45.9, 160 pairs over 4500 keys 82.8 / 70.0.
+    // 260 workgroups) 56.8 / 45.9, 160 pairs over 4500 keys 82.8 / 70.0. (The 3 us and the merge are those of an earlier combine and
+    // merge; over 84 drawn calls, 512 .. 30000 keys from HBM, the number that they give takes .8 % longer than the best of those allowed on
+    // average, at worst 5 %: 16 pairs over 1704 keys 7 ranges 10.1, 16 ranges 9.6.)
     long splits = 1, most = 1;
     if (pairs <= kMaxSplitPairs && kv_valid >= 512) {
         const long even = std::max(1L, std::min({(256 + pairs / 2) / pairs, (long)(tiles + 7) / 8, (long)kMaxSplits}));

@@ -1038,8 +1038,9 @@ static hipError_t launch_fmha_segmented(const T* Q, const T* K, const T* V, T* O
 // to do, as fmha_work_item deals the items out. An item takes 2.6 us and 1.2 us per key tile (256 queries, every K / V fragment feeding
 // two MFMAs: 4.6 and 1.75); a last round of 128-query items up to a quarter less, the emptier it is (the clock rises; 528 .. 768 items over
 // 2048 keys 94.5 .. 102.6 us, as 256-query items 99.9 .. 100.1). That weighs the queries a tile is padded by, the last round of items and, causal, the length of the
-// heaviest item against the better kernel. Over 170 drawn calls (1 .. 16 sequences, 64 .. 8192 queries, 8 .. 64 heads, causal or not, and
-// chunks over a cache) the choice is within 0.2 % of the faster one on average; a rule on the number of 256-query items that preceded it, 1.7 %. us,
+// heaviest item against the better kernel. Over 165 drawn calls (1 .. 15 sequences, 64 .. 8192 queries, 8 .. 64 heads, causal or not, and
+// chunks over a cache) the choice is within 0.2 % of the faster one on average, at worst 11 % (8 x 32/32 x 619 causal 70 / 63); a rule on the number
+// of 256-query items that preceded it, 1.7 %. us,
 // 128- / 256-query items: 13 x 64/8 x 353 causal 83 / 99, 9 x 32/32 x 317 causal 34 / 42, 16 x 32/8 x 512 causal 85 / 76, 4 x 64/8 x 152 17.0 / 13.7,
 // 3 x 16/4 x 917 36.6 / 29.1, 1 x 8/2 x 7441 228 / 183, 1 x 32/8 x 1331 44.7 / 35.6, 10 x 40/8 x 255 34.1 / 28.6, 8 x 64/8 x 638 causal 104 / 115.
 static float one_walk_us(int qb, int cus, int B, int Hq, int Sq, int Sk, int causal, int kv_valid) {

@@ -1,13 +1,11 @@
 // Shared device-side helpers for the gfx950 (MI355X, CDNA4) serving kernels.
 //
 // Everything here is written for wave64 and for the gfx950 instruction set only:
-//   * v_mfma_f32_32x32x16_f16 / v_mfma_f32_16x16x32_f16 (fp16 in, fp32 accumulate)
+//   * v_mfma_f32_16x16x32_f16 / _bf16 (16-bit values in, fp32 accumulate)
 //   * global_load_lds_dwordx4 / buffer_load_dwordx4 ... lds (16-byte global -> LDS copies that bypass the VGPRs)
 //   * ds_read_b64_tr_b16 (LDS read that transposes a 4x16 block of 16-bit values)
 //
 // Register layouts (checked on hardware):
-//   mfma 32x32x16: operand lane l holds 8 consecutive k (k = 8*(l/32) .. +7) of row/col l%32;
-//                  accumulator element 4p+q of lane l is D[8p + 4*(l/32) + q][l%32].
 //   mfma 16x16x32: operand lane l holds k = 8*(l/16) .. +7 of row/col l%16;
 //                  accumulator element q of lane l is D[4*(l/16) + q][l%16].
 //   ds_read_b64_tr_b16: inside each group of 16 lanes, input lane j supplies the four 16-bit values
@@ -22,7 +20,6 @@ typedef _Float16 half_t;
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float16v __attribute__((ext_vector_type(16)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef int int4v __attribute__((ext_vector_type(4)));
@@ -153,9 +150,6 @@ struct Elem<half_t> {
     using v4 = half4;
     using v2 = half2v;
     static __device__ __forceinline__ v8 frag(half8 raw) { return raw; }
-    static __device__ __forceinline__ float16v mfma32(v8 a, v8 b, float16v c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
     static __device__ __forceinline__ float4v mfma16(v8 a, v8 b, float4v c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
     }
@@ -166,9 +160,6 @@ struct Elem<bf16_t> {
     using v4 = bf16x4;
     using v2 = bf16x2;
     static __device__ __forceinline__ v8 frag(half8 raw) { return __builtin_bit_cast(bf16x8, raw); }
-    static __device__ __forceinline__ float16v mfma32(v8 a, v8 b, float16v c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
     static __device__ __forceinline__ float4v mfma16(v8 a, v8 b, float4v c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }

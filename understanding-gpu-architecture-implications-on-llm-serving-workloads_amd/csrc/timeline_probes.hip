@@ -14,6 +14,8 @@
 #ifdef MI355_TIMELINE
 namespace mi355 {
 
+typedef float float16v __attribute__((ext_vector_type(16)));
+
 __global__ __launch_bounds__(256) void stream_read_kernel(const float4v* __restrict__ p, long n16, float* sink) {
     float4v acc = {0.f, 0.f, 0.f, 0.f};
     const long stride = (long)gridDim.x * blockDim.x;
