@@ -328,11 +328,18 @@ def test_the_copies_of_a_call_never_take_more_than_is_asked_for_and_often_nothin
     use = lambda *c: lib.load().mi355_internal_gemm_copy_bytes(*args(*c))
     for c in ((8, 50257, 4096, "NN"), (64, 50257, 4096, "NN"), (62, 19578, 5867, "NT"), (16, 14337, 4096, "NN")):
         assert use(*c) == 0 and ask(*c) > 100 << 20, c       # read where they lie
-    # large products, and a long K whose ranges leave one CU of an XCD with twice the work of the others (3 ranges of 84 tiles: 33 workgroups)
-    for c in ((1999, 3001, 2503, "NN"), (2169, 2399, 1727, "NT"), (4097, 4097, 4097, "TN"), (751, 385, 8595, "NN"), (1029, 261, 6005, "NN"),
-              (561, 551, 5443, "NT"), (1287, 221, 5129, "NT"), (2439, 321, 3389, "NN")):
+    for c in ((1999, 3001, 2503, "NN"), (2169, 2399, 1727, "NT"), (4097, 4097, 4097, "TN")):
         assert use(*c) == ask(*c) > 0, c
     rng = random.Random(1)
     for _ in range(3000):
         c = tuple(int(lo * (hi / lo) ** rng.random()) for lo, hi in ((1, 8192), (16, 100000), (8, 16384))) + (rng.choice(("NN", "NT", "TN")),)
         assert use(*c) in (0, ask(*c)), c
+
+
+def test_the_direct_kernel_leaves_no_cu_of_an_xcd_with_twice_the_work_of_the_others(lib):
+    # an XCD's 32 CUs take an eighth of the tiles of every range, rounded up: 84 tiles in 3 ranges are 33 workgroups on most XCDs
+    for M, N, K, layout in ((751, 385, 8595, "NN"), (1029, 261, 6005, "NN"), (561, 551, 5443, "NT"), (1287, 221, 5129, "NT")):
+        variant = lib.load().mi355_internal_hgemm_direct_choice(M, N, K, lib.LAYOUTS[layout], None)
+        tile, ranges = {10: 64, 11: 128}[variant & 15], max(1, variant >> 4)
+        tiles = -(-M // tile) * -(-N // tile)
+        assert -(-tiles // 8) * ranges <= 32, (M, N, K, layout, tile, ranges)

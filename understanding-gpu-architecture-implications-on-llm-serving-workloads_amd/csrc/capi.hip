@@ -242,6 +242,12 @@ int mi355_internal_hgemm_wide_ranges(int M, int N, int K, int64_t ldb, int layou
     return k.shape == mi355::kSmallM && k.wide_ranges > 1 ? k.wide_ranges : 0;
 }
 
+int mi355_internal_hgemm_direct_choice(int M, int N, int K, int layout, float* us) {
+    const mi355::KernelChoice k = mi355::choose_direct(M, N, K, layout, true);
+    if (us != nullptr) *us = k.us;
+    return k.shape + (k.splits > 1 ? 16 * k.splits : 0);
+}
+
 int mi355_internal_fmha_decode_plan(int B, int Hq, int Hkv, int Sq, int kv_valid_len, int* splits, int* waves) {
     if (B < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv != 0 || Sq < 1 || kv_valid_len < 1 || !splits || !waves)
         return fail(MI355_ERR_BAD_ARGUMENT, "mi355_internal_fmha_decode_plan: bad argument");

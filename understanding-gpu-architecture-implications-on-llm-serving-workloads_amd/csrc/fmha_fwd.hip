@@ -585,7 +585,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     // 4 x 32/32 x 1001 74.9 / 73.1, 5 x 32/8 x 1328 160 / 152. The unrolled loop wants pair 0 in slot 0: an item that has steps for it
     // starts there, also where that means that its first pairs can only leave behind the last barrier of the item in front (a second copy
     // of the general step in front of the loop makes the 256-query instantiation spill 400 bytes a lane).
-    MI355_TL(unsigned long long tl_tiles = 0;)
+    MI355_TL(unsigned long long tl_tiles = 0, tl_end = 0, tl_between = 0;)   // cycles from an item's last barrier to the first of the next
     load_q(cur.Qh, q_wave0);
     if (cur.n_tiles > 0) issue_first_pairs();
     const bool more_items = (long)q_tiles * Hq * B * (SEG ? segments : 1) > gridDim.x;   // of the launch, than it has workgroups
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
             float4v s[4][QB];
             V8 pf[2][QB];
             V8 fr[AHEAD];
-            MI355_TL(if (round == 1) tl_w[1] = timeline::wall_clock(); const unsigned long long tl_c0 = timeline::shader_cycles();)
+            MI355_TL(if (round == 1) tl_w[1] = timeline::wall_clock(); const unsigned long long tl_c0 = timeline::shader_cycles(); if (tl_end) tl_between += tl_c0 - tl_end;)
             preload(I0{}, Dyn{}, ring & (NBUF - 1), fr);
             __builtin_amdgcn_s_setprio(1);
             mfma_phase(I0{}, I16{}, Dyn{}, ring & (NBUF - 1), s, pf, fr);               // S(0) alone
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
             wait_vmcnt<0>();
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) asm volatile("" : "+v"(qf[qb][0]), "+v"(qf[qb][1]), "+v"(qf[qb][2]), "+v"(qf[qb][3]));
-            MI355_TL(tl_w[2] = timeline::wall_clock(); tl_c[1] += timeline::shader_cycles() - tl_c0; tl_tiles += (unsigned long long)n_tiles;)
+            MI355_TL(tl_w[2] = timeline::wall_clock(); tl_end = timeline::shader_cycles(); tl_c[1] += tl_end - tl_c0; tl_tiles += (unsigned long long)n_tiles;)
         } else {
             wait_lgkmcnt<0>();
             phase_barrier();
@@ -771,7 +771,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
         if (tid == 0 && blockIdx.x < timeline::kMaxWorkgroups) {
             unsigned long long* rec = fmha_fwd_stamps + (long)blockIdx.x * timeline::kSlots;
             rec[0] = tl_w[0]; rec[1] = tl_w[1]; rec[2] = tl_w[2]; rec[3] = tl_w[3];
-            rec[4] = 0; rec[5] = tl_c[1]; rec[6] = tl_tiles; rec[7] = 0;
+            rec[4] = 0; rec[5] = tl_c[1]; rec[6] = tl_tiles; rec[7] = tl_between;
         })
 }
 

@@ -157,9 +157,9 @@ KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles
 // 32 CUs take an eighth of the tiles, of every range, rounded up: 84 tiles in 3 ranges are 252 workgroups, but 33 on most XCDs, and one CU
 // of each walks K for two of them (751 x 385 x 8595 NN 42.6 us, copies 32.3; counted over 256 CUs this was expected to take 25).
 // Fitted to 2027 timings of 190 products (1 .. 2600 rows, 64 .. 20000 columns, K 40 .. 9000, all layouts, both operands from HBM; rms 6.6 %). The
-// choice among these kernels and the aligned copies, copies_pay, takes .80 of the time of copies and of the gather that these kernels
-// replaced on average, and 4.6 % more than the fastest of them; slower than those: 3 x 17073 x 65 NN 7.2 us (gathered 5.9), 1 x 73 x 1439 NT 9.1
-// (8.2), 191 x 8893 x 1763 TN 29.6 (27.7), and with K up to 64 some by up to 8 % (441 x 6011 x 41 TN 7.4, 6.9).
+// choice among these kernels and the aligned copies, copies_pay, takes 1.4 % more than the fastest of them on average, and over 261 other drawn
+// products .80 of the time of copies and of the gather that these kernels replaced; slower than those: 269 x 2593 x 3487 NT 29.8 us (26.4),
+// 427 x 1393 x 7277 NT 41.3 (37.3), a K just over one tile against many columns (3 x 17073 x 65 NN 7.2, gathered 5.9), K up to 64 by up to 8 %.
 KernelChoice choose_direct(int M, int N, int K, int layout, bool split_ok) {
     static const int ranges[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int ktiles = (K + 63) / 64;

@@ -71,12 +71,16 @@ hipError_t split_k_workspace(size_t bytes, hipStream_t stream, char** out, std::
 }
 
 // Whether the copies of a plan are repaid: a launch, each copied operand read and written once, and the product on the kernels for
-// aligned rows, against the direct kernel, which reads the operands where they lie. us, copies / direct: 2169 x 2399 x 1727 NT
-// 34.5 / 47.7, 475 x 7131 x 4859 TN 64 / 77, 1999 x 3001 x 2503 NN 43 / 59; 99 x 9001 x 3021 NT 43 / 30, 8 x 6407 x 983 NN 19.2 / 10.5,
-// 1 x 591 x 391 NN 9.9 / 7.9, 62 x 19578 x 5867 NT 168 / 78.
+// aligned rows, against the direct kernel, which reads the operands where they lie. A product behind its copies, whose rows are no whole
+// lines, takes longer than choose_kernel expects, by up to half of a short one: the terms fitted to 185 products with copies, both operands from
+// HBM, rms 10 %. us, copies / direct: 2169 x 2399 x 1727 NT 34.5 / 47.7, 475 x 7131 x 4859 TN 64 / 77, 1999 x 3001 x 2503 NN 43 / 59, 751 x 385 x 8595
+// NN 32 / 43; 99 x 9001 x 3021 NT 43 / 30, 8 x 6407 x 983 NN 19.2 / 10.5, 683 x 615 x 2587 NN 23.2 / 16.0, 62 x 19578 x 5867 NT 168 / 78. What the choice
+// between them takes: choose_direct.
 static bool copies_pay(const GemmPackPlan& plan, int M, int N, int K, int layout) {
     const KernelChoice fast = choose_kernel(M, N, K, layout != MI355_GEMM_TN, layout == MI355_GEMM_NT, true, true, plan.b.ld % 64 == 0);
-    return fast.us + 5.3f + 2.f * (float)(plan.a.bytes + plan.b.bytes) / 5.96e6f < choose_direct(M, N, K, layout, true).us;
+    const float copied_mb = 2e-6f * (float)(plan.a.bytes + plan.b.bytes);
+    const float copies_us = 3.8f + fast.us + (fast.splits > 1 ? .47f : .755f) * fminf(fast.us, 12.f) + copied_mb / 7.67f;
+    return copies_us < choose_direct(M, N, K, layout, true).us;
 }
 
 size_t hgemm_copy_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb, int layout) {

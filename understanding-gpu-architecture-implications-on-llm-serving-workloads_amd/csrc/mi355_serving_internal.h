@@ -211,6 +211,8 @@ int mi355_internal_hgemm_silu_mul_variant(const void* A, const void* B, void* C,
 int mi355_internal_fmha_fwd_variant(const void* Q, const void* K, const void* V, void* O, float* LSE, int B, int Hq, int Hkv,
                                     int Sq, int Sk, int D, float scale, int causal, int kv_valid_len, const int64_t* strides,
                                     int dtype, int variant, void* stream);
+// the variant of the direct kernel that a product of unaligned operands takes if it is not copied, and the time it expects (us may be null)
+int mi355_internal_hgemm_direct_choice(int M, int N, int K, int layout, float* us);
 // bytes of workspace that mi355_gemm_ws uses for a call (0: it makes no copies): what the operators, the Python binding and the decoder layer
 // allocate, where mi355_gemm_workspace_bytes may ask for more
 size_t mi355_internal_gemm_copy_bytes(const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int layout);

@@ -21,7 +21,8 @@ EXPORTED_SYMBOLS = ("mi355_hgemm", "mi355_fmha_fwd", "mi355_fmha_fwd_strided", "
                     "mi355_fmha_fwd_workspace_bytes", "mi355_fmha_fwd_ws", "mi355_fmha_fwd_noalloc",
                     "mi355_last_error", "mi355_serving_version")
 # exported for tests and tuning runs, declared in csrc/mi355_serving_internal.h and not in the public header
-INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_add_variant", "mi355_internal_hgemm_choice", "mi355_internal_hgemm_wide_ranges", "mi355_internal_gemm_copy_bytes",
+INTERNAL_SYMBOLS = ("mi355_internal_hgemm_variant", "mi355_internal_hgemm_add_variant", "mi355_internal_hgemm_choice", "mi355_internal_hgemm_wide_ranges", "mi355_internal_hgemm_direct_choice",
+                    "mi355_internal_gemm_copy_bytes",
                     "mi355_internal_hgemm_silu_mul_variant", "mi355_internal_fmha_fwd_variant",
                     "mi355_internal_fmha_decode_plan", "mi355_internal_step_qkv", "mi355_internal_step_gate_up")
 
@@ -97,6 +98,8 @@ def load():
     lib.mi355_internal_hgemm_add_variant.restype = i32
     lib.mi355_internal_hgemm_choice.argtypes = [i32, i32, i32, i64, i32, ctypes.POINTER(f32)]
     lib.mi355_internal_hgemm_choice.restype = i32
+    lib.mi355_internal_hgemm_direct_choice.argtypes = [i32, i32, i32, i32, ctypes.POINTER(ctypes.c_float)]
+    lib.mi355_internal_hgemm_direct_choice.restype = i32
     lib.mi355_internal_hgemm_wide_ranges.argtypes = [i32, i32, i32, i64, i32]
     lib.mi355_internal_hgemm_wide_ranges.restype = i32
     lib.mi355_internal_hgemm_silu_mul_variant.argtypes = lib.mi355_internal_hgemm_variant.argtypes
