@@ -580,7 +580,7 @@ __global__ __launch_bounds__(512, 2) void fmha_fwd_pingpong_kernel(const T* __re
     // use of the current ones, so that the next item starts, when O has been normalised and stored (nothing waits for the stores), on
     // operands that are there. Requested together behind the last barrier, these 144 KiB and the 64 KiB of O took the CU, whose share of
     // memory's rate is ~56 GB/s from HBM, 17200 cycles from the last barrier of an item to the first of the next (4 x 32/32 x 1001, not
-    // causal; 128-query items of 13 x 64/8 x 353, causal, 8400); so they take 5700 (3200). us, before / now: 16 x 32/8 x 512 causal
+    // causal; 128-query items of 13 x 64/8 x 353, causal, 8400); so they take 5500 .. 6000 (3300 .. 3700). us, before / now: 16 x 32/8 x 512 causal
     // 86 / 76, 13 x 64/8 x 353 128-query items 102 / 83, 16 x 64/8 x 200 70 / 60, 8 x 32/8 x 1000 106 / 96, 1 x 32/8 x 4844 181 / 177, not causal
     // 4 x 32/32 x 1001 74.9 / 73.1, 5 x 32/8 x 1328 160 / 152. The unrolled loop wants pair 0 in slot 0: an item that has steps for it
     // starts there, also where that means that its first pairs can only leave behind the last barrier of the item in front (a second copy

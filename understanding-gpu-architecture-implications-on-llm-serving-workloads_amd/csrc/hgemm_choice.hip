@@ -153,7 +153,7 @@ KernelChoice choose_kernel(int M, int N, int K, bool a_kc, bool b_kc, bool tiles
 }
 
 // The direct kernel (hgemm_direct.hip) for a product: tiles and ranges of K. A K tile costs a CU .41 us on 64x64 tiles however many of
-// them share it (its LDS is busy: every operand byte is written once and read twice), .99 us on one 128x128 tile and 1.65 on two. An XCD's
+// them share it (its vector memory path is busy), .99 us on one 128x128 tile and 1.65 on two. An XCD's
 // 32 CUs take an eighth of the tiles, of every range, rounded up: 84 tiles in 3 ranges are 252 workgroups, but 33 on most XCDs, and one CU
 // of each walks K for two of them (751 x 385 x 8595 NN 42.6 us, copies 32.3; counted over 256 CUs this was expected to take 25).
 // Fitted to 2027 timings of 190 products (1 .. 2600 rows, 64 .. 20000 columns, K 40 .. 9000, all layouts, both operands from HBM; rms 6.6 %). The

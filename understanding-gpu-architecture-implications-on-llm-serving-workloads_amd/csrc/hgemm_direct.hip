@@ -8,8 +8,9 @@
 //   * no load has a condition: an offset past the last whole 16 bytes of the operand is moved back to it, and what that changes
 //     (only chunks of the last two K tiles that count) is put right on the way to LDS: elements moved down, zeros behind K;
 //   * fragments, products and the stores of C are those of the tiled kernels, four waves side by side over the tile. What bounds it is
-//     LDS: 32 (128x128 tiles: 64) KiB read and half as many written per K tile, .37 (.77) us of a CU for each tile. Rows 2 bytes off
-//     a multiple of 4 take 20 - 25 % longer than aligned ones.
+//     the CU's vector memory path, which takes 53 cycles for a load of 64 unaligned 16-byte pieces: it is busy 94 % of a CU's cycles on
+//     64x64 tiles (.41 us a K tile) and 73 .. 88 % on 128x128 (.83), LDS 29 and 25 %, the matrix pipes 14 and 24 % (1999 x 3001 x 2503 NN).
+//     Rows 2 bytes off a multiple of 4 take 20 - 25 % longer than aligned ones.
 // us per product, aligned copies in front of the tiled kernels / direct: 1 x 203 x 236 TN 8.1 / 5.3, 8 x 6407 x 983 NN 19.2 / 10.5, 397 x 965 x 313
 // NN 10.9 / 6.8, 99 x 9001 x 3021 NT 43 / 30, 62 x 19578 x 5867 NT 168 / 78; large ones stay with the copies (1999 x 3001 x 2503 NN 43 / 59).
 // Operands of fewer than 8 elements are read one element at a time.
